@@ -64,12 +64,12 @@ def variant_indices():
 
 def build_hip(force=False, jobs=None):
     headers = [os.path.join(CSRC, f) for f in ("gmm_kernel.hpp", "gmm_generic.hpp", "gmm_variants.hpp",
-                                               "gmm_variants.def")]
+                                               "gmm_variants.def", "row_kernels.hpp")]
     headers.append(os.path.join(ROOT, "include", "grouped_gemm_hip.h"))
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     obj_dir, hip_lib, extra = OBJ_DIR, HIP_LIB, []
     os.makedirs(obj_dir, exist_ok=True)
-    units = [(os.path.join(CSRC, "gmm_api.hip"), os.path.join(obj_dir, "gmm_api.o"), extra)]
+    units = [(os.path.join(CSRC, f + ".hip"), os.path.join(obj_dir, f + ".o"), extra) for f in ("gmm_api", "row_kernels")]
     for i in variant_indices():
         units.append((os.path.join(CSRC, "gmm_variant.hip"), os.path.join(obj_dir, f"gmm_variant_{i}.o"),
                       extra + [f"-DGG_VARIANT_INDEX={i}"]))

@@ -12,6 +12,7 @@
 
 #include "gmm_generic.hpp"
 #include "gmm_variants.hpp"
+#include "row_kernels.hpp"
 
 namespace gg {
 const GenericOps* generic_ops_0();
@@ -535,6 +536,17 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
   g.trans_a = 1, g.accumulate_f32 = 1;
   g.stream = stream;
   return gmm_impl(g);
+}
+
+int gg_swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t rows, int64_t cols, int dtype,
+                       void* stream) {
+  if (dtype != GG_DTYPE_BF16 && dtype != GG_DTYPE_F16) return fail(GG_EINVAL, "dtype must be GG_DTYPE_BF16 or GG_DTYPE_F16");
+  if (rows < 0 || cols < 0) return fail(GG_EINVAL, "negative dimension");
+  if (rows >= (int64_t(1) << 31) || cols >= (1 << 22)) return fail(GG_ELIMIT, "rows must be below 2^31, cols below 2^22");
+  if (rows == 0 || cols == 0) return GG_OK;
+  if (gate_up == nullptr || grad == nullptr || out == nullptr) return fail(GG_EINVAL, "gate_up, grad or out is null");
+  GG_HIP(gg::swiglu_backward(gate_up, grad, out, rows, cols, dtype, static_cast<hipStream_t>(stream)));
+  return GG_OK;
 }
 
 int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device, int64_t num_groups,

@@ -243,6 +243,27 @@ void GroupedGemmSwiGLU(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch:
   Run(a, b, c, batch_sizes, /*trans_a=*/false, trans_b, /*accumulate_f32=*/false, /*flags=*/0, rows, /*gate_up=*/true);
 }
 
+// Gradients of gate | up (rows, 2 * cols) from the gradient of silu(gate) * up (rows, cols); see
+// gg_swiglu_backward.
+torch::Tensor SwiGLUBackward(torch::Tensor gate_up, torch::Tensor grad) {
+  TORCH_CHECK(gate_up.is_cuda() && grad.is_cuda() && gate_up.device() == grad.device(),
+              "grouped_gemm: gate_up and grad must be on the same GPU");
+  TORCH_CHECK(gate_up.scalar_type() == torch::kBFloat16 || gate_up.scalar_type() == torch::kFloat16,
+              "grouped_gemm: gate_up must be bfloat16 or float16");
+  TORCH_CHECK(grad.scalar_type() == gate_up.scalar_type(), "grouped_gemm: grad must have the element type of gate_up");
+  TORCH_CHECK(gate_up.dim() == 2 && grad.dim() == 2 && gate_up.size(0) == grad.size(0) &&
+                  gate_up.size(1) == 2 * grad.size(1),
+              "grouped_gemm: gate_up must be (rows, 2 * cols) and grad (rows, cols)");
+  TORCH_CHECK(gate_up.is_contiguous() && grad.is_contiguous(), "grouped_gemm: gate_up and grad must be contiguous");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(gate_up.device());
+  torch::Tensor out = torch::empty_like(gate_up);
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(gate_up.device().index()).stream();
+  const int rc = gg_swiglu_backward(gate_up.data_ptr(), grad.data_ptr(), out.data_ptr(), grad.size(0), grad.size(1),
+                                    DtypeCode(gate_up.scalar_type()), static_cast<void*>(stream));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+  return out;
+}
+
 // c (num_experts, hidden_in, hidden_out) fp32 += per expert a_e^T @ b_e; see gg_gmm_bf16_acc_f32.
 void AccumulateWeightGradient(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes) {
   TORCH_CHECK(c.scalar_type() == torch::kFloat32, "grouped_gemm: the accumulated gradient must be float32");
@@ -301,6 +322,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gmm_swiglu", &GroupedGemmSwiGLU, "silu(a @ gate) * (a @ up) with b = [gate | up].", py::arg("a"),
         py::arg("b"), py::arg("c"), py::arg("batch_sizes"), py::arg("trans_b"), py::arg("a_rows") = py::none(),
         py::arg("c_rows") = py::none());
+  m.def("swiglu_backward", &SwiGLUBackward, "Gradients of gate | up from the gradient of silu(gate) * up.");
   m.def("size_status", &SizeStatus,
         "Bits collected since the last call: 1 a device-resident batch size was negative, 2 they summed past the "
         "rows of a (both clamped by the kernel).");

@@ -121,8 +121,8 @@ def gmm_scatter(a, w, batch_sizes, row_index, trans_b=False):
 class GroupedGemmSwiGLU(torch.autograd.Function):
     """silu(a @ gate) * (a @ up) with w = [gate | up] per expert, the activation fused into the
     GEMM's epilogue.  The backward recomputes the two products with a plain grouped GEMM (they are
-    not stored by the forward), applies the derivative elementwise and runs the two usual
-    gradient GEMMs on the result."""
+    not stored by the forward), applies the derivative in one elementwise kernel and runs the two
+    usual gradient GEMMs on the result."""
 
     @staticmethod
     def forward(ctx, a, w, batch_sizes, trans_b):
@@ -134,13 +134,15 @@ class GroupedGemmSwiGLU(torch.autograd.Function):
     def backward(ctx, grad):
         grad = grad.contiguous()
         a, w, batch_sizes = ctx.saved_tensors
-        gate_up = backend.gmm(a, w, batch_sizes, trans_b=ctx.trans_b).float()
-        gate, up = gate_up.chunk(2, dim=-1)
-        sig = torch.sigmoid(gate)
-        g32 = grad.float()
-        dgate = g32 * up * sig * (1.0 + gate * (1.0 - sig))
-        dup = g32 * gate * sig
-        dgu = torch.cat([dgate, dup], dim=-1).to(a.dtype)
+        gate_up = backend.gmm(a, w, batch_sizes, trans_b=ctx.trans_b)
+        if a.dtype == gate_up.dtype:
+            dgu = backend.backend.swiglu_backward(gate_up, grad)
+        else:   # float8 operands: rounded once, from fp32 to their type
+            gate, up = gate_up.float().chunk(2, dim=-1)
+            sig = torch.sigmoid(gate)
+            g32 = grad.float()
+            dgate = g32 * up * sig * (1.0 + gate * (1.0 - sig))
+            dgu = torch.cat([dgate, g32 * gate * sig], dim=-1).to(a.dtype)
         agrad = wgrad = None
         if ctx.needs_input_grad[0]:
             agrad = backend.gmm(dgu, w, batch_sizes, trans_b=not ctx.trans_b)

@@ -248,6 +248,16 @@ uint64_t gg_workspace_bytes_for(const gg_gmm_args* args);
 int gg_gmm_no_alloc(const gg_gmm_args* args);
 
 /*
+ * Backward of the SwiGLU epilogue between its grouped GEMMs: from gate_up (rows, 2 * cols), the
+ * products a @ gate | a @ up side by side, and grad (rows, cols), the gradient of silu(gate) * up,
+ * the gradients of both products side by side into out (rows, 2 * cols).  Computed in fp32,
+ * rounded once.  All three contiguous, of element type dtype (GG_DTYPE_BF16 or GG_DTYPE_F16).
+ * No counterpart in the reference, which has no epilogue (csrc/grouped_gemm.cu:255).
+ */
+int gg_swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t rows, int64_t cols,
+                       int dtype, void* stream);
+
+/*
  * Runs only the on-device scheduler of gg_gmm_bf16 (same device code, same
  * arguments) and writes what it derived to `table_out`, a device buffer of
  * num_groups * GG_SCHED_COLS int64: per group the problem (m, n, k), leading

@@ -1620,6 +1620,34 @@ def test_swiglu_autograd(ops, oracle, trans_b):
     assert (w.grad[1] == 0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (5, 3, 0), (257, 2, 0), (33, 100, 0), (300, 257, 0), (64, 264, 0),
+                                             (7, 2048, 0), (40, 64, 1), (40, 64, 2), (2100, 2048, 0), (0, 8, 0)])
+def test_swiglu_backward_kernel(ops, dtype, rows, cols, shift):
+    # the derivative of silu(gate) * up against float64: one rounding of the result (half a unit
+    # in the last of p significant bits is at most 2^-p of it: p = 8 in bfloat16, 11 in float16, and
+    # subnormal float16 results come in steps of 2^-24), and fp32 arithmetic
+    # before it, whose error is bounded by a few 2^-22 of the terms that may cancel.  Every access
+    # width (from the column count and from operands `shift` elements off a 16-byte boundary), more
+    # items than one pass of the grid takes, and no rows.
+    _announce("swiglu backward", dtype, rows, cols, shift)
+    g = torch.Generator().manual_seed(rows + cols)
+    def operand(*shape):
+        flat = torch.empty(shape[0] * shape[1] + shift, dtype=dtype, device="cuda")
+        t = flat[shift:].view(*shape)
+        t.copy_(torch.randn(*shape, generator=g) * 3)
+        return t
+    gate_up, grad = operand(rows, 2 * cols), operand(rows, cols)
+    out = ops.backend.backend.swiglu_backward(gate_up, grad)
+    gate, up = gate_up.double().chunk(2, dim=-1)
+    sig, d = torch.sigmoid(gate), grad.double()
+    want = torch.cat([d * up * sig * (1 + gate * (1 - sig)), d * gate * sig], dim=-1)
+    terms = torch.cat([(d * up).abs() * (1 + gate.abs()), (d * gate).abs()], dim=-1)
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    tol = half_ulp * want.abs() + 2.0 ** -20 * terms + (2.0 ** -24 if dtype == torch.float16 else 0.0)
+    assert bool(((out.double() - want).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("config", [2, 5])
 def test_fused_rows_and_swiglu_at_benchmark_shapes(ops, oracle, config):
     # the gather-fused load, the scatter-fused store and the SwiGLU epilogue at the row counts and
