@@ -549,6 +549,23 @@ int gg_swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t
   return GG_OK;
 }
 
+uint64_t gg_sum_rows_scratch_bytes(int64_t rows, int64_t num_dst) {
+  return rows < 0 || num_dst < 0 ? 0 : gg::sum_rows_scratch_bytes(rows, num_dst);
+}
+
+int gg_sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t rows, int64_t num_dst, int64_t cols,
+                int dtype, void* scratch, void* stream) {
+  if (dtype != GG_DTYPE_BF16 && dtype != GG_DTYPE_F16) return fail(GG_EINVAL, "dtype must be GG_DTYPE_BF16 or GG_DTYPE_F16");
+  if (rows < 0 || num_dst < 0 || cols < 0) return fail(GG_EINVAL, "negative dimension");
+  if (rows >= (int64_t(1) << 31) || num_dst >= (int64_t(1) << 31) || cols >= (1 << 22))
+    return fail(GG_ELIMIT, "rows must be below 2^31, cols below 2^22");
+  if (num_dst == 0 || cols == 0) return GG_OK;
+  if (dst == nullptr || scratch == nullptr || (rows > 0 && (src == nullptr || row_index == nullptr)))
+    return fail(GG_EINVAL, "src, row_index, dst or scratch is null");
+  GG_HIP(gg::sum_rows(src, row_index, dst, rows, num_dst, cols, dtype, scratch, static_cast<hipStream_t>(stream)));
+  return GG_OK;
+}
+
 int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device, int64_t num_groups,
                       int64_t tokens, int64_t hidden_in, int64_t hidden_out, int trans_a,
                       int trans_b, int64_t* table_out, void* stream_) {

@@ -11,4 +11,10 @@ namespace gg {
 hipError_t swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t rows, int64_t cols, int dt,
                            hipStream_t stream);
 
+// dst[d] = sum of the rows r of src with row_index[r] == d, in fp32, rounded once (zeros where there
+// are none); `scratch` holds sum_rows_scratch_bytes, 4-byte aligned, any contents.
+uint64_t sum_rows_scratch_bytes(int64_t rows, int64_t destinations);
+hipError_t sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t rows, int64_t destinations,
+                    int64_t cols, int dt, void* scratch, hipStream_t stream);
+
 }  // namespace gg

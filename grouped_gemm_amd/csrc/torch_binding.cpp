@@ -264,6 +264,26 @@ torch::Tensor SwiGLUBackward(torch::Tensor gate_up, torch::Tensor grad) {
   return out;
 }
 
+// out (num_dst, cols): row d is the sum of the rows of src that row_index sends there; see gg_sum_rows.
+torch::Tensor SumRows(torch::Tensor src, torch::Tensor row_index, int64_t num_dst) {
+  TORCH_CHECK(src.is_cuda() && src.dim() == 2 && src.is_contiguous(), "grouped_gemm: src must be a contiguous 2-d GPU tensor");
+  TORCH_CHECK(src.scalar_type() == torch::kBFloat16 || src.scalar_type() == torch::kFloat16,
+              "grouped_gemm: src must be bfloat16 or float16");
+  TORCH_CHECK(row_index.dim() == 1 && row_index.scalar_type() == torch::kInt32 && row_index.is_contiguous() &&
+                  row_index.device() == src.device() && row_index.size(0) == src.size(0),
+              "grouped_gemm: row_index must be a contiguous int32 tensor with one entry per row, on src's GPU");
+  TORCH_CHECK(num_dst >= 0, "grouped_gemm: negative row count");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(src.device());
+  torch::Tensor out = torch::empty({num_dst, src.size(1)}, src.options());
+  torch::Tensor scratch = torch::empty({(int64_t)gg_sum_rows_scratch_bytes(src.size(0), num_dst)},
+                                       src.options().dtype(torch::kUInt8));
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(src.device().index()).stream();
+  const int rc = gg_sum_rows(src.data_ptr(), row_index.data_ptr<int32_t>(), out.data_ptr(), src.size(0), num_dst,
+                             src.size(1), DtypeCode(src.scalar_type()), scratch.data_ptr(), static_cast<void*>(stream));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+  return out;
+}
+
 // c (num_experts, hidden_in, hidden_out) fp32 += per expert a_e^T @ b_e; see gg_gmm_bf16_acc_f32.
 void AccumulateWeightGradient(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes) {
   TORCH_CHECK(c.scalar_type() == torch::kFloat32, "grouped_gemm: the accumulated gradient must be float32");
@@ -323,6 +343,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("b"), py::arg("c"), py::arg("batch_sizes"), py::arg("trans_b"), py::arg("a_rows") = py::none(),
         py::arg("c_rows") = py::none());
   m.def("swiglu_backward", &SwiGLUBackward, "Gradients of gate | up from the gradient of silu(gate) * up.");
+  m.def("sum_rows", &SumRows, "Row d of the result is the sum of the rows of src that row_index sends there.");
   m.def("size_status", &SizeStatus,
         "Bits collected since the last call: 1 a device-resident batch size was negative, 2 they summed past the "
         "rows of a (both clamped by the kernel).");

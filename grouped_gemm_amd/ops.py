@@ -65,14 +65,17 @@ class GroupedGemmGather(torch.autograd.Function):
             # rows of x that several sorted rows came from collect several gradients: a sum, not
             # a store, so it is not fused
             sorted_grad = backend.gmm(grad, w, batch_sizes, trans_b=not ctx.trans_b)
-            xgrad = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
-            xgrad.index_add_(0, row_index.long(), sorted_grad.float())
-            xgrad = xgrad.to(x.dtype)
+            if sorted_grad.dtype == x.dtype:
+                xgrad = backend.backend.sum_rows(sorted_grad, row_index, x.shape[0])
+            else:   # float8 operands: rounded once, from fp32 to their type
+                xgrad = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
+                xgrad.index_add_(0, row_index, sorted_grad.float())
+                xgrad = xgrad.to(x.dtype)
         if ctx.needs_input_grad[1]:
             # The weight-gradient layout takes row indices on the general kernels only, which are
             # several times slower than the streaming ones: one explicit gather and the streaming
             # kernel is the faster way to the same result.
-            sorted_x = x.index_select(0, row_index.long())
+            sorted_x = x.index_select(0, row_index)
             lhs, rhs = (grad, sorted_x) if ctx.trans_b else (sorted_x, grad)
             wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
         return xgrad, wgrad, None, None, None
@@ -99,7 +102,7 @@ class GroupedGemmScatter(torch.autograd.Function):
             agrad = backend.gmm_indexed(grad, w, batch_sizes, trans_b=not ctx.trans_b, a_rows=row_index)
         if ctx.needs_input_grad[1]:
             # (as in GroupedGemmGather: an explicit gather, then the streaming weight-gradient kernel)
-            sorted_grad = grad.index_select(0, row_index.long())
+            sorted_grad = grad.index_select(0, row_index)
             lhs, rhs = (sorted_grad, a) if ctx.trans_b else (a, sorted_grad)
             wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
         return agrad, wgrad, None, None, None

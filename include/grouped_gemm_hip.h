@@ -258,6 +258,20 @@ int gg_swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t
                        int dtype, void* stream);
 
 /*
+ * The gradient of a row gather: dst[d] = the sum of the rows r of src (rows, cols) with
+ * row_index[r] == d, accumulated in fp32 and rounded once; zeros for a row of dst (num_dst, cols)
+ * that no index names.  Indices that name no row of dst are ignored.  src and dst contiguous, of
+ * element type dtype (GG_DTYPE_BF16 or GG_DTYPE_F16); row_index int32[rows] on the device.
+ * Sums of up to 8 rows are added in ascending row order, the same bits on every call; rows past
+ * that are added in the order the device meets them.  `scratch`: device memory of
+ * gg_sum_rows_scratch_bytes(rows, num_dst) bytes, 4-byte aligned, of any contents.
+ * No counterpart in the reference, which takes rows already sorted (grouped_gemm/ops.py:8).
+ */
+uint64_t gg_sum_rows_scratch_bytes(int64_t rows, int64_t num_dst);
+int gg_sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t rows, int64_t num_dst,
+                int64_t cols, int dtype, void* scratch, void* stream);
+
+/*
  * Runs only the on-device scheduler of gg_gmm_bf16 (same device code, same
  * arguments) and writes what it derived to `table_out`, a device buffer of
  * num_groups * GG_SCHED_COLS int64: per group the problem (m, n, k), leading

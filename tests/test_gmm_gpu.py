@@ -1491,6 +1491,34 @@ def test_fused_permutation_autograd(ops, oracle, trans_b):
     check_scaled(x.grad, xg_ref, "x gradient")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,destinations,cols", [(1, 1, 1), (600, 100, 3), (600, 300, 2), (40, 5, 100), (300, 1, 257),
+                                                    (64, 200, 264), (0, 3, 8), (5000, 2000, 2048)])
+def test_sum_rows_kernel(ops, dtype, rows, destinations, cols):
+    # the gradient of a row gather against float64: every access width, destinations that no row
+    # names (zeros), that up to 8 rows name (the inline slots) and that more name (the lists: 8 rows
+    # a destination on average and 300 for one), indices that name no destination, no rows.  fp32
+    # additions of n terms err by at most n 2^-24 of the terms' magnitudes, one rounding of the
+    # result by 2^-8 (bfloat16) or 2^-11 (float16) of it (2^-25 for subnormal float16 results).
+    _announce("sum rows", dtype, rows, destinations, cols)
+    g = torch.Generator().manual_seed(rows + cols)
+    src = torch.randn(rows, cols, generator=g).to(dtype).cuda()
+    index = torch.randint(0, destinations, (rows,), generator=g, dtype=torch.int32)
+    if rows > 10:
+        index[3], index[7] = -1, destinations
+    out = ops.backend.backend.sum_rows(src, index.cuda(), destinations)
+    ok = (index >= 0) & (index < destinations)
+    want = torch.zeros(destinations, cols, dtype=torch.float64)
+    size = torch.zeros(destinations, cols, dtype=torch.float64)
+    want.index_add_(0, index[ok].long(), src.double().cpu()[ok])
+    size.index_add_(0, index[ok].long(), src.double().cpu()[ok].abs())
+    most = int(torch.bincount(index[ok].long(), minlength=destinations).max()) if rows else 0
+    tol = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * want.abs() + most * 2.0 ** -24 * size + 2.0 ** -25
+    assert bool(((out.double().cpu() - want).abs() <= tol).all())
+    if 0 < most <= 8:
+        assert torch.equal(out, ops.backend.backend.sum_rows(src, index.cuda(), destinations))
+
+
 # ------------------------------------------------------------------ SwiGLU epilogue
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
