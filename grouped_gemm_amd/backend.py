@@ -106,6 +106,9 @@ def _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
 
 
 def gmm(a, b, batch_sizes, trans_a=False, trans_b=False, c=None):
+    out = backend.gmm_direct(a, b, batch_sizes, trans_a, trans_b, c)
+    if out is not None:
+        return out
     if c is None:
         c = _allocate_output(a, b, batch_sizes, trans_a, trans_b)
     if _padded_call(a, b, c, batch_sizes, trans_a, trans_b):

@@ -213,6 +213,83 @@ void GroupedGemm(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tenso
   Run(a, b, c, batch_sizes, trans_a, trans_b, /*accumulate_f32=*/false, /*flags=*/0);
 }
 
+// Whether a call runs on the streaming kernels as it is: well-formed contiguous operands whose sizes
+// and addresses need no padded copies (the rule of _padded_call in backend.py).  Everything else is
+// left to the Python side, whose checks and error messages then apply.
+bool IsDirect(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& batch_sizes, bool trans_a,
+              bool trans_b, const torch::Tensor* c) {
+  if ((trans_a && trans_b) || batch_sizes.dim() != 1 || a.dim() != 2 || b.dim() != (trans_a ? 2 : 3)) return false;
+  if (!a.is_cuda() || !b.is_cuda() || a.scalar_type() != b.scalar_type()) return false;
+  const torch::ScalarType t = a.scalar_type();
+  if (t != torch::kBFloat16 && t != torch::kFloat16 && !IsFloat8(t)) return false;
+  if (!a.is_contiguous() || !b.is_contiguous() || (c != nullptr && !c->is_contiguous())) return false;
+  const int64_t hin = a.size(1), hout = trans_a || trans_b ? b.size(1) : b.size(2);
+  if (a.size(0) == 0 || hin == 0 || hout == 0) return false;
+  const uintptr_t addresses = reinterpret_cast<uintptr_t>(a.data_ptr()) | reinterpret_cast<uintptr_t>(b.data_ptr()) |
+                              (c != nullptr ? reinterpret_cast<uintptr_t>(c->data_ptr()) : 0);
+  const int64_t mult = IsFloat8(t) ? 16 : 8;
+  if (hin % mult == 0 && hout % mult == 0 && (addresses & 15) == 0) return true;
+  return !IsFloat8(t) && hin % 2 == 0 && hout % 2 == 0 && (addresses & 3) == 0;
+}
+
+torch::Tensor AllocateOutput(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& batch_sizes,
+                             bool trans_a, bool trans_b) {
+  const auto options = a.options().dtype(OutputType(a.scalar_type()));
+  if (trans_a) return torch::empty({batch_sizes.size(0), a.size(1), b.size(1)}, options);
+  return torch::empty({a.size(0), trans_b ? b.size(1) : b.size(2)}, options);
+}
+
+// backend.gmm in one step for direct calls; nothing is returned (and nothing done) for others.
+c10::optional<torch::Tensor> GroupedGemmDirect(const torch::Tensor& a, const torch::Tensor& b,
+                                               const torch::Tensor& batch_sizes, bool trans_a, bool trans_b,
+                                               const c10::optional<torch::Tensor>& c) {
+  if (!IsDirect(a, b, batch_sizes, trans_a, trans_b, c.has_value() ? &*c : nullptr)) return c10::nullopt;
+  torch::Tensor out = c.has_value() ? *c : AllocateOutput(a, b, batch_sizes, trans_a, trans_b);
+  GroupedGemm(a, b, out, batch_sizes, trans_a, trans_b);
+  return out;
+}
+
+// ops.GroupedGemm (the reference's grouped_gemm/ops.py:8-29) as a native autograd node: a training
+// step of a small layer is bound by what the host does between the three launches, and the
+// interpreter was most of it.
+class GroupedGemmNode : public torch::autograd::Function<GroupedGemmNode> {
+ public:
+  static torch::Tensor forward(torch::autograd::AutogradContext* ctx, const torch::Tensor& a, const torch::Tensor& b,
+                               const torch::Tensor& batch_sizes, bool trans_b) {
+    ctx->save_for_backward({a, b, batch_sizes});
+    ctx->saved_data["trans_b"] = trans_b;
+    torch::Tensor out = AllocateOutput(a, b, batch_sizes, false, trans_b);
+    GroupedGemm(a, b, out, batch_sizes, false, trans_b);
+    return out;
+  }
+
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    torch::Tensor grad = grads[0].contiguous();
+    if (reinterpret_cast<uintptr_t>(grad.data_ptr()) & 15) grad = grad.clone();
+    const auto saved = ctx->get_saved_variables();
+    const torch::Tensor &a = saved[0], &b = saved[1], &batch_sizes = saved[2];
+    const bool trans_b = ctx->saved_data["trans_b"].toBool();
+    torch::Tensor agrad, bgrad;
+    if (ctx->needs_input_grad(0)) {
+      agrad = AllocateOutput(grad, b, batch_sizes, false, !trans_b);
+      GroupedGemm(grad, b, agrad, batch_sizes, false, !trans_b);
+    }
+    if (ctx->needs_input_grad(1)) {
+      const torch::Tensor &lhs = trans_b ? grad : a, &rhs = trans_b ? a : grad;
+      bgrad = AllocateOutput(lhs, rhs, batch_sizes, true, false);
+      GroupedGemm(lhs, rhs, bgrad, batch_sizes, true, false);
+    }
+    return {agrad, bgrad, torch::Tensor(), torch::Tensor()};
+  }
+};
+
+c10::optional<torch::Tensor> GroupedGemmAutograd(const torch::Tensor& a, const torch::Tensor& b,
+                                                 const torch::Tensor& batch_sizes, bool trans_b) {
+  if (!IsDirect(a, b, batch_sizes, false, trans_b, nullptr)) return c10::nullopt;
+  return GroupedGemmNode::apply(a, b, batch_sizes, trans_b);
+}
+
 // gmm with GG_FLAG_* bits, for tests that compare the ways a call can be scheduled.
 void GroupedGemmWithFlags(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes,
                           bool trans_a, bool trans_b, int64_t flags) {
@@ -332,6 +409,9 @@ torch::Tensor DebugSchedule(torch::Tensor batch_sizes, int64_t tokens, int64_t h
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gmm", &GroupedGemm, "Grouped GEMM.");
+  m.def("gmm_direct", &GroupedGemmDirect,
+        "gmm with the output allocated where c is None, for calls the streaming kernels take as they are; None for others.");
+  m.def("gmm_autograd", &GroupedGemmAutograd, "The differentiable form of gmm_direct without trans_a.");
   m.def("validate",
         [](torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes, bool trans_a,
            bool trans_b) { Validate(a, b, c, batch_sizes, trans_a, trans_b, /*on_device=*/false); },

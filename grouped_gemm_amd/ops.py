@@ -36,7 +36,9 @@ class GroupedGemm(torch.autograd.Function):
 
 
 def gmm(a, b, batch_sizes, trans_b=False):
-    return GroupedGemm.apply(a, b, batch_sizes, trans_b)
+    # (the same node in native code; None: a call that backend.gmm has to prepare or reject)
+    out = backend.backend.gmm_autograd(a, b, batch_sizes, trans_b)
+    return GroupedGemm.apply(a, b, batch_sizes, trans_b) if out is None else out
 
 
 # --------------------------------------------------- fused permutation (gather / scatter)

@@ -1966,6 +1966,30 @@ def test_needs_input_grad_is_respected(ops):
     assert a.grad is not None and b.grad is None
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("upstream", ["plain", "expanded", "off the 16-byte boundary"])
+def test_native_autograd_node_against_the_python_one(ops, trans_b, upstream):
+    # ops.gmm runs as a native node where no operand needs preparing, ops.GroupedGemm is the same
+    # node in Python: the same bits, also for gradients that arrive expanded or misaligned and where
+    # only one input wants a gradient
+    g = torch.Generator().manual_seed(17)
+    sizes = torch.tensor([40, 0, 88], dtype=torch.int64).cuda()
+    a0 = torch.randn(128, 136, generator=g).to(torch.bfloat16).cuda()
+    b0 = torch.randn(3, *((72, 136) if trans_b else (136, 72)), generator=g).to(torch.bfloat16).cuda()
+    grad = torch.randn(1 + 128 * 72, generator=g).to(torch.bfloat16).cuda()[1:].view(128, 72)
+    grad = {"plain": grad.clone(), "expanded": grad[:1, :1].expand(128, 72)}.get(upstream, grad)
+    for wants in ((True, True), (True, False), (False, True)):
+        got = []
+        for fn in (ops.gmm, ops.GroupedGemm.apply):
+            a, b = a0.clone().requires_grad_(wants[0]), b0.clone().requires_grad_(wants[1])
+            out = fn(a, b, sizes, trans_b)
+            out.backward(grad)
+            got.append((out.detach(), a.grad, b.grad))
+        for x, y in zip(*got):
+            assert (x is None and y is None) or torch.equal(x, y)
+        assert (got[0][1] is not None, got[0][2] is not None) == wants
+
+
 def test_runs_on_the_current_stream(ops, oracle):
     g = torch.Generator().manual_seed(11)
     sizes = torch.tensor([500, 12])
