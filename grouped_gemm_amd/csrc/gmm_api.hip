@@ -27,7 +27,10 @@ const GenericOps* generic_ops_3();
 namespace {
 
 using gg::Short;
+using gg::Small;
+using gg::SmallSquare;
 using gg::Wide;
+using gg::WideRaggedDepth;
 
 thread_local char g_err[512] = "";
 
@@ -264,6 +267,72 @@ IndexedRows indexed_rows(const gg_gmm_args& g) {
   return r;
 }
 
+struct TileShape {
+  int id, bm, bn;
+};
+template <typename S>
+constexpr TileShape shape_of() {
+  return TileShape{S::kId, S::BM, S::BN};
+}
+
+// Tiles of a call in a shape: those of groups of average size, which is what device-resident sizes
+// can be judged by.
+int64_t average_tiles(const gg_gmm_args& g, int bm, int bn) {
+  const int64_t tiles_n = (g.hidden_out + bn - 1) / bn;
+  if (g.trans_a) return g.num_groups * ((g.hidden_in + bm - 1) / bm) * tiles_n;
+  const int64_t rows = (g.tokens + g.num_groups - 1) / g.num_groups;
+  return g.num_groups * ((rows + bm - 1) / bm) * tiles_n;
+}
+
+// Workgroups of a full launch of one workgroup per compute unit, for the rules below.
+constexpr int kFullLaunch = 256;
+
+// Whether the streaming kernel exists in a shape: the short and the small ones for two-byte elements
+// and, with b stored transposed and the plain epilogue, fp8.
+bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
+  const bool plain = g.epilogue == GG_EPILOGUE_NONE && !r.indexed;
+  if (g.trans_a) return id == Wide::kId || (id == SmallSquare::kId && r.elem_bytes == 2);
+  return id == Wide::kId || ((id == Short::kId || id == Small::kId) && (r.elem_bytes == 2 || (g.trans_b && plain)));
+}
+
+// The tile shape of a streaming call.
+//
+// Small tiles where one round of them (two workgroups per compute unit; one for weight gradients)
+// holds the whole launch: the launch is then bound by how long one tile takes, and by how many
+// compute units pull data.  Us per launch, bf16, wide / short / small, NN layout: 8 groups x 128
+// rows, 128 -> 128: 9.6 / 8.5 / 7.4; 16 x 256, 1024 -> 1024 (512 small tiles): 20.1 / 18.5 / 17.9;
+// 20 x 168, 5592 -> 232: 60 / 53 / 29.5; past that line the small ones lose: 8 x 1024,
+// 128 -> 1024 (1024 small tiles) 12.0 / 11.1 / 11.8, 8 x 2048, 1024 -> 1024: 35.6 / 37.9 / 49.5.
+// Weight gradients, wide / small: 8 x 512, 256 x 256: 18.2 / 10.8; 8 x 1024, 128 x 1024 (64 tiles):
+// 26.5 / 17.8; 16 x 256, 1024 x 1024 (1024 tiles): 18.0 / 20.8.
+// Groups of kDeepGroups rows and more keep the wide ones: where a few of them are much deeper than
+// the rest, those are cut along the depth (plan_deep_tiles).
+// Short tiles where groups average few rows (use_short_shape), where one round of them holds the
+// launch (8 x 1024, 128 -> 1024, 256 of them, above), and where few rows of deep products leave
+// nothing to do but pull weights, for which their larger buffers are better (8 x 16, 14336 -> 4096,
+// 128 short tiles in two depth pieces each: 152 us, 256 small ones: 172 us).
+constexpr int64_t kDeepGroups = 2560;
+constexpr int64_t kDeepProduct = 6144;
+
+TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
+  if (r.ragged_depth) return shape_of<WideRaggedDepth>();
+  const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
+  if (g.trans_a) {
+    const bool small = has_shape(g, r, SmallSquare::kId) && g.tokens < kDeepGroups * g.num_groups &&
+                       average_tiles(g, SmallSquare::BM, SmallSquare::BN) <= kFullLaunch;
+    return small ? shape_of<SmallSquare>() : shape_of<Wide>();
+  }
+  const int64_t short_tiles = average_tiles(g, Short::BM, Short::BN / halves);
+  const bool streams_weights = g.tokens <= Small::BM * g.num_groups && g.hidden_in >= kDeepProduct && 2 * short_tiles >= kFullLaunch;
+  if (has_shape(g, r, Small::kId) && !streams_weights &&
+      average_tiles(g, Small::BM, Small::BN / halves) <= 2 * kFullLaunch)
+    return shape_of<Small>();
+  if (has_shape(g, r, Short::kId) && (use_short_shape(g.num_groups, g.tokens, 0) ||
+                                      short_tiles <= kFullLaunch))
+    return shape_of<Short>();
+  return shape_of<Wide>();
+}
+
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
 int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
@@ -321,19 +390,18 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
   hipStream_t stream = static_cast<hipStream_t>(g.stream);
   const int layout = trans_a ? gg::kTN : (trans_b ? gg::kNT : gg::kNN);
   const int epilogue = out_f32 ? gg::kEpiAccF32 : (swiglu ? gg::kEpiSwiGLU : gg::kEpiStore);
+  const TileShape shape = generic ? TileShape{-1, gg::kGenericTileM, gg::kGenericTileN} : pick_shape(g, route);
   // deep groups: the launch is bound by the matrix pipe, and atomic additions to c cost less of
   // its time than reading, adding and writing; shallow groups: bound by the traffic of c, the reverse
-  const int variant_epilogue = out_f32 && tokens >= (int64_t)kShallowBelow * num_groups ? gg::kEpiAccF32Atomic : epilogue;
-  // (the short tile shape exists for two-byte elements, the plain epilogue and rows in place only)
-  const bool short_shape = !generic && !swiglu && !indexed && elem_bytes == 2 && !route.ragged_depth &&
-                           use_short_shape(num_groups, tokens, trans_a);
-  const int bm = generic ? gg::kGenericTileM : (short_shape ? Short::BM : Wide::BM);
+  // (small tiles: launches too short for the difference, read-add-write only)
+  const int variant_epilogue = out_f32 && shape.id == Wide::kId && tokens >= (int64_t)kShallowBelow * num_groups
+                                   ? gg::kEpiAccF32Atomic : epilogue;
+  const int bm = shape.bm;
   // output columns per tile: half the tile's width when it holds gate and up columns
-  const int bn = (generic ? gg::kGenericTileN : (short_shape ? Short::BN : Wide::BN)) / (swiglu ? 2 : 1);
+  const int bn = shape.bn / (swiglu ? 2 : 1);
   const gg::VariantOps* variant = nullptr;
   if (!generic) {
-    const int shape = route.ragged_depth ? gg::WideRaggedDepth::kId : (short_shape ? Short::kId : Wide::kId);
-    variant = find_variant(g.dtype, layout, shape, variant_epilogue, indexed ? 1 : 0);
+    variant = find_variant(g.dtype, layout, shape.id, variant_epilogue, indexed ? 1 : 0);
     if (variant == nullptr) return fail(GG_EINVAL, "no kernel for this combination of arguments");
   }
 
@@ -385,9 +453,10 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     if (reinterpret_cast<uintptr_t>(g.workspace) & 255)
       return fail(GG_ELIMIT, "the workspace must be 256-byte aligned");
     const uint64_t slot_bytes = (uint64_t)bm * bn * (swiglu ? 2 : 1) * 4;
-    if (g.workspace_bytes < gg::kWsCounterBytes + slot_bytes)
+    constexpr uint64_t least = gg::kWsCounterBytes + (uint64_t)Wide::BM * Wide::BN * 4;
+    if (g.workspace_bytes < least)
       return fail(GG_ELIMIT, "the workspace holds %llu bytes, the smallest useful one %llu",
-                  (unsigned long long)g.workspace_bytes, (unsigned long long)(gg::kWsCounterBytes + slot_bytes));
+                  (unsigned long long)g.workspace_bytes, (unsigned long long)least);
     const uint64_t slots = (g.workspace_bytes - gg::kWsCounterBytes) / slot_bytes;
     p.workspace = static_cast<char*>(g.workspace);
     // one arrival counter per tile of the last round: at most grid / 2 of them, 1024 fit
@@ -446,7 +515,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
       const int64_t grid = tiles < 2 * info.cus ? tiles : 2 * info.cus;
       GG_HIP(generic_ops(g.dtype)->launch(layout, vec, epilogue, gp, hs, (int)grid, stream));
     } else {
-      GG_HIP(variant->launch(p, hs, info.cus, stream));
+      GG_HIP(variant->launch(p, hs, info.cus * variant->workgroups_per_cu, stream));
     }
   }
   return GG_OK;
@@ -488,17 +557,22 @@ uint64_t gg_workspace_bytes_for(const gg_gmm_args* args) {
   const gg_gmm_args& g = *args;
   if (g.dtype < GG_DTYPE_BF16 || g.dtype > GG_DTYPE_F8E5M2 || g.hidden_in <= 0 || g.hidden_out <= 0) return 0;
   const Route r = classify(g);
-  // (the kernels never cut tiles that are combined or scattered on their way out along the depth)
   // (the fix-up of depth pieces stores 4 columns at a time: whole tiles and row pieces for ragged widths)
-  if (r.generic || r.ragged_width || r.ragged_depth || r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU) return 0;
+  if (r.generic || r.ragged_width || r.ragged_depth || g.num_groups <= 0) return 0;
   if (g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ROW_PIECES)) return 0;
-  {
-    const int64_t slice = r.elem_bytes == 1 ? 2 * gg::BK : gg::BK;   // depth elements per slice
-    // (weight-gradient layout: the depth is a group's row count, and one group may hold all rows:
-    // the kernel cuts the tiles of groups much deeper than the rest, plan_deep_tiles)
-    const int64_t depth = g.trans_a ? g.tokens : g.hidden_in;
-    if ((depth + slice - 1) / slice < 2 * gg::kMinSlicesPerPiece) return 0;
-  }
+  const TileShape shape = pick_shape(g, r);
+  const int64_t slice = r.elem_bytes == 1 ? 2 * gg::BK : gg::BK;   // depth elements per slice
+  // (weight-gradient layout: the depth is a group's row count, and one group may hold all rows:
+  // the kernel cuts the tiles of groups much deeper than the rest, plan_deep_tiles)
+  const int64_t depth = g.trans_a ? g.tokens : g.hidden_in;
+  const int64_t slices = (depth + slice - 1) / slice;
+  const int rows = g.trans_a || g.tokens >= g.num_groups * shape.bm ? shape.bm : (int)((g.tokens / g.num_groups + 31) / 32 * 32);
+  const bool scattered = r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU;
+  if (scattered && shape.id == Wide::kId) return 0;
+  // (judged as for a crowded device: a call that could be cut only where it has few tiles does without)
+  if (gg::best_depth_pieces((int)slices, rows, shape.bn, kFullLaunch, 2 * kFullLaunch, gg::kMaxDepthPieces) == 1 &&
+      !(g.trans_a && slices >= 2 * gg::min_slices_per_piece(shape.bm * shape.bn)))
+    return 0;
   return GG_WORKSPACE_BYTES;
 }
 

@@ -101,10 +101,30 @@ enum : int {   // debugging switches, for comparing the ways a call can be sched
 // Workspace layout: kWsCounterBytes of int32 arrival counters (one per tile of the last round; all
 // zero before a launch and all zero again after it), then ws_slots partial tiles of BM x BN floats.
 constexpr int kWsCounterBytes = 4096;
-// Depth pieces per tile: 2 or 4.  A piece's fix-up (a partial tile written, the last piece reading
-// them all back) costs about as much as 20 depth slices, so only deep tiles are cut.
-constexpr int kMaxDepthPieces = 4;
-constexpr int kMinSlicesPerPiece = 48;
+// Into how many depth pieces `tiles` tiles of `slices` depth slices, `rows` rows and BN columns are
+// best cut, at most `most` (1: not at all), on `units` compute units.  In units of depth slices of the
+// same tile: the slices left to a piece, half as slow again where two pieces share a compute unit, and
+// the fix-up: a constant (the arrival counted, the tile loop left) and the partial tiles, written
+// by their pieces and read back by the last of them to arrive, which go through memory and slow down
+// when more than half the device does it at once.  Measured, at 0.6-0.7 us a slice: 64 tiles of 256 x
+// 256, 2 pieces: 25 us of fix-up; 16 of them, 4 pieces: 26 us; 128 of 64 rows x 256, 4 pieces: 18 us;
+// 16 rows x 256, 4 and 8 pieces: 7 and 9 us.
+constexpr int kMaxDepthPieces = 16;
+__host__ __device__ inline int best_depth_pieces(int slices, int rows, int bn, int tiles, int units, int most) {
+  int best = 1, best_cost = slices;
+  for (int pieces = 2; pieces <= most && pieces <= kMaxDepthPieces; pieces *= 2) {
+    const int all = tiles * pieces;
+    int each = (slices + pieces - 1) / pieces;
+    if (all > units) each = each * (units + all) / (2 * units);
+    const int cost = each + 10 + pieces * rows * bn / (2 * all > units ? 3500 : 8000);
+    if (cost < best_cost) best = pieces, best_cost = cost;
+  }
+  return best;
+}
+// ... and for the tiles of a weight gradient that are so deep that they set the length of the launch:
+// fewest slices per piece, most pieces.
+constexpr int min_slices_per_piece(int tile_outputs) { return tile_outputs > 128 * 128 ? 48 : 16; }
+constexpr int kMaxDeepPieces = 4;
 
 // The last round of a persistent grid is filled only partly: `tiles % grid` workgroups have a
 // tile, the others idle.  When that rest is at most half of the grid, each of its tiles is cut
@@ -121,32 +141,25 @@ struct TailPlan {
   int total;        // indices to hand out: main_tiles + rest * pieces
   bool by_depth;
 };
-template <int LAYOUT, bool DEPTH_PIECES_ALLOWED = true>
+template <int LAYOUT, int BM, int BN, int WGS_PER_CU, bool DEPTH_PIECES_ALLOWED = true>
 __device__ __forceinline__ TailPlan plan_tail(int tiles, int grid, const GmmParams& p, int bk) {
   TailPlan t;
   const int rest = tiles % grid;
   t.pieces = 1;
   t.by_depth = false;
   if (rest > 0 && 2 * rest <= grid && !(p.flags & kFlagWholeTiles)) {
-    int cand = grid / rest;
-    cand = cand > kMaxDepthPieces ? kMaxDepthPieces : cand;
     if (DEPTH_PIECES_ALLOWED && p.ws_slots > 0 && !(p.flags & kFlagRowPieces)) {
-      if (rest * cand > p.ws_slots) cand = p.ws_slots / rest;
-      cand = cand >= 4 ? 4 : cand;
-      {   // keep the pieces worth their fix-up
-        // (the depth is the same for every tile, or, in the weight-gradient layout, the group's
-        // row count: there the average over the groups stands for it)
-        const int64_t depth = LAYOUT != kTN ? (int64_t)p.hidden_in : p.tokens / (p.num_groups > 0 ? p.num_groups : 1);
-        const int nk = (int)((depth + bk - 1) / bk);
-        if (cand > nk / kMinSlicesPerPiece) cand = nk / kMinSlicesPerPiece;
-      }
-      cand &= ~1;   // 2 or 4 (3 becomes 2): the fix-up sums two pieces per step
-      if (cand >= 2) {
-        t.pieces = cand;
-        t.by_depth = true;
-      }
+      // The depth is the same for every tile, or, in the weight-gradient layout, the group's row
+      // count: there the average over the groups stands for it, as it does for the rows of a tile
+      // in the other layouts.
+      const int average = (int)(p.tokens / (p.num_groups > 0 ? p.num_groups : 1));
+      const int depth = LAYOUT != kTN ? p.hidden_in : average;
+      const int rows = LAYOUT != kTN && average < BM ? (average + 31) / 32 * 32 : BM;
+      t.pieces = best_depth_pieces((depth + bk - 1) / bk, rows, BN, rest, grid / WGS_PER_CU, min(grid, p.ws_slots) / rest);
+      t.by_depth = t.pieces > 1;
     }
-    if (!t.by_depth && LAYOUT != kTN) t.pieces = 4 * rest <= grid ? 4 : 2;
+    // (a tile of two 32-row blocks is spread over both wave rows already)
+    if (!t.by_depth && LAYOUT != kTN && BM > 64) t.pieces = 4 * rest <= grid ? 4 : 2;
   }
   t.main_tiles = t.pieces > 1 ? tiles - rest : tiles;
   t.total = t.main_tiles + (tiles - t.main_tiles) * t.pieces;
@@ -193,6 +206,10 @@ constexpr uint32_t kRsrcFlags = 0x00020000u;   // raw buffer, 32-bit data format
 // Cache policy of the output stores: non-temporal.  The output is written once and never read by
 // this kernel, so it should not push operand lines that other tiles still share out of L2.
 constexpr int kStoreStreaming = 2;
+// Cache policy of the partial tiles of depth pieces: device scope (sc1), i.e. written through to and
+// read from where all XCDs see them.  Their hand-over then needs no fence, which would write back
+// and invalidate whole L2s: 512 pieces of 16 depth slices took 100 us for theirs.
+constexpr int kDeviceScope = 16;
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
@@ -496,7 +513,9 @@ __device__ __forceinline__ void order_groups_by_depth(Sched* s, int num_groups, 
 // the tiles deeper than half that share (and deep enough to pay for their fix-up) are cut into 2
 // or 4 depth pieces, which are handed out first, one per workgroup.  Run by every thread; the
 // same answer in each.
+template <int BM, int BN>
 __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, int grid, int bk, TailPlan* plan) {
+  constexpr int MIN_SLICES = min_slices_per_piece(BM * BN);
   const int E = p.num_groups;
   const int tiles = s->tile_start[E];
   if (E == 0 || tiles == 0 || p.ws_slots <= 0 || (p.flags & (kFlagWholeTiles | kFlagRowPieces))) return;
@@ -505,7 +524,8 @@ __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, in
   const int64_t slices = ((int64_t)s->row_start[E] - s->row_start[0] + (int64_t)E * (bk / 2)) / bk;
   const int64_t share = slices * per_group / grid;
   const int deepest = (s->most_rows + bk - 1) / bk;
-  const int pieces = deepest >= 4 * kMinSlicesPerPiece ? 4 : (deepest >= 2 * kMinSlicesPerPiece ? 2 : 0);
+  int pieces = deepest / MIN_SLICES;
+  pieces = (pieces > kMaxDeepPieces ? kMaxDeepPieces : pieces) & ~1;
   if (pieces == 0 || deepest <= share) return;
   int most = grid / pieces;
   most = most < p.ws_slots / pieces ? most : p.ws_slots / pieces;
@@ -513,7 +533,7 @@ __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, in
   int front = 0;
   for (int q = 0; q < E && front < most; ++q) {
     const int depth = (s->rows[s->order[q]] + bk - 1) / bk;
-    if (2 * (int64_t)depth <= share || depth < pieces * kMinSlicesPerPiece) break;
+    if (2 * (int64_t)depth <= share || depth < pieces * MIN_SLICES) break;
     front += per_group;
   }
   front = front < most ? front : most;
@@ -1065,6 +1085,7 @@ struct GmmConfig {
                         : SCHED_OFFSET + (int)sizeof(Sched)) + 15) / 16 * 16;
   static constexpr int LDS_BYTES = TILE_RING_OFFSET + WAVES_M * WAVES_N * TILE_RING_SLOTS * kTileInfoDwords * 4;
   static_assert(LDS_BYTES <= 160 * 1024, "a compute unit has 160 KiB of LDS");
+  static constexpr int WORKGROUPS_PER_CU = 2 * LDS_BYTES <= 160 * 1024 ? 2 : 1;
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "wave tile is made of 32x32 MFMA blocks");
   static_assert(BK % 16 == 0 && STAGES >= 2, "");
 };
@@ -1255,7 +1276,9 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
 // RAGGED_DEPTH: hidden_in is even but no multiple of 8 (NN and NT, two-byte elements, plain store).
 template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N,
           int EPI = kEpiStore, bool INDEXED = false, bool RAGGED_DEPTH = false>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p, HostSizes hs) {
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
+                             (GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>::WORKGROUPS_PER_CU)) void
+gmm_kernel(GmmParams p, HostSizes hs) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
   using Cfg = GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>;
   constexpr int NT = Cfg::NT, MB = Cfg::MB, NB = Cfg::NB, KS = BK / 16;
@@ -1280,9 +1303,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
   using BFrag = std::conditional_t<Cfg::B_DEPTH_MAJOR, DepthMajorFrag<BK, 1, F8>,
                                    std::conditional_t<F8, WidthMajorFrag8<BN, NB, 1>, WidthMajorFrag<BN, BK, NB, 1>>>;
   constexpr int LOADS_PER_STAGE = ALoad::NI + BLoad::NI;   // per lane, per depth slice
-  constexpr int QUARTER_LOADS = LOADS_PER_STAGE / 4;
+  // (a slice's loads go out in four parts, one per step: loads Q1, Q2 and Q3 begin parts 2, 3 and 4)
+  constexpr int Q1 = LOADS_PER_STAGE / 4, Q2 = LOADS_PER_STAGE / 2, Q3 = LOADS_PER_STAGE * 3 / 4;
   static_assert(KS == 4 && STAGES == 2, "the step schedule below is written for BK = 64 and two buffers");
-  static_assert(LOADS_PER_STAGE % 4 == 0 && LOADS_PER_STAGE < 32, "");
+  static_assert(LOADS_PER_STAGE >= 4 && LOADS_PER_STAGE < 32, "");
   constexpr int UNITS = MB + NB;    // fragments of one 16-deep step
 
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -1304,15 +1328,15 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
   afrag.setup(wm * 32);   // wave row wm owns row blocks wm, wm + WAVES_M, ...
   bfrag.setup(wn * Cfg::WTN);
 
-  // (a tile that is combined or scattered on its way out is never cut along the depth: the
-  // fix-up of the depth pieces stores plain tiles)
-  constexpr bool DEPTH_PIECES = !(GATE_UP || INDEXED || RAGGED_DEPTH);
-  TailPlan plan = plan_tail<LAYOUT, DEPTH_PIECES>(
+  // (tiles that are combined or scattered on their way out are cut along the depth in the shapes for
+  // few rows and few tiles only: full ones would pay for it with the fix-up's scalar registers)
+  constexpr bool DEPTH_PIECES = !RAGGED_DEPTH && !((GATE_UP || INDEXED) && BM > 128);
+  TailPlan plan = plan_tail<LAYOUT, BM, BN, Cfg::WORKGROUPS_PER_CU, DEPTH_PIECES>(
       uniform(sched->tile_start[p.num_groups]) + uniform(sched->runt_start[p.num_groups]),
       (int)gridDim.x, p, BK_ELEMS);
   if constexpr (!DEPTH_PIECES) plan.by_depth = false;   // (known at compile time: no depth-piece code is kept)
   if constexpr (LAYOUT == kTN && DEPTH_PIECES) {
-    plan_deep_tiles(sched, p, (int)gridDim.x, BK_ELEMS, &plan);
+    plan_deep_tiles<BM, BN>(sched, p, (int)gridDim.x, BK_ELEMS, &plan);
     plan.pieces = uniform(plan.pieces), plan.main_tiles = uniform(plan.main_tiles), plan.total = uniform(plan.total);
   }
   const int total_tiles = plan.total;
@@ -1430,9 +1454,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
   using I2 = std::integral_constant<int, 2>;
   using I3 = std::integral_constant<int, 3>;
   using IMB = std::integral_constant<int, MB>;
-  using IQ = std::integral_constant<int, QUARTER_LOADS>;
-  using IQ2 = std::integral_constant<int, 2 * QUARTER_LOADS>;
-  using IQ3 = std::integral_constant<int, 3 * QUARTER_LOADS>;
+  using IQ1 = std::integral_constant<int, Q1>;
+  using IQ2 = std::integral_constant<int, Q2>;
+  using IQ3 = std::integral_constant<int, Q3>;
+  using ILast = std::integral_constant<int, LOADS_PER_STAGE - Q3>;   // loads of the fourth part, and so on
+  using IThird = std::integral_constant<int, Q3 - Q2>;
+  using ISecond = std::integral_constant<int, Q2 - Q1>;
 
   // Both buffers are requested up front, except the last quarter of the second slice: every
   // step issues one quarter of a slice's loads, and step 0 issues the last quarter of the
@@ -1442,7 +1469,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
   static_for<LOADS_PER_STAGE>([&](auto j) { fetch_load(j, 0); });
   fetch_advance();
   fetch_begin();
-  static_for<3 * QUARTER_LOADS>([&](auto j) { fetch_load(j, 1); });
+  static_for<Q3>([&](auto j) { fetch_load(j, 1); });
 
   int tile_t = vid;
   int tile_n = 0;   // tiles this workgroup has finished
@@ -1473,7 +1500,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
       block_barrier();
     }
   };
-  wait_vmcnt<3 * QUARTER_LOADS>();   // the first slice is in
+  wait_vmcnt<Q3>();   // the first slice is in
   block_barrier();
   if (RAGGED_DEPTH && tail_slice == 0) clear_tail(0);
   static_for<2 * UNITS>([&](auto u) {
@@ -1483,14 +1510,46 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
 
   int x = 0;   // buffer of the slice being multiplied
 
-  // Partial tile of depth piece `piece` of the tile `ti` names, as this thread sees it: a lane's
-  // 16-byte group (i, j, q) sits at ((i * NB + j) * 4 + q) * NT + thread, so one instruction of a
-  // wave moves 1 KiB of consecutive bytes.
-  auto partial_slot = [&](const TileInfo& tile, int piece) {
-    return reinterpret_cast<float*>(p.workspace + kWsCounterBytes) +
-           (int64_t)(tile.rank * tile.pieces + piece) * (BM * BN) + threadIdx.x * 4;
+  // Partial tile of depth piece `piece` of the tile `ti` names: a lane's 16-byte group (i, j, q) sits
+  // at ((i * NB + j) * 4 + q) * NT + thread, so one instruction of a wave moves 1 KiB of consecutive
+  // bytes.
+  auto partial_rsrc = [&](const TileInfo& tile, int piece) {
+    return make_rsrc(p.workspace + kWsCounterBytes + (int64_t)(tile.rank * tile.pieces + piece) * (BM * BN * 4),
+                     BM * BN * 4);
   };
+  auto partial_at = [&](int i, int j, int q) -> uint32_t { return (((i * NB + j) * 4 + q) * NT + threadIdx.x) * 16; };
   bool fix_pending = false;   // this workgroup's depth piece was the last of its tile to arrive
+
+  // Where a tile's rows of c are: a descriptor of them, or of all of c when rows go through an
+  // index, the byte offset of row `row` of the tile in it and that of one of its columns (C_OOR: no
+  // such row or column, nothing is stored).
+  constexpr int CE = ACC_F32 ? 4 : 2;   // bytes per element of c
+  constexpr uint32_t C_OOR = INDEXED ? kOutOfRangeIndexed : kOutOfRange;
+  auto c_rsrc = [&](const TileInfo& tile) {
+    if constexpr (INDEXED) return make_rsrc(p.c, p.c_bytes);
+    return make_rsrc(p.c + (tile.g.c_off + (int64_t)tile.m0 * tile.g.n) * CE,
+                     tile.rows_valid > 0 ? (uint32_t)(tile.rows_valid * tile.g.n) * (uint32_t)CE : 0u);
+  };
+  auto c_row = [&](const TileInfo& tile, int row) -> uint32_t {
+    if constexpr (INDEXED) {
+      if (row >= tile.rows_valid) return C_OOR;
+      const int r = tile.g.row0 + tile.m0 + row;
+      const uint32_t dst = p.c_rows != nullptr ? (uint32_t)p.c_rows[r] : (uint32_t)r;
+      return dst < p.c_index_rows ? dst * (uint32_t)tile.g.n * 2u : C_OOR;   // no such row: not stored
+    } else {
+      return (uint32_t)(row * tile.g.n) * (uint32_t)CE;
+    }
+  };
+  auto c_at = [&](const TileInfo& tile, uint32_t row_off, int col) -> uint32_t {
+    return col < tile.g.n && (!INDEXED || row_off != C_OOR) ? row_off + (uint32_t)col * (uint32_t)CE : C_OOR;
+  };
+  // silu(gate) * up of four element pairs, rounded
+  auto combine4 = [](const float* gate, const float* up) {
+    float o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = gate[r] / (1.0f + __expf(-gate[r])) * up[r];
+    return round4<OUT_DT>(o[0], o[1], o[2], o[3]);
+  };
 
   // One tile, for a wave that has ML row blocks with rows in them (the tile's row blocks go to
   // the wave rows alternately).  One copy of this body exists per value of ML; a tile picks
@@ -1556,19 +1615,19 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
 
     for (int kt = 0; kt < ti.nk; ++kt) {
       const int y = uniform(x ^ 1);   // (the same in every lane: keeps the LDS addresses scalar)
-      step(I0{}, I2{}, ml_tag, I2{}, IQ3{}, IQ{}, x, y);
+      step(I0{}, I2{}, ml_tag, I2{}, IQ3{}, ILast{}, x, y);
       fetch_advance();
       // every wave has all fragments of this slice in registers
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       block_barrier();
       fetch_begin();
-      step(I1{}, I0{}, ml_tag, I0{}, I0{}, IQ{}, x, x);
-      step(I2{}, I0{}, ml_tag, I0{}, IQ{}, IQ{}, x, x);
+      step(I1{}, I0{}, ml_tag, I0{}, I0{}, IQ1{}, x, x);
+      step(I2{}, I0{}, ml_tag, I0{}, IQ1{}, ISecond{}, x, x);
       // the next slice has landed for every wave (only this slice's two quarters may be pending)
-      wait_vmcnt<2 * QUARTER_LOADS>();
+      wait_vmcnt<Q2>();
       block_barrier();
       if (RAGGED_DEPTH && uniform(kt + 1 == ti.nk ? 0 : kt + 1) == tail_slice) clear_tail(y);
-      step(I3{}, I2{}, IMB{}, I0{}, IQ2{}, IQ{}, y, x);
+      step(I3{}, I2{}, IMB{}, I0{}, IQ2{}, IThird{}, y, x);
       x = uniform(y);
     }
 
@@ -1576,7 +1635,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
     // count the arrival.  The piece that arrives last adds the partial tiles up and stores the
     // sum, after the tile loop (fix_up below), where no accumulator is live any more.
     if (DEPTH_PIECES && ti.pieces > 1) {
-      float* mine = partial_slot(ti, ti.piece);
+      const __amdgpu_buffer_rsrc_t mine = partial_rsrc(ti, ti.piece);
 #pragma unroll
       for (int i = 0; i < ML; ++i)
 #pragma unroll
@@ -1584,11 +1643,12 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-            *reinterpret_cast<f32x4*>(mine + ((i * NB + j) * 4 + q) * (NT * 4)) = v;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), mine, partial_at(i, j, q), 0, kDeviceScope);
           }
-      __threadfence();   // the partial tile is visible device-wide before the arrival is counted
+      wait_vmcnt<0>();   // every wave's part has arrived before the arrival is counted
       block_barrier();
-      if (threadIdx.x == 0) sched->arrived = atomicAdd(reinterpret_cast<int*>(p.workspace) + ti.rank, 1);
+      if (threadIdx.x == 0) sched->arrived = __hip_atomic_fetch_add(reinterpret_cast<int*>(p.workspace) + ti.rank, 1, __ATOMIC_RELAXED,
+                                                                        __HIP_MEMORY_SCOPE_AGENT);
       block_barrier();
       fix_pending = uniform(sched->arrived) == ti.pieces - 1;
       if (fix_pending) {
@@ -1608,27 +1668,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
     // The accumulators stay in the accumulation registers; each value is moved out right
     // where it is converted, so the epilogue needs only a few vector registers.
     {
-      constexpr int CE = ACC_F32 ? 4 : 2;   // bytes per element of c
-      constexpr uint32_t OOR = INDEXED ? kOutOfRangeIndexed : kOutOfRange;
-      // the descriptor covers the tile's rows of c, or all of c when rows go through an index
-      const char* cbase = INDEXED ? p.c : p.c + (ti.g.c_off + (int64_t)ti.m0 * ti.g.n) * CE;
-      const uint32_t cbytes = INDEXED ? p.c_bytes
-                              : (ti.rows_valid > 0 ? (uint32_t)(ti.rows_valid * ti.g.n) * (uint32_t)CE : 0u);
-      const __amdgpu_buffer_rsrc_t rc = make_rsrc(cbase, cbytes);
-      // byte offset of row `row` of the tile in that descriptor (OOR: the row does not exist)
-      auto row_offset = [&](int row) -> uint32_t {
-        if constexpr (INDEXED) {
-          if (row >= ti.rows_valid) return OOR;
-          const int r = ti.g.row0 + ti.m0 + row;
-          const uint32_t dst = p.c_rows != nullptr ? (uint32_t)p.c_rows[r] : (uint32_t)r;
-          return dst < p.c_index_rows ? dst * (uint32_t)ti.g.n * 2u : OOR;   // no such row: not stored
-        } else {
-          return (uint32_t)(row * ti.g.n) * (uint32_t)CE;
-        }
-      };
-      auto at = [&](uint32_t row_off, int col) -> uint32_t {
-        return col < ti.g.n && (!INDEXED || row_off != OOR) ? row_off + (uint32_t)col * (uint32_t)CE : OOR;
-      };
+      constexpr uint32_t OOR = C_OOR;
+      const __amdgpu_buffer_rsrc_t rc = c_rsrc(ti);
+      auto row_offset = [&](int row) { return c_row(ti, row); };
+      auto at = [&](uint32_t row_off, int col) { return c_at(ti, row_off, col); };
       auto take4 = [&](int i, int j, int q) {
         float v[4];
 #pragma unroll
@@ -1646,17 +1689,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
           for (int jp = 0; jp < NB / 2; ++jp) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-              float o[4];
+              float gate[4], up[4];
 #pragma unroll
               for (int r = 0; r < 4; ++r) {
-                float gate, up;
-                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(gate) : "a"(acc[i][2 * jp][4 * q + r]));
-                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(up) : "a"(acc[i][2 * jp + 1][4 * q + r]));
-                o[r] = gate / (1.0f + __expf(-gate)) * up;
+                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(gate[r]) : "a"(acc[i][2 * jp][4 * q + r]));
+                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(up[r]) : "a"(acc[i][2 * jp + 1][4 * q + r]));
               }
               const int col = ti.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
-              __builtin_amdgcn_raw_buffer_store_b64(round4<OUT_DT>(o[0], o[1], o[2], o[3]), rc, at(row_off, col), 0,
-                                                    kStoreStreaming);
+              __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, at(row_off, col), 0, kStoreStreaming);
             }
             __builtin_amdgcn_sched_barrier(0);
           }
@@ -1835,12 +1875,8 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
 #pragma unroll
     for (int i = 0; i < kTileInfoDwords; ++i) words[i] = sched->fix_tile[i];
     const TileInfo ft = unpack_tile(words);
-    __threadfence();   // the other pieces' partial tiles are visible to this workgroup
     if (threadIdx.x == 0) reinterpret_cast<int*>(p.workspace)[ft.rank] = 0;   // leave the counters as they were found
-    constexpr int CE = ACC_F32 ? 4 : 2;   // bytes per element of c
-    const char* cbase = p.c + (ft.g.c_off + (int64_t)ft.m0 * ft.g.n) * CE;
-    const uint32_t cbytes = ft.rows_valid > 0 ? (uint32_t)(ft.rows_valid * ft.g.n) * (uint32_t)CE : 0u;
-    const __amdgpu_buffer_rsrc_t rc = make_rsrc(cbase, cbytes);
+    const __amdgpu_buffer_rsrc_t rc = c_rsrc(ft);
     const int live = LAYOUT == kTN ? MB : (ft.blocks - wm + WAVES_M - 1) / WAVES_M;
     for (int i = 0; i < live; ++i) {
       f32x4 sum[NB][4];
@@ -1849,15 +1885,14 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
 #pragma unroll
         for (int q = 0; q < 4; ++q) sum[j][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
       for (int piece = 0; piece < ft.pieces; piece += 2) {
-        const float* from0 = partial_slot(ft, piece) + (i * NB * 4) * (NT * 4);
-        const float* from1 = partial_slot(ft, piece + 1) + (i * NB * 4) * (NT * 4);
+        const __amdgpu_buffer_rsrc_t from0 = partial_rsrc(ft, piece), from1 = partial_rsrc(ft, piece + 1);
         f32x4 v0[NB][4], v1[NB][4];
 #pragma unroll
         for (int j = 0; j < NB; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            v0[j][q] = *reinterpret_cast<const f32x4*>(from0 + (j * 4 + q) * (NT * 4));
-            v1[j][q] = *reinterpret_cast<const f32x4*>(from1 + (j * 4 + q) * (NT * 4));
+            v0[j][q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from0, partial_at(i, j, q), 0, kDeviceScope));
+            v1[j][q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from1, partial_at(i, j, q), 0, kDeviceScope));
           }
 #pragma unroll
         for (int j = 0; j < NB; ++j)
@@ -1865,21 +1900,34 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N * 64) void gmm_kernel(GmmParams p,
           for (int q = 0; q < 4; ++q) sum[j][q] = (sum[j][q] + v0[j][q]) + v1[j][q];
       }
       // a lane owns row (l % 32) of each 32x32 block and columns 8q + 4(l/32) .. +3
-      const int row = (wm + i * WAVES_M) * 32 + (lane & 31);
+      const uint32_t row_off = c_row(ft, (wm + i * WAVES_M) * 32 + (lane & 31));
+      if constexpr (GATE_UP) {
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
+        for (int jp = 0; jp < NB / 2; ++jp)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int col = ft.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
-          const uint32_t off = col < ft.g.n ? (uint32_t)(row * ft.g.n + col) * (uint32_t)CE : kOutOfRange;
-          if constexpr (ACC_F32) {
-            const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
-            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, old + sum[j][q]), rc, off, 0, 0);
-          } else {
-            __builtin_amdgcn_raw_buffer_store_b64(
-                round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]), rc, off, 0, kStoreStreaming);
+          for (int q = 0; q < 4; ++q) {
+            float gate[4], up[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) gate[r] = sum[2 * jp][q][r], up[r] = sum[2 * jp + 1][q][r];
+            const int col = ft.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
+            __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, c_at(ft, row_off, col), 0, kStoreStreaming);
           }
-        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int col = ft.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
+            const uint32_t off = c_at(ft, row_off, col);
+            if constexpr (ACC_F32) {
+              const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
+              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, old + sum[j][q]), rc, off, 0, 0);
+            } else {
+              __builtin_amdgcn_raw_buffer_store_b64(
+                  round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]), rc, off, 0, kStoreStreaming);
+            }
+          }
+      }
     }
   }
 #endif  // __HIP_DEVICE_COMPILE__

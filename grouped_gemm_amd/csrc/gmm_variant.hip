@@ -44,7 +44,7 @@ hipError_t launch(const GmmParams& p, const HostSizes& hs, int grid, hipStream_t
                          Cfg::LDS_BYTES, stream);
 }
 
-const VariantOps kOps = {V::DT, V::LAYOUT, S::kId, V::EPI, V::INDEXED ? 1 : 0, Cfg::LDS_BYTES, &prepare, &launch};
+const VariantOps kOps = {V::DT, V::LAYOUT, S::kId, V::EPI, V::INDEXED ? 1 : 0, Cfg::LDS_BYTES, Cfg::WORKGROUPS_PER_CU, &prepare, &launch};
 
 }  // namespace
 

@@ -31,9 +31,22 @@ struct WideRaggedDepth : Wide {
   static constexpr bool RAGGED_DEPTH = true;
 };
 
+// Small tiles, for launches that have too few wide ones to fill the device: 64 x 128 outputs, two
+// workgroups per compute unit, in the layouts with a row of c per token; 128 x 128 for weight
+// gradients (whose operands run along both widths, at least 128 of each).
+struct Small {
+  static constexpr int kId = 3, BM = 64, BN = 128, WAVES_M = 2, WAVES_N = 2;
+  static constexpr bool RAGGED_DEPTH = false;
+};
+struct SmallSquare {
+  static constexpr int kId = 4, BM = 128, BN = 128, WAVES_M = 2, WAVES_N = 2;
+  static constexpr bool RAGGED_DEPTH = false;
+};
+
 struct VariantOps {
   int dt, layout, shape, epilogue, indexed;
   int lds_bytes;
+  int workgroups_per_cu;
   // raises the kernel's dynamic LDS limit on the current device
   hipError_t (*prepare)();
   hipError_t (*launch)(const GmmParams& p, const HostSizes& hs, int grid, hipStream_t stream);

@@ -170,8 +170,8 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *   accumulate_f32  1: c is fp32 and is added to (trans_a = 1 only), as gg_gmm_bf16_acc_f32.
  *   workspace, workspace_bytes
  *                 Device memory the call may use for partial results, or NULL.  When the last
- *                 round of the persistent grid is at most half full, each of its tiles is cut
- *                 into 2 or 4 pieces along the depth; a piece adds up its depth slices into an
+ *                 round of the persistent grid is at most half full, each of its tiles may be cut
+ *                 into 2 to 16 pieces along the depth; a piece adds up its depth slices into an
  *                 fp32 partial tile in the workspace, and the piece that finishes last sums the
  *                 partial tiles in piece order and stores the result, so the output does not
  *                 depend on timing.  With trans_a = 1, when a group is so much deeper than the
@@ -218,10 +218,10 @@ int gg_gmm(const gg_gmm_args* args);
 
 /*
  * Bytes of workspace the call described by `args` can make use of: 0 when no launch of it ever
- * cuts tiles along the depth (general kernels, row indices, the SwiGLU epilogue, or a product too
- * shallow for depth pieces to pay: fewer than 96 depth slices of 64 two-byte or 128 one-byte
- * elements, the depth of the trans_a layout being what one group could hold, i.e. all rows),
- * GG_WORKSPACE_BYTES otherwise.  Looks at the sizes, flags
+ * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8, or a
+ * product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte
+ * elements for full tiles, fewer for groups of few rows; the depth of the trans_a layout being what
+ * one group could hold, i.e. all rows), GG_WORKSPACE_BYTES otherwise.  Looks at the sizes, flags
  * and pointers' alignment only; args->workspace is ignored.  A caller that keeps workspaces
  * (one per stream) need not allocate one for calls this returns 0 for.  No counterpart in the
  * reference, which asks CUTLASS for its workspace size per call (csrc/grouped_gemm.cu:347-349).
@@ -289,7 +289,8 @@ int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device,
 
 /* Output tile (rows, columns) and depth slice the kernel uses for a call with these arguments
  * (calls whose groups average few rows get a shorter tile); for reports and for checking the
- * tile counts of gg_debug_schedule. */
+ * tile counts of gg_debug_schedule.  Launches with too few of these tiles to fill the device run
+ * on smaller ones, which depends on the hidden sizes as well: neither function shows those. */
 int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, int* bm, int* bn,
                   int* bk);
 

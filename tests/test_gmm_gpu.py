@@ -508,6 +508,72 @@ def test_deep_groups_of_a_weight_gradient_are_cut_first(oracle):
                 assert not bool(cut[e].any())
 
 
+# Sizes that reach every tile shape, whole and cut along the depth (the rule is pick_shape in
+# gmm_api.hip): sizes, hidden_in, hidden_out.
+_TILE_SHAPES = {
+    "wide": (list(range(1, 520, 11)), 72, 1032),                 # every count of 32-row blocks, partly filled columns
+    "short": ([(7 * e) % 61 for e in range(200)], 136, 776),
+    "short, cut": ([16, 0, 40, 1, 33, 16, 20, 2], 6400, 4096),   # few rows, deep: two pieces
+    "small": ([300, 0, 17, 195, 64, 65], 264, 392),
+    "small, cut": ([20, 0, 70, 1, 33], 4096, 200),               # up to sixteen pieces
+    "small, one slice": ([5, 130], 8, 136),
+}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("case", list(_TILE_SHAPES))
+def test_every_tile_shape_with_every_epilogue(ops, oracle, case, trans_b, dtype):
+    # plain, gathered, scattered, SwiGLU and SwiGLU with both, against the loop in fp32 on the GPU; the
+    # same bits on a second call (the fix-up of depth pieces adds in a fixed order)
+    sizes, hin, hout = _TILE_SHAPES[case]
+    _announce("tile shapes", case, trans_b, dtype)
+    g = torch.Generator().manual_seed(23)
+    bs = torch.tensor(sizes, dtype=torch.int64)
+    t = int(bs.sum())
+    a = torch.randn(t, hin, generator=g).to(dtype).cuda()
+    b = (torch.randn(len(sizes), *((hout, hin) if trans_b else (hin, hout)), generator=g) * hin ** -0.5).to(dtype).cuda()
+    rows = torch.randperm(t, generator=g).to(torch.int32).cuda()
+    dev = bs.cuda()
+    be = ops.backend
+    def scattered(fn, width):
+        c = torch.full((t, width), 7.0, dtype=dtype, device="cuda")
+        fn(c)
+        return c[rows.long()]
+    plain, swiglu = oracle.gmm_loop(a, b, bs, trans_b=trans_b), oracle.swiglu_loop(a, b, bs, trans_b=trans_b)
+    gathered = oracle.gmm_loop(a[rows.long()], b, bs, trans_b=trans_b)
+    both = oracle.swiglu_loop(a[rows.long()], b, bs, trans_b=trans_b)
+    for what, want, call in (
+            ("plain", plain, lambda: be.gmm(a, b, dev, trans_b=trans_b)),
+            ("gathered", gathered, lambda: be.gmm_indexed(a, b, dev, trans_b=trans_b, a_rows=rows)),
+            ("scattered", plain, lambda: scattered(lambda c: be.gmm_indexed(a, b, dev, trans_b=trans_b, c=c, c_rows=rows), hout)),
+            ("swiglu", swiglu, lambda: be.gmm_swiglu(a, b, dev, trans_b=trans_b)),
+            ("swiglu, both", both, lambda: scattered(lambda c: be.gmm_swiglu(a, b, dev, trans_b=trans_b, c=c, a_rows=rows, c_rows=rows), hout // 2))):
+        got = call()
+        check(got, want, f"{case}, {what}")
+        assert torch.equal(got, call()), f"{case}, {what}: not the same bits twice"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("sizes,hin,hout", [([300, 0, 17, 195], 136, 264), ([1], 8, 8), ([2000, 1500], 128, 128),
+                                            ([129] * 40, 264, 136)])
+def test_small_tiles_of_a_weight_gradient(ops, oracle, dtype, sizes, hin, hout):
+    # 128 x 128 tiles: ragged edges, an empty group, one slice, a group deep enough for depth pieces;
+    # stored and added to fp32
+    _announce("small weight gradient", dtype, sizes if len(sizes) < 9 else len(sizes), hin, hout)
+    g = torch.Generator().manual_seed(29)
+    bs = torch.tensor(sizes, dtype=torch.int64)
+    a = torch.randn(int(bs.sum()), hin, generator=g).to(dtype)
+    b = torch.randn(int(bs.sum()), hout, generator=g).to(dtype)
+    want = oracle.gmm_loop(a, b, bs, trans_a=True)
+    got = ops.backend.gmm(a.cuda(), b.cuda(), bs.cuda(), trans_a=True)
+    check(got, want, "stored")
+    assert torch.equal(got, ops.backend.gmm(a.cuda(), b.cuda(), bs.cuda(), trans_a=True))
+    c = torch.randn(len(sizes), hin, hout, generator=g)
+    acc = ops.backend.accumulate_weight_gradient(a.cuda(), b.cuda(), bs.cuda(), c.cuda())
+    check(acc, c + want, "accumulated")
+
+
 def test_c_abi_without_workspace_cuts_rows_bit_exactly(oracle):
     # gg_gmm_bf16 brings no workspace: the tiles of the last round are cut along their rows, which
     # leaves the depth order of every output element alone, so the result equals the whole-tile
