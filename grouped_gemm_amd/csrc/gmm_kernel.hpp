@@ -1681,10 +1681,22 @@ gmm_kernel(GmmParams p, HostSizes hs) {
       };
       if constexpr (GATE_UP) {
         // Blocks 2 jp and 2 jp + 1 of a wave hold the gate and the up value of the same 32 output
-        // columns, element for element: silu(gate) * up in fp32, one rounding, 8 bytes per lane.
+        // columns, element for element: silu(gate) * up in fp32, one rounding, then through the wave's
+        // LDS strip (32 rows x the wave's output columns) so that stores are 16 bytes per lane and
+        // whole lines: the 8-byte pieces the lanes hold, 16 bytes of a line per row and instruction,
+        // were written at that size past L2 (16 x 1024 rows, 2048 -> 4096: 637 -> 574 us; decode,
+        // 8 x 16 rows, 4096 -> 14336: 357 -> 348).
+        static_assert(Cfg::STAGED_EPILOGUE, "the gate | up epilogue uses the waves' LDS strips");
+        constexpr int OUTW = Cfg::WTN / 2, CHUNKS = OUTW / 8, ROWS = 64 / CHUNKS, PITCH = Cfg::EPILOGUE_PITCH;
+        char* strip = smem + Cfg::EPILOGUE_OFFSET + wave * Cfg::EPILOGUE_WAVE_BYTES;
+        const int in_row = lane & 31, in_half = lane >> 5;
+        const int out_row = lane / CHUNKS, out_chunk = lane % CHUNKS;
+        const int col = ti.n0 + wn * OUTW + out_chunk * 8;
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
-          const uint32_t row_off = row_offset((wm + i * WAVES_M) * 32 + (lane & 31));
+          uint32_t row_off[32 / ROWS];
+#pragma unroll
+          for (int r = 0; r < 32 / ROWS; ++r) row_off[r] = row_offset((wm + i * WAVES_M) * 32 + r * ROWS + out_row);
 #pragma unroll
           for (int jp = 0; jp < NB / 2; ++jp) {
 #pragma unroll
@@ -1695,11 +1707,16 @@ gmm_kernel(GmmParams p, HostSizes hs) {
                 asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(gate[r]) : "a"(acc[i][2 * jp][4 * q + r]));
                 asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(up[r]) : "a"(acc[i][2 * jp + 1][4 * q + r]));
               }
-              const int col = ti.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
-              __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, at(row_off, col), 0, kStoreStreaming);
+              *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jp * 32 + 8 * q + 4 * in_half) * 2) =
+                  combine4(gate, up);
             }
-            __builtin_amdgcn_sched_barrier(0);
           }
+#pragma unroll
+          for (int r = 0; r < 32 / ROWS; ++r) {
+            const u32x4 v = *reinterpret_cast<const u32x4*>(strip + (r * ROWS + out_row) * PITCH + out_chunk * 16);
+            __builtin_amdgcn_raw_buffer_store_b128(v, rc, at(row_off[r], col), 0, kStoreStreaming);
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
       } else if constexpr (ACC_F32) {
         if constexpr (EPI == kEpiAccF32Atomic) {
