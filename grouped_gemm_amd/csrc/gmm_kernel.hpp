@@ -1649,6 +1649,9 @@ gmm_kernel(GmmParams p, HostSizes hs) {
       block_barrier();
       if (threadIdx.x == 0) sched->arrived = __hip_atomic_fetch_add(reinterpret_cast<int*>(p.workspace) + ti.rank, 1, __ATOMIC_RELAXED,
                                                                         __HIP_MEMORY_SCOPE_AGENT);
+      // (the barrier alone orders nothing: without the wait another wave could read the word before
+      // it is written, and would then add up a tile that is not complete, or leave its part out)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       block_barrier();
       fix_pending = uniform(sched->arrived) == ti.pieces - 1;
       if (fix_pending) {
