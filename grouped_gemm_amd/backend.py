@@ -23,12 +23,15 @@ import sys as _sys
 _sys.modules.setdefault("grouped_gemm_backend", backend)
 
 
-def _allocate_output(a, b, batch_sizes, trans_a, trans_b):
+def _check_ranks(a, b, batch_sizes, trans_a, trans_b):
     assert not (trans_a and trans_b)
     assert batch_sizes.ndim == 1, "Expected 1d tensor for batch_sizes"
     assert a.ndim == 2, "Expected 2d tensor for 'a'"
     assert b.ndim == (2 if trans_a else 3)
 
+
+def _allocate_output(a, b, batch_sizes, trans_a, trans_b):
+    _check_ranks(a, b, batch_sizes, trans_a, trans_b)
     shape = (
         (batch_sizes.shape[0], a.shape[1], b.shape[1])
         if trans_a else
@@ -46,8 +49,8 @@ def _output_dtype(dtype):
 # start on a 16-byte boundary, would run on the extension's general kernels, which are many times
 # slower than the streaming ones (calling the extension directly gets exactly that, copy-free).
 # gmm instead copies such operands into zero-padded, aligned tensors, runs the streaming kernels
-# on those and copies the result back: three extra passes over the operands, still several times
-# faster.  Zeros along the depth add nothing to any sum; padded output columns are dropped.
+# on those and copies the result back: one pass over each, still several times faster.  Zeros along
+# the depth add nothing to any sum; padded output columns are dropped.
 # Needing no copies: two-byte operands on 4-byte boundaries whose hidden sizes are both even.
 
 
@@ -55,54 +58,108 @@ def _round_up(x, m):
     return (x + m - 1) // m * m
 
 
-def _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
-    """gmm through zero-padded copies; returns False when the operands are not the well-formed GPU
-    tensors this path assumes (the plain call then runs and raises what it has to raise)."""
-    if not (a.is_cuda and b.is_cuda and c.is_cuda and a.dtype == b.dtype and a.dim() == 2 and
-            b.dim() == (2 if trans_a else 3) and c.dtype == _output_dtype(a.dtype) and batch_sizes.dim() == 1):
+def _needs_padding(a, b, c, batch_sizes, trans_a, trans_b):
+    """Whether gmm goes through zero-padded copies; False when the operands are not the well-formed
+    GPU tensors that way assumes (the plain call then runs and raises what it has to raise).  `c`:
+    the output, or None for one still to be allocated."""
+    if not (a.is_cuda and b.is_cuda and a.dtype == b.dtype and a.dim() == 2 and
+            b.dim() == (2 if trans_a else 3) and batch_sizes.dim() == 1):
+        return False
+    if not (a.device == b.device and a.dtype in (torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.float8_e5m2)):
         return False
     hin = a.shape[1]
     hout = b.shape[1] if (trans_a or trans_b) else b.shape[2]
     experts = batch_sizes.shape[0]
     if trans_a:
-        consistent = a.shape[0] == b.shape[0] and tuple(c.shape) == (experts, hin, hout)
+        consistent = a.shape[0] == b.shape[0]
+        out_shape = (experts, hin, hout)
     else:
-        consistent = (tuple(b.shape) == ((experts, hout, hin) if trans_b else (experts, hin, hout)) and
-                      tuple(c.shape) == (a.shape[0], hout))
+        consistent = tuple(b.shape) == ((experts, hout, hin) if trans_b else (experts, hin, hout))
+        out_shape = (a.shape[0], hout)
+    if c is not None:
+        consistent = (consistent and tuple(c.shape) == out_shape and c.device == a.device and
+                      c.dtype == _output_dtype(a.dtype) and c.is_contiguous())
     if not consistent or hin == 0 or hout == 0 or a.shape[0] == 0:
         return False
     # (tensors that are not contiguous are rejected by the extension, as by the reference)
-    if not (a.is_contiguous() and b.is_contiguous() and c.is_contiguous()):
+    if not (a.is_contiguous() and b.is_contiguous()):
         return False
+    operands = (a, b) if c is None else (a, b, c)
     mult = 16 if a.element_size() == 1 else 8
-    aligned = all(t.data_ptr() % 16 == 0 for t in (a, b, c))
-    if hin % mult == 0 and hout % mult == 0 and aligned:
+    if hin % mult == 0 and hout % mult == 0 and all(t.data_ptr() % 16 == 0 for t in operands):
         return False
-    if a.element_size() == 2 and all(t.data_ptr() % 4 == 0 for t in (a, b, c)) and hout % 2 == 0 and hin % 2 == 0:
-        return False   # the streaming kernels take these as they are
+    # (otherwise the streaming kernels take these as they are)
+    return not (a.element_size() == 2 and all(t.data_ptr() % 4 == 0 for t in operands) and hout % 2 == 0 and hin % 2 == 0)
+
+
+def _padded(t, rows, cols):
+    if t.shape[-2] == rows and t.shape[-1] == cols and t.data_ptr() % 16 == 0:
+        return t
+    return backend.pad_rows(t, rows, cols)
+
+
+def _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
+    """gmm through zero-padded copies, for operands that _needs_padding accepts."""
+    hin = a.shape[1]
+    hout = b.shape[1] if (trans_a or trans_b) else b.shape[2]
+    mult = 16 if a.element_size() == 1 else 8
     hin_p, hout_p = _round_up(hin, mult), _round_up(hout, mult)
-
-    def padded(t, shape):
-        if tuple(t.shape) == tuple(shape) and t.data_ptr() % 16 == 0:
-            return t
-        out = t.new_zeros(shape)
-        out[tuple(slice(0, n) for n in t.shape)] = t
-        return out
-
-    a_p = padded(a, (a.shape[0], hin_p))
+    a_p = _padded(a, a.shape[0], hin_p)
     if trans_a:
-        b_p = padded(b, (b.shape[0], hout_p))
-        c_p = c.new_empty((experts, hin_p, hout_p))   # every element is written
-        backend.gmm(a_p, b_p, c_p, batch_sizes, True, False)
-        c.copy_(c_p[:, :hin, :hout])
+        b_p = _padded(b, b.shape[0], hout_p)
     else:
-        b_p = padded(b, (experts, hout_p, hin_p) if trans_b else (experts, hin_p, hout_p))
-        # rows past sum(batch_sizes) are not written by the kernel and must keep what c holds
-        c_p = padded(c, (c.shape[0], hout_p))
-        backend.gmm(a_p, b_p, c_p, batch_sizes, False, trans_b)
-        if c_p is not c:
-            c.copy_(c_p[:, :hout])
-    return True
+        b_p = _padded(b, hout_p, hin_p) if trans_b else _padded(b, hin_p, hout_p)
+    return _padded_product(a_p, b_p, c, batch_sizes, trans_a, trans_b and not trans_a, hin, hout)
+
+
+def _padded_product(a_p, b_p, c, batch_sizes, trans_a, trans_b, hin, hout):
+    """The product of padded operands as an unpadded tensor: into c, or a new one where c is None."""
+    hin_p, hout_p = a_p.shape[1], b_p.shape[1] if (trans_a or trans_b) else b_p.shape[2]
+    dtype = _output_dtype(a_p.dtype)
+    if trans_a:
+        experts = batch_sizes.shape[0]
+        if c is None:
+            c = torch.empty(experts, hin, hout, dtype=dtype, device=a_p.device)
+        whole = hin == hin_p and hout == hout_p and c.data_ptr() % 16 == 0
+        c_p = c if whole else torch.empty(experts, hin_p, hout_p, dtype=dtype, device=a_p.device)   # all of it is written
+    else:
+        given = c is not None
+        if c is None:
+            c = torch.empty(a_p.shape[0], hout, dtype=dtype, device=a_p.device)
+        # rows past sum(batch_sizes) are not written by the kernel and must keep what a given c holds
+        if given or hout == hout_p:
+            c_p = _padded(c, c.shape[0], hout_p)
+        else:
+            c_p = torch.empty(c.shape[0], hout_p, dtype=dtype, device=a_p.device)
+    backend.gmm(a_p, b_p, c_p, batch_sizes, trans_a, trans_b)
+    if c_p is not c:
+        backend.unpad_rows(c_p, c)
+    return c
+
+
+def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
+    """Both gradients of gmm(a, b, batch_sizes, trans_b=trans_b), each None where it is not wanted."""
+    if want_a and want_b and _needs_padding(grad, b, None, batch_sizes, False, not trans_b) and \
+            a.device == grad.device and a.dtype == grad.dtype and a.is_contiguous() and \
+            tuple(a.shape) == (grad.shape[0], b.shape[2 if trans_b else 1]):
+        # (one padded copy of the gradient serves both products)
+        hin, hout = a.shape[1], grad.shape[1]
+        mult = 16 if a.element_size() == 1 else 8
+        hin_p, hout_p = _round_up(hin, mult), _round_up(hout, mult)
+        grad_p = _padded(grad, grad.shape[0], hout_p)
+        b_p = _padded(b, hout_p, hin_p) if trans_b else _padded(b, hin_p, hout_p)
+        agrad = _padded_product(grad_p, b_p, None, batch_sizes, False, not trans_b, hout, hin)
+        del b_p
+        a_p = _padded(a, a.shape[0], hin_p)
+        if trans_b:
+            return agrad, _padded_product(grad_p, a_p, None, batch_sizes, True, False, hout, hin)
+        return agrad, _padded_product(a_p, grad_p, None, batch_sizes, True, False, hin, hout)
+    agrad = gmm(grad, b, batch_sizes, trans_a=False, trans_b=not trans_b) if want_a else None
+    bgrad = None
+    if want_b:
+        lhs, rhs = (grad, a) if trans_b else (a, grad)
+        bgrad = gmm(lhs, rhs, batch_sizes, trans_a=True, trans_b=False)
+    return agrad, bgrad
 
 
 def gmm(a, b, batch_sizes, trans_a=False, trans_b=False, c=None):
@@ -110,9 +167,11 @@ def gmm(a, b, batch_sizes, trans_a=False, trans_b=False, c=None):
     if out is not None:
         return out
     if c is None:
+        _check_ranks(a, b, batch_sizes, trans_a, trans_b)
+    if _needs_padding(a, b, c, batch_sizes, trans_a, trans_b):
+        return _padded_call(a, b, c, batch_sizes, trans_a, trans_b)
+    if c is None:
         c = _allocate_output(a, b, batch_sizes, trans_a, trans_b)
-    if _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
-        return c
     backend.gmm(a, b, c, batch_sizes, trans_a, trans_b)
     return c
 

@@ -640,6 +640,41 @@ int gg_sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t ro
   return GG_OK;
 }
 
+static int check_repitch(const void* src, const void* dst, int64_t batches, int64_t small_rows, int64_t small_cols,
+                         int64_t large_rows, int64_t large_cols, int elem_bytes) {
+  if (batches < 0 || small_rows < 0 || small_cols < 0) return fail(GG_EINVAL, "negative dimension");
+  if (large_rows < small_rows || large_cols < small_cols) return fail(GG_EINVAL, "the padded tensor must be the larger one");
+  if (large_cols >= (int64_t(1) << 23) || large_rows >= (int64_t(1) << 31) ||
+      (large_rows > 0 && batches >= (int64_t(1) << 32) / large_rows))
+    return fail(GG_ELIMIT, "rows must be below 2^31, all batches' below 2^32, columns below 2^23");
+  if (elem_bytes != 1 && elem_bytes != 2) return fail(GG_EINVAL, "elements of 1 or 2 bytes");
+  if (src == nullptr || dst == nullptr) return fail(GG_EINVAL, "src or dst is null");
+  return GG_OK;
+}
+
+int gg_pad_rows(const void* src, void* dst, int64_t batches, int64_t src_rows, int64_t src_cols, int64_t dst_rows,
+                int64_t dst_cols, int elem_bytes, void* stream) {
+  const int rc = check_repitch(src, dst, batches, src_rows, src_cols, dst_rows, dst_cols, elem_bytes);
+  if (rc != GG_OK) return rc;
+  if ((dst_cols * elem_bytes) % 16 != 0 || (reinterpret_cast<uintptr_t>(dst) & 15))
+    return fail(GG_ELIMIT, "dst must have rows of whole 16-byte chunks, on a 16-byte boundary");
+  if (reinterpret_cast<uintptr_t>(src) & (uintptr_t)(elem_bytes - 1)) return fail(GG_ELIMIT, "src must be aligned to its elements");
+  if (batches == 0 || dst_rows == 0 || dst_cols == 0) return GG_OK;
+  GG_HIP(gg::pad_rows(src, dst, batches, src_rows, src_cols, dst_rows, dst_cols, elem_bytes, static_cast<hipStream_t>(stream)));
+  return GG_OK;
+}
+
+int gg_unpad_rows(const void* src, void* dst, int64_t batches, int64_t src_rows, int64_t src_cols, int64_t dst_rows,
+                  int64_t dst_cols, void* stream) {
+  const int rc = check_repitch(src, dst, batches, dst_rows, dst_cols, src_rows, src_cols, 2);
+  if (rc != GG_OK) return rc;
+  if ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 1)
+    return fail(GG_ELIMIT, "src and dst must be aligned to their elements");
+  if (batches == 0 || dst_rows == 0 || dst_cols == 0) return GG_OK;
+  GG_HIP(gg::unpad_rows(src, dst, batches, src_rows, src_cols, dst_rows, dst_cols, static_cast<hipStream_t>(stream)));
+  return GG_OK;
+}
+
 int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device, int64_t num_groups,
                       int64_t tokens, int64_t hidden_in, int64_t hidden_out, int trans_a,
                       int trans_b, int64_t* table_out, void* stream_) {

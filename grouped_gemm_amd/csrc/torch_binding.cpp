@@ -361,6 +361,35 @@ torch::Tensor SumRows(torch::Tensor src, torch::Tensor row_index, int64_t num_ds
   return out;
 }
 
+// t (batch, rows, cols) or (rows, cols), zero-padded to `rows` x `cols` per batch; see gg_pad_rows.
+torch::Tensor PadRows(torch::Tensor t, int64_t rows, int64_t cols) {
+  TORCH_CHECK(t.is_cuda() && t.is_contiguous() && (t.dim() == 2 || t.dim() == 3) && t.element_size() <= 2,
+              "grouped_gemm: pad_rows needs a contiguous 2-d or 3-d GPU tensor of 1 or 2 byte elements");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(t.device());
+  const int64_t batches = t.dim() == 3 ? t.size(0) : 1;
+  torch::Tensor out = t.dim() == 3 ? torch::empty({batches, rows, cols}, t.options()) : torch::empty({rows, cols}, t.options());
+  if (out.numel() == 0) return out;
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+  const int rc = gg_pad_rows(t.data_ptr(), out.data_ptr(), batches, t.size(-2), t.size(-1), rows, cols, (int)t.element_size(),
+                             static_cast<void*>(stream));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+  return out;
+}
+
+// c = the upper left corner of every batch of t; see gg_unpad_rows.
+void UnpadRows(torch::Tensor t, torch::Tensor c) {
+  TORCH_CHECK(t.is_cuda() && c.is_cuda() && t.device() == c.device() && t.is_contiguous() && c.is_contiguous() &&
+                  t.dim() == c.dim() && (t.dim() == 2 || (t.dim() == 3 && t.size(0) == c.size(0))) &&
+                  t.scalar_type() == c.scalar_type() && t.element_size() == 2,
+              "grouped_gemm: unpad_rows needs two contiguous GPU tensors of the same two-byte type, 2-d or of as many batches");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(t.device());
+  if (c.numel() == 0) return;
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
+  const int rc = gg_unpad_rows(t.data_ptr(), c.data_ptr(), t.dim() == 3 ? t.size(0) : 1, t.size(-2), t.size(-1), c.size(-2),
+                               c.size(-1), static_cast<void*>(stream));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+}
+
 // c (num_experts, hidden_in, hidden_out) fp32 += per expert a_e^T @ b_e; see gg_gmm_bf16_acc_f32.
 void AccumulateWeightGradient(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes) {
   TORCH_CHECK(c.scalar_type() == torch::kFloat32, "grouped_gemm: the accumulated gradient must be float32");
@@ -424,6 +453,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("c_rows") = py::none());
   m.def("swiglu_backward", &SwiGLUBackward, "Gradients of gate | up from the gradient of silu(gate) * up.");
   m.def("sum_rows", &SumRows, "Row d of the result is the sum of the rows of src that row_index sends there.");
+  m.def("pad_rows", &PadRows, "A zero-padded copy with `rows` rows of `cols` elements per batch.");
+  m.def("unpad_rows", &UnpadRows, "The second tensor = the upper left corner of every batch of the first.");
   m.def("size_status", &SizeStatus,
         "Bits collected since the last call: 1 a device-resident batch size was negative, 2 they summed past the "
         "rows of a (both clamped by the kernel).");

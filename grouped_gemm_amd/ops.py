@@ -22,16 +22,8 @@ class GroupedGemm(torch.autograd.Function):
     def backward(ctx, grad):
         grad = grad.contiguous()
         a, b, batch_sizes = ctx.saved_tensors
-        trans_b = ctx.trans_b
-
-        agrad = None
-        if ctx.needs_input_grad[0]:
-            agrad = backend.gmm(grad, b, batch_sizes, trans_a=False, trans_b=not trans_b)
-
-        bgrad = None
-        if ctx.needs_input_grad[1]:
-            lhs, rhs = (grad, a) if trans_b else (a, grad)
-            bgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True, trans_b=False)
+        agrad, bgrad = backend.gradients(grad, a, b, batch_sizes, ctx.trans_b, ctx.needs_input_grad[0],
+                                         ctx.needs_input_grad[1])
         return agrad, bgrad, None, None
 
 

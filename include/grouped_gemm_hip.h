@@ -272,6 +272,22 @@ int gg_sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t ro
                 int64_t cols, int dtype, void* scratch, void* stream);
 
 /*
+ * Operands whose rows the streaming kernels cannot take (hidden sizes that are not multiples of 8,
+ * or addresses off the 16-byte boundary) laid out again: dst (batches, dst_rows, dst_cols) gets src
+ * (batches, src_rows, src_cols) in the upper left corner of every batch and zeros elsewhere.
+ * Elements of elem_bytes (1 or 2), both tensors dense, dst on a 16-byte boundary with rows of whole
+ * 16-byte chunks, dst_rows >= src_rows and dst_cols >= src_cols.
+ * gg_unpad_rows is the way back: dst (batches, dst_rows, dst_cols) gets the upper left corner of
+ * every batch of src (batches, src_rows, src_cols); elements of two bytes, dst_rows <= src_rows and
+ * dst_cols <= src_cols.
+ * No counterpart in the reference, whose cuBLAS path takes any size (csrc/grouped_gemm.cu:373-394).
+ */
+int gg_pad_rows(const void* src, void* dst, int64_t batches, int64_t src_rows, int64_t src_cols,
+                int64_t dst_rows, int64_t dst_cols, int elem_bytes, void* stream);
+int gg_unpad_rows(const void* src, void* dst, int64_t batches, int64_t src_rows, int64_t src_cols,
+                  int64_t dst_rows, int64_t dst_cols, void* stream);
+
+/*
  * Runs only the on-device scheduler of gg_gmm_bf16 (same device code, same
  * arguments) and writes what it derived to `table_out`, a device buffer of
  * num_groups * GG_SCHED_COLS int64: per group the problem (m, n, k), leading

@@ -1585,6 +1585,53 @@ def test_sum_rows_kernel(ops, dtype, rows, destinations, cols):
         assert torch.equal(out, ops.backend.backend.sum_rows(src, index.cuda(), destinations))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("batches,rows,cols,shift", [(1, 1, 1, 0), (3, 5, 7, 1), (2, 9, 33, 3), (4, 30, 257, 5), (1, 700, 4093, 2),
+                                                     (5, 16, 64, 1), (8, 401, 1365, 0)])
+def test_pad_and_unpad_rows(ops, dtype, batches, rows, cols, shift):
+    # copies, so the same bytes: every offset of a row from the 4-byte boundaries, rows shorter than
+    # one 16-byte chunk, chunks of the dense side that hold several row boundaries, padded rows, and
+    # both sides off the 16-byte boundary by `shift` elements
+    mult = 16 if dtype == torch.float8_e4m3fn else 8
+    rows_p, cols_p = (rows + 7) // 8 * 8, (cols + mult - 1) // mult * mult
+    _announce("pad", dtype, batches, rows, cols, shift)
+    raw = {1: torch.uint8, 2: torch.int16}[dtype.itemsize]
+    g = torch.Generator().manual_seed(rows + cols)
+    values = torch.randint(0, 127, (batches * rows * cols + shift,), generator=g).to(raw)
+    dense = values.cuda()[shift:].view(dtype).view(batches, rows, cols)
+    padded = ops.backend.backend.pad_rows(dense, rows_p, cols_p)
+    want = torch.zeros(batches, rows_p, cols_p, dtype=raw)
+    want[:, :rows, :cols] = values[shift:].view(batches, rows, cols)
+    assert torch.equal(padded.view(raw).cpu(), want)
+    if dtype != torch.bfloat16:
+        return
+    around = torch.full((batches * rows * cols + shift + 9,), 21, dtype=raw).cuda()
+    back = around[shift:shift + batches * rows * cols].view(dtype).view(batches, rows, cols)
+    ops.backend.backend.unpad_rows(padded, back)
+    assert torch.equal(back.view(raw).cpu(), values[shift:].view(batches, rows, cols))
+    assert bool((around[:shift] == 21).all()) and bool((around[shift + batches * rows * cols:] == 21).all())
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("hin,hout", [(65, 131), (264, 77), (51, 264), (30, 45)])
+def test_odd_sizes_forward_and_gradients(ops, oracle, hin, hout, trans_b):
+    # both gradients share one padded copy of theirs; one of the sizes, or both, not a multiple of 8
+    _announce("odd gradients", hin, hout, trans_b)
+    sizes = torch.tensor([70, 0, 300, 3])
+    g = torch.Generator().manual_seed(hin + hout)
+    a = torch.randn(int(sizes.sum()), hin, generator=g).to(torch.bfloat16)
+    b = torch.randn(4, *((hout, hin) if trans_b else (hin, hout)), generator=g).to(torch.bfloat16)
+    grad = torch.randn(a.shape[0], hout, generator=g).to(torch.bfloat16)
+    da, db = a.cuda().requires_grad_(True), b.cuda().requires_grad_(True)
+    out = ops.gmm(da, db, sizes.cuda(), trans_b)
+    out.backward(grad.cuda())
+    for got, want, what in zip((out.detach(), da.grad, db.grad), oracle.gmm_autograd_loop(a, b, sizes, trans_b, grad),
+                               ("out", "agrad", "bgrad")):
+        check(got, want, what)
+    only_b = torch.autograd.grad(ops.gmm(da.detach(), db, sizes.cuda(), trans_b), db, grad.cuda())[0]
+    assert torch.equal(only_b, db.grad)
+
+
 # ------------------------------------------------------------------ SwiGLU epilogue
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
