@@ -1303,8 +1303,19 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   using BFrag = std::conditional_t<Cfg::B_DEPTH_MAJOR, DepthMajorFrag<BK, 1, F8>,
                                    std::conditional_t<F8, WidthMajorFrag8<BN, NB, 1>, WidthMajorFrag<BN, BK, NB, 1>>>;
   constexpr int LOADS_PER_STAGE = ALoad::NI + BLoad::NI;   // per lane, per depth slice
-  // (a slice's loads go out in four parts, one per step: loads Q1, Q2 and Q3 begin parts 2, 3 and 4)
-  constexpr int Q1 = LOADS_PER_STAGE / 4, Q2 = LOADS_PER_STAGE / 2, Q3 = LOADS_PER_STAGE * 3 / 4;
+  // A slice's loads go out in three parts, in steps 1, 2 and 3, or in four, in steps 1 to 3 and step 0
+  // of the slice after: loads T1, T2 and T3 begin parts 2, 3 and 4.  With three parts all loads of the
+  // next tile's first two slices precede the stores of a tile, and the first wait of the next tile lets
+  // those stores pass (counters go down in the order of issue); with a part of the loads behind the
+  // stores it waits for the memory to take the whole tile.  That pays where tiles are shallow and
+  // where the launch is bound by memory: weight gradients, 256 groups x 256 rows, 2048 x 7168: 2555 ->
+  // 2502 us, 64 x 768, 2048 x 1408: 294 -> 280; two rows each of 256 groups, 7168 -> 2048 (short
+  // tiles): 1039 -> 1016.  Full tiles of deep products run 0.3 % (bf16) to 1.3 % (fp8) faster with
+  // the steadier four parts (8 x 4096 rows, 4096 -> 14336).
+  constexpr bool THREE_PARTS = LAYOUT == kTN || BM < 256;
+  constexpr int T1 = THREE_PARTS ? LOADS_PER_STAGE / 3 : LOADS_PER_STAGE / 4;
+  constexpr int T2 = THREE_PARTS ? LOADS_PER_STAGE * 2 / 3 : LOADS_PER_STAGE / 2;
+  constexpr int T3 = THREE_PARTS ? LOADS_PER_STAGE : LOADS_PER_STAGE * 3 / 4;
   static_assert(KS == 4 && STAGES == 2, "the step schedule below is written for BK = 64 and two buffers");
   static_assert(LOADS_PER_STAGE >= 4 && LOADS_PER_STAGE < 32, "");
   constexpr int UNITS = MB + NB;    // fragments of one 16-deep step
@@ -1454,22 +1465,20 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   using I2 = std::integral_constant<int, 2>;
   using I3 = std::integral_constant<int, 3>;
   using IMB = std::integral_constant<int, MB>;
-  using IQ1 = std::integral_constant<int, Q1>;
-  using IQ2 = std::integral_constant<int, Q2>;
-  using IQ3 = std::integral_constant<int, Q3>;
-  using ILast = std::integral_constant<int, LOADS_PER_STAGE - Q3>;   // loads of the fourth part, and so on
-  using IThird = std::integral_constant<int, Q3 - Q2>;
-  using ISecond = std::integral_constant<int, Q2 - Q1>;
+  using IT1 = std::integral_constant<int, T1>;
+  using IT2 = std::integral_constant<int, T2>;
+  using ISecond = std::integral_constant<int, T2 - T1>;   // loads of the second part
+  using IThird = std::integral_constant<int, T3 - T2>;
+  using IT3 = std::integral_constant<int, T3>;
+  using ILast = std::integral_constant<int, LOADS_PER_STAGE - T3>;
 
-  // Both buffers are requested up front, except the last quarter of the second slice: every
-  // step issues one quarter of a slice's loads, and step 0 issues the last quarter of the
-  // slice that was begun in the steps before it.
+  // Both buffers are requested up front, except what step 0 issues.
   fetch_setup();
   fetch_begin();
   static_for<LOADS_PER_STAGE>([&](auto j) { fetch_load(j, 0); });
   fetch_advance();
   fetch_begin();
-  static_for<Q3>([&](auto j) { fetch_load(j, 1); });
+  static_for<T3>([&](auto j) { fetch_load(j, 1); });
 
   int tile_t = vid;
   int tile_n = 0;   // tiles this workgroup has finished
@@ -1500,7 +1509,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
       block_barrier();
     }
   };
-  wait_vmcnt<Q3>();   // the first slice is in
+  wait_vmcnt<T3>();   // the first slice is in
   block_barrier();
   if (RAGGED_DEPTH && tail_slice == 0) clear_tail(0);
   static_for<2 * UNITS>([&](auto u) {
@@ -1551,6 +1560,12 @@ gmm_kernel(GmmParams p, HostSizes hs) {
     return round4<OUT_DT>(o[0], o[1], o[2], o[3]);
   };
 
+  // Row blocks this wave has stored of the tile before (0: none, or all of it has arrived), and the
+  // store instructions of one (at least; more of them only make the wait that counts them stricter).
+  int stored = 0;
+  constexpr int STORES = ACC_F32 ? 8 : (GATE_UP ? Cfg::WTN / 32 : (Cfg::STAGED_EPILOGUE ? NB / 2 * 4 : NB * 4));
+  static_assert(T2 + STORES * MB < 64, "vmcnt is a 6-bit field");
+
   // One tile, for a wave that has ML row blocks with rows in them (the tile's row blocks go to
   // the wave rows alternately).  One copy of this body exists per value of ML; a tile picks
   // its copy once, so no accumulator ever lives across a choice.
@@ -1560,9 +1575,9 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   //   step 1  barrier: X goes to the fetch cursor, which starts the slice two ahead into it
   //   step 3  barrier: Y is complete for every wave; reads the fragments of the next slice's
   //           steps 0 and 1 from Y (all MB of A's: the next slice may be the next tile's)
-  // Every step issues a quarter of a slice's loads (step 0 the last quarter of the slice begun
-  // in steps 1-3 before it), so the memory pipe sees a steady trickle, and X is released two
-  // steps before Y is needed, so loads stay in flight across the hand-over.
+  // Steps 1 to 3 (and 0) each issue a part of a slice's loads, so the memory pipe sees a steady
+  // trickle, and X is released two steps before Y is needed, so loads stay in flight across the
+  // hand-over.
   auto tile_body = [&](auto ml_tag) {
     constexpr int ML = decltype(ml_tag)::value;
     constexpr int SLOTS = ML * NB;    // MFMAs per 16-deep step
@@ -1615,19 +1630,26 @@ gmm_kernel(GmmParams p, HostSizes hs) {
 
     for (int kt = 0; kt < ti.nk; ++kt) {
       const int y = uniform(x ^ 1);   // (the same in every lane: keeps the LDS addresses scalar)
-      step(I0{}, I2{}, ml_tag, I2{}, IQ3{}, ILast{}, x, y);
+      step(I0{}, I2{}, ml_tag, I2{}, IT3{}, ILast{}, x, y);
       fetch_advance();
       // every wave has all fragments of this slice in registers
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       block_barrier();
       fetch_begin();
-      step(I1{}, I0{}, ml_tag, I0{}, I0{}, IQ1{}, x, x);
-      step(I2{}, I0{}, ml_tag, I0{}, IQ1{}, ISecond{}, x, x);
-      // the next slice has landed for every wave (only this slice's two quarters may be pending)
-      wait_vmcnt<Q2>();
+      step(I1{}, I0{}, ml_tag, I0{}, I0{}, IT1{}, x, x);
+      step(I2{}, I0{}, ml_tag, I0{}, IT1{}, ISecond{}, x, x);
+      // the next slice has landed for every wave (only the two parts just issued may be pending and,
+      // THREE_PARTS, in a tile's first slice the stores of the tile before)
+      if (THREE_PARTS && kt == 0 && uniform(stored) == MB) {
+        wait_vmcnt<T2 + STORES * MB>();
+      } else if (THREE_PARTS && kt == 0 && uniform(stored) > 0) {
+        wait_vmcnt<T2 + STORES>();
+      } else {
+        wait_vmcnt<T2>();
+      }
       block_barrier();
       if (RAGGED_DEPTH && uniform(kt + 1 == ti.nk ? 0 : kt + 1) == tail_slice) clear_tail(y);
-      step(I3{}, I2{}, IMB{}, I0{}, IQ2{}, IThird{}, y, x);
+      step(I3{}, I2{}, IMB{}, I0{}, IT2{}, IThird{}, y, x);
       x = uniform(y);
     }
 
@@ -1646,6 +1668,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), mine, partial_at(i, j, q), 0, kDeviceScope);
           }
       wait_vmcnt<0>();   // every wave's part has arrived before the arrival is counted
+      stored = 0;
       block_barrier();
       if (threadIdx.x == 0) sched->arrived = __hip_atomic_fetch_add(reinterpret_cast<int*>(p.workspace) + ti.rank, 1, __ATOMIC_RELAXED,
                                                                         __HIP_MEMORY_SCOPE_AGENT);
@@ -1804,6 +1827,30 @@ gmm_kernel(GmmParams p, HostSizes hs) {
         // an even width that is not a multiple of 8: rows of c then start on 4-byte boundaries
         // only, and the last 16-byte chunk of a row holds 2, 4 or 6 columns
         const bool ragged_width = uniform(ti.g.n & 7) != 0;
+        // One strip behind: the reads of a strip return while the next one is converted (the LDS
+        // serves a wave in order, so the next strip's writes need not wait for them).
+        u32x4 held[4];
+        uint32_t held_off[4];
+        int held_col = 0;
+        auto store_held = [&]() {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const u32x4 v = held[r];
+            // (whole chunks only: for widths that are multiples of 8 the same as col < n)
+            __builtin_amdgcn_raw_buffer_store_b128(v, rc, held_col + 8 <= ti.g.n ? at(held_off[r], held_col) : OOR, 0,
+                                                   kStoreStreaming);
+            if (ragged_width) {
+              const int valid = ti.g.n - held_col;   // columns of this lane's chunk that exist
+              const uint32_t off = at(held_off[r], held_col);
+              if (valid > 0 && valid < 8 && off != OOR) {
+                if (valid & 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, rc, off, 0, kStoreStreaming);
+                if (valid & 2)
+                  __builtin_amdgcn_raw_buffer_store_b32((valid & 4) ? v[2] : v[0], rc, off + ((valid & 4) ? 8u : 0u), 0,
+                                                        kStoreStreaming);
+              }
+            }
+          }
+        };
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
           uint32_t row_off[4];
@@ -1817,31 +1864,19 @@ gmm_kernel(GmmParams p, HostSizes hs) {
               for (int q = 0; q < 4; ++q)
                 *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jj * 32 + 8 * q + 4 * in_half) * 2) =
                     take4(i, 2 * jp + jj, q);
+            if (i + jp > 0) store_held();
+            held_col = ti.n0 + wn * Cfg::WTN + jp * 64 + out_chunk * 8;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const u32x4 v = *reinterpret_cast<const u32x4*>(strip + (r * 8 + out_row) * PITCH + out_chunk * 16);
-              const int col = ti.n0 + wn * Cfg::WTN + jp * 64 + out_chunk * 8;
-              // (whole chunks only: for widths that are multiples of 8 the same as col < n)
-              __builtin_amdgcn_raw_buffer_store_b128(v, rc, col + 8 <= ti.g.n ? at(row_off[r], col) : OOR, 0,
-                                                     kStoreStreaming);
-              {
-                if (ragged_width) {
-                  const int valid = ti.g.n - col;   // columns of this lane's chunk that exist
-                  const uint32_t off = at(row_off[r], col);
-                  if (valid > 0 && valid < 8 && off != OOR) {
-                    if (valid & 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, rc, off, 0, kStoreStreaming);
-                    if (valid & 2)
-                      __builtin_amdgcn_raw_buffer_store_b32((valid & 4) ? v[2] : v[0], rc, off + ((valid & 4) ? 8u : 0u), 0,
-                                                            kStoreStreaming);
-                  }
-                }
-              }
+              held[r] = *reinterpret_cast<const u32x4*>(strip + (r * 8 + out_row) * PITCH + out_chunk * 16);
+              held_off[r] = row_off[r];
             }
             // keep the conversion of one strip from being hoisted over the stores of the
             // previous one: few accumulators are live in vector registers at a time
             __builtin_amdgcn_sched_barrier(0);
           }
         }
+        store_held();
       } else {
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
@@ -1857,6 +1892,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
           }
         }
       }
+      stored = ML;
     }
   };
 
