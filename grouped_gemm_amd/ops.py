@@ -92,13 +92,16 @@ class GroupedGemmScatter(torch.autograd.Function):
         grad = grad.contiguous()
         a, w, batch_sizes, row_index = ctx.saved_tensors
         agrad = wgrad = None
-        if ctx.needs_input_grad[0]:
-            agrad = backend.gmm_indexed(grad, w, batch_sizes, trans_b=not ctx.trans_b, a_rows=row_index)
         if ctx.needs_input_grad[1]:
-            # (as in GroupedGemmGather: an explicit gather, then the streaming weight-gradient kernel)
+            # (as in GroupedGemmGather: an explicit gather, then the streaming weight-gradient kernel;
+            # the input gradient takes the sorted rows too where they are there)
             sorted_grad = grad.index_select(0, row_index)
             lhs, rhs = (sorted_grad, a) if ctx.trans_b else (a, sorted_grad)
             wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
+            if ctx.needs_input_grad[0]:
+                agrad = backend.gmm(sorted_grad, w, batch_sizes, trans_b=not ctx.trans_b)
+        elif ctx.needs_input_grad[0]:
+            agrad = backend.gmm_indexed(grad, w, batch_sizes, trans_b=not ctx.trans_b, a_rows=row_index)
         return agrad, wgrad, None, None, None
 
 
