@@ -275,13 +275,14 @@ constexpr TileShape shape_of() {
   return TileShape{S::kId, S::BM, S::BN};
 }
 
-// Tiles of a call in a shape: those of groups of average size, which is what device-resident sizes
-// can be judged by.
-int64_t average_tiles(const gg_gmm_args& g, int bm, int bn) {
+// Tiles of a call in a shape, as far as that can be told without the sizes, which may be on the
+// device only.  Groups are ragged: each has on average half a tile row more than its rows fill (groups of
+// 64 rows on average are as often 65 and more, two rows of 64 x 128 tiles, as 64 and fewer).
+int64_t expected_tiles(const gg_gmm_args& g, int bm, int bn) {
   const int64_t tiles_n = (g.hidden_out + bn - 1) / bn;
   if (g.trans_a) return g.num_groups * ((g.hidden_in + bm - 1) / bm) * tiles_n;
-  const int64_t rows = (g.tokens + g.num_groups - 1) / g.num_groups;
-  return g.num_groups * ((rows + bm - 1) / bm) * tiles_n;
+  const int64_t tile_rows = (2 * g.tokens / bm + g.num_groups) / 2;
+  return (tile_rows > g.num_groups ? tile_rows : g.num_groups) * tiles_n;
 }
 
 // Workgroups of a full launch of one workgroup per compute unit, for the rules below.
@@ -297,35 +298,38 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 
 // The tile shape of a streaming call.
 //
-// Small tiles where one round of them (two workgroups per compute unit; one for weight gradients)
-// holds the whole launch: the launch is then bound by how long one tile takes, and by how many
-// compute units pull data.  Us per launch, bf16, wide / short / small, NN layout: 8 groups x 128
-// rows, 128 -> 128: 9.6 / 8.5 / 7.4; 16 x 256, 1024 -> 1024 (512 small tiles): 20.1 / 18.5 / 17.9;
-// 20 x 168, 5592 -> 232: 60 / 53 / 29.5; past that line the small ones lose: 8 x 1024,
-// 128 -> 1024 (1024 small tiles) 12.0 / 11.1 / 11.8, 8 x 2048, 1024 -> 1024: 35.6 / 37.9 / 49.5.
+// Small tiles where two of three compute units would have at most one of them and the others two
+// (one for weight gradients, and for deep products, whose tiles suffer most from sharing): such a
+// launch is bound by how long one tile takes, and by how many compute units pull data.  Short tiles where
+// one round of them holds the launch, where groups average few rows (use_short_shape), and where few
+// rows of deep products leave nothing to do but pull weights, for which their larger buffers are
+// better than small tiles' (8 x 16, 14336 -> 4096, 128 short tiles in two depth pieces each: 152 us, 256
+// small ones: 172 us).  Us per launch, bf16, NN layout, row counts drawn at random around the average,
+// wide / short / small, and the expected number of small and of short tiles: 29 x 238 rows, 280 -> 152
+// (244, 68): 11.8 / 10.6 / 9.5; 4 x 512, 512 -> 1024 (272, 72): 13.0 / 12.2 / 11.6; 8 x 700, 512 -> 512 (364, 94):
+// 13.4 / 12.5 / 11.9; 16 x 200, 3072 -> 768 (348, 99): 38.3 / 32.8 / 35.3; 32 x 128, 2048 -> 768 (480, 144): 30.4 /
+// 29.8 / 32.7; 16 x 256, 2048 -> 1024 (576, 160): 31.2 / 30.8 / 38.8; 64 x 64, 1024 -> 1024 (768, 256): 28.1 / 26.8 /
+// 42.2; 32 x 250, 1024 -> 1024 (1256, 312): 30.2 / 32.6 / 42.3; 32 x 128, 768 -> 2048 (1280, 384): 24.3 / 29.9 / 36.9.
 // Weight gradients, wide / small: 8 x 512, 256 x 256: 18.2 / 10.8; 8 x 1024, 128 x 1024 (64 tiles):
-// 26.5 / 17.8; 16 x 256, 1024 x 1024 (1024 tiles): 18.0 / 20.8.
-// Groups of kDeepGroups rows and more keep the wide ones: where a few of them are much deeper than
-// the rest, those are cut along the depth (plan_deep_tiles).
-// Short tiles where groups average few rows (use_short_shape), where one round of them holds the
-// launch (8 x 1024, 128 -> 1024, 256 of them, above), and where few rows of deep products leave
-// nothing to do but pull weights, for which their larger buffers are better (8 x 16, 14336 -> 4096,
-// 128 short tiles in two depth pieces each: 152 us, 256 small ones: 172 us).
+// 26.5 / 17.8; 16 x 256, 1024 x 1024 (1024 tiles): 18.0 / 20.8.  Groups of kDeepGroups rows and more keep the
+// wide ones: where a few of them are much deeper than the rest, those are cut along the depth
+// (plan_deep_tiles).
 constexpr int64_t kDeepGroups = 2560;
-constexpr int64_t kDeepProduct = 6144;
+constexpr int64_t kDeepProduct = 6144;       // weights are pulled through short tiles
+constexpr int64_t kDeepForSharing = 3072;    // small tiles one to a compute unit
 
 TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   if (r.ragged_depth) return shape_of<WideRaggedDepth>();
   const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
   if (g.trans_a) {
     const bool small = has_shape(g, r, SmallSquare::kId) && g.tokens < kDeepGroups * g.num_groups &&
-                       average_tiles(g, SmallSquare::BM, SmallSquare::BN) <= kFullLaunch;
+                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <= kFullLaunch;
     return small ? shape_of<SmallSquare>() : shape_of<Wide>();
   }
-  const int64_t short_tiles = average_tiles(g, Short::BM, Short::BN / halves);
+  const int64_t short_tiles = expected_tiles(g, Short::BM, Short::BN / halves);
   const bool streams_weights = g.tokens <= Small::BM * g.num_groups && g.hidden_in >= kDeepProduct && 2 * short_tiles >= kFullLaunch;
-  if (has_shape(g, r, Small::kId) && !streams_weights &&
-      average_tiles(g, Small::BM, Small::BN / halves) <= 2 * kFullLaunch)
+  const int64_t most_small = g.hidden_in >= kDeepForSharing ? kFullLaunch : kFullLaunch * 3 / 2;
+  if (has_shape(g, r, Small::kId) && !streams_weights && expected_tiles(g, Small::BM, Small::BN / halves) <= most_small)
     return shape_of<Small>();
   if (has_shape(g, r, Short::kId) && (use_short_shape(g.num_groups, g.tokens, 0) ||
                                       short_tiles <= kFullLaunch))
