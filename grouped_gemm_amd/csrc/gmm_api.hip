@@ -298,9 +298,9 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 
 // The tile shape of a streaming call.
 //
-// Small tiles where two of three compute units would have at most one of them and the others two
-// (one for weight gradients, and for deep products, whose tiles suffer most from sharing): such a
-// launch is bound by how long one tile takes, and by how many compute units pull data.  Short tiles where
+// NN and NT layouts: small tiles up to one and a half of them per compute unit (one for deep
+// products, whose tiles suffer most from sharing): such a launch is bound by how long one tile takes,
+// and by how many compute units pull data.  Short tiles where
 // one round of them holds the launch, where groups average few rows (use_short_shape), and where few
 // rows of deep products leave nothing to do but pull weights, for which their larger buffers are
 // better than small tiles' (8 x 16, 14336 -> 4096, 128 short tiles in two depth pieces each: 152 us, 256
@@ -310,10 +310,13 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 13.4 / 12.5 / 11.9; 16 x 200, 3072 -> 768 (348, 99): 38.3 / 32.8 / 35.3; 32 x 128, 2048 -> 768 (480, 144): 30.4 /
 // 29.8 / 32.7; 16 x 256, 2048 -> 1024 (576, 160): 31.2 / 30.8 / 38.8; 64 x 64, 1024 -> 1024 (768, 256): 28.1 / 26.8 /
 // 42.2; 32 x 250, 1024 -> 1024 (1256, 312): 30.2 / 32.6 / 42.3; 32 x 128, 768 -> 2048 (1280, 384): 24.3 / 29.9 / 36.9.
-// Weight gradients, wide / small: 8 x 512, 256 x 256: 18.2 / 10.8; 8 x 1024, 128 x 1024 (64 tiles):
-// 26.5 / 17.8; 16 x 256, 1024 x 1024 (1024 tiles): 18.0 / 20.8.  Groups of kDeepGroups rows and more keep the
-// wide ones: where a few of them are much deeper than the rest, those are cut along the depth
-// (plan_deep_tiles).
+// Weight gradients: small tiles up to two rounds of them.  Wide / small, groups of even and of Zipf (0.8)
+// depths: 8 x 512 rows, 512 x 1024 (256 small tiles): 19.4 / 12.4 and 30.8 / 17.3; 16 x 512, 768 x 640 (480): 19.4 /
+// 18.1 and 39.0 / 24.9; 16 x 1024, 512 x 1024 (512): 28.3 / 25.2 and 70.7 / 40.6 (the deepest group's tiles set the
+// length of the launch: four times as many take a quarter of the time each); past that line even
+// depths lose: 64 x 256, 256 x 768 (768): 18.3 / 20.0; 16 x 256, 1024 x 1024 (1024): 19.7 / 22.6.  Groups of
+// kDeepGroups rows and more keep the wide ones: where a few of them are much deeper than the rest,
+// those are cut along the depth (plan_deep_tiles).
 constexpr int64_t kDeepGroups = 2560;
 constexpr int64_t kDeepProduct = 6144;       // weights are pulled through short tiles
 constexpr int64_t kDeepForSharing = 3072;    // small tiles one to a compute unit
@@ -323,7 +326,7 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
   if (g.trans_a) {
     const bool small = has_shape(g, r, SmallSquare::kId) && g.tokens < kDeepGroups * g.num_groups &&
-                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <= kFullLaunch;
+                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <= 2 * kFullLaunch;
     return small ? shape_of<SmallSquare>() : shape_of<Wide>();
   }
   const int64_t short_tiles = expected_tiles(g, Short::BM, Short::BN / halves);

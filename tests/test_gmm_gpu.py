@@ -556,9 +556,10 @@ def test_every_tile_shape_with_every_epilogue(ops, oracle, case, trans_b, dtype)
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sizes,hin,hout", [([300, 0, 17, 195], 136, 264), ([1], 8, 8), ([2000, 1500], 128, 128),
-                                            ([129] * 40, 264, 136)])
+                                            ([129] * 40, 264, 136), ([40] * 30 + [0, 1100], 304, 520)])
 def test_small_tiles_of_a_weight_gradient(ops, oracle, dtype, sizes, hin, hout):
-    # 128 x 128 tiles: ragged edges, an empty group, one slice, a group deep enough for depth pieces;
+    # 128 x 128 tiles: ragged edges, an empty group, one slice, a group deep enough for depth pieces, two
+    # rounds with one group much deeper than the rest;
     # stored and added to fp32
     _announce("small weight gradient", dtype, sizes if len(sizes) < 9 else len(sizes), hin, hout)
     g = torch.Generator().manual_seed(29)
