@@ -1309,8 +1309,8 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   // those stores pass (counters go down in the order of issue); with a part of the loads behind the
   // stores it waits for the memory to take the whole tile.  That pays where tiles are shallow and
   // where the launch is bound by memory: weight gradients, 256 groups x 256 rows, 2048 x 7168: 2555 ->
-  // 2502 us, 64 x 768, 2048 x 1408: 294 -> 280; two rows each of 256 groups, 7168 -> 2048 (short
-  // tiles): 1039 -> 1016.  Full tiles of deep products run 0.3 % (bf16) to 1.3 % (fp8) faster with
+  // 2502 us, 64 x 768, 2048 x 1408: 290 -> 280; two rows each of 256 groups, 7168 -> 2048 (short
+  // tiles): 0 to 3 % by the box.  Full tiles of deep products run 0.3 % (bf16) to 1.3 % (fp8) faster with
   // the steadier four parts (8 x 4096 rows, 4096 -> 14336).
   constexpr bool THREE_PARTS = LAYOUT == kTN || BM < 256;
   constexpr int T1 = THREE_PARTS ? LOADS_PER_STAGE / 3 : LOADS_PER_STAGE / 4;
