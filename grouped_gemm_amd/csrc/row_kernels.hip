@@ -82,8 +82,9 @@ struct RowSumScratch {
   int32_t* list_next;   // [rows] 1 + next row of the same list, 0: none
 };
 
-__global__ __launch_bounds__(kRowThreads) void clear_words_kernel(int32_t* words, uint32_t n) {
-  for (uint32_t i = blockIdx.x * kRowThreads + threadIdx.x; i < n; i += gridDim.x * kRowThreads) words[i] = 0;
+// (64-bit numbers: two words per destination may be close to 2^32, past which a step would wrap around)
+__global__ __launch_bounds__(kRowThreads) void clear_words_kernel(int32_t* words, uint64_t n) {
+  for (uint64_t i = blockIdx.x * kRowThreads + threadIdx.x; i < n; i += gridDim.x * kRowThreads) words[i] = 0;
 }
 
 __global__ __launch_bounds__(kRowThreads) void invert_index_kernel(const int32_t* row_index, uint32_t rows,
@@ -238,9 +239,9 @@ __global__ __launch_bounds__(kRowThreads) void unpad_rows_kernel(const T* src, T
   }
 }
 
-uint32_t row_blocks(uint32_t items) {
-  const uint32_t all = (items + kRowThreads - 1) / kRowThreads;
-  return all < kRowBlocks ? all : kRowBlocks;
+uint32_t row_blocks(uint64_t items) {
+  const uint64_t all = (items + kRowThreads - 1) / kRowThreads;
+  return all < kRowBlocks ? (uint32_t)all : kRowBlocks;
 }
 
 template <int DT>
@@ -312,7 +313,7 @@ hipError_t sum_rows(const void* src, const int32_t* row_index, void* dst, int64_
   s.list_head = s.count + destinations;
   s.slots = s.list_head + destinations;
   s.list_next = s.slots + destinations * kInlineRows;
-  const uint32_t words = (uint32_t)(2 * destinations);
+  const uint64_t words = 2 * (uint64_t)destinations;
   hipLaunchKernelGGL(clear_words_kernel, dim3(row_blocks(words)), dim3(kRowThreads), 0, stream, s.count, words);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
