@@ -1762,6 +1762,42 @@ def test_swiglu_autograd(ops, oracle, trans_b):
     assert (w.grad[1] == 0).all()
 
 
+def _nearest_to_a_rounding_boundary(factor):
+    """Per element of `factor` (float64): the float16 number in [1, 2) whose product with it lies nearest to the
+    middle between two float16 numbers (about 2^-23 of it away on average), where an error of a few 2^-25 decides
+    how the product is rounded."""
+    best = torch.ones_like(factor)
+    nearest = torch.full_like(factor, 2.0)
+    for m in range(1024):
+        mantissa = torch.frexp(factor * (1 + m / 1024.0))[0].abs() * 2048     # in [1024, 2048): 11 bits before the point
+        off = (mantissa - mantissa.floor() - 0.5).abs()
+        best = torch.where(off < nearest, torch.full_like(best, 1 + m / 1024.0), best)
+        nearest = torch.minimum(off, nearest)
+    return best.half()
+
+
+@pytest.mark.parametrize("sizes", [[4096] * 8, [40] * 700, [60, 64, 33]])
+def test_swiglu_epilogue_divides_in_full_precision(ops, sizes):
+    # silu(gate) * up of known pre-activations (rows times an identity), `up` chosen so that the product lies as
+    # near to a rounding boundary of float16 as it can: then the share of outputs that are not the correctly
+    # rounded ones measures the epilogue's fp32 error.  It has to be that of the plain formula in fp32 with
+    # a correctly rounded division; the reciprocal alone in its place (one unit in the last place) gives a fifth
+    # more.  Wide, short and small tiles.
+    _announce("swiglu precision", len(sizes))
+    rows, n = sum(sizes), 64
+    g = torch.Generator(device="cuda").manual_seed(31)
+    gate = (torch.randn(rows, n, generator=g, device="cuda") * 2).half()
+    gate = torch.where(gate.abs() < 0.05, torch.full_like(gate, 0.7), gate)   # (results far from subnormal numbers)
+    silu = gate.double() / (1 + torch.exp(-gate.double()))
+    up = _nearest_to_a_rounding_boundary(silu)
+    eye = torch.eye(2 * n, dtype=torch.float16, device="cuda").expand(len(sizes), -1, -1).contiguous()
+    got = ops.backend.gmm_swiglu(torch.cat([gate, up], dim=1), eye, torch.tensor(sizes).cuda())
+    want = (silu * up.double()).half()
+    plain = (gate.float() / (1 + torch.exp2(gate.float() * -1.44269504)) * up.float()).half()
+    wrong, plain_wrong = int((got != want).sum()), int((plain != want).sum())
+    assert wrong <= 1.03 * plain_wrong + 4 * plain_wrong ** 0.5, (wrong, plain_wrong)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,cols,shift", [(1, 1, 0), (5, 3, 0), (257, 2, 0), (33, 100, 0), (300, 257, 0), (64, 264, 0),
                                              (7, 2048, 0), (40, 64, 1), (40, 64, 2), (2100, 2048, 0), (0, 8, 0)])
