@@ -38,7 +38,8 @@ struct Halves {
 // gradient of the product once, writes the gradients of both.  Bound by memory, so one pass and
 // accesses of up to 16 bytes (VEC elements); items are numbered along the rows, so consecutive lanes
 // touch consecutive memory.  16384 rows x 4096 columns, bf16: 113 us, 5.9 TB/s of the 671 MB it has
-// to move; the same formula as thirteen elementwise passes with fp32 intermediates took 1710 us.
+// to move; the same formula as thirteen elementwise passes with fp32 intermediates took 1710 us.  The
+// full exponential: the short one, whose error grows with |gate|, is 1 % faster here, 8 % at 4096 x 1408 (12 us).
 template <int DT, int VEC>
 __global__ __launch_bounds__(kRowThreads) void swiglu_backward_kernel(const uint16_t* gate_up, const uint16_t* grad,
                                                                       uint16_t* out, uint32_t cols, uint32_t items) {
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(kRowThreads) void swiglu_backward_kernel(const uint
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       const float gate = widen<DT>(g.v[e]), up = widen<DT>(u.v[e]), up_grad = widen<DT>(d.v[e]);
-      const float sig = 1.0f / (1.0f + __expf(-gate));
+      const float sig = 1.0f / (1.0f + expf(-gate));
       dg.v[e] = narrow<DT>(up_grad * up * sig * (1.0f + gate * (1.0f - sig)));
       du.v[e] = narrow<DT>(up_grad * gate * sig);
     }

@@ -1826,6 +1826,25 @@ def test_swiglu_backward_kernel(ops, dtype, rows, cols, shift):
     assert bool(((out.double() - want).abs() <= tol).all())
 
 
+def test_swiglu_backward_has_the_full_exponential(ops):
+    # as test_swiglu_epilogue_divides_in_full_precision, for the gradient of `up`: grad * silu(gate) with `grad`
+    # chosen so that the product lies next to a rounding boundary.  The kernel's fp32 error has to be that of
+    # torch.sigmoid; an exponential whose error grows with |gate| rounds a quarter more of them the wrong way.
+    _announce("swiglu backward precision")
+    rows, n = 16384, 64
+    g = torch.Generator(device="cuda").manual_seed(37)
+    gate = (torch.randn(rows, n, generator=g, device="cuda") * 2).half()
+    gate = torch.where(gate.abs() < 0.05, torch.full_like(gate, 0.7), gate)
+    silu = gate.double() / (1 + torch.exp(-gate.double()))
+    grad = _nearest_to_a_rounding_boundary(silu)
+    out = ops.backend.backend.swiglu_backward(torch.cat([gate, torch.ones_like(gate)], dim=1), grad)[:, n:]
+    want = (silu * grad.double()).half()
+    plain = (grad.float() * gate.float() * torch.sigmoid(gate.float())).half()
+    wrong, plain_wrong = int((out != want).sum()), int((plain != want).sum())
+    print("rounded the other way:", wrong, "torch:", plain_wrong, flush=True)
+    assert wrong <= 1.03 * plain_wrong + 4 * plain_wrong ** 0.5, (wrong, plain_wrong)
+
+
 @pytest.mark.parametrize("config", [2, 5])
 def test_fused_rows_and_swiglu_at_benchmark_shapes(ops, oracle, config):
     # the gather-fused load, the scatter-fused store and the SwiGLU epilogue at the row counts and
