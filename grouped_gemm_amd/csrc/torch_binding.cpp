@@ -133,21 +133,45 @@ void Validate(const torch::Tensor& a, const torch::Tensor& b, const torch::Tenso
   }
 }
 
-// Workspace for the depth pieces of a call's last round (see gg_gmm): one per device and stream,
-// allocated and zeroed at the first call there that can use one (gg_workspace_bytes_for) and kept
-// for the life of the process.  Calls on one
-// stream run one after the other, so they can share it; the kernels leave its counters zero.
+bool IsCapturing(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
+// Workspace for the depth pieces of a call's last round (see gg_gmm).
+//
+// Outside a graph capture: one per device and stream, allocated and zeroed at the first call there that can
+// use one (gg_workspace_bytes_for) and kept for the life of the process.  Calls on one stream run one after
+// the other, so they can share it; the kernels leave its counters zero.
+//
+// A captured call runs at every replay, on whatever stream and beside whatever other graphs the program
+// chooses, and what it allocates is the graph's pool's, which graphs may share.  It takes a workspace for
+// itself alone, which its graph's later calls and no others can get again, and clears the counters as a
+// part of the graph (a fill of 4 KiB ahead of the launch).
 torch::Tensor Workspace(const torch::Device& device, hipStream_t stream) {
+  constexpr int64_t kCounterBytes = 4096;   // the arrival counters at its beginning, see gg_gmm_args.workspace
+  const auto bytes = torch::dtype(torch::kUInt8).device(device);
+  if (IsCapturing(stream)) {
+    torch::Tensor ws = torch::empty({(int64_t)GG_WORKSPACE_BYTES}, bytes);
+    ws.narrow(0, 0, kCounterBytes).zero_();
+    return ws;
+  }
   static std::mutex mu;
   static std::map<std::pair<int, hipStream_t>, torch::Tensor> cache;
-  std::lock_guard<std::mutex> lock(mu);
-  auto key = std::make_pair((int)device.index(), stream);
-  auto it = cache.find(key);
-  if (it == cache.end()) {
-    torch::Tensor ws = torch::zeros({(int64_t)GG_WORKSPACE_BYTES}, torch::dtype(torch::kUInt8).device(device));
-    it = cache.emplace(key, ws).first;
+  const auto key = std::make_pair((int)device.index(), stream);
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = cache.find(key);
+    if (it != cache.end()) return it->second;
   }
-  return it->second;
+  // (allocated with the lock released: the allocation may have to wait for another thread)
+  torch::Tensor ws = torch::zeros({(int64_t)GG_WORKSPACE_BYTES}, bytes);
+  std::lock_guard<std::mutex> lock(mu);
+  return cache.emplace(key, ws).first->second;
 }
 
 // One int32 word per device that the kernels OR GG_STATUS_* bits into when device-resident

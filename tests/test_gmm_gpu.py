@@ -1016,6 +1016,82 @@ def test_hip_graph_capture_of_the_first_call_in_a_process():
     assert res.returncode == 0 and "cold capture ok" in res.stdout, res.stdout[-2000:] + res.stderr[-4000:]
 
 
+_SEVERAL_GRAPHS = r"""
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from grouped_gemm import backend
+g = torch.Generator(device="cuda").manual_seed(41)
+def call(sizes, hin, hout, swiglu):
+    a = torch.randn(sum(sizes), hin, generator=g, device="cuda").to(torch.bfloat16)
+    b = (torch.randn(len(sizes), hin, (2 if swiglu else 1) * hout, generator=g, device="cuda") * hin ** -0.5).to(torch.bfloat16)
+    bs = torch.tensor(sizes).cuda()
+    out = torch.zeros(sum(sizes), hout, dtype=torch.bfloat16, device="cuda")
+    return out, (lambda: backend.gmm_swiglu(a, b, bs, c=out)) if swiglu else (lambda: backend.gmm(a, b, bs, c=out))
+# calls whose tiles are all cut along the depth: plain and SwiGLU, short and small tiles
+calls = [call([16, 0, 40, 1, 33, 16, 20, 2], 6400, 4096, False), call([16, 0, 40, 1, 33, 16, 20, 2], 6400, 2048, True),
+         call([20, 0, 70, 1, 33], 4096, 200, False), call([20, 0, 70, 1, 33], 4096, 208, True)]
+torch.cuda.synchronize()
+
+def capture(pool, *fns):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, pool=pool):
+        for fn in fns:
+            fn()
+    return graph
+def temporaries():       # what an earlier graph of the pool leaves in every free block of it at each replay
+    blocks = [torch.full((48 << 20,), 3, dtype=torch.int32, device="cuda") for _ in range(2)]
+    return [b.add_(1) for b in blocks][0][:1].clone()
+
+# the library's first calls that cut tiles are captured: three graphs in one pool (the second with two calls)
+# after one that only has temporaries, then each call in a graph with a pool of its own
+pool = torch.cuda.graph_pool_handle()
+earlier = capture(pool, temporaries)
+shared = [capture(pool, calls[0][1]), capture(pool, calls[1][1], calls[2][1]), capture(pool, calls[3][1])]
+outputs = [[0], [1, 2], [3]]
+own = [capture(None, fn) for _, fn in calls]
+
+want = []
+for out, fn in calls:
+    out.fill_(7.0); fn(); torch.cuda.synchronize(); want.append(out.clone())
+def same(i, what):
+    torch.cuda.synchronize()
+    assert torch.equal(calls[i][0], want[i]), (i, what)
+    calls[i][0].fill_(7.0)
+    torch.cuda.synchronize()
+for order in ([2, 1, 0], [1, 1, 2], [0, 2, 1, 0]):   # the last one captured is replayed first
+    for n in order:
+        for replays in (1, 2):
+            for i in outputs[n]:
+                calls[i][0].fill_(7.0)
+            earlier.replay()
+            for _ in range(replays):
+                shared[n].replay()
+            for i in outputs[n]:
+                same(i, ("one pool", order, n))
+        calls[n][1](); same(n, "eager between the replays")
+print("graphs in one pool ok", flush=True)
+streams = [torch.cuda.Stream() for _ in calls]
+for _ in range(10):                                  # all at once, on streams of their own
+    for _ in range(3):
+        for graph, stream in zip(own, streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+    for i in range(len(calls)):
+        same(i, "several streams")
+print("several graphs ok")
+"""
+
+
+def test_hip_graphs_that_share_a_pool_or_run_side_by_side():
+    # Captured calls that cut tiles along the depth bring a workspace per call: replays in any order, after
+    # another graph of the pool has written over its temporaries, beside eager calls and beside each other on
+    # several streams all give the bits of the eager calls.
+    import subprocess
+    import sys
+    res = subprocess.run([sys.executable, "-u", "-c", _SEVERAL_GRAPHS, ROOT], capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0 and "several graphs ok" in res.stdout, res.stdout[-2000:] + res.stderr[-4000:]
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_traceable_operator_under_torch_compile(ops, trans_b):
     # one graph, no breaks (fullgraph), forward and both gradients bit-equal to the autograd
