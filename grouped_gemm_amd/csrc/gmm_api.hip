@@ -127,12 +127,16 @@ static __device__ __align__(256) unsigned char scratch[GG_WORKSPACE_BYTES];
 // Most workgroups a launch may have for the static scratch to hold one partial tile each.
 constexpr int kStaticScratchGrid = (GG_WORKSPACE_BYTES - gg::kWsCounterBytes) / (256 * 256 * 4);
 
+// gg_size_status_word: zero when the library is loaded.
+static __device__ int32_t size_status_word;
+
 __global__ void clear_counters_kernel(int* counters) { counters[threadIdx.x] = 0; }
 
 struct DeviceInfo {
   int cus = 0;
   bool ok = false;
-  unsigned char* scratch = nullptr;   // device address of `scratch` on this device
+  unsigned char* scratch = nullptr;   // device addresses of `scratch` and `size_status_word` on this device
+  int32_t* size_status = nullptr;
 };
 
 // Per device, once: the architecture check and the LDS limit of every kernel variant.
@@ -151,7 +155,10 @@ int device_info(DeviceInfo* out) {
     for (int i = 0; i < kNumVariants; ++i) GG_HIP(kVariantGetters[i]()->prepare());
     void* scratch_address = nullptr;
     GG_HIP(hipGetSymbolAddress(&scratch_address, HIP_SYMBOL(scratch)));
+    void* status_address = nullptr;
+    GG_HIP(hipGetSymbolAddress(&status_address, HIP_SYMBOL(size_status_word)));
     cache[dev].scratch = static_cast<unsigned char*>(scratch_address);
+    cache[dev].size_status = static_cast<int32_t*>(status_address);
     cache[dev].cus = prop.multiProcessorCount;
     cache[dev].ok = true;
   }
@@ -539,6 +546,11 @@ int gg_version(void) { return 200; }
 int gg_init(void) {
   DeviceInfo info;
   return device_info(&info);
+}
+
+int32_t* gg_size_status_word(void) {
+  DeviceInfo info;
+  return device_info(&info) == GG_OK ? info.size_status : nullptr;
 }
 
 int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, int* bm, int* bn,

@@ -174,17 +174,15 @@ torch::Tensor Workspace(const torch::Device& device, hipStream_t stream) {
   return cache.emplace(key, ws).first->second;
 }
 
-// One int32 word per device that the kernels OR GG_STATUS_* bits into when device-resident
-// batch_sizes had to be clamped (negative, or summing past the rows of a): what a host-resident
-// size vector would have been rejected for.  Read (and cleared) through size_status().
-torch::Tensor SizeStatusWord(const torch::Device& device) {
-  static std::mutex mu;
-  static std::map<int, torch::Tensor> cache;
-  std::lock_guard<std::mutex> lock(mu);
-  auto it = cache.find((int)device.index());
-  if (it == cache.end())
-    it = cache.emplace((int)device.index(), torch::zeros({1}, torch::dtype(torch::kInt32).device(device))).first;
-  return it->second;
+// The library's int32 word of the current device that the kernels OR GG_STATUS_* bits into when
+// device-resident batch_sizes had to be clamped (negative, or summing past the rows of a): what a
+// host-resident size vector would have been rejected for.  Read (and cleared) through size_status().
+// (No tensor: one made during a graph capture would lie in that graph's pool, under other graphs' temporaries,
+// and be cleared by its replays.)
+int32_t* SizeStatusWord() {
+  int32_t* word = gg_size_status_word();
+  TORCH_CHECK(word != nullptr, "grouped_gemm: ", gg_last_error());
+  return word;
 }
 
 void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& batch_sizes,
@@ -224,7 +222,7 @@ void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c,
     g.workspace_bytes = (uint64_t)ws.numel();
   }
   g.stream = static_cast<void*>(stream);
-  if (sizes.is_cuda()) g.size_status = SizeStatusWord(a.device()).data_ptr<int32_t>();
+  if (sizes.is_cuda()) g.size_status = SizeStatusWord();
   const int rc = gg_gmm(&g);
   TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
 }
@@ -435,7 +433,7 @@ int64_t SizeStatus(torch::Device device) {
   TORCH_CHECK(device.is_cuda(), "grouped_gemm: size_status is kept per GPU");
   c10::hip::HIPGuardMasqueradingAsCUDA guard(device);
   if (!device.has_index()) device = torch::Device(device.type(), c10::hip::current_device());
-  torch::Tensor word = SizeStatusWord(device);
+  torch::Tensor word = torch::from_blob(SizeStatusWord(), {1}, torch::dtype(torch::kInt32).device(device));
   const int64_t bits = word.item<int32_t>();
   if (bits != 0) word.zero_();
   return bits;

@@ -10,7 +10,7 @@
  *
  * All functions return 0 on success and a negative GG_E* code on failure;
  * gg_last_error() then holds a message for the calling thread
- * (gg_workspace_bytes_for returns a size).  No entry point synchronises the device or
+ * (gg_workspace_bytes_for returns a size, gg_size_status_word an address).  No entry point synchronises the device or
  * allocates device memory.
  */
 #ifndef GROUPED_GEMM_HIP_H_
@@ -69,6 +69,13 @@ extern "C" {
  * device; call this first where that first call must not happen inside a HIP graph capture.
  */
 int gg_init(void);
+
+/*
+ * A device word for gg_gmm_args.size_status that nothing else owns: one int32 per device inside the
+ * library, zero when it is loaded, at the same address until the process ends, so that captured calls and
+ * eager ones can name it.  NULL (and a message) where gg_init fails.  The library never clears it.
+ */
+int32_t* gg_size_status_word(void);
 
 /*
  * Grouped GEMM, bf16 in, fp32 accumulate, bf16 out, alpha = 1, beta = 0.

@@ -2134,6 +2134,46 @@ def test_clamped_device_sizes_are_reported(ops, oracle):
         check(out[:rows], oracle.gmm_loop(a.cpu(), b.cpu(), torch.tensor(used))[:rows], f"clamped {sizes}")
 
 
+_STATUS_UNDER_CAPTURE = r"""
+import sys, torch
+sys.path.insert(0, sys.argv[1])
+from grouped_gemm import backend
+be = backend.backend
+a = torch.randn(100, 64, device="cuda").to(torch.bfloat16)
+b = torch.randn(3, 64, 64, device="cuda").to(torch.bfloat16)
+out = torch.zeros(100, 64, dtype=torch.bfloat16, device="cuda")
+sizes = torch.tensor([30, 30, 40]).cuda()
+too_many = torch.tensor([60, 30, 40]).cuda()
+pool = torch.cuda.graph_pool_handle()
+def capture(fn):
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, pool=pool):
+        fn()
+    return graph
+earlier = capture(lambda: [torch.full((64,), 4, dtype=torch.int32, device="cuda") for _ in range(64)] and None)
+graph = capture(lambda: backend.gmm(a, b, sizes, c=out))      # the library's first call
+earlier.replay()
+assert be.size_status(torch.device("cuda", 0)) == 0, "another graph's temporaries in the word"
+backend.gmm(a, b, too_many)
+graph.replay()
+assert be.size_status(torch.device("cuda", 0)) == be.status_rows_past_end, "a replay cleared the word"
+sizes.copy_(torch.tensor([-1, 30, 40]))
+for _ in range(2):
+    graph.replay()
+    assert be.size_status(torch.device("cuda", 0)) == be.status_negative_size
+assert be.size_status(torch.device("cuda", 0)) == 0
+print("status ok")
+"""
+
+
+def test_size_status_of_captured_calls():
+    # the status word belongs to no graph, also where the library's first call is captured
+    import subprocess
+    import sys
+    res = subprocess.run([sys.executable, "-u", "-c", _STATUS_UNDER_CAPTURE, ROOT], capture_output=True, text=True, timeout=100)
+    assert res.returncode == 0 and "status ok" in res.stdout, res.stdout[-2000:] + res.stderr[-4000:]
+
+
 def test_all_experts_empty(ops):
     a = torch.zeros(0, 64, dtype=torch.bfloat16, device="cuda")
     b = torch.randn(4, 64, 72, device="cuda").to(torch.bfloat16)
