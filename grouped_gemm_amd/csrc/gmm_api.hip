@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -347,6 +348,27 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   return shape_of<Wide>();
 }
 
+// Whether tiles of a call may be cut along the depth: what gg_workspace_bytes_for promises and what a launch is
+// allowed.  Judged as for a crowded device (the sizes, and so the tiles of the last round, may be known on the
+// device only): a call that could be cut only where its last round holds few tiles does without.
+bool may_cut_depth(const gg_gmm_args& g, const Route& r, const TileShape& shape) {
+  // (the fix-up of depth pieces stores 4 columns at a time: whole tiles and row pieces for ragged widths.
+  // Ragged depths: the kernel looks for the ragged chunks in the slice hidden_in / 64 of tiles that start
+  // at depth 0.)
+  if (r.generic || r.ragged_width || r.ragged_depth || g.num_groups <= 0) return false;
+  if (g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ROW_PIECES)) return false;
+  const bool scattered = r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU;
+  if (scattered && shape.id == Wide::kId) return false;
+  const int64_t slice = r.elem_bytes == 1 ? 2 * gg::BK : gg::BK;   // depth elements per slice
+  // (weight-gradient layout: the depth is a group's row count, and one group may hold all rows:
+  // the kernel cuts the tiles of groups much deeper than the rest, plan_deep_tiles)
+  const int64_t depth = g.trans_a ? g.tokens : g.hidden_in;
+  const int slices = (int)std::min<int64_t>((depth + slice - 1) / slice, 1 << 16);
+  if (g.trans_a && slices >= 2 * gg::min_slices_per_piece(shape.bm * shape.bn)) return true;
+  const int rows = g.trans_a || g.tokens >= g.num_groups * shape.bm ? shape.bm : (int)((g.tokens / g.num_groups + 31) / 32 * 32);
+  return gg::best_depth_pieces(slices, rows, shape.bn, kFullLaunch, 2 * kFullLaunch, gg::kMaxDepthPieces) > 1;
+}
+
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
 int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
@@ -442,10 +464,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
                 GG_FLAG_ROW_PIECES == gg::kFlagRowPieces && GG_FLAG_GROUP_ORDER == gg::kFlagGroupOrder,
                 "the header's flags are the kernel's");
   p.flags = g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ONE_CLASS | GG_FLAG_ROW_PIECES | GG_FLAG_GROUP_ORDER);
-  // (ragged widths: the fix-up of depth pieces stores 4 columns at a time; ragged depths: the
-  // kernel looks for the ragged chunks in the slice hidden_in / 64 of tiles that start at depth 0.
-  // Whole tiles and row pieces only, for both.)
-  const bool no_depth_pieces = route.ragged_width || route.ragged_depth;
+  const bool depth_pieces = !generic && may_cut_depth(g, route, shape);
   p.sched_out = nullptr;
   if (static_scratch) {
     if (g.workspace != nullptr)
@@ -457,13 +476,13 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     p.ws_slots = (int32_t)(((uint64_t)GG_WORKSPACE_BYTES - gg::kWsCounterBytes) /
                            ((uint64_t)bm * bn * (swiglu ? 2 : 1) * 4));
     if (p.ws_slots > 1024) p.ws_slots = 1024;
-    if (no_depth_pieces) p.ws_slots = 0;
+    if (!depth_pieces) p.ws_slots = 0;
     // Every call on this device shares the array and finds what the last call left: the arrival
     // counters must start at zero (a fill kernel, not a memset: callers may be capturing a graph).
     hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(gg::kWsCounterBytes / 4), 0, stream,
                        reinterpret_cast<int*>(info.scratch));
     GG_HIP(hipGetLastError());
-  } else if (g.workspace != nullptr && !generic && !no_depth_pieces) {
+  } else if (g.workspace != nullptr && !generic && !route.ragged_width && !route.ragged_depth) {
     if (reinterpret_cast<uintptr_t>(g.workspace) & 255)
       return fail(GG_ELIMIT, "the workspace must be 256-byte aligned");
     const uint64_t slot_bytes = (uint64_t)bm * bn * (swiglu ? 2 : 1) * 4;
@@ -474,7 +493,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     const uint64_t slots = (g.workspace_bytes - gg::kWsCounterBytes) / slot_bytes;
     p.workspace = static_cast<char*>(g.workspace);
     // one arrival counter per tile of the last round: at most grid / 2 of them, 1024 fit
-    p.ws_slots = slots > 1024 ? 1024 : (int32_t)slots;
+    p.ws_slots = !depth_pieces ? 0 : (slots > 1024 ? 1024 : (int32_t)slots);
   }
 
   const int64_t tiles_n = (hidden_out + bn - 1) / bn;
@@ -576,23 +595,7 @@ uint64_t gg_workspace_bytes_for(const gg_gmm_args* args) {
   const gg_gmm_args& g = *args;
   if (g.dtype < GG_DTYPE_BF16 || g.dtype > GG_DTYPE_F8E5M2 || g.hidden_in <= 0 || g.hidden_out <= 0) return 0;
   const Route r = classify(g);
-  // (the fix-up of depth pieces stores 4 columns at a time: whole tiles and row pieces for ragged widths)
-  if (r.generic || r.ragged_width || r.ragged_depth || g.num_groups <= 0) return 0;
-  if (g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ROW_PIECES)) return 0;
-  const TileShape shape = pick_shape(g, r);
-  const int64_t slice = r.elem_bytes == 1 ? 2 * gg::BK : gg::BK;   // depth elements per slice
-  // (weight-gradient layout: the depth is a group's row count, and one group may hold all rows:
-  // the kernel cuts the tiles of groups much deeper than the rest, plan_deep_tiles)
-  const int64_t depth = g.trans_a ? g.tokens : g.hidden_in;
-  const int64_t slices = (depth + slice - 1) / slice;
-  const int rows = g.trans_a || g.tokens >= g.num_groups * shape.bm ? shape.bm : (int)((g.tokens / g.num_groups + 31) / 32 * 32);
-  const bool scattered = r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU;
-  if (scattered && shape.id == Wide::kId) return 0;
-  // (judged as for a crowded device: a call that could be cut only where it has few tiles does without)
-  if (gg::best_depth_pieces((int)slices, rows, shape.bn, kFullLaunch, 2 * kFullLaunch, gg::kMaxDepthPieces) == 1 &&
-      !(g.trans_a && slices >= 2 * gg::min_slices_per_piece(shape.bm * shape.bn)))
-    return 0;
-  return GG_WORKSPACE_BYTES;
+  return !r.generic && may_cut_depth(g, r, pick_shape(g, r)) ? GG_WORKSPACE_BYTES : 0;
 }
 
 int gg_gmm_no_alloc(const gg_gmm_args* args) {

@@ -176,7 +176,8 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *                 epilogue hook (alpha = 1, beta = 0, csrc/grouped_gemm.cu:255).
  *   accumulate_f32  1: c is fp32 and is added to (trans_a = 1 only), as gg_gmm_bf16_acc_f32.
  *   workspace, workspace_bytes
- *                 Device memory the call may use for partial results, or NULL.  When the last
+ *                 Device memory the call may use for partial results, or NULL (not used where
+ *                 gg_workspace_bytes_for returns 0).  When the last
  *                 round of the persistent grid is at most half full, each of its tiles may be cut
  *                 into 2 to 16 pieces along the depth; a piece adds up its depth slices into an
  *                 fp32 partial tile in the workspace, and the piece that finishes last sums the

@@ -862,6 +862,41 @@ def test_c_abi_workspace_sizes(oracle):
     assert lib.gg_gmm(ctypes.byref(args)) == -2 and b"workspace" in lib.gg_last_error()
 
 
+# sizes, hidden_in, hidden_out, trans_a, SwiGLU: calls too shallow for depth pieces as gg_workspace_bytes_for judges them,
+# most of them with a last round of a few tiles, which the cost of a cut alone would let the kernel cut
+_NEVER_CUT = [([16640], 4096, 1024, False, False), ([4200, 4200], 5760, 2048, False, False), ([300, 300], 1280, 256, False, False),
+              ([20] * 4, 1408, 1024, False, False), ([20] * 4, 1408, 512, False, True), ([700, 700], 512, 264, True, False),
+              ([700], 256, 384, True, False)]
+
+
+@pytest.mark.parametrize("case", range(len(_NEVER_CUT)))
+def test_no_workspace_bytes_means_no_depth_pieces(case):
+    # where gg_workspace_bytes_for returns 0, a workspace (of the caller's, or the static scratch of
+    # gg_gmm_no_alloc) changes nothing: no partial tile is written and the bits are those of a call without one
+    sizes, hin, hout, trans_a, swiglu = _NEVER_CUT[case]
+    _announce("never cut", sizes, hin, hout, trans_a, swiglu)
+    lib = _c_abi()
+    lib.gg_gmm_no_alloc.argtypes = [ctypes.c_void_p]
+    lib.gg_workspace_bytes_for.argtypes, lib.gg_workspace_bytes_for.restype = [ctypes.c_void_p], ctypes.c_uint64
+    g = torch.Generator(device="cuda").manual_seed(43 + case)
+    bs = torch.tensor(sizes).cuda()
+    t = sum(sizes)
+    a = torch.randn(t, hin, generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(*((t, hout) if trans_a else (len(sizes), hin, hout * (2 if swiglu else 1))), generator=g, device="cuda").to(torch.bfloat16)
+    ws = torch.zeros(1024 + 256 * 256 * 256, dtype=torch.float32, device="cuda")
+    out = []
+    for entry, workspace in ((lib.gg_gmm, None), (lib.gg_gmm, ws), (lib.gg_gmm_no_alloc, None)):
+        c = torch.full((len(sizes), hin, hout) if trans_a else (t, hout), 7.0, dtype=torch.bfloat16, device="cuda")
+        args = _gmm_args(lib, a, b, c, bs, True, t, hin, hout, trans_a, False, workspace=workspace)
+        args.epilogue = int(swiglu)
+        assert lib.gg_workspace_bytes_for(ctypes.byref(args)) == 0
+        assert entry(ctypes.byref(args)) == 0, lib.gg_last_error()
+        out.append(c)
+    torch.cuda.synchronize()
+    assert not bool(ws.any()), "a partial tile in the workspace"
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False)])
 def test_groups_are_isolated_from_each_other(ops, layout):
     # NaNs in the rows of one group (and in its weights) must show up in that group's output
