@@ -486,7 +486,10 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     if (reinterpret_cast<uintptr_t>(g.workspace) & 255)
       return fail(GG_ELIMIT, "the workspace must be 256-byte aligned");
     const uint64_t slot_bytes = (uint64_t)bm * bn * (swiglu ? 2 : 1) * 4;
-    constexpr uint64_t least = gg::kWsCounterBytes + (uint64_t)Wide::BM * Wide::BN * 4;
+    // (one tile of the wide shape, or of the short one where groups average few rows: what a caller can tell
+    // without the rules of pick_shape, whose tiles are no larger)
+    const bool few_rows = !swiglu && !indexed && elem_bytes == 2 && use_short_shape(num_groups, tokens, trans_a);
+    const uint64_t least = gg::kWsCounterBytes + (few_rows ? (uint64_t)Short::BM * Short::BN : (uint64_t)Wide::BM * Wide::BN) * 4;
     if (g.workspace_bytes < least)
       return fail(GG_ELIMIT, "the workspace holds %llu bytes, the smallest useful one %llu",
                   (unsigned long long)g.workspace_bytes, (unsigned long long)least);

@@ -188,7 +188,9 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *                 round's).  The first 4096 bytes (arrival counters) must be zero
  *                 before the first call and are zero again after every call; the rest needs no
  *                 initialisation.  GG_WORKSPACE_BYTES serves every call; a smaller workspace
- *                 (at least 4096 + one 256 KiB tile) serves fewer pieces; 256-byte aligned.
+ *                 (at least 4096 + one 256 KiB tile; plain calls on two-byte operands whose
+ *                 groups average few rows, see gg_tile_shape: 128 KiB) serves fewer pieces;
+ *                 256-byte aligned.
  *                 Calls that share a workspace must not overlap in time (same stream is enough).
  *   flags         GG_FLAG_* bits.
  */

@@ -862,6 +862,30 @@ def test_c_abi_workspace_sizes(oracle):
     assert lib.gg_gmm(ctypes.byref(args)) == -2 and b"workspace" in lib.gg_last_error()
 
 
+def test_c_abi_smallest_workspace_for_few_rows(oracle):
+    # groups that average few rows: a workspace with room for one 128 x 256 tile is enough, on short tiles (the
+    # first case, cut along the depth) and on small ones; other calls need 256 x 256, and SwiGLU and row indices too
+    lib = _c_abi()
+    for sizes, hin, hout in (([16, 0, 40, 1, 33, 16, 20, 2], 6400, 4096), ([20, 0, 70, 1, 33], 4096, 208)):
+        _announce("smallest workspace", sizes, hin, hout)
+        g = torch.Generator().manual_seed(47)
+        bs, t = torch.tensor(sizes), sum(sizes)
+        a = torch.randn(t, hin, generator=g).to(torch.bfloat16).cuda()
+        b = (torch.randn(len(sizes), hin, hout, generator=g) * hin ** -0.5).to(torch.bfloat16).cuda()
+        want = oracle.gmm_loop(a, b, bs)
+        for nbytes, epilogue, rc in ((4096 + 128 * 1024, 0, 0), (4096 + 128 * 1024 - 256, 0, -2), (4096 + 256 * 1024, 1, 0),
+                                     (4096 + 256 * 1024 - 256, 1, -2)):
+            ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+            c = torch.full((t, hout // (1 + epilogue)), 7.0, dtype=torch.bfloat16, device="cuda")
+            args = _gmm_args(lib, a, b, c, bs.cuda(), True, t, hin, c.shape[1], 0, 0, workspace=ws)
+            args.epilogue = epilogue
+            assert lib.gg_gmm(ctypes.byref(args)) == rc, (nbytes, epilogue, lib.gg_last_error())
+            torch.cuda.synchronize()
+            if rc == 0 and epilogue == 0:
+                check(c, want, f"workspace of {nbytes} bytes")
+            assert not ws[:4096].any()
+
+
 # sizes, hidden_in, hidden_out, trans_a, SwiGLU: calls too shallow for depth pieces as gg_workspace_bytes_for judges them,
 # most of them with a last round of a few tiles, which the cost of a cut alone would let the kernel cut
 _NEVER_CUT = [([16640], 4096, 1024, False, False), ([4200, 4200], 5760, 2048, False, False), ([300, 300], 1280, 256, False, False),
