@@ -67,89 +67,350 @@ __global__ __launch_bounds__(kRowThreads) void swiglu_backward_kernel(const uint
 // Rows that name the same destination, summed: the inverse of a gather.  An index names each
 // destination a few times (top-k routing), in any order, so its inverse is built on the way: per
 // destination a count and kInlineRows slots for the rows that name it, filled with one atomic
-// per row; rows past those (an index may name a row any number of times) hang on a list per
-// destination.  The slots are put in ascending order by whoever sums them, so the sums of up to
-// kInlineRows rows do not depend on timing.
+// per row.  The slots are put in ascending order by whoever sums them, so the sums do not depend on timing.
 //
-// Bound by reading every row once: 49152 rows x 2048 columns onto 8192 destinations (six each), bf16:
-// 51 us, 4.6 TB/s, and 9 us for the two kernels that build the inverse.  Adding the rows to a cleared
-// fp32 tensor atom by atom, with a conversion on either side, took 481 us.
-constexpr int kInlineRows = 8;
+// Bound by reading every row once: 49152 rows x 2048 columns onto 8192 destinations (six each), bf16: 48 us in
+// five launches, 36 of them here (6.5 TB/s); by atomics on a cleared fp32 tensor, with a conversion on
+// either side, 484.  Sixteen rows each, 65536 onto 4096: 68 us.
+//
+// An index may name a row any number of times (padding rows that all name row 0).  Destinations of more
+// rows than slots, the heavy ones, are left to two more kernels, which end at once where there are none
+// (5 us of the 48): one lists their further rows, the other sums them.  65536 rows, 32 and 300 to a
+// destination: 67 and 113 us (by atomics 604 and 587); 4096 of the 49152 rows on one destination: 136 (520), all of them:
+// 394 (1356; as one chain of dependent loads 26000).
+constexpr int kInlineRows = 16;
+constexpr int kWaveRows = 64;       // heavy destinations of up to this many rows are summed by single waves,
+constexpr int kListedRows = 1024;   // ... of up to this many by workgroups that sort the rows in LDS
 
 struct RowSumScratch {
-  int32_t* count;       // [destinations] rows that name it; zero before use
-  int32_t* list_head;   // [destinations] 1 + first row of its list, 0: none; zero before use
-  int32_t* slots;       // [destinations][kInlineRows]
-  int32_t* list_next;   // [rows] 1 + next row of the same list, 0: none
+  int32_t* count;     // [destinations] rows that name it; zero before use
+  int32_t* cursor;    // [kCursorWords] zero before use
+  int32_t* slots;     // [destinations][kInlineRows] the first rows that name it
+  int32_t* base;      // [destinations] heavy ones: where their further rows begin in `rest`
+  int32_t* arrival;   // [rows] how many rows of the same destination were met before the row
+  int32_t* rest;      // [rows] the further rows of heavy destinations, one destination after another
+  int32_t* heavy;     // [2][most_heavy(rows)] heavy destinations: up to kWaveRows rows; up to kListedRows, others from the back
 };
+enum : int { kRestUsed = 0, kHeavyWave = 1, kHeavyListed = 2, kHeavyLong = 3, kCursorWords = 4 };
+__host__ __device__ constexpr int64_t most_heavy(int64_t rows) { return rows / (kInlineRows + 1); }
 
-// (64-bit numbers: two words per destination may be close to 2^32, past which a step would wrap around)
+// (64-bit numbers: the words may be close to 2^32, past which a step would wrap around)
 __global__ __launch_bounds__(kRowThreads) void clear_words_kernel(int32_t* words, uint64_t n) {
   for (uint64_t i = blockIdx.x * kRowThreads + threadIdx.x; i < n; i += gridDim.x * kRowThreads) words[i] = 0;
 }
 
+__device__ __forceinline__ int lanes_below(uint64_t mask) {   // lanes of `mask` ahead of this one
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+}
+
+// Atomics of one wave on one address follow each other at 11 ns: the rows of the destinations that the
+// first lanes name are counted together (all 49152 rows on one destination: 559 -> 11 us), the others one by one.
 __global__ __launch_bounds__(kRowThreads) void invert_index_kernel(const int32_t* row_index, uint32_t rows,
                                                                    uint32_t destinations, RowSumScratch s) {
   for (uint32_t r = blockIdx.x * kRowThreads + threadIdx.x; r < rows; r += gridDim.x * kRowThreads) {
     const uint32_t d = (uint32_t)row_index[r];
-    if (d >= destinations) continue;   // names no row
-    const int at = atomicAdd(&s.count[d], 1);
-    if (at < kInlineRows) {
-      s.slots[(uint64_t)d * kInlineRows + at] = (int32_t)r;
-    } else {
-      s.list_next[r] = atomicExch(&s.list_head[d], (int32_t)r + 1);
+    int at = 0;
+    bool counted = d >= destinations;   // names no row
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+      if (counted) continue;
+      const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);   // of the lanes not counted yet
+      const uint64_t same = __ballot(d == first);
+      if (d == first) {
+        const int before = lanes_below(same);
+        int begin = 0;
+        if (before == 0) begin = atomicAdd(&s.count[d], __popcll(same));
+        at = __builtin_amdgcn_readfirstlane(begin) + before;   // (the lane ahead of all of `same`)
+        counted = true;
+      }
+    }
+    if (!counted) at = atomicAdd(&s.count[d], 1);
+    s.arrival[r] = at;
+    if (d < destinations && at < kInlineRows) s.slots[(uint64_t)d * kInlineRows + at] = (int32_t)r;
+  }
+}
+
+// The VEC columns from `col` on of the up to N rows in `slots`, in ascending order of the rows; eight
+// loads in flight.
+template <int DT, int VEC, int N>
+__device__ __forceinline__ void sum_few_rows(const uint16_t* src, const int32_t* slots, int count, uint32_t cols, uint32_t col,
+                                             float* sum) {
+  using V = Halves<VEC>;
+  constexpr int32_t NONE = 0x7fffffff;
+  constexpr int IN_FLIGHT = 8;
+  int32_t row[N];
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int32_t r = slots[k];   // (not written past the count)
+    row[k] = k < count ? r : NONE;
+  }
+  // odd-even transposition, N rounds
+#pragma unroll
+  for (int round = 0; round < N; ++round)
+#pragma unroll
+    for (int k = round & 1; k + 1 < N; k += 2) {
+      const int32_t lo = min(row[k], row[k + 1]), hi = max(row[k], row[k + 1]);
+      row[k] = lo, row[k + 1] = hi;
+    }
+#pragma unroll
+  for (int at = 0; at < N; at += IN_FLIGHT) {
+    V v[IN_FLIGHT];
+#pragma unroll
+    for (int k = 0; k < IN_FLIGHT; ++k)
+      if (row[at + k] != NONE) v[k] = *reinterpret_cast<const V*>(src + (uint64_t)row[at + k] * cols + col);
+#pragma unroll
+    for (int k = 0; k < IN_FLIGHT; ++k)
+      if (row[at + k] != NONE)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sum[e] += widen<DT>(v[k].v[e]);
+  }
+}
+
+// Enters the heavy ones of the destinations first .. first + number - 1 into the list; one
+// atomic per wave and list, not one per destination.
+__device__ __forceinline__ void list_heavy_destinations(uint32_t first, uint32_t number, uint32_t rows, const RowSumScratch& s) {
+  const uint32_t step = gridDim.x * kRowThreads, lane = threadIdx.x & 63;
+  for (uint32_t wave = blockIdx.x * kRowThreads + (threadIdx.x & ~63u); wave < number; wave += step) {   // (whole waves)
+    const uint32_t d = first + wave + lane;
+    const int count = wave + lane < number ? s.count[d] : 0;
+    if (__ballot(count > kInlineRows) == 0) continue;
+    const int list = count <= kInlineRows ? kRestUsed : (count <= kWaveRows ? kHeavyWave : (count <= kListedRows ? kHeavyListed : kHeavyLong));
+    const int more = count > kInlineRows ? count - kInlineRows : 0;
+    int upto = more;
+#pragma unroll
+    for (int distance = 1; distance < 64; distance <<= 1) {
+      const int o = __shfl_up(upto, distance);
+      if ((int)lane >= distance) upto += o;
+    }
+    int begin = lane == 63 ? atomicAdd(&s.cursor[kRestUsed], upto) : 0;
+    begin = __shfl(begin, 63);
+    if (more > 0) s.base[d] = begin + upto - more;
+#pragma unroll
+    for (int l = kHeavyWave; l <= kHeavyLong; ++l) {
+      const uint64_t mask = __ballot(list == l);
+      if (mask == 0) continue;
+      begin = lane == 0 ? atomicAdd(&s.cursor[l], __popcll(mask)) : 0;
+      const int64_t at = __shfl(begin, 0) + lanes_below(mask), most = most_heavy(rows);
+      if (list == l) s.heavy[l == kHeavyWave ? at : (l == kHeavyListed ? most + at : 2 * most - 1 - at)] = (int32_t)d;
     }
   }
 }
 
 // One item: VEC columns of one destination row, summed in fp32 and rounded once; a destination
-// that no row names gets zeros.  All loads of an item's rows are in flight together.
+// that no row names gets zeros.
 template <int DT, int VEC>
 __global__ __launch_bounds__(kRowThreads) void sum_rows_kernel(const uint16_t* src, uint16_t* dst, uint32_t cols,
-                                                               uint32_t first, uint32_t items, RowSumScratch s) {
-  using V = Halves<VEC>;
-  constexpr int32_t NONE = 0x7fffffff;
+                                                               uint32_t first, uint32_t items, uint32_t rows, RowSumScratch s) {
   const uint32_t per_row = cols / VEC;
+  if (rows > kInlineRows) list_heavy_destinations(first, items / per_row, rows, s);
   for (uint32_t i = blockIdx.x * kRowThreads + threadIdx.x; i < items; i += gridDim.x * kRowThreads) {
     const uint32_t d = first + i / per_row, col = i % per_row * VEC;
     const int count = s.count[d];
-    int32_t row[kInlineRows];
-#pragma unroll
-    for (int k = 0; k < kInlineRows; ++k) {
-      const int32_t r = s.slots[(uint64_t)d * kInlineRows + k];   // (not written past the count)
-      row[k] = k < count ? r : NONE;
-    }
-    // ascending: odd-even transposition, kInlineRows rounds
-#pragma unroll
-    for (int round = 0; round < kInlineRows; ++round)
-#pragma unroll
-      for (int k = round & 1; k + 1 < kInlineRows; k += 2) {
-        const int32_t lo = min(row[k], row[k + 1]), hi = max(row[k], row[k + 1]);
-        row[k] = lo, row[k + 1] = hi;
-      }
-    V v[kInlineRows];
-#pragma unroll
-    for (int k = 0; k < kInlineRows; ++k)
-      if (row[k] != NONE) v[k] = *reinterpret_cast<const V*>(src + (uint64_t)row[k] * cols + col);
+    const int32_t* slots = s.slots + (uint64_t)d * kInlineRows;
     float sum[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) sum[e] = 0.0f;
-#pragma unroll
-    for (int k = 0; k < kInlineRows; ++k)
-      if (row[k] != NONE)
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) sum[e] += widen<DT>(v[k].v[e]);
-    if (count > kInlineRows) {
-      for (int32_t next = s.list_head[d]; next != 0; next = s.list_next[next - 1]) {
-        const V more = *reinterpret_cast<const V*>(src + (uint64_t)(next - 1) * cols + col);
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) sum[e] += widen<DT>(more.v[e]);
-      }
+    if (count <= 8) {
+      sum_few_rows<DT, VEC, 8>(src, slots, count, cols, col, sum);
+    } else if (count <= kInlineRows) {
+      sum_few_rows<DT, VEC, kInlineRows>(src, slots, count, cols, col, sum);
+    } else {
+      continue;
     }
-    V out;
+    Halves<VEC> out;
 #pragma unroll
     for (int e = 0; e < VEC; ++e) out.v[e] = narrow<DT>(sum[e]);
-    *reinterpret_cast<V*>(dst + (uint64_t)d * cols + col) = out;
+    *reinterpret_cast<Halves<VEC>*>(dst + (uint64_t)d * cols + col) = out;
+  }
+}
+
+__global__ __launch_bounds__(kRowThreads) void list_heavy_rows_kernel(const int32_t* row_index, uint32_t rows, RowSumScratch s) {
+  if (s.cursor[kRestUsed] == 0) return;
+  for (uint32_t r = blockIdx.x * kRowThreads + threadIdx.x; r < rows; r += gridDim.x * kRowThreads) {
+    const int at = s.arrival[r];
+    if (at >= kInlineRows) s.rest[s.base[row_index[r]] + at - kInlineRows] = (int32_t)r;
+  }
+}
+
+// The heavy destinations, eight loads in flight per thread.  Which rows a thread adds, and in which order,
+// depends on the index alone.
+//
+// Up to kWaveRows rows: a wave takes 64 column items; each lane holds a row, counts the rows below it and
+// hands it to the lane of that number.
+//
+// More rows: a workgroup takes ITEMS column items, its PARTS groups of ITEMS threads a share of the rows each,
+// and the groups' sums are added up in order at the end.  Up to kListedRows rows are sorted in LDS (a thread
+// counts the rows below its own) and dealt to the groups in turn.  Of more rows, those of a window of the
+// index are marked in a bitmap in LDS, and the groups take its words (rows 32 w .. 32 w + 31) in turn.
+template <int ITEMS>
+struct HeavyTask {
+  static constexpr int PARTS = kRowThreads / ITEMS;
+  uint32_t d, slice, item, part;
+  int count;
+  __device__ __forceinline__ HeavyTask(uint32_t d_, uint32_t slice_, int count_)
+      : d(d_), slice(slice_), item(slice_ * ITEMS + threadIdx.x % ITEMS), part(threadIdx.x / ITEMS), count(count_) {}
+};
+constexpr int kListedItems = 32, kLongItems = 4;
+constexpr uint32_t kWindowWords = 4096, kWindowRows = 32 * kWindowWords;
+
+template <int DT, int VEC>
+struct HeavySum {
+  static constexpr int IN_FLIGHT = 8;
+  using V = Halves<VEC>;
+  const uint16_t* src;
+  uint16_t* dst;
+  uint32_t cols;
+  float sum[VEC];
+
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) sum[e] = 0.0f;
+  }
+  __device__ __forceinline__ void add(const uint32_t* row, int have, uint32_t item) {
+    V v[IN_FLIGHT];
+#pragma unroll
+    for (int k = 0; k < IN_FLIGHT; ++k)
+      if (k < have) v[k] = *reinterpret_cast<const V*>(src + (uint64_t)row[k] * cols + item * VEC);
+#pragma unroll
+    for (int k = 0; k < IN_FLIGHT; ++k)
+      if (k < have)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sum[e] += widen<DT>(v[k].v[e]);
+  }
+  // The groups' sums in order, through `words`; ends with a barrier.
+  template <int ITEMS>
+  __device__ __forceinline__ void finish(const HeavyTask<ITEMS>& t, uint32_t* words) {
+    constexpr int WIDTH = ITEMS * VEC, PARTS = HeavyTask<ITEMS>::PARTS;
+    static_assert(kWindowWords >= PARTS * WIDTH && WIDTH <= kRowThreads, "");
+    float* parts = reinterpret_cast<float*>(words);
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) parts[t.part * WIDTH + tid % ITEMS * VEC + e] = sum[e];
+    __syncthreads();
+    const uint32_t col = t.slice * WIDTH + tid;
+    if (tid < WIDTH && col < cols) {
+      float all = 0.0f;
+#pragma unroll
+      for (int k = 0; k < PARTS; ++k) all += parts[k * WIDTH + tid];
+      dst[(uint64_t)t.d * cols + col] = narrow<DT>(all);
+    }
+    __syncthreads();
+  }
+};
+
+template <int DT, int VEC>
+__global__ __launch_bounds__(kRowThreads, 4) void sum_heavy_rows_kernel(const uint16_t* src, uint16_t* dst, uint32_t cols,
+                                                                        uint32_t rows, RowSumScratch s) {
+  using Sum = HeavySum<DT, VEC>;
+  constexpr int IN_FLIGHT = Sum::IN_FLIGHT;
+  __shared__ __attribute__((aligned(16))) uint32_t words[kWindowWords];
+  static_assert(kWindowWords >= 2 * kListedRows, "");
+  const int tid = threadIdx.x;
+  const uint32_t per_row = cols / VEC;
+  const int64_t most = most_heavy(rows);
+  Sum sum{src, dst, cols};
+  // the rows of destination d, in the order the device met them
+  auto row_at = [&](uint32_t d, int base, int i) -> uint32_t {
+    return i < kInlineRows ? s.slots[(uint64_t)d * kInlineRows + i] : s.rest[base + i - kInlineRows];
+  };
+
+  const uint32_t lane = tid & 63, groups = (per_row + 63) / 64;
+  const uint64_t wave_tasks = (uint64_t)s.cursor[kHeavyWave] * groups;
+  for (uint64_t task = blockIdx.x * (kRowThreads / 64) + tid / 64; task < wave_tasks; task += gridDim.x * (kRowThreads / 64)) {
+    const uint32_t d = s.heavy[task / groups], item = (uint32_t)(task % groups) * 64 + lane;
+    const int count = s.count[d];
+    const int mine = (int)lane < count ? (int)row_at(d, s.base[d], lane) : 0x7fffffff;
+    int below = 0;
+    for (int k = 0; k < count; ++k) below += __shfl(mine, k) < mine ? 1 : 0;
+    const int sorted = __builtin_amdgcn_ds_permute(4 * ((int)lane < count ? below : (int)lane), mine);
+    sum.clear();
+    for (int at = 0; at < count; at += IN_FLIGHT) {
+      uint32_t row[IN_FLIGHT];
+#pragma unroll
+      for (int k = 0; k < IN_FLIGHT; ++k) row[k] = (uint32_t)__shfl(sorted, at + k);   // (past the count: not used)
+      if (item < per_row) sum.add(row, min(IN_FLIGHT, count - at), item);
+    }
+    if (item >= per_row) continue;
+    Halves<VEC> out;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) out.v[e] = narrow<DT>(sum.sum[e]);
+    *reinterpret_cast<Halves<VEC>*>(dst + (uint64_t)d * cols + item * VEC) = out;
+  }
+
+  // (from here on every thread of a workgroup has the same tasks)
+  const uint32_t listed_slices = (per_row + kListedItems - 1) / kListedItems;
+  const uint64_t listed_tasks = (uint64_t)s.cursor[kHeavyListed] * listed_slices;
+  for (uint64_t task = blockIdx.x; task < listed_tasks; task += gridDim.x) {
+    const uint32_t d = s.heavy[most + (int64_t)(task / listed_slices)];
+    const HeavyTask<kListedItems> t(d, (uint32_t)(task % listed_slices), s.count[d]);
+    const int base = s.base[d];
+    uint32_t *listed = words, *sorted = words + kListedRows;
+    for (int i = tid; i < (t.count + 3) / 4 * 4; i += kRowThreads) listed[i] = i < t.count ? row_at(d, base, i) : ~0u;
+    __syncthreads();
+    for (int i = tid; i < t.count; i += kRowThreads) {
+      const uint32_t mine = listed[i];
+      int below = 0;
+      for (int k = 0; k < t.count; k += 4) {
+        const u32x4 other = *reinterpret_cast<const u32x4*>(listed + k);
+        below += (other[0] < mine) + (other[1] < mine) + (other[2] < mine) + (other[3] < mine);
+      }
+      sorted[below] = mine;
+    }
+    __syncthreads();
+    sum.clear();
+    for (int at = t.part; at < t.count && t.item < per_row; at += t.PARTS * IN_FLIGHT) {
+      uint32_t row[IN_FLIGHT];
+      int have = 0;
+#pragma unroll
+      for (int k = 0; k < IN_FLIGHT; ++k)
+        if (at + k * t.PARTS < t.count) row[k] = sorted[at + k * t.PARTS], have = k + 1;
+      sum.add(row, have, t.item);
+    }
+    __syncthreads();   // (the sums go where the rows are)
+    sum.finish(t, words);
+  }
+
+  const uint32_t long_slices = (per_row + kLongItems - 1) / kLongItems;
+  const uint64_t long_tasks = (uint64_t)s.cursor[kHeavyLong] * long_slices;
+  for (uint64_t task = blockIdx.x; task < long_tasks; task += gridDim.x) {
+    const uint32_t d = s.heavy[2 * most - 1 - (int64_t)(task / long_slices)];
+    const HeavyTask<kLongItems> t(d, (uint32_t)(task % long_slices), s.count[d]);
+    const int base = s.base[d];
+    sum.clear();
+    for (uint32_t first = 0; first < rows; first += kWindowRows) {
+      const uint32_t used = min(kWindowWords, (rows - first + 31) / 32);
+      for (uint32_t w = tid; w < used; w += kRowThreads) words[w] = 0;
+      __syncthreads();
+      for (uint32_t i = tid; i < (uint32_t)t.count; i += kRowThreads * IN_FLIGHT) {
+        uint32_t at[IN_FLIGHT];
+#pragma unroll
+        for (int k = 0; k < IN_FLIGHT; ++k)   // (rows ahead of the window, and no rows: far past its end)
+          at[k] = i + k * kRowThreads < (uint32_t)t.count ? row_at(d, base, (int)(i + k * kRowThreads)) - first : ~0u;
+#pragma unroll
+        for (int k = 0; k < IN_FLIGHT; ++k)
+          if (at[k] < kWindowRows) atomicOr(&words[at[k] / 32], 1u << (at[k] % 32));
+      }
+      __syncthreads();
+      uint32_t w = t.part, bits = w < used ? words[w] : 0;
+      while (w < used && t.item < per_row) {
+        uint32_t row[IN_FLIGHT];
+        int have = 0;
+#pragma unroll
+        for (int k = 0; k < IN_FLIGHT; ++k) {
+          while (bits == 0 && w < used) {
+            w += t.PARTS;
+            bits = w < used ? words[w] : 0;
+          }
+          if (bits != 0) {
+            row[k] = first + w * 32 + (__ffs(bits) - 1), have = k + 1;
+            bits &= bits - 1;
+          }
+        }
+        sum.add(row, have, t.item);
+      }
+      __syncthreads();
+    }
+    sum.finish(t, words);
   }
 }
 
@@ -272,27 +533,29 @@ hipError_t launch_swiglu_backward(const uint16_t* gate_up, const uint16_t* grad,
   return hipSuccess;
 }
 
-template <int DT>
-hipError_t launch_sum_rows(const uint16_t* src, uint16_t* dst, int64_t destinations, int64_t cols, int vec,
-                           const RowSumScratch& s, hipStream_t stream) {
-  const int64_t slab = (int64_t(1) << 30) / (cols / vec);
+// Workgroups of the kernel for heavy destinations, at most: four per compute unit.
+constexpr int64_t kHeavyBlocks = 1024;
+
+template <int DT, int VEC>
+hipError_t launch_sum_rows(const uint16_t* src, uint16_t* dst, int64_t rows, int64_t destinations, int64_t cols,
+                           const int32_t* row_index, const RowSumScratch& s, hipStream_t stream) {
+  const int64_t per_row = cols / VEC, slab = (int64_t(1) << 30) / per_row;
   for (int64_t first = 0; first < destinations; first += slab) {
-    const int64_t count = destinations - first < slab ? destinations - first : slab;
-    const uint32_t items = (uint32_t)(count * (cols / vec));
-#define GG_LAUNCH(V)                                                                                              \
-  hipLaunchKernelGGL((sum_rows_kernel<DT, V>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream, src, dst, \
-                     (uint32_t)cols, (uint32_t)first, items, s)
-    switch (vec) {
-      case 8: GG_LAUNCH(8); break;
-      case 4: GG_LAUNCH(4); break;
-      case 2: GG_LAUNCH(2); break;
-      default: GG_LAUNCH(1); break;
-    }
-#undef GG_LAUNCH
+    const uint32_t items = (uint32_t)((destinations - first < slab ? destinations - first : slab) * per_row);
+    hipLaunchKernelGGL((sum_rows_kernel<DT, VEC>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream, src, dst,
+                       (uint32_t)cols, (uint32_t)first, items, (uint32_t)rows, s);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
-  return hipSuccess;
+  if (most_heavy(rows) == 0) return hipSuccess;
+  hipLaunchKernelGGL(list_heavy_rows_kernel, dim3(row_blocks((uint32_t)rows)), dim3(kRowThreads), 0, stream, row_index,
+                     (uint32_t)rows, s);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return err;
+  const int64_t tasks = most_heavy(rows) * ((per_row + kLongItems - 1) / kLongItems);   // no fewer than there can be
+  hipLaunchKernelGGL((sum_heavy_rows_kernel<DT, VEC>), dim3(tasks < kHeavyBlocks ? (uint32_t)tasks : (uint32_t)kHeavyBlocks),
+                     dim3(kRowThreads), 0, stream, src, dst, (uint32_t)cols, (uint32_t)rows, s);
+  return hipGetLastError();
 }
 
 int access_width(uintptr_t bits) {   // elements per access that divide every address and pitch in `bits`
@@ -304,17 +567,20 @@ int access_width(uintptr_t bits) {   // elements per access that divide every ad
 }  // namespace
 
 uint64_t sum_rows_scratch_bytes(int64_t rows, int64_t destinations) {
-  return (uint64_t)(destinations * (2 + kInlineRows) + rows) * sizeof(int32_t);
+  return (uint64_t)(destinations * (2 + kInlineRows) + kCursorWords + 2 * rows + 2 * most_heavy(rows)) * sizeof(int32_t);
 }
 
 hipError_t sum_rows(const void* src, const int32_t* row_index, void* dst, int64_t rows, int64_t destinations,
                     int64_t cols, int dt, void* scratch, hipStream_t stream) {
   RowSumScratch s;
   s.count = static_cast<int32_t*>(scratch);
-  s.list_head = s.count + destinations;
-  s.slots = s.list_head + destinations;
-  s.list_next = s.slots + destinations * kInlineRows;
-  const uint64_t words = 2 * (uint64_t)destinations;
+  s.cursor = s.count + destinations;
+  s.slots = s.cursor + kCursorWords;
+  s.base = s.slots + destinations * kInlineRows;
+  s.arrival = s.base + destinations;
+  s.rest = s.arrival + rows;
+  s.heavy = s.rest + rows;
+  const uint64_t words = (uint64_t)destinations + kCursorWords;
   hipLaunchKernelGGL(clear_words_kernel, dim3(row_blocks(words)), dim3(kRowThreads), 0, stream, s.count, words);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
@@ -325,8 +591,16 @@ hipError_t sum_rows(const void* src, const int32_t* row_index, void* dst, int64_
     if (err != hipSuccess) return err;
   }
   const int vec = access_width(reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst) | (uintptr_t)(2 * cols));
-  auto launch = dt == kBF16 ? &launch_sum_rows<kBF16> : &launch_sum_rows<kF16>;
-  return launch(static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), destinations, cols, vec, s, stream);
+#define GG_LAUNCH(V)                                                                                  \
+  (dt == kBF16 ? &launch_sum_rows<kBF16, V> : &launch_sum_rows<kF16, V>)(                             \
+      static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), rows, destinations, cols, row_index, s, stream)
+  switch (vec) {
+    case 8: return GG_LAUNCH(8);
+    case 4: return GG_LAUNCH(4);
+    case 2: return GG_LAUNCH(2);
+    default: return GG_LAUNCH(1);
+  }
+#undef GG_LAUNCH
 }
 
 hipError_t swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t rows, int64_t cols, int dt,

@@ -272,8 +272,8 @@ int gg_swiglu_backward(const void* gate_up, const void* grad, void* out, int64_t
  * row_index[r] == d, accumulated in fp32 and rounded once; zeros for a row of dst (num_dst, cols)
  * that no index names.  Indices that name no row of dst are ignored.  src and dst contiguous, of
  * element type dtype (GG_DTYPE_BF16 or GG_DTYPE_F16); row_index int32[rows] on the device.
- * Sums of up to 8 rows are added in ascending row order, the same bits on every call; rows past
- * that are added in the order the device meets them.  `scratch`: device memory of
+ * The order of the additions depends on row_index alone (ascending rows for up to 64 of them), so the
+ * bits are the same on every call.  `scratch`: device memory of
  * gg_sum_rows_scratch_bytes(rows, num_dst) bytes, 4-byte aligned, of any contents.
  * No counterpart in the reference, which takes rows already sorted (grouped_gemm/ops.py:8).
  */

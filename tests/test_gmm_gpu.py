@@ -1721,6 +1721,63 @@ def test_sum_rows_kernel(ops, dtype, rows, destinations, cols):
         assert torch.equal(out, ops.backend.backend.sum_rows(src, index.cuda(), destinations))
 
 
+def _index_with_counts(counts, generator):
+    """A shuffled index in which destination d comes counts[d] times."""
+    index = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))
+    return index[torch.randperm(index.numel(), generator=generator)].to(torch.int32)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols", [1, 3, 70, 100, 264])
+@pytest.mark.parametrize("counts", [[8, 9, 16, 17, 0, 64, 65, 1023, 1024, 1025, 1], [0] * 5 + [700] + [3] * 40, [17], [1025],
+                                    [0, 140000, 20, 300], [12] * 900 + [30] * 1500 + [70] * 50, [16] * 5000 + [20] * 5000])
+def test_sum_rows_of_many_rows(ops, dtype, cols, counts):
+    # destinations that many rows name, against float64: the limits of the slots and of the rows sorted in LDS, rows on both sides of a window of the bitmap (131072 rows), more heavy destinations
+    # than workgroups, every access width, with the tolerance of test_sum_rows_kernel; the same bits on every call
+    _announce("sum rows, heavy", dtype, cols, len(counts), max(counts))
+    g = torch.Generator().manual_seed(len(counts) + cols)
+    index = _index_with_counts(counts, g)
+    if index.numel() > 1000:
+        index[5], index[900] = -1, len(counts)
+    src = torch.randn(index.numel(), cols, generator=g).to(dtype)
+    dev, didx = src.cuda(), index.cuda()
+    out = ops.backend.backend.sum_rows(dev, didx, len(counts))
+    ok = (index >= 0) & (index < len(counts))
+    want = torch.zeros(len(counts), cols, dtype=torch.float64).index_add_(0, index[ok].long(), src[ok].double())
+    size = torch.zeros(len(counts), cols, dtype=torch.float64).index_add_(0, index[ok].long(), src[ok].double().abs())
+    most = torch.bincount(index[ok].long(), minlength=len(counts)).double().unsqueeze(1)
+    tol = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * want.abs() + most * 2.0 ** -24 * size + 2.0 ** -25
+    assert bool(((out.double().cpu() - want).abs() <= tol).all())
+    for _ in range(3):
+        assert torch.equal(out, ops.backend.backend.sum_rows(dev, didx, len(counts)))
+
+
+@pytest.mark.parametrize("padding", [0, 4096, 49152])
+def test_sum_rows_time_does_not_follow_the_heaviest_row(ops, padding):
+    # an index whose padding rows all name row 0 (any number of them is allowed) must not turn the sum into one long
+    # chain: no slower than adding the rows to a cleared fp32 tensor by atomics, conversions included
+    _announce("sum rows, time", padding)
+    g = torch.Generator(device="cuda").manual_seed(53)
+    index = torch.arange(49152, device="cuda") % 8192
+    index[:padding] = 0
+    index = index[torch.randperm(49152, generator=g, device="cuda")].to(torch.int32)
+    src = torch.randn(49152, 2048, generator=g, device="cuda").to(torch.bfloat16)
+
+    def median_ms(fn):
+        times = []
+        for n in range(9):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record(); fn(); stop.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(stop))
+        return sorted(times[2:])[3]
+
+    atomics = median_ms(lambda: torch.zeros(8192, 2048, device="cuda").index_add_(0, index, src.float()).to(torch.bfloat16))
+    ours = median_ms(lambda: ops.backend.backend.sum_rows(src, index, 8192))
+    print("ms:", ours, "by atomics:", atomics, flush=True)
+    assert ours <= 1.2 * atomics, (ours, atomics)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("batches,rows,cols,shift", [(1, 1, 1, 0), (3, 5, 7, 1), (2, 9, 33, 3), (4, 30, 257, 5), (1, 700, 4093, 2),
                                                      (5, 16, 64, 1), (8, 401, 1365, 0)])
