@@ -669,9 +669,8 @@ static int check_repitch(const void* src, const void* dst, int64_t batches, int6
                          int64_t large_rows, int64_t large_cols, int elem_bytes) {
   if (batches < 0 || small_rows < 0 || small_cols < 0) return fail(GG_EINVAL, "negative dimension");
   if (large_rows < small_rows || large_cols < small_cols) return fail(GG_EINVAL, "the padded tensor must be the larger one");
-  if (large_cols >= (int64_t(1) << 23) || large_rows >= (int64_t(1) << 31) ||
-      (large_rows > 0 && batches >= (int64_t(1) << 32) / large_rows))
-    return fail(GG_ELIMIT, "rows must be below 2^31, all batches' below 2^32, columns below 2^23");
+  if (large_cols >= (int64_t(1) << 23) || large_rows >= (int64_t(1) << 31))
+    return fail(GG_ELIMIT, "a batch's rows must be below 2^31, columns below 2^23");
   if (elem_bytes != 1 && elem_bytes != 2) return fail(GG_EINVAL, "elements of 1 or 2 bytes");
   if (src == nullptr || dst == nullptr) return fail(GG_EINVAL, "src or dst is null");
   return GG_OK;

@@ -614,18 +614,28 @@ hipError_t swiglu_backward(const void* gate_up, const void* grad, void* out, int
 
 namespace {
 
+// Batches whose rows, `rows` each, are numbered in 32 bits together: what one launch may cover.
+int64_t batches_of_a_launch(int64_t batches, int64_t rows) {
+  const int64_t most = ((int64_t(1) << 32) - 1) / rows;
+  return batches < most ? batches : most;
+}
+
 template <typename T>
 hipError_t launch_pad_rows(const T* src, T* dst, int64_t batches, int64_t src_rows, int64_t src_cols, int64_t dst_rows,
                            int64_t dst_cols, hipStream_t stream) {
-  const int64_t per_row = dst_cols / (16 / (int64_t)sizeof(T)), rows = batches * dst_rows;
+  const int64_t per_row = dst_cols / (16 / (int64_t)sizeof(T)), together = batches_of_a_launch(batches, dst_rows);
   // (32-bit item numbers: larger tensors go in slabs of rows)
   const int64_t slab = (int64_t(1) << 30) / per_row;
-  for (int64_t first = 0; first < rows; first += slab) {
-    const uint32_t items = (uint32_t)((rows - first < slab ? rows - first : slab) * per_row);
-    hipLaunchKernelGGL((pad_rows_kernel<T>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream, src, dst,
-                       (uint32_t)src_rows, (uint32_t)src_cols, (uint32_t)dst_rows, (uint32_t)dst_cols, (uint32_t)first, items);
-    const hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  for (int64_t batch = 0; batch < batches; batch += together) {
+    const int64_t rows = (batches - batch < together ? batches - batch : together) * dst_rows;
+    for (int64_t first = 0; first < rows; first += slab) {
+      const uint32_t items = (uint32_t)((rows - first < slab ? rows - first : slab) * per_row);
+      hipLaunchKernelGGL((pad_rows_kernel<T>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream,
+                         src + batch * src_rows * src_cols, dst + batch * dst_rows * dst_cols, (uint32_t)src_rows,
+                         (uint32_t)src_cols, (uint32_t)dst_rows, (uint32_t)dst_cols, (uint32_t)first, items);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+    }
   }
   return hipSuccess;
 }
@@ -634,18 +644,22 @@ template <typename T>
 hipError_t launch_unpad_rows(const T* src, T* dst, int64_t batches, int64_t src_rows, int64_t src_cols, int64_t dst_rows,
                              int64_t dst_cols, hipStream_t stream) {
   constexpr int64_t VEC = 16 / sizeof(T), SLAB = int64_t(1) << 30;
-  const int64_t total = batches * dst_rows * dst_cols;
-  for (int64_t first = 0; first < total; first += SLAB) {
-    const int64_t count = total - first < SLAB ? total - first : SLAB;
-    const int64_t row = first / dst_cols;
-    T* to = dst + first;
-    const int64_t head = (int64_t)(reinterpret_cast<uintptr_t>(to) % 16 / sizeof(T));
-    const uint32_t items = (uint32_t)((head + count + VEC - 1) / VEC);
-    hipLaunchKernelGGL((unpad_rows_kernel<T>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream, src, to,
-                       (uint32_t)src_rows, (uint32_t)src_cols, (uint32_t)dst_rows, (uint32_t)dst_cols, (uint32_t)row,
-                       (uint32_t)(first - row * dst_cols), (uint32_t)head, (uint32_t)count, items);
-    const hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
+  const int64_t together = batches_of_a_launch(batches, dst_rows);
+  for (int64_t batch = 0; batch < batches; batch += together) {
+    const int64_t total = (batches - batch < together ? batches - batch : together) * dst_rows * dst_cols;
+    for (int64_t first = 0; first < total; first += SLAB) {
+      const int64_t count = total - first < SLAB ? total - first : SLAB;
+      const int64_t row = first / dst_cols;
+      T* to = dst + batch * dst_rows * dst_cols + first;
+      const int64_t head = (int64_t)(reinterpret_cast<uintptr_t>(to) % 16 / sizeof(T));
+      const uint32_t items = (uint32_t)((head + count + VEC - 1) / VEC);
+      hipLaunchKernelGGL((unpad_rows_kernel<T>), dim3(row_blocks(items)), dim3(kRowThreads), 0, stream,
+                         src + batch * src_rows * src_cols, to, (uint32_t)src_rows, (uint32_t)src_cols, (uint32_t)dst_rows,
+                         (uint32_t)dst_cols, (uint32_t)row, (uint32_t)(first - row * dst_cols), (uint32_t)head,
+                         (uint32_t)count, items);
+      const hipError_t err = hipGetLastError();
+      if (err != hipSuccess) return err;
+    }
   }
   return hipSuccess;
 }

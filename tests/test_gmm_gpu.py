@@ -1805,6 +1805,28 @@ def test_pad_and_unpad_rows(ops, dtype, batches, rows, cols, shift):
     assert bool((around[:shift] == 21).all()) and bool((around[shift + batches * rows * cols:] == 21).all())
 
 
+def test_pad_and_unpad_more_than_4g_rows(ops):
+    # 65537 matrices of 65536 rows of one column, as the padded copies of that many experts' weights: row
+    # numbers over all batches do not fit 32 bits (77 GB in all)
+    _announce("pad, more than 2^32 rows")
+    batches, rows = 65537, 65536
+    number = torch.arange(rows, dtype=torch.int16, device="cuda")
+    src = torch.empty(batches, rows, 1, dtype=torch.bfloat16, device="cuda")
+    raw = src.view(torch.int16)
+    torch.add(number.view(1, rows, 1), (torch.arange(batches, device="cuda") * 7).to(torch.int16).view(batches, 1, 1), out=raw)
+    padded = ops.backend.backend.pad_rows(src, rows, 8)
+    for batch in (0, 1, 32768, batches - 2, batches - 1):
+        got = padded[batch].view(torch.int16)
+        assert torch.equal(got[:, :1], raw[batch]) and not bool(got[:, 1:].any()), batch
+    back = torch.zeros_like(src)
+    ops.backend.backend.unpad_rows(padded, back)
+    del padded
+    for batch in range(0, batches, 4096):
+        assert torch.equal(back[batch:batch + 4096].view(torch.int16), raw[batch:batch + 4096]), batch
+    del src, raw, back
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
 @pytest.mark.parametrize("hin,hout", [(65, 131), (264, 77), (51, 264), (30, 45)])
 def test_odd_sizes_forward_and_gradients(ops, oracle, hin, hout, trans_b):
