@@ -585,6 +585,16 @@ int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, 
   return GG_OK;
 }
 
+int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn) {
+  if (args == nullptr || args->struct_bytes != sizeof(gg_gmm_args) || args->num_groups <= 0 || args->hidden_out <= 0)
+    return fail(GG_EINVAL, "args do not describe a call with an output");
+  const Route route = classify(*args);
+  const TileShape shape = route.generic ? TileShape{-1, 0, 0} : pick_shape(*args, route);
+  if (bm) *bm = shape.bm;
+  if (bn) *bn = shape.bn / (args->epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1);
+  return GG_OK;
+}
+
 int gg_gmm(const gg_gmm_args* args) {
   if (args == nullptr) return fail(GG_EINVAL, "args is null");
   if (args->struct_bytes != sizeof(gg_gmm_args))

@@ -236,8 +236,8 @@ void GroupedGemm(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tenso
 }
 
 // Whether a call runs on the streaming kernels as it is: well-formed contiguous operands whose sizes
-// and addresses need no padded copies (the rule of _padded_call in backend.py).  Everything else is
-// left to the Python side, whose checks and error messages then apply.
+// and addresses need no padded copies (of a well-formed call, what _needs_padding in backend.py says no to).
+// Everything else is left to the Python side, whose checks and error messages then apply.
 bool IsDirect(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& batch_sizes, bool trans_a,
               bool trans_b, const torch::Tensor* c) {
   if ((trans_a && trans_b) || batch_sizes.dim() != 1 || a.dim() != 2 || b.dim() != (trans_a ? 2 : 3)) return false;

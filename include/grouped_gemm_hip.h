@@ -320,6 +320,10 @@ int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device,
 int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, int* bm, int* bn,
                   int* bk);
 
+/* Output tile (rows, columns of c) that the call described by `args` runs on, 0 x 0 for the general
+ * kernels; looks at what gg_workspace_bytes_for looks at. */
+int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn);
+
 /* Message of the last failure on the calling thread ("" if none). */
 const char* gg_last_error(void);
 

@@ -457,16 +457,19 @@ def test_deep_groups_of_a_weight_gradient_are_cut_first(oracle):
     # zero.  Against the oracle, against whole tiles (fp32 summation order apart), the same bits
     # on every call, zero-row groups all zero.
     lib = _c_abi()
-    cases = [  # sizes, hidden_in, hidden_out, tiles cut, pieces each
-        ([14000, 300, 200, 0, 150, 6500, 100, 120], 264, 520, 6, 4),   # the group of 6500 rows is too shallow for 4 pieces
-        ([7000, 100, 6800], 136, 264, 4, 2),                           # two deep groups, 2 pieces
-        ([64] * 50 + [20000] + [64] * 50, 256, 256, 1, 4),
-        ([13000, 50, 12800], 1024, 2048, 64, 4),                       # more deep tiles than a round has room for
-        ([6080, 100, 90], 264, 520, 0, 0),                             # 95 slices: too shallow to pay for a fix-up
-        ([7000, 7000, 7000, 7000], 2048, 4096, 0, 0),                  # deep, but no deeper than a workgroup's share
+    cases = [  # sizes, hidden_in, hidden_out, tile side, tiles cut, pieces each (0: none, of the last round's either)
+        ([14000, 300, 200, 0, 150, 6500, 100, 120], 264, 520, 256, 6, 4),   # the group of 6500 rows is too shallow for 4 pieces
+        ([7000, 100, 6800], 136, 264, 256, 4, 2),                           # two deep groups, 2 pieces
+        ([64] * 50 + [20000] + [64] * 50, 256, 256, 128, 4, 4),
+        ([13000, 50, 12800], 1024, 2048, 256, 64, 4),                       # more deep tiles than a round has room for
+        ([6080, 100, 90], 264, 520, 128, 15, 4),                            # 95 slices: deep enough for small tiles,
+        ([6080, 3000, 3000], 2048, 2048, 256, 0, 0),                        # too shallow for wide ones (a last round of 192)
+        ([2100, 100, 90], 264, 520, 128, 15, 2),                            # 33 slices
+        ([1980, 100, 90], 264, 520, 128, 0, 0),                             # 31 slices: too shallow for small tiles
+        ([7000, 7000, 7000, 7000], 2048, 4096, 256, 0, 0),                  # deep, but no deeper than a workgroup's share
     ]
-    slot = 256 * 256
-    for idx, (sizes, hin, hout, cut_tiles, pieces) in enumerate(cases):
+    for idx, (sizes, hin, hout, side, cut_tiles, pieces) in enumerate(cases):
+        slot = side * side
         _announce("deep groups first", sizes if len(sizes) < 10 else len(sizes), hin, hout)
         g = torch.Generator().manual_seed(300 + idx)
         bs = torch.tensor(sizes, dtype=torch.int64)
@@ -475,17 +478,15 @@ def test_deep_groups_of_a_weight_gradient_are_cut_first(oracle):
         b = torch.randn(t, hout, generator=g).to(torch.bfloat16).cuda()
         dbs = bs.cuda() if idx % 2 else bs
         shape = (len(sizes), hin, hout)
-        ws = torch.zeros(1024 + 256 * slot, dtype=torch.float32, device="cuda")
+        ws = torch.zeros(1024 + 256 * 256 * 256, dtype=torch.float32, device="cuda")
         cut = torch.full(shape, 7.0, dtype=torch.bfloat16, device="cuda")
         args = _gmm_args(lib, a, b, cut, dbs, bool(idx % 2), t, hin, hout, True, False, workspace=ws)
         assert lib.gg_gmm(ctypes.byref(args)) == 0, lib.gg_last_error()
         torch.cuda.synchronize()
         assert not bool(ws[:1024].any()), "arrival counters left nonzero"
-        # (a launch with fewer tiles than workgroups may also cut its last round: the deep-group
-        # cut comes instead of that one, so the count below is either the one or the other)
-        used = int((ws[1024:].view(256, slot) != 0).any(dim=1).sum())
-        if cut_tiles:
-            assert used == cut_tiles * pieces, f"case {idx}: {used} partial tiles in the workspace"
+        assert _tile(lib, args) == (side, side)
+        used = int((ws[1024:].view(-1, slot) != 0).any(dim=1).sum())
+        assert used == cut_tiles * pieces, f"case {idx}: {used} partial tiles in the workspace"
         whole = torch.full(shape, 7.0, dtype=torch.bfloat16, device="cuda")
         args = _gmm_args(lib, a, b, whole, dbs, bool(idx % 2), t, hin, hout, True, False, workspace=ws, flags=1)
         assert lib.gg_gmm(ctypes.byref(args)) == 0, lib.gg_last_error()
@@ -508,16 +509,53 @@ def test_deep_groups_of_a_weight_gradient_are_cut_first(oracle):
                 assert not bool(cut[e].any())
 
 
-# Sizes that reach every tile shape, whole and cut along the depth (the rule is pick_shape in
-# gmm_api.hip): sizes, hidden_in, hidden_out.
+# Sizes that reach every tile shape, whole and cut along the depth (the rules are pick_shape in gmm_api.hip and
+# plan_tail in gmm_kernel.hpp): sizes, hidden_in, hidden_out, tile rows and columns, partial tiles of a cut call
+# (tiles times pieces; 0: not cut).  hidden_out is a multiple of 16: half of it, for gate | up, is one of 8.
 _TILE_SHAPES = {
-    "wide": (list(range(1, 520, 11)), 72, 1032),                 # every count of 32-row blocks, partly filled columns
-    "short": ([(7 * e) % 61 for e in range(200)], 136, 776),
-    "short, cut": ([16, 0, 40, 1, 33, 16, 20, 2], 6400, 4096),   # few rows, deep: two pieces
-    "small": ([300, 0, 17, 195, 64, 65], 264, 392),
-    "small, cut": ([20, 0, 70, 1, 33], 4096, 200),               # up to sixteen pieces
-    "small, one slice": ([5, 130], 8, 136),
+    "wide": (list(range(1, 520, 11)), 72, 1040, 256, 256, 0),                 # every count of 32-row blocks, partly filled columns
+    "wide, cut": ([1100, 1000], 6400, 8192, 256, 256, 32 * 4),                # plain calls only
+    "short": ([(7 * e) % 61 for e in range(200)], 136, 784, 128, 256, 0),
+    "short, cut": ([16, 0, 40, 1, 33, 16, 20, 2], 6400, 4096, 128, 256, 7 * 16 * 2),   # few rows, deep
+    "small": ([300, 0, 17, 195, 64, 65], 264, 400, 64, 128, 0),
+    "small, cut": ([20, 0, 70, 1, 33], 4096, 208, 64, 128, 5 * 2 * 8),
+    "small, cut in sixteen": ([20, 0, 1, 33], 6400, 208, 64, 128, 3 * 2 * 16),
+    "small, one slice": ([5, 130], 8, 144, 64, 128, 0),
 }
+# ... and for fp8 with b stored transposed (other layouts run wide tiles only): 128 depth values a slice
+_TILE_SHAPES_F8 = {
+    "wide": (list(range(1, 520, 11)), 144, 1040, 256, 256, 0),
+    "wide, cut": ([1100, 1000], 12800, 8192, 256, 256, 32 * 4),
+    "short": ([(7 * e) % 61 for e in range(200)], 144, 784, 128, 256, 0),
+    "short, cut": ([16, 0, 40, 1, 33, 16, 20, 2], 12800, 4096, 128, 256, 7 * 16 * 2),
+    "small": ([300, 0, 17, 195, 64, 65], 272, 400, 64, 128, 0),
+    "small, cut": ([20, 0, 70, 1, 33], 8192, 208, 64, 128, 5 * 2 * 8),
+}
+
+
+def _tile(lib, args):
+    bm, bn = ctypes.c_int(), ctypes.c_int()
+    lib.gg_debug_tile.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_int)]
+    assert lib.gg_debug_tile(ctypes.byref(args), ctypes.byref(bm), ctypes.byref(bn)) == 0, lib.gg_last_error()
+    return bm.value, bn.value
+
+
+def _check_tiles(a, b, bs, c, tile, partial_tiles, swiglu=False, a_rows=None, c_rows=None, trans_b=False, dtype=0):
+    """The call once more through the C ABI, with a workspace of its own: the tile shape, and the partial
+    tiles it leaves in the workspace, are the ones the case is there for."""
+    lib = _c_abi()
+    ws = torch.zeros(1024 + 256 * 256 * 256, dtype=torch.float32, device="cuda")
+    args = _gmm_args(lib, a, b, c, bs, True, a.shape[0], a.shape[1], c.shape[1], False, trans_b, workspace=ws, dtype=dtype)
+    args.epilogue = int(swiglu)
+    for rows, field, count, tensor in ((a_rows, "a_row_index", "a_num_rows", a), (c_rows, "c_row_index", "c_num_rows", c)):
+        if rows is not None:
+            setattr(args, field, rows.data_ptr())
+            setattr(args, count, tensor.shape[0])
+    assert _tile(lib, args) == (tile[0], tile[1] // (1 + int(swiglu)))
+    assert lib.gg_gmm(ctypes.byref(args)) == 0, lib.gg_last_error()
+    torch.cuda.synchronize()
+    assert int((ws[1024:].view(-1, tile[0] * tile[1]) != 0).any(dim=1).sum()) == partial_tiles
+    assert not bool(ws[:1024].any()), "arrival counters left nonzero"
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -525,15 +563,15 @@ _TILE_SHAPES = {
 @pytest.mark.parametrize("case", list(_TILE_SHAPES))
 def test_every_tile_shape_with_every_epilogue(ops, oracle, case, trans_b, dtype):
     # plain, gathered, scattered, SwiGLU and SwiGLU with both, against the loop in fp32 on the GPU; the
-    # same bits on a second call (the fix-up of depth pieces adds in a fixed order)
-    sizes, hin, hout = _TILE_SHAPES[case]
+    # same bits on a second call (the fix-up of depth pieces adds in a fixed order); tiles and cut as named
+    sizes, hin, hout, bm, bn, partial_tiles = _TILE_SHAPES[case]
     _announce("tile shapes", case, trans_b, dtype)
-    g = torch.Generator().manual_seed(23)
+    g = torch.Generator(device="cuda").manual_seed(23)
     bs = torch.tensor(sizes, dtype=torch.int64)
     t = int(bs.sum())
-    a = torch.randn(t, hin, generator=g).to(dtype).cuda()
-    b = (torch.randn(len(sizes), *((hout, hin) if trans_b else (hin, hout)), generator=g) * hin ** -0.5).to(dtype).cuda()
-    rows = torch.randperm(t, generator=g).to(torch.int32).cuda()
+    a = torch.randn(t, hin, generator=g, device="cuda").to(dtype)
+    b = (torch.randn(len(sizes), *((hout, hin) if trans_b else (hin, hout)), generator=g, device="cuda") * hin ** -0.5).to(dtype)
+    rows = torch.randperm(t, generator=g, device="cuda").to(torch.int32)
     dev = bs.cuda()
     be = ops.backend
     def scattered(fn, width):
@@ -543,15 +581,34 @@ def test_every_tile_shape_with_every_epilogue(ops, oracle, case, trans_b, dtype)
     plain, swiglu = oracle.gmm_loop(a, b, bs, trans_b=trans_b), oracle.swiglu_loop(a, b, bs, trans_b=trans_b)
     gathered = oracle.gmm_loop(a[rows.long()], b, bs, trans_b=trans_b)
     both = oracle.swiglu_loop(a[rows.long()], b, bs, trans_b=trans_b)
-    for what, want, call in (
-            ("plain", plain, lambda: be.gmm(a, b, dev, trans_b=trans_b)),
-            ("gathered", gathered, lambda: be.gmm_indexed(a, b, dev, trans_b=trans_b, a_rows=rows)),
-            ("scattered", plain, lambda: scattered(lambda c: be.gmm_indexed(a, b, dev, trans_b=trans_b, c=c, c_rows=rows), hout)),
-            ("swiglu", swiglu, lambda: be.gmm_swiglu(a, b, dev, trans_b=trans_b)),
-            ("swiglu, both", both, lambda: scattered(lambda c: be.gmm_swiglu(a, b, dev, trans_b=trans_b, c=c, a_rows=rows, c_rows=rows), hout // 2))):
+    for what, want, gate_up, a_rows, c_rows, call in (
+            ("plain", plain, False, None, None, lambda: be.gmm(a, b, dev, trans_b=trans_b)),
+            ("gathered", gathered, False, rows, None, lambda: be.gmm_indexed(a, b, dev, trans_b=trans_b, a_rows=rows)),
+            ("scattered", plain, False, None, rows, lambda: scattered(lambda c: be.gmm_indexed(a, b, dev, trans_b=trans_b, c=c, c_rows=rows), hout)),
+            ("swiglu", swiglu, True, None, None, lambda: be.gmm_swiglu(a, b, dev, trans_b=trans_b)),
+            ("swiglu, both", both, True, rows, rows,
+             lambda: scattered(lambda c: be.gmm_swiglu(a, b, dev, trans_b=trans_b, c=c, a_rows=rows, c_rows=rows), hout // 2))):
         got = call()
         check(got, want, f"{case}, {what}")
         assert torch.equal(got, call()), f"{case}, {what}: not the same bits twice"
+        cut = partial_tiles if what == "plain" or bm < 256 else 0    # (wide tiles that are combined or scattered stay whole)
+        _check_tiles(a, b, dev, torch.empty_like(got), (bm, bn), cut, gate_up, a_rows, c_rows, trans_b, int(dtype == torch.float16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("case", list(_TILE_SHAPES_F8))
+def test_every_tile_shape_float8(ops, oracle, case, dtype):
+    sizes, hin, hout, bm, bn, partial_tiles = _TILE_SHAPES_F8[case]
+    _announce("tile shapes, fp8", case, dtype)
+    g = torch.Generator(device="cuda").manual_seed(59)
+    bs = torch.tensor(sizes, dtype=torch.int64)
+    a = torch.randn(int(bs.sum()), hin, generator=g, device="cuda").to(dtype)
+    b = torch.randn(len(sizes), hout, hin, generator=g, device="cuda").to(dtype)
+    got = ops.backend.gmm(a, b, bs.cuda(), trans_b=True)
+    check(got, oracle.gmm_loop(a, b, bs, trans_b=True), case)
+    assert torch.equal(got, ops.backend.gmm(a, b, bs.cuda(), trans_b=True))
+    _check_tiles(a, b, bs.cuda(), torch.empty_like(got), (bm, bn), partial_tiles, trans_b=True,
+                 dtype=2 if dtype == torch.float8_e4m3fn else 3)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -1698,7 +1755,7 @@ def test_fused_permutation_autograd(ops, oracle, trans_b):
                                                     (64, 200, 264), (0, 3, 8), (5000, 2000, 2048)])
 def test_sum_rows_kernel(ops, dtype, rows, destinations, cols):
     # the gradient of a row gather against float64: every access width, destinations that no row
-    # names (zeros), that up to 8 rows name (the inline slots) and that more name (the lists: 8 rows
+    # names (zeros), that up to 8 and up to 16 rows name (the slots) and that more name (8 rows
     # a destination on average and 300 for one), indices that name no destination, no rows.  fp32
     # additions of n terms err by at most n 2^-24 of the terms' magnitudes, one rounding of the
     # result by 2^-8 (bfloat16) or 2^-11 (float16) of it (2^-25 for subnormal float16 results).
@@ -1803,6 +1860,34 @@ def test_pad_and_unpad_rows(ops, dtype, batches, rows, cols, shift):
     ops.backend.backend.unpad_rows(padded, back)
     assert torch.equal(back.view(raw).cpu(), values[shift:].view(batches, rows, cols))
     assert bool((around[:shift] == 21).all()) and bool((around[shift + batches * rows * cols:] == 21).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False)])
+def test_direct_and_padded_calls_are_told_apart_alike(ops, layout, dtype):
+    # the rule for calls that run as they are is in the extension (gmm_direct), the one for calls that need
+    # padded copies in backend.py: every well-formed call is one or the other, for each size, alignment and given c
+    trans_a, trans_b = layout
+    be = ops.backend
+
+    def operand(shift, *shape, of=dtype):
+        flat = torch.zeros(int(np.prod(shape)) * of.itemsize + shift, dtype=torch.uint8, device="cuda")
+        return flat[shift:].view(of).view(*shape)
+
+    sizes = torch.tensor([3, 0, 6]).cuda()
+    step = dtype.itemsize
+    for hin in (8, 9, 10, 12, 16, 24, 32):
+        for hout in (8, 11, 14, 16, 24, 32):
+            for shifts in ((0, 0, None), (0, 0, 0), (step, 0, 0), (0, step, None), (4, 4, 4), (0, 4, 2), (8, 0, 4), (16, 0, 16)):
+                a = operand(shifts[0], 9, hin)
+                b = operand(shifts[1], *((9, hout) if trans_a else (3, hout, hin) if trans_b else (3, hin, hout)))
+                c = None
+                if shifts[2] is not None:
+                    c = operand(shifts[2], *((3, hin, hout) if trans_a else (9, hout)), of=be._output_dtype(dtype))
+                direct = be.backend.gmm_direct(a, b, sizes, trans_a, trans_b, c) is not None
+                assert direct != be._needs_padding(a, b, c, sizes, trans_a, trans_b), (hin, hout, shifts)
+                if c is None and not trans_a:
+                    assert direct == (be.backend.gmm_autograd(a, b, sizes, trans_b) is not None)
 
 
 def test_pad_and_unpad_more_than_4g_rows(ops):

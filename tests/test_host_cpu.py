@@ -274,6 +274,46 @@ def test_workspace_bytes_for_needs_no_device():
     assert want(dtype=2, hidden_in=12288) == full and want(dtype=2, hidden_in=12160) == 0
 
 
+def test_tile_shapes_need_no_device():
+    """The tile shape each call of the GPU tests of tile shapes runs on, so that a moved threshold cannot leave a
+    shape without a test; and the general kernels, where a half of gate | up is no multiple of 8."""
+    from test_gmm_gpu import _TILE_SHAPES, _TILE_SHAPES_F8
+    lib = ctypes.CDLL(HIP_LIB)
+    lib.gg_debug_tile.argtypes = [ctypes.c_void_p] * 3
+    lib.gg_workspace_bytes_for.argtypes = [ctypes.c_void_p]
+    lib.gg_workspace_bytes_for.restype = ctypes.c_uint64
+
+    def call(sizes, hin, hout, **kw):
+        g, bm, bn = _Args(), ctypes.c_int(-1), ctypes.c_int(-1)
+        g.struct_bytes = ctypes.sizeof(_Args)
+        g.a, g.b, g.c = 4096, 8192, 12288
+        g.num_groups, g.tokens, g.hidden_in, g.hidden_out = len(sizes), sum(sizes), hin, hout
+        for k, v in kw.items():
+            setattr(g, k, v)
+        assert lib.gg_debug_tile(ctypes.byref(g), ctypes.byref(bm), ctypes.byref(bn)) == 0
+        return (bm.value, bn.value), lib.gg_workspace_bytes_for(ctypes.byref(g)) > 0
+
+    for sizes, hin, hout, bm, bn, partial_tiles in _TILE_SHAPES.values():
+        scattered_cut = partial_tiles > 0 and bm < 256
+        for dtype in (0, 1):
+            for trans_b in (0, 1):
+                kw = dict(dtype=dtype, trans_b=trans_b)
+                assert call(sizes, hin, hout, **kw) == ((bm, bn), partial_tiles > 0)
+                assert call(sizes, hin, hout, a_row_index=64, **kw) == ((bm, bn), scattered_cut)
+                assert call(sizes, hin, hout // 2, epilogue=1, **kw) == ((bm, bn // 2), scattered_cut)
+                assert call(sizes, hin, hout // 2, epilogue=1, a_row_index=64, c_row_index=64, **kw) == ((bm, bn // 2), scattered_cut)
+    for sizes, hin, hout, bm, bn, partial_tiles in _TILE_SHAPES_F8.values():
+        for dtype in (2, 3):
+            assert call(sizes, hin, hout, dtype=dtype, trans_b=1) == ((bm, bn), partial_tiles > 0)
+            assert call(sizes, hin, hout, dtype=dtype)[0] == (256, 256)
+    assert call([300, 200], 264, 196, epilogue=1) == ((0, 0), False)
+    # weight gradients: small tiles up to two rounds of them, where groups are not deep
+    assert call([129] * 40, 264, 136, trans_a=1)[0] == (128, 128)
+    assert call([64] * 256, 256, 768, trans_a=1)[0] == (256, 256)
+    assert call([3000] * 4, 256, 256, trans_a=1)[0] == (256, 256)
+    assert lib.gg_debug_tile(None, None, None) == -1
+
+
 def test_row_index_bounds_reach_every_kernel():
     """The C ABI hands the row counts that bound a row index to the general kernels as it does to
     the streaming ones (checked in the sources: no GPU test feeds bad indices on purpose)."""
