@@ -318,6 +318,7 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 13.4 / 12.5 / 11.9; 16 x 200, 3072 -> 768 (348, 99): 38.3 / 32.8 / 35.3; 32 x 128, 2048 -> 768 (480, 144): 30.4 /
 // 29.8 / 32.7; 16 x 256, 2048 -> 1024 (576, 160): 31.2 / 30.8 / 38.8; 64 x 64, 1024 -> 1024 (768, 256): 28.1 / 26.8 /
 // 42.2; 32 x 250, 1024 -> 1024 (1256, 312): 30.2 / 32.6 / 42.3; 32 x 128, 768 -> 2048 (1280, 384): 24.3 / 29.9 / 36.9.
+// (The line of one round of short tiles is not sharp: 5 x 409, 272 -> 3520 (952, 252), b stored transposed: 16.7 / 17.8.)
 // Weight gradients: small tiles up to two rounds of them.  Wide / small, groups of even and of Zipf (0.8)
 // depths: 8 x 512 rows, 512 x 1024 (256 small tiles): 19.4 / 12.4 and 30.8 / 17.3; 16 x 512, 768 x 640 (480): 19.4 /
 // 18.1 and 39.0 / 24.9; 16 x 1024, 512 x 1024 (512): 28.3 / 25.2 and 70.7 / 40.6 (the deepest group's tiles set the

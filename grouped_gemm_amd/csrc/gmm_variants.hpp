@@ -10,11 +10,11 @@ namespace gg {
 
 constexpr int BK = 64, STAGES = 2;
 
-// Tile shapes.  Wide: 256 x 256 outputs per workgroup, 2 x 2 waves of 128 x 128.  Short: 128 x 256,
-// 1 x 4 waves of 128 x 64, for calls whose groups average few rows: with at most 128 rows per
-// group all four waves then share the rows instead of two of them idling (measured 4-7 % faster
-// below about 100 rows per group, slower from 128 on).  The weight-gradient layout always uses the
-// wide shape: its ragged dimension is the depth, not the rows.
+// Tile shapes; which one a call runs on is decided in gmm_api.hip (pick_shape), where both sides of each line are.
+// Wide: 256 x 256 outputs per workgroup, 2 x 2 waves of 128 x 128.  Short: 128 x 256, 1 x 4 waves of 128 x 64, in
+// the layouts with a row of c per token, for calls whose groups average few rows (with at most 128 rows per
+// group all four waves then share the rows instead of two of them idling: 4-7 % faster below about 100 rows per
+// group, slower from 128 on) and for launches that one round of short tiles holds.
 struct Wide {
   static constexpr int kId = 0, BM = 256, BN = 256, WAVES_M = 2, WAVES_N = 2;
   static constexpr bool RAGGED_DEPTH = false;
