@@ -8,6 +8,7 @@
 // torch's current HIP stream.
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <torch/extension.h>
 
 #include <map>
@@ -133,13 +134,28 @@ void Validate(const torch::Tensor& a, const torch::Tensor& b, const torch::Tenso
   }
 }
 
-bool IsCapturing(hipStream_t stream) {
+// Number of the capture that `stream` is in, 0: in none.
+unsigned long long CaptureNumber(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+  unsigned long long number = 0;
+  if (hipStreamGetCaptureInfo(stream, &status, &number) != hipSuccess) {
     (void)hipGetLastError();
-    return false;
+    return 0;
   }
-  return status != hipStreamCaptureStatusNone;
+  return status == hipStreamCaptureStatusNone ? 0 : number;
+}
+
+// Whether a tensor made during a capture belongs to the graph that is captured, i.e. lies in a pool that the
+// allocator keeps for it.  It does in torch's own captures (torch.cuda.graph), not in one that was begun past
+// torch: there the allocator would give the memory to others while the graph still uses it.
+bool BelongsToGraph(const torch::Tensor& t) {
+  namespace allocator = c10::hip::HIPCachingAllocator;
+  if (allocator::get()->name() != "native") return true;   // (the stream-ordered one makes it a node of the graph)
+  const size_t at = reinterpret_cast<size_t>(t.data_ptr());
+  for (const auto& segment : allocator::snapshot().segments)
+    if (at >= segment.address && at - segment.address < segment.total_size)
+      return segment.owner_private_pool_id.first != 0 || segment.owner_private_pool_id.second != 0;
+  return false;
 }
 
 // Workspace for the depth pieces of a call's last round (see gg_gmm).
@@ -151,12 +167,21 @@ bool IsCapturing(hipStream_t stream) {
 // A captured call runs at every replay, on whatever stream and beside whatever other graphs the program
 // chooses, and what it allocates is the graph's pool's, which graphs may share.  It takes a workspace for
 // itself alone, which its graph's later calls and no others can get again, and clears the counters as a
-// part of the graph (a fill of 4 KiB ahead of the launch).
+// part of the graph (a fill of 4 KiB ahead of the launch).  Where the graph cannot own one (BelongsToGraph; asked
+// once per capture and thread) there is none, an undefined tensor: the call keeps its tiles whole.
 torch::Tensor Workspace(const torch::Device& device, hipStream_t stream) {
   constexpr int64_t kCounterBytes = 4096;   // the arrival counters at its beginning, see gg_gmm_args.workspace
   const auto bytes = torch::dtype(torch::kUInt8).device(device);
-  if (IsCapturing(stream)) {
+  if (const unsigned long long capture = CaptureNumber(stream)) {
+    thread_local unsigned long long asked = 0;
+    thread_local bool owned = false;
+    if (asked == capture && !owned) return torch::Tensor();
     torch::Tensor ws = torch::empty({(int64_t)GG_WORKSPACE_BYTES}, bytes);
+    if (asked != capture) {
+      owned = BelongsToGraph(ws);
+      asked = capture;
+      if (!owned) return torch::Tensor();
+    }
     ws.narrow(0, 0, kCounterBytes).zero_();
     return ws;
   }
@@ -216,10 +241,13 @@ void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c,
   g.b_num_rows = trans_a ? (int32_t)b.size(0) : 0;
   g.flags = (int32_t)flags;
   // a workspace only for calls that can cut tiles along the depth (deep products, weight gradients)
+  torch::Tensor workspace;   // (held until the call is enqueued)
   if (gg_workspace_bytes_for(&g) > 0) {
-    torch::Tensor ws = Workspace(a.device(), stream);
-    g.workspace = ws.data_ptr();
-    g.workspace_bytes = (uint64_t)ws.numel();
+    workspace = Workspace(a.device(), stream);
+    if (workspace.defined()) {
+      g.workspace = workspace.data_ptr();
+      g.workspace_bytes = (uint64_t)workspace.numel();
+    }
   }
   g.stream = static_cast<void*>(stream);
   if (sizes.is_cuda()) g.size_status = SizeStatusWord();

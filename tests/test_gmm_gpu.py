@@ -1208,6 +1208,48 @@ def test_hip_graphs_that_share_a_pool_or_run_side_by_side():
     assert res.returncode == 0 and "several graphs ok" in res.stdout, res.stdout[-2000:] + res.stderr[-4000:]
 
 
+def test_capture_begun_past_torch(ops, oracle):
+    # A capture through the HIP runtime alone: torch's allocator keeps nothing for that graph, so a captured call may
+    # not hold on to memory of its (replays would write over whatever tensor got it next).  The call then keeps
+    # its tiles whole; every tensor made after the capture is as it was after the replays.
+    hip = ctypes.CDLL("libamdhip64.so")
+    sizes, hin, hout = [20, 0, 70, 1, 33], 4096, 208
+    _announce("capture past torch", sizes, hin, hout)
+    g = torch.Generator().manual_seed(61)
+    bs, t = torch.tensor(sizes), sum(sizes)
+    a = torch.randn(t, hin, generator=g).to(torch.bfloat16).cuda()
+    b = (torch.randn(len(sizes), hin, hout, generator=g) * hin ** -0.5).to(torch.bfloat16).cuda()
+    dev, c = bs.cuda(), torch.zeros(t, hout, dtype=torch.bfloat16, device="cuda")
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ops.backend.gmm(a, b, dev, c=c)          # (eager: with the stream's own workspace)
+    torch.cuda.synchronize()
+    eager = c.clone()
+    graph, executable = ctypes.c_void_p(), ctypes.c_void_p()
+    relaxed = 2
+    with torch.cuda.stream(stream):
+        handle = ctypes.c_void_p(stream.cuda_stream)
+        assert hip.hipStreamBeginCapture(handle, relaxed) == 0
+        for _ in range(2):
+            ops.backend.gmm(a, b, dev, c=c)
+        assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(executable), graph, None, None, ctypes.c_size_t(0)) == 0
+    after = [torch.full((16 << 20,), 5, dtype=torch.int32, device="cuda") for _ in range(6)]    # 64 MiB each
+    for _ in range(3):
+        c.fill_(7.0)
+        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(executable, handle) == 0
+        torch.cuda.synchronize()
+        check(c, oracle.gmm_loop(a.cpu(), b.cpu(), bs), "replay")
+        assert float((c.float() - eager.float()).abs().max()) <= 2 ** -7 * float(eager.float().abs().max())
+        assert all(bool((x == 5).all()) for x in after), "a replay wrote into another tensor"
+    assert hip.hipGraphExecDestroy(executable) == 0 and hip.hipGraphDestroy(graph) == 0
+    with torch.cuda.stream(stream):
+        ops.backend.gmm(a, b, dev, c=c)
+    torch.cuda.synchronize()
+    assert torch.equal(c, eager)
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_traceable_operator_under_torch_compile(ops, trans_b):
     # one graph, no breaks (fullgraph), forward and both gradients bit-equal to the autograd
