@@ -119,6 +119,20 @@ bool order_by_tile_rows(int64_t num_groups, int64_t tokens, int64_t tiles_n, int
          (tokens / bm + num_groups / 2) * tiles_n >= (int64_t)kByTileRowsRounds * grid;
 }
 
+// Whether the output goes out through L2 (kStoreMerging) instead of past it: where its rows do not start on
+// 64-byte boundaries, so that stores meet inside sectors, and where the launch is bound by them.  Us per launch, past
+// L2 / through it.  Weight gradients always are: 32 x 128 rows, 776 x 1032: 39.9 / 26.9; 64 x 128, 1032 x
+// 2040: 174 / 104; 128 x 4, 2040 x 2040 (1.07 GB): 662 / 278; 8 x 2048, 2040 x 4088: 233 / 229; 32 x 128, 264 x 392: 12.5 / 13.0.
+// Other layouts only if shallow and with many rows to a group, as L2 then does not hold what other tiles share, and
+// what is left in it at the end of a launch is written then: 32 x 2048 rows, 392 -> 520: 72.8 / 61.7; 8 x
+// 1024, 1048 -> 2040: 58.9 / 52.0; 32 x 512, 1000 -> 1000: 52.5 / 50.7; 64 x 128, 1000 -> 2000: 58.7 / 64.6; 8 x 2048, 2040 -> 4088:
+// 254 / 265.  (Rows that do start there: 64 x 128, 1024 x 2048: 70 / 90.)
+constexpr int64_t kShallowProduct = 1536;
+bool merge_stores(const gg_gmm_args& g) {
+  if ((reinterpret_cast<uintptr_t>(g.c) | (uint64_t)g.hidden_out * 2) % 64 == 0 || g.accumulate_f32) return false;
+  return g.trans_a || (g.hidden_in <= kShallowProduct && 2 * g.tokens >= g.hidden_in * g.num_groups);
+}
+
 // Scratch of gg_gmm_no_alloc: the workspace of gg_gmm (arrival counters, then partial tiles) as a
 // static array, one copy per device that loads this library, held until the process ends.  In
 // host code `scratch` is only a handle for hipGetSymbolAddress; kernels get the address that
@@ -465,6 +479,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
                 GG_FLAG_ROW_PIECES == gg::kFlagRowPieces && GG_FLAG_GROUP_ORDER == gg::kFlagGroupOrder,
                 "the header's flags are the kernel's");
   p.flags = g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ONE_CLASS | GG_FLAG_ROW_PIECES | GG_FLAG_GROUP_ORDER);
+  if (merge_stores(g)) p.flags |= gg::kFlagMergeStores;
   const bool depth_pieces = !generic && may_cut_depth(g, route, shape);
   p.sched_out = nullptr;
   if (static_scratch) {

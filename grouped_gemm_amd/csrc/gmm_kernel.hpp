@@ -96,6 +96,7 @@ enum : int {   // debugging switches, for comparing the ways a call can be sched
   kFlagRowPieces = 4,     // ignore the workspace: cut along the rows only
   kFlagGroupOrder = 8,    // NN and NT layouts: never hand out the groups' tiles by tile rows
   kFlagByTileRows = 16,   // set by the host side (never by callers): hand them out by tile rows
+  kFlagMergeStores = 32,  // set by the host side: kStoreMerging instead of kStoreStreaming (merge_stores in gmm_api.hip)
 };
 
 // Workspace layout: kWsCounterBytes of int32 arrival counters (one per tile of the last round; all
@@ -206,6 +207,10 @@ constexpr uint32_t kRsrcFlags = 0x00020000u;   // raw buffer, 32-bit data format
 // Cache policy of the output stores: non-temporal.  The output is written once and never read by
 // this kernel, so it should not push operand lines that other tiles still share out of L2.
 constexpr int kStoreStreaming = 2;
+// ... and write-back, for rows of c that do not start on 64-byte boundaries: L2 then puts the parts of a 64-byte
+// sector that different stores bring together.  A sector written past L2 in parts costs a read and two writes of
+// memory: 1.4 TB/s against 4.1 for whole sectors (1 GiB, 8 rows x 128 bytes per instruction), 2.9 where L2 merges.
+constexpr int kStoreMerging = 0;
 // Cache policy of the partial tiles of depth pieces: device scope (sc1), i.e. written through to and
 // read from where all XCDs see them.  Their hand-over then needs no fence, which would write back
 // and invalidate whole L2s: 512 pieces of 16 depth slices took 100 us for theirs.
@@ -1729,10 +1734,17 @@ gmm_kernel(GmmParams p, HostSizes hs) {
         const int col = ti.n0 + wn * OUTW + out_chunk * 8;
         u32x4 held[32 / ROWS];   // (one strip behind, as below)
         uint32_t held_off[32 / ROWS];
+        const bool merge = uniform(p.flags & kFlagMergeStores) != 0;
         auto store_held = [&]() {
+          if (merge) {
 #pragma unroll
-          for (int r = 0; r < 32 / ROWS; ++r)
-            __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, at(held_off[r], col), 0, kStoreStreaming);
+            for (int r = 0; r < 32 / ROWS; ++r)
+              __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, at(held_off[r], col), 0, kStoreMerging);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 32 / ROWS; ++r)
+              __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, at(held_off[r], col), 0, kStoreStreaming);
+          }
         };
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
@@ -1845,26 +1857,34 @@ gmm_kernel(GmmParams p, HostSizes hs) {
         // an even width that is not a multiple of 8: rows of c then start on 4-byte boundaries
         // only, and the last 16-byte chunk of a row holds 2, 4 or 6 columns
         const bool ragged_width = uniform(ti.g.n & 7) != 0;
+        const bool merge = uniform(p.flags & kFlagMergeStores) != 0;
         // One strip behind: the reads of a strip return while the next one is converted (the LDS
         // serves a wave in order, so the next strip's writes need not wait for them).
         u32x4 held[4];
         uint32_t held_off[4];
         int held_col = 0;
         auto store_held = [&]() {
+          // (whole chunks only: for widths that are multiples of 8 the same as col < n)
+          auto chunk_at = [&](int r) { return held_col + 8 <= ti.g.n ? at(held_off[r], held_col) : OOR; };
+          if (merge) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const u32x4 v = held[r];
-            // (whole chunks only: for widths that are multiples of 8 the same as col < n)
-            __builtin_amdgcn_raw_buffer_store_b128(v, rc, held_col + 8 <= ti.g.n ? at(held_off[r], held_col) : OOR, 0,
-                                                   kStoreStreaming);
-            if (ragged_width) {
+            for (int r = 0; r < 4; ++r) __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, chunk_at(r), 0, kStoreMerging);
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, chunk_at(r), 0, kStoreStreaming);
+          }
+          if (ragged_width) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const u32x4 v = held[r];
               const int valid = ti.g.n - held_col;   // columns of this lane's chunk that exist
               const uint32_t off = at(held_off[r], held_col);
               if (valid > 0 && valid < 8 && off != OOR) {
-                if (valid & 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, rc, off, 0, kStoreStreaming);
+                if (valid & 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{v[0], v[1]}, rc, off, 0, kStoreMerging);
                 if (valid & 2)
                   __builtin_amdgcn_raw_buffer_store_b32((valid & 4) ? v[2] : v[0], rc, off + ((valid & 4) ? 8u : 0u), 0,
-                                                        kStoreStreaming);
+                                                        kStoreMerging);
               }
             }
           }
@@ -1984,7 +2004,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) gate[r] = sum[2 * jp][q][r], up[r] = sum[2 * jp + 1][q][r];
             const int col = ft.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
-            __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, c_at(ft, row_off, col), 0, kStoreStreaming);
+            __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, c_at(ft, row_off, col), 0, kStoreMerging);
           }
       } else {
 #pragma unroll
@@ -1998,7 +2018,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, old + sum[j][q]), rc, off, 0, 0);
             } else {
               __builtin_amdgcn_raw_buffer_store_b64(
-                  round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]), rc, off, 0, kStoreStreaming);
+                  round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]), rc, off, 0, kStoreMerging);
             }
           }
       }

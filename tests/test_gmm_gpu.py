@@ -1518,6 +1518,38 @@ def test_even_depths_that_are_no_multiple_of_8_stream(ops, oracle, trans_b, dtyp
               f"case {idx}, gathered and scattered")
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "swiglu"])
+@pytest.mark.parametrize("hout", [8, 96, 200, 352])
+def test_rows_of_c_off_64_byte_boundaries(ops, oracle, layout, hout):
+    # Rows of c that do not start on 64-byte boundaries, by their width or by where c starts, are stored
+    # through L2 (shallow products, weight gradients), others past it: the same bits, nothing beside them.
+    _announce("rows off 64-byte boundaries", layout, hout)
+    sizes = torch.tensor([70, 0, 33, 260, 1, 148], dtype=torch.int64)
+    hin, t = 136, int(sizes.sum())
+    g = torch.Generator().manual_seed(hout)
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16)
+    a = draw(t, hin)
+    b = {"nn": (6, hin, hout), "nt": (6, hout, hin), "tn": (t, hout), "swiglu": (6, hin, 2 * hout)}[layout]
+    b = draw(*b)
+    shape = (6, hin, hout) if layout == "tn" else (t, hout)
+    results = []
+    for shift in (0, 8, 32):   # elements: a 64-byte boundary, 16 bytes past one, the next one
+        room = int(np.prod(shape))
+        buffer = torch.full((room + 128,), 3.0, dtype=torch.bfloat16, device="cuda")
+        first = (-buffer.data_ptr() // 2) % 32 + 32 + shift
+        c = buffer[first:first + room].view(*shape)
+        if layout == "swiglu":
+            ops.backend.gmm_swiglu(a.cuda(), b.cuda(), sizes, c=c)
+        else:
+            ops.backend.gmm(a.cuda(), b.cuda(), sizes, trans_a=layout == "tn", trans_b=layout == "nt", c=c)
+        assert (buffer[:first] == 3).all() and (buffer[first + room:] == 3).all(), shift
+        results.append(c.clone())
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+    want = oracle.swiglu_loop(a, b, sizes) if layout == "swiglu" else \
+        oracle.gmm_loop(a, b, sizes, trans_a=layout == "tn", trans_b=layout == "nt")
+    check(results[0], want, f"{layout} {hout}")
+
+
 def test_padded_copies_leave_tail_rows_alone(ops, oracle):
     # sum(batch_sizes) < rows of a: the rows of c past the sum keep their contents on this path too
     g = torch.Generator().manual_seed(64)
