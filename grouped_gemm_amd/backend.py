@@ -137,8 +137,21 @@ def _padded_product(a_p, b_p, c, batch_sizes, trans_a, trans_b, hin, hout):
     return c
 
 
+def _cropped(t, shape):
+    """The upper left corner of every batch of t."""
+    if t.shape == shape:
+        return t
+    c = torch.empty(shape, dtype=t.dtype, device=t.device)
+    backend.unpad_rows(t, c)
+    return c
+
+
 def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
     """Both gradients of gmm(a, b, batch_sizes, trans_b=trans_b), each None where it is not wanted."""
+    if want_a and want_b:
+        both = backend.gmm_gradients(grad, a, b, batch_sizes, trans_b)   # (one launch)
+        if both is not None:
+            return both
     if want_a and want_b and _needs_padding(grad, b, None, batch_sizes, False, not trans_b) and \
             a.device == grad.device and a.dtype == grad.dtype and a.is_contiguous() and \
             tuple(a.shape) == (grad.shape[0], b.shape[2 if trans_b else 1]):
@@ -148,12 +161,9 @@ def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
         hin_p, hout_p = _round_up(hin, mult), _round_up(hout, mult)
         grad_p = _padded(grad, grad.shape[0], hout_p)
         b_p = _padded(b, hout_p, hin_p) if trans_b else _padded(b, hin_p, hout_p)
-        agrad = _padded_product(grad_p, b_p, None, batch_sizes, False, not trans_b, hout, hin)
-        del b_p
         a_p = _padded(a, a.shape[0], hin_p)
-        if trans_b:
-            return agrad, _padded_product(grad_p, a_p, None, batch_sizes, True, False, hout, hin)
-        return agrad, _padded_product(a_p, grad_p, None, batch_sizes, True, False, hin, hout)
+        agrad_p, bgrad_p = backend.gmm_gradients(grad_p, a_p, b_p, batch_sizes, trans_b)
+        return _cropped(agrad_p, a.shape), _cropped(bgrad_p, b.shape)
     agrad = gmm(grad, b, batch_sizes, trans_a=False, trans_b=not trans_b) if want_a else None
     bgrad = None
     if want_b:

@@ -62,6 +62,11 @@ def variant_indices():
     return [int(m) for m in re.findall(r"^GG_VARIANT\((\d+),", text, flags=re.M)]
 
 
+def pair_indices():
+    text = open(os.path.join(CSRC, "gmm_variants.def")).read()
+    return [int(m) for m in re.findall(r"^GG_PAIR\((\d+),", text, flags=re.M)]
+
+
 def build_hip(force=False, jobs=None):
     headers = [os.path.join(CSRC, f) for f in ("gmm_kernel.hpp", "gmm_generic.hpp", "gmm_variants.hpp",
                                                "gmm_variants.def", "row_kernels.hpp")]
@@ -70,6 +75,8 @@ def build_hip(force=False, jobs=None):
     obj_dir, hip_lib, extra = OBJ_DIR, HIP_LIB, []
     os.makedirs(obj_dir, exist_ok=True)
     units = [(os.path.join(CSRC, f + ".hip"), os.path.join(obj_dir, f + ".o"), extra) for f in ("gmm_api", "row_kernels")]
+    for i in pair_indices():   # (the largest units first)
+        units.append((os.path.join(CSRC, "gmm_pair.hip"), os.path.join(obj_dir, f"gmm_pair_{i}.o"), extra + [f"-DGG_PAIR_INDEX={i}"]))
     for i in variant_indices():
         units.append((os.path.join(CSRC, "gmm_variant.hip"), os.path.join(obj_dir, f"gmm_variant_{i}.o"),
                       extra + [f"-DGG_VARIANT_INDEX={i}"]))

@@ -21,8 +21,10 @@ const GenericOps* generic_ops_1();
 const GenericOps* generic_ops_2();
 const GenericOps* generic_ops_3();
 #define GG_VARIANT(index, DT_, LAYOUT_, SHAPE_, EPI_, INDEXED_) const VariantOps* variant_ops_##index();
+#define GG_PAIR(index, DT_, LAYOUT_, SHAPE1_, SHAPE2_) const PairOps* pair_ops_##index();
 #include "gmm_variants.def"
 #undef GG_VARIANT
+#undef GG_PAIR
 }  // namespace gg
 
 namespace {
@@ -55,6 +57,14 @@ const gg::VariantOps* (*const kVariantGetters[])() = {
 #include "gmm_variants.def"
 #undef GG_VARIANT
 };
+const gg::PairOps* (*const kPairGetters[])() = {
+#define GG_VARIANT(index, DT_, LAYOUT_, SHAPE_, EPI_, INDEXED_)
+#define GG_PAIR(index, DT_, LAYOUT_, SHAPE1_, SHAPE2_) &gg::pair_ops_##index,
+#include "gmm_variants.def"
+#undef GG_VARIANT
+#undef GG_PAIR
+};
+constexpr int kNumPairs = sizeof(kPairGetters) / sizeof(kPairGetters[0]);
 constexpr int kNumVariants = sizeof(kVariantGetters) / sizeof(kVariantGetters[0]);
 
 static_assert(GG_DTYPE_BF16 == gg::kBF16 && GG_DTYPE_F16 == gg::kF16 && GG_DTYPE_F8E4M3 == gg::kF8E4M3 &&
@@ -75,6 +85,14 @@ const gg::VariantOps* find_variant(int dt, int layout, int shape, int epilogue, 
     if (v->dt == dt && v->layout == layout && v->shape == shape && v->epilogue == epilogue &&
         v->indexed == indexed)
       return v;
+  }
+  return nullptr;
+}
+
+const gg::PairOps* find_pair(int dt, int layout, int shape1, int shape2) {
+  for (int i = 0; i < kNumPairs; ++i) {
+    const gg::PairOps* v = kPairGetters[i]();
+    if (v->dt == dt && v->layout == layout && v->shape1 == shape1 && v->shape2 == shape2) return v;
   }
   return nullptr;
 }
@@ -168,6 +186,7 @@ int device_info(DeviceInfo* out) {
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
       return fail(GG_EHIP, "this library is built for gfx950 only, device is %s", prop.gcnArchName);
     for (int i = 0; i < kNumVariants; ++i) GG_HIP(kVariantGetters[i]()->prepare());
+    for (int i = 0; i < kNumPairs; ++i) GG_HIP(kPairGetters[i]()->prepare());
     void* scratch_address = nullptr;
     GG_HIP(hipGetSymbolAddress(&scratch_address, HIP_SYMBOL(scratch)));
     void* status_address = nullptr;
@@ -384,8 +403,20 @@ bool may_cut_depth(const gg_gmm_args& g, const Route& r, const TileShape& shape)
   return gg::best_depth_pieces(slices, rows, shape.bn, kFullLaunch, 2 * kFullLaunch, gg::kMaxDepthPieces) > 1;
 }
 
+// A call that has been checked, and how it is launched.
+struct Plan {
+  bool empty = true;   // nothing to write
+  gg::GmmParams p{};
+  Route route;
+  TileShape shape;
+  const gg::VariantOps* variant = nullptr;   // nullptr: the general kernels
+  IndexedRows index_rows;
+  int epilogue, layout, cus;
+  int bn;              // output columns per tile
+};
+
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
-int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
+int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
   const int64_t hidden_in = g.hidden_in, hidden_out = g.hidden_out;
   const int trans_a = g.trans_a != 0, trans_b = g.trans_b != 0;
@@ -456,7 +487,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     if (variant == nullptr) return fail(GG_EINVAL, "no kernel for this combination of arguments");
   }
 
-  gg::GmmParams p{};
+  gg::GmmParams& p = out->p;
   p.a = static_cast<const char*>(g.a);
   p.b = static_cast<const char*>(g.b);
   p.c = static_cast<char*>(g.c);
@@ -515,62 +546,117 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
     p.ws_slots = !depth_pieces ? 0 : (slots > 1024 ? 1024 : (int32_t)slots);
   }
 
-  const int64_t tiles_n = (hidden_out + bn - 1) / bn;
-  const int64_t tiles_m_fixed = (hidden_in + bm - 1) / bm;   // weight-gradient layout
+  out->route = route;
+  out->shape = shape;
+  out->variant = variant;
+  out->index_rows = index_rows;
+  out->epilogue = epilogue;
+  out->layout = layout;
+  out->cus = info.cus;
+  out->bn = bn;
+  out->empty = false;
+  return GG_OK;
+}
+
+// The part of a call that one launch takes, groups first .. first + count - 1: into plan->p (and hs: their
+// host-resident sizes, which start at row *row).  *tiles: how many there are, at most.
+int plan_launch(const gg_gmm_args& g, Plan* plan, int64_t first, int64_t count, int64_t* row, gg::HostSizes* hs, int64_t* tiles) {
+  gg::GmmParams& p = plan->p;
+  const int bm = plan->shape.bm;
+  const int64_t tiles_n = (g.hidden_out + plan->bn - 1) / plan->bn;
+  const int64_t tiles_m_fixed = (g.hidden_in + bm - 1) / bm;   // weight-gradient layout
+  p.first_group = (int32_t)first;
+  p.num_groups = (int32_t)count;
+  if (g.batch_sizes_on_device) {
+    p.sizes_dev = g.batch_sizes;
+    p.row_base = 0;
+    // upper bound for any size vector (the device clips rows to `tokens`)
+    *tiles = g.trans_a ? count * tiles_m_fixed * tiles_n : (g.tokens / bm + count) * tiles_n;
+  } else {
+    p.sizes_dev = nullptr;
+    p.row_base = *row;
+    *tiles = 0;
+    for (int64_t i = 0; i < count; ++i) {
+      const int64_t m = g.batch_sizes[first + i];
+      hs->v[i] = (int32_t)m;
+      *row += m;
+      *tiles += g.trans_a ? tiles_m_fixed * tiles_n : ((m + bm - 1) / bm) * tiles_n;
+    }
+  }
+  if (*tiles >= (int64_t(1) << 31)) return fail(GG_ELIMIT, "too many output tiles for one launch");
+  p.flags &= ~gg::kFlagByTileRows;
+  if (plan->variant != nullptr && !g.trans_a && !(p.flags & gg::kFlagGroupOrder) && count >= kByTileRowsGroups &&
+      order_by_tile_rows(g.num_groups, g.tokens, tiles_n, bm, plan->cus, g.hidden_in))
+    p.flags |= gg::kFlagByTileRows;
+  return GG_OK;
+}
+
+int launch_call(const gg_gmm_args& g, Plan* plan) {
+  if (plan->empty) return GG_OK;
+  hipStream_t stream = static_cast<hipStream_t>(g.stream);
   // At most GG_MAX_GROUPS_PER_LAUNCH groups per launch.  A launch sees all operands and the rows
   // its groups start at: handed over by the host for host-resident sizes, summed up by the kernel
   // itself from the sizes of the groups before it for device-resident ones.
   int64_t row = 0;
-  for (int64_t first = 0; first < num_groups; first += GG_MAX_GROUPS_PER_LAUNCH) {
-    const int64_t count = num_groups - first < GG_MAX_GROUPS_PER_LAUNCH
-                              ? num_groups - first : GG_MAX_GROUPS_PER_LAUNCH;
+  for (int64_t first = 0; first < g.num_groups; first += GG_MAX_GROUPS_PER_LAUNCH) {
+    const int64_t count = g.num_groups - first < GG_MAX_GROUPS_PER_LAUNCH
+                              ? g.num_groups - first : GG_MAX_GROUPS_PER_LAUNCH;
     gg::HostSizes hs;
-    p.first_group = (int32_t)first;
-    p.num_groups = (int32_t)count;
     int64_t tiles;
-    if (g.batch_sizes_on_device) {
-      p.sizes_dev = g.batch_sizes;
-      p.row_base = 0;
-      // upper bound for any size vector (the device clips rows to `tokens`)
-      tiles = trans_a ? count * tiles_m_fixed * tiles_n : (tokens / bm + count) * tiles_n;
-    } else {
-      p.sizes_dev = nullptr;
-      p.row_base = row;
-      tiles = 0;
-      for (int64_t i = 0; i < count; ++i) {
-        const int64_t m = g.batch_sizes[first + i];
-        hs.v[i] = (int32_t)m;
-        row += m;
-        tiles += trans_a ? tiles_m_fixed * tiles_n : ((m + bm - 1) / bm) * tiles_n;
-      }
-    }
-    if (tiles >= (int64_t(1) << 31)) return fail(GG_ELIMIT, "too many output tiles for one launch");
+    const int rc = plan_launch(g, plan, first, count, &row, &hs, &tiles);
+    if (rc != GG_OK) return rc;
     if (tiles == 0) continue;
-    p.flags &= ~gg::kFlagByTileRows;
-    if (!generic && !trans_a && !(p.flags & gg::kFlagGroupOrder) && count >= kByTileRowsGroups &&
-        order_by_tile_rows(num_groups, tokens, tiles_n, bm, info.cus, hidden_in))
-      p.flags |= gg::kFlagByTileRows;
     // the full grid also for few tiles: the last round's tiles may be cut into pieces for
     // the workgroups that would otherwise idle
-    if (generic) {
+    if (plan->variant == nullptr) {
       gg::GenericParams gp;
-      gp.p = p;
+      gp.p = plan->p;
       gp.p.workspace = nullptr;
       gp.p.ws_slots = 0;
       gp.a_rows = g.a_row_index;
       gp.b_rows = g.b_row_index;
       gp.c_rows = g.c_row_index;
-      gp.a_num_rows = index_rows.a;
-      gp.b_num_rows = index_rows.b;
-      gp.c_num_rows = index_rows.c;
+      gp.a_num_rows = plan->index_rows.a;
+      gp.b_num_rows = plan->index_rows.b;
+      gp.c_num_rows = plan->index_rows.c;
       // light workgroups (28 KiB of LDS): two per compute unit
-      const int64_t grid = tiles < 2 * info.cus ? tiles : 2 * info.cus;
-      GG_HIP(generic_ops(g.dtype)->launch(layout, vec, epilogue, gp, hs, (int)grid, stream));
+      const int64_t grid = tiles < 2 * plan->cus ? tiles : 2 * plan->cus;
+      GG_HIP(generic_ops(g.dtype)->launch(plan->layout, plan->route.vec, plan->epilogue, gp, hs, (int)grid, stream));
     } else {
-      GG_HIP(variant->launch(p, hs, info.cus * variant->workgroups_per_cu, stream));
+      GG_HIP(plan->variant->launch(plan->p, hs, plan->cus * plan->variant->workgroups_per_cu, stream));
     }
   }
   return GG_OK;
+}
+
+int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
+  Plan plan;
+  const int rc = plan_call(g, static_scratch, &plan);
+  return rc != GG_OK ? rc : launch_call(g, &plan);
+}
+
+// Groups of few rows and large weights: the first product does nothing but read weights, the second nothing but
+// write gradients, and reads queue behind writes.  Us, two launches and one: 134 x 58 rows, 600 x 8960: 765 / 800;
+// 108 x 23, 3792 x 9328: 3295 / 3356; 116 x 6, 2688 x 10304: 2025 / 2144; 70 x 12, 824 x 6416: 390 / 405; and with smaller ones
+// (MB of weights) 38 x 19, 1944 x 2496 (369): 205 / 200; 83 x 29, 168 x 4152 (116): 89 / 88; 27 x 51, 1024 x 1032 (57): 49 / 48;
+// 6 x 95, 208 x 2880 (7): 25 / 20.
+constexpr int64_t kPairWeightBytes = int64_t(128) << 20;
+bool reads_then_writes(const gg_gmm_args& g) {
+  return use_short_shape(g.num_groups, g.tokens, 0) && g.num_groups * g.hidden_in * g.hidden_out * 2 > kPairWeightBytes;
+}
+
+// The kernel that runs both calls in one launch, or nullptr: a product with plain rows and epilogue and a weight
+// gradient, over the same groups, in tile shapes of about the same weight, sharing no workspace.
+const gg::PairOps* pair_kernel(const gg_gmm_args& g1, const Plan& p1, const gg_gmm_args& g2, const Plan& p2) {
+  if (p1.empty || p2.empty || p1.variant == nullptr || p2.variant == nullptr) return nullptr;
+  if (g1.trans_a || !g2.trans_a || p1.epilogue != gg::kEpiStore || p2.epilogue != gg::kEpiStore) return nullptr;
+  if (p1.route.indexed || p2.route.indexed || g1.dtype != g2.dtype || g1.stream != g2.stream) return nullptr;
+  if (g1.batch_sizes != g2.batch_sizes || g1.batch_sizes_on_device != g2.batch_sizes_on_device ||
+      g1.num_groups != g2.num_groups || g1.tokens != g2.tokens || g1.num_groups > GG_MAX_GROUPS_PER_LAUNCH)
+    return nullptr;
+  if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace == p2.p.workspace) return nullptr;
+  if (reads_then_writes(g1)) return nullptr;
+  return find_pair(g1.dtype, p1.layout, p1.shape.id, p2.shape.id);
 }
 
 }  // namespace
@@ -617,6 +703,30 @@ int gg_gmm(const gg_gmm_args* args) {
     return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is %u, this library expects %zu", args->struct_bytes,
                 sizeof(gg_gmm_args));
   return gmm_impl(*args);
+}
+
+int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) {
+  if (first == nullptr || second == nullptr) return fail(GG_EINVAL, "args is null");
+  if (first->struct_bytes != sizeof(gg_gmm_args) || second->struct_bytes != sizeof(gg_gmm_args))
+    return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is not the %zu this library expects", sizeof(gg_gmm_args));
+  Plan p1, p2;
+  int rc = plan_call(*first, false, &p1);
+  if (rc == GG_OK) rc = plan_call(*second, false, &p2);
+  if (rc != GG_OK) return rc;
+  const gg::PairOps* pair = pair_kernel(*first, p1, *second, p2);
+  if (pair != nullptr) {
+    gg::HostSizes hs;
+    int64_t row1 = 0, row2 = 0, tiles1, tiles2;
+    rc = plan_launch(*first, &p1, 0, first->num_groups, &row1, &hs, &tiles1);
+    if (rc == GG_OK) rc = plan_launch(*second, &p2, 0, second->num_groups, &row2, &hs, &tiles2);
+    if (rc != GG_OK) return rc;
+    if (tiles1 > 0 && tiles2 > 0) {
+      GG_HIP(pair->launch(p1.p, p2.p, hs, p1.cus * pair->workgroups_per_cu, static_cast<hipStream_t>(first->stream)));
+      return GG_OK;
+    }
+  }
+  rc = launch_call(*first, &p1);
+  return rc == GG_OK ? launch_call(*second, &p2) : rc;
 }
 
 uint64_t gg_workspace_bytes_for(const gg_gmm_args* args) {

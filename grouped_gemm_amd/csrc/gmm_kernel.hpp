@@ -356,7 +356,7 @@ __device__ __forceinline__ GroupTiles group_tiles(int rows, int hidden_in, int h
 // clamped to [0, tokens] before it enters a sum, so no size vector can make a sum overflow or a
 // group start before row 0 or end past row `tokens`.
 template <int LAYOUT, int BM, int BN>
-__device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, const HostSizes& hs) {
+__device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, const HostSizes& hs, int w) {
   const int lane = threadIdx.x;
   if (lane >= 64) return;
   const int E = p.num_groups;
@@ -456,7 +456,7 @@ __device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, con
   }
   // What the host would have rejected in host-resident sizes is reported for device-resident
   // ones: one workgroup ORs what its first wave saw into the caller's status word.
-  if (p.status != nullptr && blockIdx.x == 0) {
+  if (p.status != nullptr && w == 0) {
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) bad |= __shfl_xor(bad, d);
     if (lane == 0 && bad != 0) atomicOr(p.status, bad);
@@ -703,7 +703,7 @@ template <int LAYOUT, int BM, int BN>
 __global__ __launch_bounds__(64) void schedule_dump_kernel(GmmParams p, HostSizes hs) {
   __shared__ Sched s;
   __shared__ uint64_t sort_keys[kMaxGroups];
-  build_schedule<LAYOUT, BM, BN>(&s, p, hs);
+  build_schedule<LAYOUT, BM, BN>(&s, p, hs, (int)blockIdx.x);
   __syncthreads();
   const bool ordered = LAYOUT == kTN || (p.flags & kFlagByTileRows) != 0;
   if (LAYOUT == kTN) {
@@ -1273,6 +1273,66 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
   return ti;
 }
 
+// What a launch does beside this product (the PART of gmm_tiles).
+template <int WGS_PER_CU_>
+struct Alone {   // nothing
+  static constexpr int WGS_PER_CU = WGS_PER_CU_;   // workgroups a compute unit has room for
+  static constexpr bool FIRST = false, SECOND = false;
+};
+template <int WGS_PER_CU_>
+struct FirstOfPair {   // its workgroups are followed by those of a second product (gmm_pair_kernel)
+  static constexpr int WGS_PER_CU = WGS_PER_CU_;
+  static constexpr bool FIRST = true, SECOND = false;
+};
+// ... and this is the second one: a weight gradient whose workgroups start where the first product's have ended.
+// The first one's last round leaves `early` workgroups per XCD without a tile; as many of the second's, the
+// first of each XCD (an XCD starts its workgroups in order as its compute units become free), begin a tile of the
+// first earlier than the rest, and are given `extra` more tiles: as many as end both soonest.
+// Costs of a tile in depth slices of full tiles: the slices left to a piece and 3 of tile turnover for the first
+// product, 4 of stores for the second one; short tiles' slices are five eighths as long.
+// 8 x 1024 rows, 5464 -> 2048 and the weight gradient: 461 us in two launches, 409 in one without extra tiles, 376.
+struct Head {
+  int early, extra;
+};
+// None where tiles of the second are shallow: they are bound by their stores, and slow the first down (32 x 128 rows,
+// 2048 -> 768: 62 us without, 65 to 72 with 1 to 4 extra tiles).
+constexpr int kHeadSlices = 8;
+constexpr int kMaxExtra = 12;
+template <int WGS_PER_CU_, int LAYOUT1, int BM1, int BN1>
+struct SecondOfPair {
+  static constexpr int WGS_PER_CU = WGS_PER_CU_;
+  static constexpr bool FIRST = false, SECOND = true;
+  const GmmParams& first;
+
+  // (after build_schedule and a barrier; the same answer in every wave)
+  __device__ __forceinline__ Head head(const Sched* s, const GmmParams& p, int grid, int bk) const {
+    int tile_rows = 0;
+    for (int e = threadIdx.x & 63; e < p.num_groups; e += 64) tile_rows += (s->rows[e] + BM1 - 1) / BM1;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) tile_rows += __shfl_xor(tile_rows, d);
+    const TailPlan plan = plan_tail<LAYOUT1, BM1, BN1, WGS_PER_CU>(uniform(tile_rows) * ((first.hidden_out + BN1 - 1) / BN1),
+                                                                    grid, first, bk);
+    Head h{0, 0};
+    if (grid % 8 != 0) return h;
+    h.early = grid / 8 - (plan.total % grid + 7) / 8;
+    const int slices2 = ((int)(p.tokens / p.num_groups) + bk - 1) / bk;
+    if (h.early == 0 || slices2 < kHeadSlices) return h;
+    const int slices1 = (first.hidden_in + bk - 1) / bk / (plan.by_depth ? plan.pieces : 1);
+    const int cost1 = (BM1 > 128 ? slices1 : slices1 * 5 / 8) + 3, cost2 = slices2 + 4;
+    const int tiles = uniform(s->tile_start[p.num_groups]), n = h.early * 8;
+    int best = 1 << 30;
+    for (int extra = 0; extra <= kMaxExtra && extra * n <= tiles; ++extra) {
+      const int rounds = (tiles - extra * n) / grid, rest = (tiles - extra * n) % grid;   // (of the last round, the early ones first)
+      const int late = (rounds + (rest > n ? 1 : 0)) * cost2;
+      const int soon = (extra + rounds + (rest > 0 ? 1 : 0)) * cost2 - cost1;
+      const int end = late > soon ? late : soon;
+      if (end < best) best = end, h.extra = extra;
+    }
+    return h;
+  }
+};
+
+// The tiles of one product that workgroup w of G works on.
 // DT: element type of a and b (and of c unless it is the fp32 accumulator).
 // EPI: what happens to a finished tile (kEpi*): stored in the element type; added to an fp32 c
 // (gradient accumulation, weight-gradient layout); or, with gate | up columns in b, combined to
@@ -1280,11 +1340,8 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
 // INDEXED: rows of a are fetched and rows of c stored through p.a_rows / p.c_rows (NN and NT).
 // RAGGED_DEPTH: hidden_in is even but no multiple of 8 (NN and NT, two-byte elements, plain store).
 template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N,
-          int EPI = kEpiStore, bool INDEXED = false, bool RAGGED_DEPTH = false>
-__global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
-                             (GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>::WORKGROUPS_PER_CU)) void
-gmm_kernel(GmmParams p, HostSizes hs) {
-#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
+          int EPI, bool INDEXED, bool RAGGED_DEPTH, typename PART>
+__device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& hs, char* smem, const int w, const int G, const PART& part) {
   using Cfg = GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>;
   constexpr int NT = Cfg::NT, MB = Cfg::MB, NB = Cfg::NB, KS = BK / 16;
   constexpr bool ACC_F32 = EPI == kEpiAccF32 || EPI == kEpiAccF32Atomic, GATE_UP = EPI == kEpiSwiGLU;
@@ -1325,9 +1382,8 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   static_assert(LOADS_PER_STAGE >= 4 && LOADS_PER_STAGE < 32, "");
   constexpr int UNITS = MB + NB;    // fragments of one 16-deep step
 
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
   Sched* sched = reinterpret_cast<Sched*>(smem + Cfg::SCHED_OFFSET);
-  build_schedule<LAYOUT, BM, BNS>(sched, p, hs);
+  build_schedule<LAYOUT, BM, BNS>(sched, p, hs, w);
   __syncthreads();
   if constexpr (LAYOUT == kTN) {
     order_groups_by_depth(sched, p.num_groups, reinterpret_cast<uint64_t*>(smem));
@@ -1347,13 +1403,19 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   // (tiles that are combined or scattered on their way out are cut along the depth in the shapes for
   // few rows and few tiles only: full ones would pay for it with the fix-up's scalar registers)
   constexpr bool DEPTH_PIECES = !RAGGED_DEPTH && !((GATE_UP || INDEXED) && BM > 128);
-  TailPlan plan = plan_tail<LAYOUT, BM, BN, Cfg::WORKGROUPS_PER_CU, DEPTH_PIECES>(
-      uniform(sched->tile_start[p.num_groups]) + uniform(sched->runt_start[p.num_groups]),
-      (int)gridDim.x, p, BK_ELEMS);
+  const int all_tiles = uniform(sched->tile_start[p.num_groups]) + uniform(sched->runt_start[p.num_groups]);
+  // SECOND: indices below head_tiles go to the workgroups that start early, the others to all of them
+  Head head{0, 0};
+  if constexpr (PART::SECOND) head = part.head(sched, p, G, BK_ELEMS);
+  int head_step = uniform(head.early) * 8, head_tiles = head_step * uniform(head.extra);
+  TailPlan plan = plan_tail<LAYOUT, BM, BN, PART::WGS_PER_CU, DEPTH_PIECES>(all_tiles - head_tiles, G, p, BK_ELEMS);
+  if constexpr (PART::SECOND) plan.main_tiles += head_tiles, plan.total += head_tiles;
   if constexpr (!DEPTH_PIECES) plan.by_depth = false;   // (known at compile time: no depth-piece code is kept)
   if constexpr (LAYOUT == kTN && DEPTH_PIECES) {
-    plan_deep_tiles<BM, BN>(sched, p, (int)gridDim.x, BK_ELEMS, &plan);
+    plan_deep_tiles<BM, BN>(sched, p, G, BK_ELEMS, &plan);
     plan.pieces = uniform(plan.pieces), plan.main_tiles = uniform(plan.main_tiles), plan.total = uniform(plan.total);
+    // (cut deep tiles go out first, at most one piece to a workgroup)
+    if (PART::SECOND && uniform(sched->front_tiles) > 0) head_tiles = 0;
   }
   const int total_tiles = plan.total;
 
@@ -1362,22 +1424,42 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   // deals them evenly to all XCDs: runs of G / 8 would put them on the first few, each of which
   // reaches only its share of the memory bandwidth (6 tiles of 128 depth slices, all on one XCD:
   // 51 us, one to an XCD: 36 us; 30 tiles of 100 slices: 141 -> 83 us; 200 tiles and more, and tiles
-  // of a few slices, within 2 % either way).
-  const int G = gridDim.x;
-  const int w = blockIdx.x;
-  int vid = w;
+  // of a few slices, within 2 % either way).  In a pair the last round is dealt evenly as well, so that the
+  // workgroups without a tile in it are spread over the XCDs (alone that is neutral, 0.98 to 1.01 of the time).
+  int first_t = w;
+  const int full = head_tiles + (total_tiles - head_tiles) / G * G;   // (pairs) where the last round begins
+  int last_t = full + w;                                              // (pairs) this workgroup's index in it
   if (G % 8 == 0) {
-    const int run = total_tiles < G ? (total_tiles + 7) / 8 : G / 8;
-    vid = w / 8 < run ? (w % 8) * run + w / 8 : total_tiles;
+    const int x = w % 8, s = w / 8;
+    if constexpr (PART::FIRST || PART::SECOND) {
+      const int run = (total_tiles - full + 7) / 8;
+      last_t = s < run ? full + x * run + s : total_tiles;
+      first_t = head_tiles + x * (G / 8) + s;
+      if (first_t >= full) first_t = last_t;
+      if (PART::SECOND && head_tiles > 0 && s < head_step / 8) first_t = x * (head_step / 8) + s;
+    } else {
+      const int run = total_tiles < G ? (total_tiles + 7) / 8 : G / 8;
+      first_t = s < run ? x * run + s : total_tiles;
+    }
   }
-  if (vid >= total_tiles) return;
+  if (first_t >= total_tiles) return;
+  first_t = uniform(first_t);
+  // The index of this workgroup's tile after tile t (total_tiles and more: none)
+  auto next_index = [&](int t) {
+    if constexpr (!PART::FIRST && !PART::SECOND) return uniform(t + G);
+    if (PART::SECOND && t < head_tiles) {
+      const int mine = head_tiles + (G % 8 == 0 ? (w % 8) * (G / 8) + w / 8 : w);
+      return uniform(t + head_step < head_tiles ? t + head_step : (mine < full ? mine : last_t));
+    }
+    return uniform(t + G < full ? t + G : (t < full ? last_t : total_tiles));
+  };
 
   // Two cursors walk this workgroup's tiles: the fetch cursor runs STAGES depth slices
   // ahead of the compute cursor and crosses into the next tile on its own, so the first
   // slices of a tile are already in flight while the previous tile is being stored.
   ALoad aload;
   BLoad bload;
-  int fetch_t = vid, fetch_kt = 0;
+  int fetch_t = first_t, fetch_kt = 0;
   TileCursor fetch_cur;
   TileInfo fti;
   // The compute cursor does not look its tiles up again: the fetch cursor, which is one or two
@@ -1446,7 +1528,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
     // slice descriptors below are computed lane by lane and the branch becomes a masked one)
     fetch_kt = uniform(fetch_kt + 1);
     if (fetch_kt == uniform(fti.nk) && uniform((int)fti.valid) != 0) {
-      fetch_t = uniform(fetch_t + G);
+      fetch_t = next_index(fetch_t);
       fetch_kt = 0;
       fetch_setup();
     }
@@ -1485,7 +1567,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
   fetch_begin();
   static_for<T3>([&](auto j) { fetch_load(j, 1); });
 
-  int tile_t = vid;
+  int tile_t = first_t;
   int tile_n = 0;   // tiles this workgroup has finished
   auto next_tile = [&]() {
     int32_t words[kTileInfoDwords];
@@ -1798,14 +1880,18 @@ gmm_kernel(GmmParams p, HostSizes hs) {
                   asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[i][j][4 * q + r]));
                 *reinterpret_cast<f32x4*>(strip + in_row * PITCH + (8 * q + 4 * in_half) * 4) = v;
               }
-              const int col = ti.n0 + wn * Cfg::WTN + j * 32 + (lane & 31);
+              // (offsets from one per block on: worked out per instruction they do not change from tile to
+              // tile, and the compiler keeps them in more registers than there are: reloading those it
+              // spilled waits for the atomics ahead of them: 2.9 % of 8 x 4096 rows, 4096 x 14336)
+              int at_lane = lane;
+              asm volatile("" : "+v"(at_lane));
+              const int col = ti.n0 + wn * Cfg::WTN + j * 32 + (at_lane & 31);
+              uint32_t off = col < ti.g.n ? (uint32_t)(((wm + i * WAVES_M) * 32 + (at_lane >> 5)) * ti.g.n + col) * 4u : kOutOfRange;
 #pragma unroll
               for (int r = 0; r < 16; ++r) {
-                const int srow = r * 2 + (lane >> 5);
-                const float v = *reinterpret_cast<const float*>(strip + srow * PITCH + (lane & 31) * 4);
-                const int row = (wm + i * WAVES_M) * 32 + srow;
-                const uint32_t off = col < ti.g.n ? (uint32_t)(row * ti.g.n + col) * 4u : kOutOfRange;
+                const float v = *reinterpret_cast<const float*>(strip + (r * 2 + (lane >> 5)) * PITCH + (lane & 31) * 4);
                 __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rc, off, 0, 0);
+                off += (uint32_t)ti.g.n * 8u;   // two rows (stays out of range: widths are below 2^20 here)
               }
               __builtin_amdgcn_sched_barrier(0);
             }
@@ -1951,7 +2037,7 @@ gmm_kernel(GmmParams p, HostSizes hs) {
         tile_body(std::integral_constant<int, 1>{});
       }
     }
-    tile_t = uniform(tile_t + G);
+    tile_t = next_index(tile_t);
     if (tile_t >= total_tiles) break;
     tile_n = uniform(tile_n + 1);
     ti = next_tile();
@@ -2024,7 +2110,51 @@ gmm_kernel(GmmParams p, HostSizes hs) {
       }
     }
   }
-#endif  // __HIP_DEVICE_COMPILE__
+}
+
+template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N,
+          int EPI = kEpiStore, bool INDEXED = false, bool RAGGED_DEPTH = false>
+__global__ __launch_bounds__(WAVES_M* WAVES_N * 64,
+                             (GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>::WORKGROUPS_PER_CU)) void
+gmm_kernel(GmmParams p, HostSizes hs) {
+#if defined(__HIP_DEVICE_COMPILE__)  // the host pass only needs the launch stub
+  using Cfg = GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  gmm_tiles<DT, LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N, EPI, INDEXED, RAGGED_DEPTH>(p, hs, smem, (int)blockIdx.x,
+                                                                                        (int)gridDim.x, Alone<Cfg::WORKGROUPS_PER_CU>{});
+#endif
+}
+
+// Both gradients of a product in one launch: workgroups 0 .. G - 1 work on the input gradient (shape S1, layout
+// LAYOUT1), G .. 2 G - 1 on the weight gradient (S2).  A compute unit has room for one of them, so the
+// second half starts as the first half ends: compute units that the first product's last round leaves idle begin
+// the second product at once, and what a launch takes to start and to drain (4 of the 8 us of a small one)
+// passes once.  Us, two launches and one: 8 x 128 rows, 128 x 128: 15.6 / 11.2; 32 x 128, 768 x 2048: 67 / 61; 8 x
+// 1024, 2048 x 5464: 461 / 376; 64 Zipf groups, 49152 rows, 2048 x 1408: 623 / 611; 43 x 848, 5696 x 2752: 2097 / 2110.
+template <int LAYOUT1, typename S1, typename S2, int BK, int STAGES>
+struct PairConfig {
+  using First = GmmConfig<LAYOUT1, S1::BM, S1::BN, BK, STAGES, S1::WAVES_M, S1::WAVES_N>;
+  using Second = GmmConfig<kTN, S2::BM, S2::BN, BK, STAGES, S2::WAVES_M, S2::WAVES_N>;
+  static_assert(First::NT == Second::NT, "");
+  static constexpr int NT = First::NT;
+  static constexpr int LDS_BYTES = First::LDS_BYTES > Second::LDS_BYTES ? First::LDS_BYTES : Second::LDS_BYTES;
+  static constexpr int WORKGROUPS_PER_CU = 2 * LDS_BYTES <= 160 * 1024 ? 2 : 1;
+};
+template <int DT, int LAYOUT1, typename S1, typename S2, int BK, int STAGES>
+__global__ __launch_bounds__((PairConfig<LAYOUT1, S1, S2, BK, STAGES>::NT), (PairConfig<LAYOUT1, S1, S2, BK, STAGES>::WORKGROUPS_PER_CU)) void
+gmm_pair_kernel(GmmParams p1, GmmParams p2, HostSizes hs) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  constexpr int WGS = PairConfig<LAYOUT1, S1, S2, BK, STAGES>::WORKGROUPS_PER_CU;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int G = (int)gridDim.x / 2, w = (int)blockIdx.x;
+  if (w < G) {
+    gmm_tiles<DT, LAYOUT1, S1::BM, S1::BN, BK, STAGES, S1::WAVES_M, S1::WAVES_N, kEpiStore, false, false>(
+        p1, hs, smem, w, G, FirstOfPair<WGS>{});
+  } else {
+    gmm_tiles<DT, kTN, S2::BM, S2::BN, BK, STAGES, S2::WAVES_M, S2::WAVES_N, kEpiStore, false, false>(
+        p2, hs, smem, w - G, G, SecondOfPair<WGS, LAYOUT1, S1::BM, S1::BN>{p1});
+  }
+#endif
 }
 
 }  // namespace gg

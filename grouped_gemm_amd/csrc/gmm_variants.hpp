@@ -52,6 +52,15 @@ struct VariantOps {
   hipError_t (*launch)(const GmmParams& p, const HostSizes& hs, int grid, hipStream_t stream);
 };
 
+// Both gradients of a product in one launch (gmm_pair_kernel).
+struct PairOps {
+  int dt, layout, shape1, shape2;
+  int workgroups_per_cu;
+  hipError_t (*prepare)();
+  // grid: workgroups of each of the two products
+  hipError_t (*launch)(const GmmParams& p1, const GmmParams& p2, const HostSizes& hs, int grid, hipStream_t stream);
+};
+
 // The kernels of gmm_generic.hpp for one element type (gmm_generic_variant.hip).
 struct GenericParams;
 struct GenericOps {

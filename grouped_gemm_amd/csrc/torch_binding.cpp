@@ -13,6 +13,7 @@
 
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <utility>
 
 #include "../../include/grouped_gemm_hip.h"
@@ -162,14 +163,15 @@ bool BelongsToGraph(const torch::Tensor& t) {
 //
 // Outside a graph capture: one per device and stream, allocated and zeroed at the first call there that can
 // use one (gg_workspace_bytes_for) and kept for the life of the process.  Calls on one stream run one after
-// the other, so they can share it; the kernels leave its counters zero.
+// the other, so they can share it; the kernels leave its counters zero.  Two calls in one launch (gg_gmm_pair) run
+// at the same time: the second one's is another, `which` = 1, made at the first pair whose both halves can use one.
 //
 // A captured call runs at every replay, on whatever stream and beside whatever other graphs the program
 // chooses, and what it allocates is the graph's pool's, which graphs may share.  It takes a workspace for
 // itself alone, which its graph's later calls and no others can get again, and clears the counters as a
 // part of the graph (a fill of 4 KiB ahead of the launch).  Where the graph cannot own one (BelongsToGraph; asked
 // once per capture and thread) there is none, an undefined tensor: the call keeps its tiles whole.
-torch::Tensor Workspace(const torch::Device& device, hipStream_t stream) {
+torch::Tensor Workspace(const torch::Device& device, hipStream_t stream, int which = 0) {
   constexpr int64_t kCounterBytes = 4096;   // the arrival counters at its beginning, see gg_gmm_args.workspace
   const auto bytes = torch::dtype(torch::kUInt8).device(device);
   if (const unsigned long long capture = CaptureNumber(stream)) {
@@ -186,8 +188,8 @@ torch::Tensor Workspace(const torch::Device& device, hipStream_t stream) {
     return ws;
   }
   static std::mutex mu;
-  static std::map<std::pair<int, hipStream_t>, torch::Tensor> cache;
-  const auto key = std::make_pair((int)device.index(), stream);
+  static std::map<std::tuple<int, hipStream_t, int>, torch::Tensor> cache;
+  const auto key = std::make_tuple((int)device.index(), stream, which);
   {
     std::lock_guard<std::mutex> lock(mu);
     const auto it = cache.find(key);
@@ -210,13 +212,11 @@ int32_t* SizeStatusWord() {
   return word;
 }
 
-void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& batch_sizes,
-         bool trans_a, bool trans_b, bool accumulate_f32, int64_t flags, const RowIndices& rows = RowIndices(),
-         bool gate_up = false) {
-  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
-  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
-  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(a.device().index()).stream();
-  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+// The C ABI's arguments for a validated call on the current device and `stream`, without a workspace.  `sizes`:
+// contiguous batch_sizes, which have to live until the call is enqueued.
+gg_gmm_args Arguments(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& sizes,
+                      bool trans_a, bool trans_b, bool accumulate_f32, int64_t flags, const RowIndices& rows, bool gate_up,
+                      hipStream_t stream) {
   gg_gmm_args g = {};
   g.struct_bytes = sizeof(g);
   g.dtype = DtypeCode(a.scalar_type());
@@ -240,18 +240,51 @@ void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c,
   g.c_num_rows = trans_a ? 0 : c.size(0);
   g.b_num_rows = trans_a ? (int32_t)b.size(0) : 0;
   g.flags = (int32_t)flags;
-  // a workspace only for calls that can cut tiles along the depth (deep products, weight gradients)
-  torch::Tensor workspace;   // (held until the call is enqueued)
-  if (gg_workspace_bytes_for(&g) > 0) {
-    workspace = Workspace(a.device(), stream);
-    if (workspace.defined()) {
-      g.workspace = workspace.data_ptr();
-      g.workspace_bytes = (uint64_t)workspace.numel();
-    }
-  }
   g.stream = static_cast<void*>(stream);
   if (sizes.is_cuda()) g.size_status = SizeStatusWord();
+  return g;
+}
+
+// A workspace for calls that can cut tiles along the depth (deep products, weight gradients) and only for
+// them; the tensor has to live until the call is enqueued.
+torch::Tensor AttachWorkspace(gg_gmm_args* g, const torch::Device& device, hipStream_t stream, int which = 0) {
+  torch::Tensor workspace;
+  if (gg_workspace_bytes_for(g) > 0) {
+    workspace = Workspace(device, stream, which);
+    if (workspace.defined()) {
+      g->workspace = workspace.data_ptr();
+      g->workspace_bytes = (uint64_t)workspace.numel();
+    }
+  }
+  return workspace;
+}
+
+void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& batch_sizes,
+         bool trans_a, bool trans_b, bool accumulate_f32, int64_t flags, const RowIndices& rows = RowIndices(),
+         bool gate_up = false) {
+  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(a.device().index()).stream();
+  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+  gg_gmm_args g = Arguments(a, b, c, sizes, trans_a, trans_b, accumulate_f32, flags, rows, gate_up, stream);
+  const torch::Tensor workspace = AttachWorkspace(&g, a.device(), stream);
   const int rc = gg_gmm(&g);
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+}
+
+// Both gradients of a product, agrad = grad @ b (or b^T) and bgrad = lhs^T @ rhs, all validated.
+void RunGradients(const torch::Tensor& grad, const torch::Tensor& b, const torch::Tensor& agrad, bool trans_b,
+                  const torch::Tensor& lhs, const torch::Tensor& rhs, const torch::Tensor& bgrad,
+                  const torch::Tensor& batch_sizes) {
+  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(grad.device().index()).stream();
+  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+  gg_gmm_args g1 = Arguments(grad, b, agrad, sizes, false, trans_b, false, 0, RowIndices(), false, stream);
+  gg_gmm_args g2 = Arguments(lhs, rhs, bgrad, sizes, true, false, false, 0, RowIndices(), false, stream);
+  const torch::Tensor workspace1 = AttachWorkspace(&g1, grad.device(), stream);
+  const torch::Tensor workspace2 = AttachWorkspace(&g2, grad.device(), stream, workspace1.defined() ? 1 : 0);
+  const int rc = gg_gmm_pair(&g1, &g2);
   TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
 }
 
@@ -299,6 +332,29 @@ c10::optional<torch::Tensor> GroupedGemmDirect(const torch::Tensor& a, const tor
   return out;
 }
 
+// Both gradients of gmm(a, b, batch_sizes, trans_b=trans_b); the launches of both are one where the library has
+// a kernel for the two (gg_gmm_pair).
+std::pair<torch::Tensor, torch::Tensor> BothGradients(const torch::Tensor& grad, const torch::Tensor& a, const torch::Tensor& b,
+                                                      const torch::Tensor& batch_sizes, bool trans_b) {
+  const torch::Tensor &lhs = trans_b ? grad : a, &rhs = trans_b ? a : grad;
+  torch::Tensor agrad = AllocateOutput(grad, b, batch_sizes, false, !trans_b);
+  Validate(grad, b, agrad, batch_sizes, false, !trans_b, /*on_device=*/true);
+  torch::Tensor bgrad = AllocateOutput(lhs, rhs, batch_sizes, true, false);
+  Validate(lhs, rhs, bgrad, batch_sizes, true, false, /*on_device=*/true);
+  RunGradients(grad, b, agrad, !trans_b, lhs, rhs, bgrad, batch_sizes);
+  return {agrad, bgrad};
+}
+
+// ... for operands that the streaming kernels take as they are; nothing is returned (and nothing done) for others.
+c10::optional<std::pair<torch::Tensor, torch::Tensor>> GroupedGemmGradients(const torch::Tensor& grad, const torch::Tensor& a,
+                                                                            const torch::Tensor& b,
+                                                                            const torch::Tensor& batch_sizes, bool trans_b) {
+  const torch::Tensor &lhs = trans_b ? grad : a, &rhs = trans_b ? a : grad;
+  if (!IsDirect(grad, b, batch_sizes, false, !trans_b, nullptr) || !IsDirect(lhs, rhs, batch_sizes, true, false, nullptr))
+    return c10::nullopt;
+  return BothGradients(grad, a, b, batch_sizes, trans_b);
+}
+
 // ops.GroupedGemm (the reference's grouped_gemm/ops.py:8-29) as a native autograd node: a training
 // step of a small layer is bound by what the host does between the three launches, and the
 // interpreter was most of it.
@@ -321,11 +377,12 @@ class GroupedGemmNode : public torch::autograd::Function<GroupedGemmNode> {
     const torch::Tensor &a = saved[0], &b = saved[1], &batch_sizes = saved[2];
     const bool trans_b = ctx->saved_data["trans_b"].toBool();
     torch::Tensor agrad, bgrad;
-    if (ctx->needs_input_grad(0)) {
+    if (ctx->needs_input_grad(0) && ctx->needs_input_grad(1)) {
+      std::tie(agrad, bgrad) = BothGradients(grad, a, b, batch_sizes, trans_b);
+    } else if (ctx->needs_input_grad(0)) {
       agrad = AllocateOutput(grad, b, batch_sizes, false, !trans_b);
       GroupedGemm(grad, b, agrad, batch_sizes, false, !trans_b);
-    }
-    if (ctx->needs_input_grad(1)) {
+    } else if (ctx->needs_input_grad(1)) {
       const torch::Tensor &lhs = trans_b ? grad : a, &rhs = trans_b ? a : grad;
       bgrad = AllocateOutput(lhs, rhs, batch_sizes, true, false);
       GroupedGemm(lhs, rhs, bgrad, batch_sizes, true, false);
@@ -491,6 +548,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gmm_direct", &GroupedGemmDirect,
         "gmm with the output allocated where c is None, for calls the streaming kernels take as they are; None for others.");
   m.def("gmm_autograd", &GroupedGemmAutograd, "The differentiable form of gmm_direct without trans_a.");
+  m.def("gmm_gradients", &GroupedGemmGradients,
+        "Both gradients of gmm, for operands the streaming kernels take as they are; None for others.");
   m.def("validate",
         [](torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes, bool trans_a,
            bool trans_b) { Validate(a, b, c, batch_sizes, trans_a, trans_b, /*on_device=*/false); },

@@ -54,24 +54,23 @@ class GroupedGemmGather(torch.autograd.Function):
     def backward(ctx, grad):
         grad = grad.contiguous()
         x, w, batch_sizes, row_index = ctx.saved_tensors
-        xgrad = wgrad = None
+        xgrad = wgrad = sorted_x = None
+        if ctx.needs_input_grad[1]:
+            # The weight-gradient layout takes row indices on the general kernels only, which are
+            # several times slower than the streaming ones: one explicit gather and the streaming
+            # kernel is the faster way to the same result.
+            sorted_x = x.index_select(0, row_index)
+        sorted_grad, wgrad = backend.gradients(grad, sorted_x, w, batch_sizes, ctx.trans_b, ctx.needs_input_grad[0],
+                                               ctx.needs_input_grad[1])
         if ctx.needs_input_grad[0]:
             # rows of x that several sorted rows came from collect several gradients: a sum, not
             # a store, so it is not fused
-            sorted_grad = backend.gmm(grad, w, batch_sizes, trans_b=not ctx.trans_b)
             if sorted_grad.dtype == x.dtype:
                 xgrad = backend.backend.sum_rows(sorted_grad, row_index, x.shape[0])
             else:   # float8 operands: rounded once, from fp32 to their type
                 xgrad = torch.zeros(x.shape, dtype=torch.float32, device=x.device)
                 xgrad.index_add_(0, row_index, sorted_grad.float())
                 xgrad = xgrad.to(x.dtype)
-        if ctx.needs_input_grad[1]:
-            # The weight-gradient layout takes row indices on the general kernels only, which are
-            # several times slower than the streaming ones: one explicit gather and the streaming
-            # kernel is the faster way to the same result.
-            sorted_x = x.index_select(0, row_index)
-            lhs, rhs = (grad, sorted_x) if ctx.trans_b else (sorted_x, grad)
-            wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
         return xgrad, wgrad, None, None, None
 
 
@@ -96,10 +95,7 @@ class GroupedGemmScatter(torch.autograd.Function):
             # (as in GroupedGemmGather: an explicit gather, then the streaming weight-gradient kernel;
             # the input gradient takes the sorted rows too where they are there)
             sorted_grad = grad.index_select(0, row_index)
-            lhs, rhs = (sorted_grad, a) if ctx.trans_b else (a, sorted_grad)
-            wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
-            if ctx.needs_input_grad[0]:
-                agrad = backend.gmm(sorted_grad, w, batch_sizes, trans_b=not ctx.trans_b)
+            agrad, wgrad = backend.gradients(sorted_grad, a, w, batch_sizes, ctx.trans_b, ctx.needs_input_grad[0], True)
         elif ctx.needs_input_grad[0]:
             agrad = backend.gmm_indexed(grad, w, batch_sizes, trans_b=not ctx.trans_b, a_rows=row_index)
         return agrad, wgrad, None, None, None
@@ -143,12 +139,7 @@ class GroupedGemmSwiGLU(torch.autograd.Function):
             g32 = grad.float()
             dgate = g32 * up * sig * (1.0 + gate * (1.0 - sig))
             dgu = torch.cat([dgate, g32 * gate * sig], dim=-1).to(a.dtype)
-        agrad = wgrad = None
-        if ctx.needs_input_grad[0]:
-            agrad = backend.gmm(dgu, w, batch_sizes, trans_b=not ctx.trans_b)
-        if ctx.needs_input_grad[1]:
-            lhs, rhs = (dgu, a) if ctx.trans_b else (a, dgu)
-            wgrad = backend.gmm(lhs, rhs, batch_sizes, trans_a=True)
+        agrad, wgrad = backend.gradients(dgu, a, w, batch_sizes, ctx.trans_b, ctx.needs_input_grad[0], ctx.needs_input_grad[1])
         return agrad, wgrad, None, None
 
 

@@ -227,6 +227,16 @@ typedef struct gg_gmm_args {
 int gg_gmm(const gg_gmm_args* args);
 
 /*
+ * Two independent calls, neither of which reads what the other writes: the same results as
+ * gg_gmm(first) followed by gg_gmm(second), in one launch where that is possible (a product with plain
+ * rows and epilogue, then a weight gradient over the same batch_sizes, stream and tokens, two-byte elements:
+ * the two gradients of a product).  Compute units that run out of tiles of the first then go on with the
+ * second.  The two must not share a workspace; where they do, they are launched one after the other.
+ * No counterpart in the reference, whose backward makes two calls (grouped_gemm/ops.py:19-29).
+ */
+int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second);
+
+/*
  * Bytes of workspace the call described by `args` can make use of: 0 when no launch of it ever
  * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8, or a
  * product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte

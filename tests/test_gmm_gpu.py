@@ -2540,6 +2540,75 @@ def test_gpu_validation_errors(ops):
         ops.backend.gmm(a, b, bs, trans_a=True, trans_b=True)
 
 
+@pytest.mark.parametrize("on_device", [False, True])
+@pytest.mark.parametrize("experts,rows,hin,hout,trans_b,skew", [
+    (8, 1024, 128, 128, False, 0),       # small tiles of both
+    (6, 570, 208, 2880, False, 0),       # one round of the first, cut along the depth
+    (32, 4096, 768, 2048, True, 0),      # short tiles that leave workgroups idle, shallow weight gradient
+    (8, 8192, 2048, 1368, False, 0),     # extra tiles for the workgroups that start early
+    (4, 4600, 1032, 264, True, 0),       # a row width off 64-byte boundaries
+    (8, 16000, 264, 520, False, 3),      # deep groups of the weight gradient, cut and first
+    (3, 40, 8, 16, True, 1),             # less than a tile
+    (5, 300, 130, 262, False, 0),        # even sizes
+])
+def test_both_gradients_in_one_launch(ops, oracle, experts, rows, hin, hout, trans_b, skew, on_device):
+    # The pair launch against the two calls: the same tiles, pieces and sums, so the same bits, except where
+    # the last round is cut differently (fp32 sums in another order); rows past the last group are not touched by
+    # either, and an expert without rows gets a gradient of zeros.
+    _announce("pair", experts, rows, hin, hout, trans_b, skew, on_device)
+    g = torch.Generator().manual_seed(rows)
+    share = torch.rand(experts, generator=g) ** (1 + 4 * skew)
+    share[experts // 2] = 0
+    sizes = torch.bincount(torch.multinomial(share, rows - 3, replacement=True, generator=g), minlength=experts)
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    a, grad = draw(rows, hin), draw(rows, hout)
+    b = draw(*((experts, hout, hin) if trans_b else (experts, hin, hout)))
+    bs = sizes.cuda() if on_device else sizes
+    used = rows - 3
+    lhs, rhs = (grad, a) if trans_b else (a, grad)
+    want_a = oracle.gmm_loop(grad, b, sizes, trans_b=not trans_b)
+    want_b = oracle.gmm_loop(lhs, rhs, sizes, trans_a=True)
+    first = None
+    for _ in range(3):   # (the workspaces' counters are left as they were found)
+        agrad, bgrad = ops.backend.backend.gmm_gradients(grad, a, b, bs, trans_b)
+        check(agrad[:used], want_a[:used], "input gradient")
+        check(bgrad, want_b, "weight gradient")
+        assert not bgrad[experts // 2].any()
+        first = first or (agrad.clone(), bgrad.clone())
+        assert torch.equal(agrad[:used], first[0][:used]) and torch.equal(bgrad, first[1])
+    alone_a = ops.backend.gmm(grad, b, bs, trans_b=not trans_b)[:used].float()
+    alone_b = ops.backend.gmm(lhs, rhs, bs, trans_a=True).float()
+    # one rounding of c may fall the other way: 2 ** -8 of an element, few of them
+    for got, alone in ((first[0][:used].float(), alone_a), (first[1].float(), alone_b)):
+        assert ((got - alone).abs() <= 2.0 ** -7 * alone.abs() + 1e-4 * alone.abs().max()).all()
+
+
+def test_both_gradients_in_one_launch_inside_a_graph(ops):
+    sizes = torch.tensor([700, 0, 300, 500], dtype=torch.int64).cuda()
+    g = torch.Generator().manual_seed(41)
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    a, b, grad = draw(1500, 264), draw(4, 264, 6400), draw(1500, 6400)
+    run = lambda: ops.backend.backend.gmm_gradients(grad, a, b, sizes, False)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        agrad, bgrad = run()
+    for new_sizes in ([700, 0, 300, 500], [1500, 0, 0, 0], [1, 2, 3, 1494], [375] * 4):
+        _announce("pair replay", new_sizes)
+        sizes.copy_(torch.tensor(new_sizes, dtype=torch.int64))
+        agrad.fill_(7.0)
+        bgrad.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = run()
+        assert torch.equal(agrad, eager[0]) and torch.equal(bgrad, eager[1]), new_sizes
+
+
 def test_needs_input_grad_is_respected(ops):
     a = torch.randn(64, 32, device="cuda").to(torch.bfloat16).requires_grad_(True)
     b = torch.randn(2, 32, 40, device="cuda").to(torch.bfloat16)
