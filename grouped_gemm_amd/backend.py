@@ -54,8 +54,13 @@ def _output_dtype(dtype):
 # Needing no copies: two-byte operands on 4-byte boundaries whose hidden sizes are both even.
 
 
-def _round_up(x, m):
-    return (x + m - 1) // m * m
+def _padded_size(n, itemsize):
+    """The hidden size that n is padded to: what the streaming kernels need (16-byte rows), and where that adds
+    little, rows of whole lines (128 bytes), or sectors (64), which neither loads nor stores share with the
+    next row.  8 x 1024 rows, 2047 -> 5461, forward and gradients, padded to 5464 / 5504: 910 / 877 us."""
+    align = 128 if n * itemsize >= 2048 else (64 if n * itemsize >= 512 else 16)
+    m = align // itemsize
+    return (n + m - 1) // m * m
 
 
 def _needs_padding(a, b, c, batch_sizes, trans_a, trans_b):
@@ -102,8 +107,7 @@ def _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
     """gmm through zero-padded copies, for operands that _needs_padding accepts."""
     hin = a.shape[1]
     hout = b.shape[1] if (trans_a or trans_b) else b.shape[2]
-    mult = 16 if a.element_size() == 1 else 8
-    hin_p, hout_p = _round_up(hin, mult), _round_up(hout, mult)
+    hin_p, hout_p = _padded_size(hin, a.element_size()), _padded_size(hout, a.element_size())
     a_p = _padded(a, a.shape[0], hin_p)
     if trans_a:
         b_p = _padded(b, b.shape[0], hout_p)
@@ -157,8 +161,7 @@ def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
             tuple(a.shape) == (grad.shape[0], b.shape[2 if trans_b else 1]):
         # (one padded copy of the gradient serves both products)
         hin, hout = a.shape[1], grad.shape[1]
-        mult = 16 if a.element_size() == 1 else 8
-        hin_p, hout_p = _round_up(hin, mult), _round_up(hout, mult)
+        hin_p, hout_p = _padded_size(hin, a.element_size()), _padded_size(hout, a.element_size())
         grad_p = _padded(grad, grad.shape[0], hout_p)
         b_p = _padded(b, hout_p, hin_p) if trans_b else _padded(b, hin_p, hout_p)
         a_p = _padded(a, a.shape[0], hin_p)
