@@ -416,7 +416,8 @@ struct Plan {
 };
 
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
-int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out) {
+// gate_up: where gate | up are kept beside c (SwiGLU epilogue), or nullptr.
+int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_up = nullptr) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
   const int64_t hidden_in = g.hidden_in, hidden_out = g.hidden_out;
   const int trans_a = g.trans_a != 0, trans_b = g.trans_b != 0;
@@ -471,7 +472,7 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out) {
   if (rc != GG_OK) return rc;
   hipStream_t stream = static_cast<hipStream_t>(g.stream);
   const int layout = trans_a ? gg::kTN : (trans_b ? gg::kNT : gg::kNN);
-  const int epilogue = out_f32 ? gg::kEpiAccF32 : (swiglu ? gg::kEpiSwiGLU : gg::kEpiStore);
+  const int epilogue = out_f32 ? gg::kEpiAccF32 : (gate_up != nullptr ? gg::kEpiSwiGLUKeep : (swiglu ? gg::kEpiSwiGLU : gg::kEpiStore));
   const TileShape shape = generic ? TileShape{-1, gg::kGenericTileM, gg::kGenericTileN} : pick_shape(g, route);
   // deep groups: the launch is bound by the matrix pipe, and atomic additions to c cost less of
   // its time than reading, adding and writing; shallow groups: bound by the traffic of c, the reverse
@@ -491,6 +492,7 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out) {
   p.a = static_cast<const char*>(g.a);
   p.b = static_cast<const char*>(g.b);
   p.c = static_cast<char*>(g.c);
+  p.gate_up = static_cast<char*>(gate_up);
   p.tokens = tokens;
   p.hidden_in = (int32_t)hidden_in;
   p.hidden_out = (int32_t)hidden_out;
@@ -703,6 +705,22 @@ int gg_gmm(const gg_gmm_args* args) {
     return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is %u, this library expects %zu", args->struct_bytes,
                 sizeof(gg_gmm_args));
   return gmm_impl(*args);
+}
+
+int gg_keeps_gate_up(const gg_gmm_args* args) {
+  if (args == nullptr || args->struct_bytes != sizeof(gg_gmm_args)) return 0;
+  if (args->epilogue != GG_EPILOGUE_SWIGLU || (args->dtype != GG_DTYPE_BF16 && args->dtype != GG_DTYPE_F16)) return 0;
+  const Route r = classify(*args);
+  return !r.generic && !r.indexed ? 1 : 0;
+}
+
+int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up) {
+  if (!gg_keeps_gate_up(args)) return fail(GG_EINVAL, "gate | up cannot be kept by this call (gg_keeps_gate_up)");
+  if (gate_up == nullptr || (reinterpret_cast<uintptr_t>(gate_up) & 15))
+    return fail(GG_EINVAL, "gate_up must be on a 16-byte boundary");
+  Plan plan;
+  const int rc = plan_call(*args, false, &plan, gate_up);
+  return rc != GG_OK ? rc : launch_call(*args, &plan);
 }
 
 int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) {

@@ -72,6 +72,7 @@ struct GmmParams {
   uint32_t c_bytes;
   uint32_t a_index_rows;   // rows of a and of c in memory: an index that names no row of them is a
   uint32_t c_index_rows;   // missing row (read as zeros, not stored)
+  char* gate_up;           // kEpiSwiGLUKeep: (tokens, 2 hidden_out), rows like those of c
   int32_t* status;         // device word that collects kStatus* bits about the sizes, or nullptr
 };
 
@@ -88,6 +89,7 @@ enum : int {
   // by the matrix pipe (deep groups: 3.35 -> 3.16 ms at 8 x 4096 rows, 4096 x 14336), much slower
   // when it is bound by the traffic of c itself (256 x 256 rows, 2048 x 7168: 7.0 -> 11.7 ms)
   kEpiAccF32Atomic = 3,
+  kEpiSwiGLUKeep = 4,   // kEpiSwiGLU that also stores gate | up, rounded, for the gradient
 };
 
 enum : int {   // debugging switches, for comparing the ways a call can be scheduled
@@ -1344,7 +1346,7 @@ template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, i
 __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& hs, char* smem, const int w, const int G, const PART& part) {
   using Cfg = GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>;
   constexpr int NT = Cfg::NT, MB = Cfg::MB, NB = Cfg::NB, KS = BK / 16;
-  constexpr bool ACC_F32 = EPI == kEpiAccF32 || EPI == kEpiAccF32Atomic, GATE_UP = EPI == kEpiSwiGLU;
+  constexpr bool ACC_F32 = EPI == kEpiAccF32 || EPI == kEpiAccF32Atomic, KEEP = EPI == kEpiSwiGLUKeep, GATE_UP = EPI == kEpiSwiGLU || KEEP;
   // One-byte elements (NT layout only: both operands depth-contiguous).  The tile movers see them
   // as two-byte elements, two to one: same bytes per row and slice, BK_ELEMS depth values a slice.
   constexpr bool F8 = is_f8(DT);
@@ -1352,6 +1354,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   static_assert(!F8 || !GATE_UP || LAYOUT == kNT, "fp8 with gate | up rows streams in the NT layout only");
   static_assert(!ACC_F32 || LAYOUT == kTN, "the fp32 accumulator is the weight gradient's");
   static_assert(!(GATE_UP || INDEXED) || LAYOUT != kTN, "row indices and gate | up are for the NN and NT layouts");
+  static_assert(!KEEP || (!F8 && !INDEXED), "gate | up are kept for two-byte elements and rows in place");
   static_assert(!GATE_UP || NB % 2 == 0, "a wave needs the gate and the up block of its columns");
   constexpr int BNS = GATE_UP ? BN / 2 : BN;   // output columns per tile, what the schedule counts in
   // (width-major tiles of one-byte elements: half as many two-byte elements per depth row, twice
@@ -1626,6 +1629,11 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
     return make_rsrc(p.c + (tile.g.c_off + (int64_t)tile.m0 * tile.g.n) * CE,
                      tile.rows_valid > 0 ? (uint32_t)(tile.rows_valid * tile.g.n) * (uint32_t)CE : 0u);
   };
+  // ... and, KEEP, of the gate | up rows beside them, twice as long
+  auto gate_up_rsrc = [&](const TileInfo& tile) {
+    return make_rsrc(p.gate_up + (tile.g.c_off + (int64_t)tile.m0 * tile.g.n) * 4,
+                     tile.rows_valid > 0 ? (uint32_t)(tile.rows_valid * tile.g.n) * 4u : 0u);
+  };
   auto c_row = [&](const TileInfo& tile, int row) -> uint32_t {
     if constexpr (INDEXED) {
       if (row >= tile.rows_valid) return C_OOR;
@@ -1817,22 +1825,58 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         u32x4 held[32 / ROWS];   // (one strip behind, as below)
         uint32_t held_off[32 / ROWS];
         const bool merge = uniform(p.flags & kFlagMergeStores) != 0;
-        auto store_held = [&]() {
+        // What is held, to columns at_col .. +7 of the rows at held_off.
+        auto store_held_to = [&](const __amdgpu_buffer_rsrc_t& to, int at_col) {
+          auto chunk_at = [&](int r) {
+            return col < ti.g.n && (!INDEXED || held_off[r] != C_OOR) ? held_off[r] + (uint32_t)at_col * 2u : OOR;
+          };
           if (merge) {
 #pragma unroll
             for (int r = 0; r < 32 / ROWS; ++r)
-              __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, at(held_off[r], col), 0, kStoreMerging);
+              __builtin_amdgcn_raw_buffer_store_b128(held[r], to, chunk_at(r), 0, kStoreMerging);
           } else {
 #pragma unroll
             for (int r = 0; r < 32 / ROWS; ++r)
-              __builtin_amdgcn_raw_buffer_store_b128(held[r], rc, at(held_off[r], col), 0, kStoreStreaming);
+              __builtin_amdgcn_raw_buffer_store_b128(held[r], to, chunk_at(r), 0, kStoreStreaming);
           }
+        };
+        auto hold_strip = [&](const uint32_t* row_off) {
+#pragma unroll
+          for (int r = 0; r < 32 / ROWS; ++r) {
+            held[r] = *reinterpret_cast<const u32x4*>(strip + (r * ROWS + out_row) * PITCH + out_chunk * 16);
+            held_off[r] = row_off[r];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        auto into_strip = [&](int jp, int q, u32x2 v) {
+          *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jp * 32 + 8 * q + 4 * in_half) * 2) = v;
         };
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
           uint32_t row_off[32 / ROWS];
 #pragma unroll
           for (int r = 0; r < 32 / ROWS; ++r) row_off[r] = row_offset((wm + i * WAVES_M) * 32 + r * ROWS + out_row);
+          if constexpr (KEEP) {
+            // The gate columns, then the up columns, as the plain epilogue would store them (16 x 1024 rows,
+            // 2048 -> 4096: 520 us, 590 with them; the product that the backward would run for them: 490).
+            const __amdgpu_buffer_rsrc_t rg = gate_up_rsrc(ti);
+            uint32_t keep_off[32 / ROWS];
+#pragma unroll
+            for (int r = 0; r < 32 / ROWS; ++r) keep_off[r] = 2 * row_off[r];
+#pragma unroll
+            for (int part = 0; part < 2; ++part) {
+#pragma unroll
+              for (int jp = 0; jp < NB / 2; ++jp)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) into_strip(jp, q, take4(i, 2 * jp + part, q));
+              if (part == 1) {
+                store_held_to(rg, col);
+              } else if (i > 0) {
+                store_held_to(rc, col);
+              }
+              hold_strip(keep_off);
+            }
+          }
 #pragma unroll
           for (int jp = 0; jp < NB / 2; ++jp) {
 #pragma unroll
@@ -1843,19 +1887,17 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
                 asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(gate[r]) : "a"(acc[i][2 * jp][4 * q + r]));
                 asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(up[r]) : "a"(acc[i][2 * jp + 1][4 * q + r]));
               }
-              *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jp * 32 + 8 * q + 4 * in_half) * 2) =
-                  combine4(gate, up);
+              into_strip(jp, q, combine4(gate, up));
             }
           }
-          if (i > 0) store_held();
-#pragma unroll
-          for (int r = 0; r < 32 / ROWS; ++r) {
-            held[r] = *reinterpret_cast<const u32x4*>(strip + (r * ROWS + out_row) * PITCH + out_chunk * 16);
-            held_off[r] = row_off[r];
+          if constexpr (KEEP) {
+            store_held_to(gate_up_rsrc(ti), ti.g.n + col);
+          } else {
+            if (i > 0) store_held_to(rc, col);
           }
-          __builtin_amdgcn_sched_barrier(0);
+          hold_strip(row_off);
         }
-        store_held();
+        store_held_to(rc, col);
       } else if constexpr (ACC_F32) {
         if constexpr (EPI == kEpiAccF32Atomic) {
           // c += product in fp32, by atomic additions that return nothing: the wave fires them and
@@ -2091,6 +2133,13 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
             for (int r = 0; r < 4; ++r) gate[r] = sum[2 * jp][q][r], up[r] = sum[2 * jp + 1][q][r];
             const int col = ft.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
             __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, c_at(ft, row_off, col), 0, kStoreMerging);
+            if constexpr (KEEP) {
+              const __amdgpu_buffer_rsrc_t rg = gate_up_rsrc(ft);
+              const uint32_t gate_off = col < ft.g.n ? 2 * row_off + (uint32_t)col * 2u : C_OOR;
+              const uint32_t up_off = col < ft.g.n ? 2 * row_off + (uint32_t)(ft.g.n + col) * 2u : C_OOR;
+              __builtin_amdgcn_raw_buffer_store_b64(round4<OUT_DT>(gate[0], gate[1], gate[2], gate[3]), rg, gate_off, 0, kStoreMerging);
+              __builtin_amdgcn_raw_buffer_store_b64(round4<OUT_DT>(up[0], up[1], up[2], up[3]), rg, up_off, 0, kStoreMerging);
+            }
           }
       } else {
 #pragma unroll

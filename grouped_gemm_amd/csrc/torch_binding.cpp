@@ -427,6 +427,28 @@ void GroupedGemmSwiGLU(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch:
   Run(a, b, c, batch_sizes, /*trans_a=*/false, trans_b, /*accumulate_f32=*/false, /*flags=*/0, rows, /*gate_up=*/true);
 }
 
+// The same for a gradient to come: c, and gate | up (tokens, 2 * hidden_out) as gmm(a, b) would give them; nothing (and
+// nothing done) for calls whose kernels do not keep them.
+c10::optional<std::pair<torch::Tensor, torch::Tensor>> GroupedGemmSwiGLUKeep(const torch::Tensor& a, const torch::Tensor& b,
+                                                                             const torch::Tensor& batch_sizes, bool trans_b) {
+  if (!IsDirect(a, b, batch_sizes, false, trans_b, nullptr) || IsFloat8(a.scalar_type())) return c10::nullopt;
+  const int64_t cols = trans_b ? b.size(1) : b.size(2);
+  if (cols % 16 != 0) return c10::nullopt;   // (odd numbers of columns are rejected, others run on the general kernels)
+  torch::Tensor c = torch::empty({a.size(0), cols / 2}, a.options());
+  Validate(a, b, c, batch_sizes, false, trans_b, /*on_device=*/true, RowIndices(), /*gate_up=*/true);
+  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(a.device().index()).stream();
+  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+  gg_gmm_args g = Arguments(a, b, c, sizes, false, trans_b, false, 0, RowIndices(), true, stream);
+  if (!gg_keeps_gate_up(&g)) return c10::nullopt;
+  torch::Tensor gate_up = torch::empty({a.size(0), cols}, a.options());
+  const torch::Tensor workspace = AttachWorkspace(&g, a.device(), stream);
+  const int rc = gg_gmm_keep_gate_up(&g, gate_up.data_ptr());
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+  return std::make_pair(c, gate_up);
+}
+
 // Gradients of gate | up (rows, 2 * cols) from the gradient of silu(gate) * up (rows, cols); see
 // gg_swiglu_backward.
 torch::Tensor SwiGLUBackward(torch::Tensor gate_up, torch::Tensor grad) {
@@ -560,6 +582,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gmm_swiglu", &GroupedGemmSwiGLU, "silu(a @ gate) * (a @ up) with b = [gate | up].", py::arg("a"),
         py::arg("b"), py::arg("c"), py::arg("batch_sizes"), py::arg("trans_b"), py::arg("a_rows") = py::none(),
         py::arg("c_rows") = py::none());
+  m.def("gmm_swiglu_keep", &GroupedGemmSwiGLUKeep, "gmm_swiglu, and gate | up for its gradient; None where they are not kept.");
   m.def("swiglu_backward", &SwiGLUBackward, "Gradients of gate | up from the gradient of silu(gate) * up.");
   m.def("sum_rows", &SumRows, "Row d of the result is the sum of the rows of src that row_index sends there.");
   m.def("pad_rows", &PadRows, "A zero-padded copy with `rows` rows of `cols` elements per batch.");

@@ -237,6 +237,15 @@ int gg_gmm(const gg_gmm_args* args);
 int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second);
 
 /*
+ * gg_gmm with GG_EPILOGUE_SWIGLU that also stores the two products, rounded to the element type, for the
+ * gradient (gg_swiglu_backward): gate_up (tokens, 2 * hidden_out), gate first, rows like those of c, 16-byte
+ * aligned.  For calls for which gg_keeps_gate_up returns 1: two-byte elements, no row indices, sizes and
+ * alignment that the streaming kernels take.  No counterpart in the reference.
+ */
+int gg_keeps_gate_up(const gg_gmm_args* args);
+int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up);
+
+/*
  * Bytes of workspace the call described by `args` can make use of: 0 when no launch of it ever
  * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8, or a
  * product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte

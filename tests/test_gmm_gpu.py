@@ -2149,6 +2149,52 @@ def _nearest_to_a_rounding_boundary(factor):
     return best.half()
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("experts,rows,hin,hout,dtype", [
+    (5, 2600, 264, 1304, torch.bfloat16),     # full tiles, a partly filled last column
+    (3, 4100, 512, 256, torch.float16),       # ... of every count of 32-row blocks
+    (8, 700, 192, 520, torch.bfloat16),       # one round of short tiles
+    (4, 90, 128, 72, torch.float16),          # small tiles
+    (8, 120, 7168, 2048, torch.bfloat16),     # short tiles cut along the depth
+    (2, 40, 6400, 128, torch.float16),        # small ones
+])
+def test_swiglu_keeps_gate_and_up(ops, experts, rows, hin, hout, dtype, trans_b):
+    # The products kept beside the activation against a plain launch (another tile shape may add up in
+    # another order: half a unit of the element type each, and fp32 sums), the activation bit for bit.
+    _announce("keep gate | up", experts, rows, hin, hout, dtype, trans_b)
+    g = torch.Generator().manual_seed(rows)
+    share = torch.rand(experts, generator=g) + 0.02
+    share[experts // 2] = 0
+    sizes = torch.bincount(torch.multinomial(share, rows - 2, replacement=True, generator=g), minlength=experts).cuda()
+    used = rows - 2
+    a = torch.randn(rows, hin, generator=g).to(dtype).cuda()
+    w = (torch.randn(*((experts, 2 * hout, hin) if trans_b else (experts, hin, 2 * hout)), generator=g) * hin ** -0.5).to(dtype).cuda()
+    for _ in range(2):
+        c, gate_up = ops.backend.backend.gmm_swiglu_keep(a, w, sizes, trans_b)
+        assert torch.equal(c[:used], ops.backend.gmm_swiglu(a, w, sizes, trans_b=trans_b)[:used])
+        want = ops.backend.gmm(a, w, sizes, trans_b=trans_b)[:used].float()
+        unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        assert ((gate_up[:used].float() - want).abs() <= 2 * unit * want.abs() + 1e-5 * hin ** 0.5).all()
+
+
+def test_swiglu_gradients_from_kept_and_recomputed_products(ops):
+    # The memory rule: kept where no larger than the operands; both ways give the same gradients.
+    g = torch.Generator().manual_seed(5)
+    sizes = torch.tensor([300, 0, 212], dtype=torch.int64).cuda()
+    for hin, hout, kept in ((256, 264, True), (64, 640, False)):
+        draw = lambda *shape: (torch.randn(*shape, generator=g) * 0.2).to(torch.bfloat16).cuda().requires_grad_(True)
+        a, w = draw(512, hin), draw(3, hin, 2 * hout)
+        upstream = draw(512, hout).detach()
+        out = ops.gmm_swiglu(a, w, sizes)
+        assert len(out.grad_fn.saved_tensors) == (4 if kept else 3)
+        again = ops.GroupedGemmSwiGLU.apply(a, w, sizes, False)
+        assert len(again.grad_fn.saved_tensors) == 3
+        for x, y in zip(torch.autograd.grad(out, (a, w), upstream), torch.autograd.grad(again, (a, w), upstream)):
+            check(x, y.float(), f"gradients, {hin} -> {hout}")
+    with torch.no_grad():
+        assert ops.gmm_swiglu(a, w, sizes).grad_fn is None
+
+
 @pytest.mark.parametrize("sizes", [[4096] * 8, [40] * 700, [60, 64, 33]])
 def test_swiglu_epilogue_divides_in_full_precision(ops, sizes):
     # silu(gate) * up of known pre-activations (rows times an identity), `up` chosen so that the product lies as
