@@ -344,7 +344,11 @@ __device__ __forceinline__ GroupTiles group_tiles(int rows, int hidden_in, int h
     g.tiles_m = (rows + BM - 1) / BM;
     g.height = BM;
     if (g.tiles_m > 0) {
-      g.height = ((rows + g.tiles_m - 1) / g.tiles_m + 31) / 32 * 32;
+      // rows / tiles_m rounded up to whole blocks: 1 .. BM / 32 of them, counted instead of divided out
+      int blocks = 1;
+#pragma unroll
+      for (int h = 1; h < BM / 32; ++h) blocks += (uint32_t)(h * 32) * (uint32_t)g.tiles_m < (uint32_t)rows ? 1 : 0;
+      g.height = blocks * 32;
       const int last_blocks = (rows - (g.tiles_m - 1) * g.height + 31) / 32;
       g.runt = g.tiles_m >= 2 && 2 * last_blocks <= g.height / 32 && !(flags & kFlagOneClass) ? 1 : 0;
     }
@@ -353,10 +357,28 @@ __device__ __forceinline__ GroupTiles group_tiles(int rows, int hidden_in, int h
   return g;
 }
 
-// Run by the first wave of a workgroup.  Each lane owns up to 8 consecutive groups; one
-// wave-wide scan of int64 row counts and one of the two int32 tile counts.  Every size is
-// clamped to [0, tokens] before it enters a sum, so no size vector can make a sum overflow or a
-// group start before row 0 or end past row `tokens`.
+// Inclusive scan over the lanes of a wave by `op`, whose identity is 0: data-parallel moves, a few cycles
+// each, where a shuffle goes through LDS.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROW_MASK, 0xf, false);
+}
+template <typename OP>
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x, OP op) {
+  x = op(x, dpp_or_zero<0x111, 0xf>(x));   // row_shr:1, 2, 4, 8: inside rows of 16 lanes
+  x = op(x, dpp_or_zero<0x112, 0xf>(x));
+  x = op(x, dpp_or_zero<0x114, 0xf>(x));
+  x = op(x, dpp_or_zero<0x118, 0xf>(x));
+  x = op(x, dpp_or_zero<0x142, 0xa>(x));   // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3
+  return op(x, dpp_or_zero<0x143, 0xc>(x));
+}
+
+// Run by the first wave of a workgroup.  Each lane owns up to 8 consecutive groups; one wave-wide scan of row
+// counts and one of each of the two tile counts.  Every size is clamped to [0, tokens] before it enters a
+// sum, and sums of rows stay at 2^32 - 1 once they are there (tokens is below 2^31), so no size vector can make a
+// sum overflow or a group start before row 0 or end past row `tokens`.
+// Every launch starts with this: 2.4 us of the 7 of a small one, most of it in divisions, 1.3 without them
+// and with data-parallel moves for the scans.
 template <int LAYOUT, int BM, int BN>
 __device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, const HostSizes& hs, int w) {
   const int lane = threadIdx.x;
@@ -364,97 +386,84 @@ __device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, con
   const int E = p.num_groups;
   const int per = (E + 63) >> 6;
   const int e0 = lane * per;
+  const uint32_t tokens = (uint32_t)p.tokens;
   int bad = 0;   // kStatus* bits seen by this lane
   auto clamp = [&](int64_t v) {
     if (v < 0) bad |= kStatusNegativeSize;
     if (v > p.tokens) bad |= kStatusRowsPastEnd;
-    return v < 0 ? (int64_t)0 : (v > p.tokens ? p.tokens : v);
+    return v < 0 ? 0u : (v > p.tokens ? tokens : (uint32_t)v);
   };
+  auto add = [](uint32_t x, uint32_t y) { return x + y; };
+  auto add_sat = [](uint32_t x, uint32_t y) { return __builtin_elementwise_add_sat(x, y); };
+  auto larger = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
   // rows taken by the groups before this launch's first one
-  int64_t base = p.row_base;
+  uint32_t base = (uint32_t)(p.row_base < (int64_t)0xffffffffll ? p.row_base : (int64_t)0xffffffffll);
   if (p.sizes_dev != nullptr && p.first_group > 0) {
-    int64_t part = 0;
-    for (int i = lane; i < p.first_group; i += 64) part += clamp(p.sizes_dev[i]);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) part += __shfl_xor(part, d);
-    base = part;
+    uint32_t part = 0;
+    for (int i = lane; i < p.first_group; i += 64) part = add_sat(part, clamp(p.sizes_dev[i]));
+    base = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(part, add_sat), 63);
   }
-  int64_t sz[8];
-  int64_t sum = 0;
+  uint32_t sz[8];
+  uint32_t sum = 0;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int e = e0 + i;
-    int64_t v = 0;
-    if (i < per && e < E) {
-      v = p.sizes_dev != nullptr ? p.sizes_dev[p.first_group + e] : (int64_t)hs.v[e];
-      v = clamp(v);
+    sz[i] = 0;
+    if (i < per) {   // (the same in every lane: groups that no lane has cost nothing)
+      const int e = e0 + i;
+      if (e < E) sz[i] = clamp(p.sizes_dev != nullptr ? p.sizes_dev[p.first_group + e] : (int64_t)hs.v[e]);
+      sum = add_sat(sum, sz[i]);
     }
-    sz[i] = v;
-    sum += v;
   }
-  int64_t incl = sum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int64_t o = __shfl_up(incl, d);
-    if (lane >= d) incl += o;
-  }
-  int64_t run = base + incl - sum;
-  int rows[8];
-  int tsum = 0, rsum = 0;
+  // (what the lanes before this one add up to, not this one's sum less: sums may be at their limit)
+  uint32_t run = wave_scan(sum, add_sat);
+  const uint32_t all = add_sat(base, (uint32_t)__builtin_amdgcn_readlane((int)run, 63));
+  run = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)run, 0x138, 0xf, 0xf, false);   // wave_shr:1
+  run = add_sat(base, run);
+  uint32_t main_tiles[8], runt_tiles[8];
+  uint32_t tsum = 0, rsum = 0, most = 0;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int e = e0 + i;
-    const int64_t start = run < p.tokens ? run : p.tokens;
-    const int64_t left = p.tokens - start;
-    const int r = (int)(sz[i] < left ? sz[i] : left);
-    rows[i] = r;
-    if (i < per && e < E) {
-      s->row_start[e] = (int)start;
-      s->rows[e] = r;
-      const GroupTiles g = group_tiles<LAYOUT, BM, BN>(r, p.hidden_in, p.hidden_out, p.flags);
-      tsum += g.main_rows * g.tiles_n;
-      rsum += g.runt * g.tiles_n;
-    }
-    run += sz[i];
-  }
-  int tincl = tsum, rincl = rsum;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int o = __shfl_up(tincl, d);
-    const int o2 = __shfl_up(rincl, d);
-    if (lane >= d) {
-      tincl += o;
-      rincl += o2;
+    main_tiles[i] = runt_tiles[i] = 0;
+    if (i < per) {
+      const int e = e0 + i;
+      const uint32_t start = run < tokens ? run : tokens, left = tokens - start;
+      const uint32_t rows = sz[i] < left ? sz[i] : left;
+      if (e < E) {
+        s->row_start[e] = (int)start;
+        s->rows[e] = (int)rows;
+        const GroupTiles g = group_tiles<LAYOUT, BM, BN>((int)rows, p.hidden_in, p.hidden_out, p.flags);
+        main_tiles[i] = (uint32_t)(g.main_rows * g.tiles_n);
+        runt_tiles[i] = (uint32_t)(g.runt * g.tiles_n);
+        most = larger(most, rows);
+      }
+      tsum += main_tiles[i];
+      rsum += runt_tiles[i];
+      run = add_sat(run, sz[i]);
     }
   }
-  int trun = tincl - tsum, rrun = rincl - rsum;
+  const uint32_t tincl = wave_scan(tsum, add), rincl = LAYOUT == kTN ? 0u : wave_scan(rsum, add);
+  most = wave_scan(most, larger);
+  uint32_t trun = tincl - tsum, rrun = rincl - rsum;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const int e = e0 + i;
-    if (i < per && e < E) {
-      s->tile_start[e] = trun;
-      s->runt_start[e] = rrun;
-      const GroupTiles g = group_tiles<LAYOUT, BM, BN>(rows[i], p.hidden_in, p.hidden_out, p.flags);
-      trun += g.main_rows * g.tiles_n;
-      rrun += g.runt * g.tiles_n;
+    if (i < per) {
+      const int e = e0 + i;
+      if (e < E) {
+        s->tile_start[e] = (int)trun;
+        s->runt_start[e] = (int)rrun;
+      }
+      trun += main_tiles[i];
+      rrun += runt_tiles[i];
     }
-  }
-  int most = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) most = rows[i] > most ? rows[i] : most;
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    const int o = __shfl_xor(most, d);
-    most = o > most ? o : most;
   }
   if (lane == 63) {
     s->front_tiles = 0;
     s->front_pieces = 1;
-    s->most_rows = most;
-    s->row_start[E] = (int)(run < p.tokens ? run : p.tokens);
-    s->tile_start[E] = tincl;
-    s->runt_start[E] = rincl;
-    if (run > p.tokens) bad |= kStatusRowsPastEnd;
+    s->most_rows = (int)most;
+    s->row_start[E] = (int)(all < tokens ? all : tokens);
+    s->tile_start[E] = (int)tincl;
+    s->runt_start[E] = (int)rincl;
+    if (all > tokens) bad |= kStatusRowsPastEnd;
   }
   // What the host would have rejected in host-resident sizes is reported for device-resident
   // ones: one workgroup ORs what its first wave saw into the caller's status word.
@@ -478,10 +487,16 @@ __device__ __forceinline__ void order_groups_by_depth(Sched* s, int num_groups, 
     for (int e = threadIdx.x; e < num_groups; e += blockDim.x) {
       const int mine = s->rows[e];
       int before = 0;
-      for (int j = 0; j < num_groups; ++j) {
-        const int other = s->rows[j];   // (the same address in every lane: a broadcast read)
-        before += (other > mine || (other == mine && j < e)) ? 1 : 0;
+      auto count = [&](int other, int j) { before += (other > mine || (other == mine && j < e)) ? 1 : 0; };
+      int j = 0;
+      for (; j + 8 <= num_groups; j += 8) {   // (eight reads in flight, the same addresses in every lane)
+        int other[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) other[k] = s->rows[j + k];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) count(other[k], j + k);
       }
+      for (; j < num_groups; ++j) count(s->rows[j], j);
       s->order[before] = (int16_t)e;
     }
     __syncthreads();
@@ -1231,7 +1246,9 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
   // read through the first lane: everything derived from these stays in scalar registers
   const int rows = uniform(sched->rows[e]);
   ti.g = group_geometry<LAYOUT>(p, p.first_group + e, uniform(sched->row_start[e]), rows);
-  const GroupTiles gt = group_tiles<LAYOUT, BM, BN>(rows, p.hidden_in, p.hidden_out, p.flags);
+  GroupTiles gt = group_tiles<LAYOUT, BM, BN>(rows, p.hidden_in, p.hidden_out, p.flags);
+  gt.height = uniform(gt.height);
+  gt.main_rows = uniform(gt.main_rows);
   int tm, tn;
   if (cur.cls == 0) {
     tile_coords(u, gt.main_rows, gt.tiles_n, p.group_m, &tm, &tn);

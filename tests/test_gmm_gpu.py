@@ -806,6 +806,25 @@ def test_schedule_saturates_huge_and_negative_sizes(ops):
             assert (got[:, 6:9] >= 0).all()
 
 
+@pytest.mark.parametrize("groups", [1, 2, 15, 17, 63, 64, 65, 127, 129, 255, 257, 511, 512])
+def test_schedule_sums_over_lanes(ops, groups):
+    # A wave sums up to eight groups per lane: rows and starts clipped at `tokens` against Python's integers, at
+    # every number of groups where lanes or rows of lanes are partly filled, also with sums past 2^32.
+    rng = np.random.default_rng(groups)
+    for tokens in (3000, (1 << 31) - 1):
+        sizes = rng.integers(0, 2 * tokens // groups + 2, groups)
+        sizes[rng.integers(groups)] = -7
+        if groups > 2:
+            sizes[rng.integers(groups)] = tokens + 5
+        got = ops.backend.debug_schedule(torch.from_numpy(sizes).cuda(), tokens, 8, 8).cpu().numpy()
+        start = 0
+        for e, size in enumerate(sizes.tolist()):
+            size = min(max(size, 0), tokens)
+            begin = min(start, tokens)
+            assert got[e, 6] == begin * 8 and got[e, 11] == min(size, tokens - begin), (groups, tokens, e)
+            start += size
+
+
 # ----------------------------------------------------------------- C ABI, directly
 
 def _c_abi():
