@@ -357,9 +357,13 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 18.1 and 39.0 / 24.9; 16 x 1024, 512 x 1024 (512): 28.3 / 25.2 and 70.7 / 40.6 (the deepest group's tiles set the
 // length of the launch: four times as many take a quarter of the time each); past that line even
 // depths lose: 64 x 256, 256 x 768 (768): 18.3 / 20.0; 16 x 256, 1024 x 1024 (1024): 19.7 / 22.6.  Groups of
+// kMiddlingGroups rows gain up to four rounds of small tiles, where the depth of a tile counts for more than its
+// traffic (both gradients in one launch): 9 x 613, 1792 x 960 (1008): 79 / 66; 11 x 980, 1088 x 1088 (891): 82 / 73; 6 x 1784, 1792 x 1088
+// (756): 120 / 111; 15 x 1627, 2368 x 256 (570): 91 / 96; of fewer rows 26 x 318, 192 x 1312 (572): 30 / 38.  Groups of
 // kDeepGroups rows and more keep the wide ones: where a few of them are much deeper than the rest,
 // those are cut along the depth (plan_deep_tiles).
 constexpr int64_t kDeepGroups = 2560;
+constexpr int64_t kMiddlingGroups = 512;
 constexpr int64_t kDeepProduct = 6144;       // weights are pulled through short tiles
 constexpr int64_t kDeepForSharing = 3072;    // small tiles one to a compute unit
 
@@ -368,7 +372,8 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
   if (g.trans_a) {
     const bool small = has_shape(g, r, SmallSquare::kId) && g.tokens < kDeepGroups * g.num_groups &&
-                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <= 2 * kFullLaunch;
+                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <=
+                           (g.tokens >= kMiddlingGroups * g.num_groups && !g.accumulate_f32 ? 4 : 2) * kFullLaunch;
     return small ? shape_of<SmallSquare>() : shape_of<Wide>();
   }
   const int64_t short_tiles = expected_tiles(g, Short::BM, Short::BN / halves);
@@ -658,6 +663,9 @@ const gg::PairOps* pair_kernel(const gg_gmm_args& g1, const Plan& p1, const gg_g
     return nullptr;
   if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace == p2.p.workspace) return nullptr;
   if (reads_then_writes(g1)) return nullptr;
+  // (small tiles have a compute unit each to themselves here, half as many as alone: too few to pull the weights of
+  // deep products.  14 x 221 rows, 11392 -> 384: 118 / 130)
+  if (p1.shape.id == Small::kId && g1.hidden_in > kDeepForSharing) return nullptr;
   return find_pair(g1.dtype, p1.layout, p1.shape.id, p2.shape.id);
 }
 

@@ -2615,6 +2615,9 @@ def test_gpu_validation_errors(ops):
     (8, 16000, 264, 520, False, 3),      # deep groups of the weight gradient, cut and first
     (3, 40, 8, 16, True, 1),             # less than a tile
     (5, 300, 130, 262, False, 0),        # even sizes
+    (14, 584, 960, 1280, False, 0),      # small tiles, then full ones
+    (9, 5519, 1792, 960, True, 1),       # full tiles, then small ones, four rounds of them
+    (5, 1000, 704, 400, True, 0),        # short tiles, then small ones
 ])
 def test_both_gradients_in_one_launch(ops, oracle, experts, rows, hin, hout, trans_b, skew, on_device):
     # The pair launch against the two calls: the same tiles, pieces and sums, so the same bits, except where
