@@ -48,16 +48,18 @@ def _output_dtype(dtype):
 # Hidden sizes that are not multiples of 8 elements (16 for float8), and operands that do not
 # start on a 16-byte boundary, would run on the extension's general kernels, which are many times
 # slower than the streaming ones (calling the extension directly gets exactly that, copy-free).
-# gmm instead copies such operands into zero-padded, aligned tensors, runs the streaming kernels
-# on those and copies the result back: one pass over each, still several times faster.  Zeros along
-# the depth add nothing to any sum; padded output columns are dropped.
+# gmm instead copies operands whose rows cannot be read as they are into tensors with zero-padded, aligned
+# rows and runs the streaming kernels on those: one pass over each, still several times faster.  Zeros along
+# the depth add nothing to any sum.  Results of two-byte types are written where they belong, whatever their
+# rows are; for float8, whose kernels need whole chunks, all three are padded and the result is copied back.
 # Needing no copies: two-byte operands on 4-byte boundaries whose hidden sizes are both even.
 
 
 def _padded_size(n, itemsize):
     """The hidden size that n is padded to: what the streaming kernels need (16-byte rows), and where that adds
     little, rows of whole lines (128 bytes), or sectors (64), which neither loads nor stores share with the
-    next row.  8 x 1024 rows, 2047 -> 5461, forward and gradients, padded to 5464 / 5504: 910 / 869 us."""
+    next row.  8 x 1024 rows, 2047 -> 5461, forward and gradients, padded to 5464 / 5504: 910 / 869 us
+    (with results padded too)."""
     align = 128 if n * itemsize >= 2048 else (64 if n * itemsize >= 512 else 16)
     m = align // itemsize
     return (n + m - 1) // m * m
@@ -103,10 +105,23 @@ def _padded(t, rows, cols):
     return backend.pad_rows(t, rows, cols)
 
 
+def _lined(t):
+    """t, or a copy of it with zero-padded rows that the streaming kernels can read."""
+    if t.shape[-1] % 8 == 0 and t.data_ptr() % 16 == 0:
+        return t
+    return backend.pad_rows(t, t.shape[-2], _padded_size(t.shape[-1], t.element_size()))
+
+
 def _padded_call(a, b, c, batch_sizes, trans_a, trans_b):
-    """gmm through zero-padded copies, for operands that _needs_padding accepts."""
+    """gmm for operands that _needs_padding accepts."""
     hin = a.shape[1]
     hout = b.shape[1] if (trans_a or trans_b) else b.shape[2]
+    if a.element_size() == 2:
+        # (only what cannot be read as it is gets copied, and the result needs no copy)
+        if c is None:
+            c = _allocate_output(a, b, batch_sizes, trans_a, trans_b)
+        backend.gmm_strided(_lined(a), _lined(b), c, batch_sizes, trans_a, trans_b and not trans_a, hin, hout)
+        return c
     hin_p, hout_p = _padded_size(hin, a.element_size()), _padded_size(hout, a.element_size())
     a_p = _padded(a, a.shape[0], hin_p)
     if trans_a:
@@ -141,15 +156,6 @@ def _padded_product(a_p, b_p, c, batch_sizes, trans_a, trans_b, hin, hout):
     return c
 
 
-def _cropped(t, shape):
-    """The upper left corner of every batch of t."""
-    if t.shape == shape:
-        return t
-    c = torch.empty(shape, dtype=t.dtype, device=t.device)
-    backend.unpad_rows(t, c)
-    return c
-
-
 def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
     """Both gradients of gmm(a, b, batch_sizes, trans_b=trans_b), each None where it is not wanted."""
     if want_a and want_b:
@@ -157,16 +163,10 @@ def gradients(grad, a, b, batch_sizes, trans_b, want_a, want_b):
         if both is not None:
             return both
     if want_a and want_b and _needs_padding(grad, b, None, batch_sizes, False, not trans_b) and \
-            a.device == grad.device and a.dtype == grad.dtype and a.is_contiguous() and \
+            a.device == grad.device and a.dtype == grad.dtype and a.element_size() == 2 and a.is_contiguous() and \
             tuple(a.shape) == (grad.shape[0], b.shape[2 if trans_b else 1]):
         # (one padded copy of the gradient serves both products)
-        hin, hout = a.shape[1], grad.shape[1]
-        hin_p, hout_p = _padded_size(hin, a.element_size()), _padded_size(hout, a.element_size())
-        grad_p = _padded(grad, grad.shape[0], hout_p)
-        b_p = _padded(b, hout_p, hin_p) if trans_b else _padded(b, hin_p, hout_p)
-        a_p = _padded(a, a.shape[0], hin_p)
-        agrad_p, bgrad_p = backend.gmm_gradients(grad_p, a_p, b_p, batch_sizes, trans_b)
-        return _cropped(agrad_p, a.shape), _cropped(bgrad_p, b.shape)
+        return backend.gmm_gradients_strided(_lined(grad), _lined(a), _lined(b), batch_sizes, trans_b, a.shape[1], grad.shape[1])
     agrad = gmm(grad, b, batch_sizes, trans_a=False, trans_b=not trans_b) if want_a else None
     bgrad = None
     if want_b:

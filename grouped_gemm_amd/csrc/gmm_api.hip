@@ -294,6 +294,30 @@ Route classify(const gg_gmm_args& g) {
   return r;
 }
 
+// gg_gmm_strided: rows of a and b on 16-byte boundaries, further apart than they are long.
+struct Strides {
+  int64_t a, b;
+};
+
+bool strides_fit(const gg_gmm_args& g, const Strides& s) {
+  if (g.dtype != GG_DTYPE_BF16 && g.dtype != GG_DTYPE_F16) return false;
+  if (g.epilogue != GG_EPILOGUE_NONE || g.accumulate_f32 || g.a_row_index || g.b_row_index || g.c_row_index) return false;
+  if ((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 15) return false;
+  const int64_t b_row = g.trans_b ? g.hidden_in : g.hidden_out;
+  // (whole chunks of 8: what a chunk reads past the end of a row is its padding)
+  return s.a % 8 == 0 && s.b % 8 == 0 && s.a >= g.hidden_in && s.b >= b_row && s.a < (1 << 22) && s.b < (1 << 22);
+}
+
+Route strided_route(const gg_gmm_args& g) {
+  gg_gmm_args aligned = g;   // (the streaming kernels' route, whatever the sizes and c)
+  aligned.hidden_in = (g.hidden_in + 7) / 8 * 8;
+  aligned.hidden_out = (g.hidden_out + 7) / 8 * 8;
+  aligned.c = reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(g.c) + 15) / 16 * 16);
+  Route r = classify(aligned);
+  r.address_bits = (r.address_bits & ~(uintptr_t)15) | (reinterpret_cast<uintptr_t>(g.c) & 15);
+  return r;
+}
+
 // Rows of a, b and c in memory, the bounds a row index is held against: an index that names no
 // row is a missing row (zeros on the way in, nothing stored on the way out) on every kernel.
 struct IndexedRows {
@@ -422,7 +446,8 @@ struct Plan {
 
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
 // gate_up: where gate | up are kept beside c (SwiGLU epilogue), or nullptr.
-int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_up = nullptr) {
+// strides: where rows of a and b are further apart than they are long (gg_gmm_strided).
+int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_up = nullptr, const Strides* strides = nullptr) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
   const int64_t hidden_in = g.hidden_in, hidden_out = g.hidden_out;
   const int trans_a = g.trans_a != 0, trans_b = g.trans_b != 0;
@@ -453,7 +478,8 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
   if (hidden_out == 0 || (trans_a ? hidden_in == 0 : tokens == 0)) return GG_OK;
   if (g.c == nullptr) return fail(GG_EINVAL, "c is null");
   if (tokens > 0 && (g.a == nullptr || g.b == nullptr)) return fail(GG_EINVAL, "a or b is null");
-  const Route route = classify(g);
+  if (strides != nullptr && !strides_fit(g, *strides)) return fail(GG_EINVAL, "row strides do not fit the call (gg_gmm_strided)");
+  const Route route = strides != nullptr ? strided_route(g) : classify(g);
   const uintptr_t address_bits = route.address_bits;
   if (address_bits & (uintptr_t)(elem_bytes - 1) || reinterpret_cast<uintptr_t>(g.c) & (out_f32 ? 3 : 1))
     return fail(GG_ELIMIT, "a, b and c must be aligned to their element size");
@@ -502,6 +528,8 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
   p.hidden_in = (int32_t)hidden_in;
   p.hidden_out = (int32_t)hidden_out;
   p.b_cols = (int32_t)(swiglu ? 2 * hidden_out : hidden_out);
+  p.lda = (int32_t)(strides != nullptr ? strides->a : hidden_in);
+  p.ldb = (int32_t)(strides != nullptr ? strides->b : (trans_a ? hidden_out : (trans_b ? hidden_in : p.b_cols)));
   p.a_rows = g.a_row_index;
   p.c_rows = g.c_row_index;
   static_assert(GG_STATUS_NEGATIVE_SIZE == gg::kStatusNegativeSize && GG_STATUS_ROWS_PAST_END == gg::kStatusRowsPastEnd,
@@ -518,6 +546,7 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
                 "the header's flags are the kernel's");
   p.flags = g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ONE_CLASS | GG_FLAG_ROW_PIECES | GG_FLAG_GROUP_ORDER);
   if (merge_stores(g)) p.flags |= gg::kFlagMergeStores;
+  if (strides != nullptr && (hidden_out % 8 != 0 || (reinterpret_cast<uintptr_t>(g.c) & 15))) p.flags |= gg::kFlagAnyRows;
   const bool depth_pieces = !generic && may_cut_depth(g, route, shape);
   p.sched_out = nullptr;
   if (static_scratch) {
@@ -731,13 +760,21 @@ int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up) {
   return rc != GG_OK ? rc : launch_call(*args, &plan);
 }
 
-int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) {
+int gg_gmm_strided(const gg_gmm_args* args, int64_t a_row, int64_t b_row) {
+  if (args == nullptr || args->struct_bytes != sizeof(gg_gmm_args)) return fail(GG_EINVAL, "args is null or of another size");
+  const Strides strides{a_row, b_row};
+  Plan plan;
+  const int rc = plan_call(*args, false, &plan, nullptr, &strides);
+  return rc != GG_OK ? rc : launch_call(*args, &plan);
+}
+
+static int run_pair(const gg_gmm_args* first, const Strides* strides1, const gg_gmm_args* second, const Strides* strides2) {
   if (first == nullptr || second == nullptr) return fail(GG_EINVAL, "args is null");
   if (first->struct_bytes != sizeof(gg_gmm_args) || second->struct_bytes != sizeof(gg_gmm_args))
     return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is not the %zu this library expects", sizeof(gg_gmm_args));
   Plan p1, p2;
-  int rc = plan_call(*first, false, &p1);
-  if (rc == GG_OK) rc = plan_call(*second, false, &p2);
+  int rc = plan_call(*first, false, &p1, nullptr, strides1);
+  if (rc == GG_OK) rc = plan_call(*second, false, &p2, nullptr, strides2);
   if (rc != GG_OK) return rc;
   const gg::PairOps* pair = pair_kernel(*first, p1, *second, p2);
   if (pair != nullptr) {
@@ -753,6 +790,14 @@ int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) {
   }
   rc = launch_call(*first, &p1);
   return rc == GG_OK ? launch_call(*second, &p2) : rc;
+}
+
+int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) { return run_pair(first, nullptr, second, nullptr); }
+
+int gg_gmm_pair_strided(const gg_gmm_args* first, int64_t a_row1, int64_t b_row1, const gg_gmm_args* second, int64_t a_row2,
+                        int64_t b_row2) {
+  const Strides strides1{a_row1, b_row1}, strides2{a_row2, b_row2};
+  return run_pair(first, &strides1, second, &strides2);
 }
 
 uint64_t gg_workspace_bytes_for(const gg_gmm_args* args) {
@@ -881,6 +926,8 @@ int gg_debug_schedule(const int64_t* batch_sizes, int batch_sizes_on_device, int
   p.group_m = band_height(num_groups, tokens, trans_a);
   p.num_groups = (int32_t)num_groups;
   p.b_cols = (int32_t)hidden_out;
+  p.lda = (int32_t)hidden_in;
+  p.ldb = (int32_t)(trans_b ? hidden_in : hidden_out);
   p.sched_out = table_out;
   const int layout = trans_a ? gg::kTN : (trans_b ? gg::kNT : gg::kNN);
   const bool short_shape = use_short_shape(num_groups, tokens, trans_a);

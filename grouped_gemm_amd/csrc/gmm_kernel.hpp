@@ -65,6 +65,8 @@ struct GmmParams {
   int32_t flags;       // kFlag* bits
   int32_t ws_slots;    // partial-tile slots the workspace holds (0: no depth pieces)
   int32_t b_cols;      // columns of one group's b in memory: hidden_out, or twice that for gate | up
+  int32_t lda, ldb;    // elements from one row of a (of b) in memory to the next: more than a row has in copies
+                       // that are padded to whole lines, with zeros where the rows run along the depth
   // the variants with row indices only:
   const int32_t* a_rows;   // row r of the left operand is row a_rows[r] of a, or nullptr (rows in place)
   const int32_t* c_rows;   // row r of the output goes to row c_rows[r] of c, or nullptr
@@ -98,6 +100,7 @@ enum : int {   // debugging switches, for comparing the ways a call can be sched
   kFlagRowPieces = 4,     // ignore the workspace: cut along the rows only
   kFlagGroupOrder = 8,    // NN and NT layouts: never hand out the groups' tiles by tile rows
   kFlagByTileRows = 16,   // set by the host side (never by callers): hand them out by tile rows
+  kFlagAnyRows = 64,      // set by the host side: rows of c on 2-byte boundaries, of any length
   kFlagMergeStores = 32,  // set by the host side: kStoreMerging instead of kStoreStreaming (merge_stores in gmm_api.hip)
 };
 
@@ -688,15 +691,15 @@ __device__ __forceinline__ GroupGeom group_geometry(const GmmParams& p, int e, i
     g.m = p.hidden_in;
     g.n = p.hidden_out;
     g.k = rows;
-    g.a_off = hin * start;
-    g.b_off = start * hout;
+    g.a_off = start * p.lda;
+    g.b_off = start * p.ldb;
     g.c_off = (int64_t)e * hin * hout;
   } else {
     g.m = rows;
     g.n = p.hidden_out;
     g.k = p.hidden_in;
-    g.a_off = start * hin;
-    g.b_off = (int64_t)e * hin * p.b_cols;
+    g.a_off = start * p.lda;
+    g.b_off = (int64_t)e * (LAYOUT == kNT ? (int64_t)p.b_cols : hin) * p.ldb;
     g.c_off = start * hout;
   }
   return g;
@@ -1503,15 +1506,16 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       fetch_n = uniform(fetch_n + 1);
     }
     const int depth = fti.depth;
+    // (an odd depth has a zero behind it: buffers end after whole dwords)
+    const int along = ES == 2 ? depth + (depth & 1) : depth / 2;   // depth of rows along it, in two-byte elements
     if constexpr (INDEXED) {
       const int first = fti.g.row0 + fti.m0;
       aload.setup_gather(p.a, p.a_bytes, p.a_rows != nullptr ? p.a_rows + first : nullptr, p.a_index_rows, first,
                          fti.g.k * ES / 2, depth > 0 ? fti.rows_valid : 0, depth * ES / 2);
     } else if constexpr (Cfg::A_DEPTH_MAJOR) {
-      aload.setup(p.a + (fti.g.a_off + (int64_t)fti.m0 * fti.g.k) * ES, fti.g.k * ES / 2, fti.rows_valid,
-                  depth * ES / 2);
+      aload.setup(p.a + (fti.g.a_off + (int64_t)fti.m0 * p.lda) * ES, p.lda * ES / 2, fti.rows_valid, along);
     } else {
-      aload.setup(p.a + fti.g.a_off * ES, fti.g.m * ES / 2, depth, fti.m0 * ES / 2, fti.g.m * ES / 2);
+      aload.setup(p.a + fti.g.a_off * ES, p.lda * ES / 2, depth, fti.m0 * ES / 2, fti.g.m * ES / 2);
     }
     if constexpr (GATE_UP && Cfg::B_DEPTH_MAJOR) {
       bload.setup_gate_up(p.b + (fti.g.b_off + (int64_t)fti.n0 * fti.g.k) * ES, fti.g.k * ES / 2,
@@ -1519,10 +1523,11 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
     } else if constexpr (GATE_UP) {
       bload.setup_gate_up(p.b + fti.g.b_off * 2, 2 * fti.g.n, depth, fti.n0, fti.g.n);
     } else if constexpr (Cfg::B_DEPTH_MAJOR) {
-      bload.setup(p.b + (fti.g.b_off + (int64_t)fti.n0 * fti.g.k) * ES, fti.g.k * ES / 2,
-                  fti.valid && depth > 0 ? min(BN, fti.g.n - fti.n0) : 0, depth * ES / 2);
+      bload.setup(p.b + (fti.g.b_off + (int64_t)fti.n0 * p.ldb) * ES, p.ldb * ES / 2,
+                  fti.valid && depth > 0 ? min(BN, fti.g.n - fti.n0) : 0, along);
     } else {
-      bload.setup(p.b + fti.g.b_off * ES, fti.g.n * ES / 2, depth, fti.n0 * ES / 2, fti.g.n * ES / 2);
+      // (rows of b are as long as they are apart where row indices are used: a scalar register less)
+      bload.setup(p.b + fti.g.b_off * ES, (INDEXED ? fti.g.n : p.ldb) * ES / 2, depth, fti.n0 * ES / 2, fti.g.n * ES / 2);
     }
   };
   // Slices past the depth (or past the last tile) are fetched with an empty descriptor:
@@ -1663,6 +1668,29 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   };
   auto c_at = [&](const TileInfo& tile, uint32_t row_off, int col) -> uint32_t {
     return col < tile.g.n && (!INDEXED || row_off != C_OOR) ? row_off + (uint32_t)col * (uint32_t)CE : C_OOR;
+  };
+  // Rows of c on 2-byte boundaries and of any length (outputs of odd width, written where they belong: a padded
+  // copy of them costs a pass more than the product's own): whole chunks at once, which global memory takes on
+  // any boundary, the last ones of a row by elements.  8 x 1024 rows, 2047 -> 5461, forward and gradients: 834 us with
+  // padded results copied back (120 of them the copies), 760 so.
+  constexpr bool ANY_ROWS = EPI == kEpiStore && !INDEXED && !RAGGED_DEPTH && !F8;
+  auto store_any = [&](const TileInfo& tile, uint32_t row_off, int col, int most, u32x4 v) {
+    struct Chunk {
+      u32x4 v;
+    } __attribute__((packed, aligned(2)));
+    const int left = row_off < (uint32_t)(tile.rows_valid * tile.g.n) * 2u ? tile.g.n - col : 0;
+    uint16_t* to = reinterpret_cast<uint16_t*>(p.c + (tile.g.c_off + (int64_t)tile.m0 * tile.g.n) * 2 + row_off) + col;
+    if (most == 8 && left >= 8) {
+      reinterpret_cast<Chunk*>(to)->v = v;
+    } else {
+      uint64_t low = (uint64_t)v[1] << 32 | v[0], high = (uint64_t)v[3] << 32 | v[2];
+#pragma unroll 1
+      for (int e = left < most ? left : most; e > 0; --e) {
+        *to++ = (uint16_t)low;
+        low = low >> 16 | high << 48;
+        high >>= 16;
+      }
+    }
   };
   // silu(gate) * up of four element pairs, rounded.  gate / (1 + exp(-gate)), the division by Markstein's
   // scheme: the hardware's reciprocal (one unit in the last place; of a quarter of the divisor, whose reciprocal
@@ -2002,6 +2030,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         // an even width that is not a multiple of 8: rows of c then start on 4-byte boundaries
         // only, and the last 16-byte chunk of a row holds 2, 4 or 6 columns
         const bool ragged_width = uniform(ti.g.n & 7) != 0;
+        const bool any_rows = ANY_ROWS && uniform(p.flags & kFlagAnyRows) != 0;
         const bool merge = uniform(p.flags & kFlagMergeStores) != 0;
         // One strip behind: the reads of a strip return while the next one is converted (the LDS
         // serves a wave in order, so the next strip's writes need not wait for them).
@@ -2009,6 +2038,11 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         uint32_t held_off[4];
         int held_col = 0;
         auto store_held = [&]() {
+          if (any_rows) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) store_any(ti, held_off[r], held_col, 8, held[r]);
+            return;
+          }
           // (whole chunks only: for widths that are multiples of 8 the same as col < n)
           auto chunk_at = [&](int r) { return held_col + 8 <= ti.g.n ? at(held_off[r], held_col) : OOR; };
           if (merge) {
@@ -2075,7 +2109,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           }
         }
       }
-      stored = ML;
+      stored = ANY_ROWS && (p.flags & kFlagAnyRows) != 0 ? 0 : ML;   // (not every store is sent there: nothing to count on)
     }
   };
 
@@ -2165,7 +2199,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           for (int q = 0; q < 4; ++q) {
             const int col = ft.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
             const uint32_t off = c_at(ft, row_off, col);
-            if constexpr (ACC_F32) {
+            if (ANY_ROWS && (p.flags & kFlagAnyRows) != 0) {
+              const u32x2 v = round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]);
+              store_any(ft, row_off, col, 4, u32x4{v[0], v[1], 0u, 0u});
+            } else if constexpr (ACC_F32) {
               const f32x4 old = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rc, off, 0, 0));
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, old + sum[j][q]), rc, off, 0, 0);
             } else {

@@ -397,6 +397,82 @@ c10::optional<torch::Tensor> GroupedGemmAutograd(const torch::Tensor& a, const t
   return GroupedGemmNode::apply(a, b, batch_sizes, trans_b);
 }
 
+// Operands whose rows are further apart than they are long (gg_gmm_strided): a (tokens, a row), b (experts, rows,
+// a row), or (tokens, a row) with trans_a; c as for gmm with the given hidden sizes.
+void CheckStrided(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& batch_sizes,
+                  bool trans_a, bool trans_b, int64_t hin, int64_t hout) {
+  TORCH_CHECK(a.is_cuda() && b.is_cuda() && c.is_cuda() && a.device() == b.device() && a.device() == c.device() &&
+                  a.is_contiguous() && b.is_contiguous() && c.is_contiguous(),
+              "grouped_gemm: a, b and c must be contiguous tensors on the same GPU");
+  TORCH_CHECK((a.scalar_type() == torch::kBFloat16 || a.scalar_type() == torch::kFloat16) && b.scalar_type() == a.scalar_type() &&
+                  c.scalar_type() == a.scalar_type(),
+              "grouped_gemm: a, b and c must all be bfloat16 or float16");
+  TORCH_CHECK(batch_sizes.dim() == 1 && batch_sizes.scalar_type() == torch::kInt64 &&
+                  (batch_sizes.is_cpu() || (batch_sizes.device() == a.device() && batch_sizes.is_contiguous())),
+              "grouped_gemm: batch_sizes must be 1-d int64 on the host or on a's GPU");
+  TORCH_CHECK(!(trans_a && trans_b), "grouped_gemm: trans_a and trans_b cannot both be set");
+  const int64_t experts = batch_sizes.size(0), tokens = a.dim() == 2 ? a.size(0) : -1;
+  const int64_t b_rows = trans_a ? tokens : (trans_b ? hout : hin), b_row = trans_b ? hin : hout;
+  TORCH_CHECK(tokens >= 0 && a.size(1) >= hin && b.dim() == (trans_a ? 2 : 3) && (trans_a || b.size(0) == experts) &&
+                  b.size(-2) == b_rows && b.size(-1) >= b_row,
+              "grouped_gemm: a or b does not hold operands of these hidden sizes");
+  TORCH_CHECK(trans_a ? c.dim() == 3 && c.size(0) == experts && c.size(1) == hin && c.size(2) == hout
+                      : c.dim() == 2 && c.size(0) == tokens && c.size(1) == hout,
+              "grouped_gemm: c does not have the shape of the product");
+}
+
+// Arguments of such a call, with a workspace where the same call on multiples of 8 would have one.
+gg_gmm_args StridedArguments(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& sizes,
+                             bool trans_a, bool trans_b, int64_t hin, int64_t hout, hipStream_t stream, int which,
+                             torch::Tensor* workspace) {
+  gg_gmm_args g = Arguments(a, b, c, sizes, trans_a, trans_b, false, 0, RowIndices(), false, stream);
+  gg_gmm_args whole = g;
+  whole.hidden_in = (hin + 7) / 8 * 8;
+  whole.hidden_out = (hout + 7) / 8 * 8;
+  whole.c = nullptr;
+  *workspace = AttachWorkspace(&whole, a.device(), stream, which);
+  g.workspace = whole.workspace;
+  g.workspace_bytes = whole.workspace_bytes;
+  g.hidden_in = hin;
+  g.hidden_out = hout;
+  return g;
+}
+
+void GroupedGemmStrided(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes, bool trans_a,
+                        bool trans_b, int64_t hin, int64_t hout) {
+  CheckStrided(a, b, c, batch_sizes, trans_a, trans_b, hin, hout);
+  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(a.device());
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(a.device().index()).stream();
+  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+  torch::Tensor workspace;
+  const gg_gmm_args g = StridedArguments(a, b, c, sizes, trans_a, trans_b, hin, hout, stream, 0, &workspace);
+  const int rc = gg_gmm_strided(&g, a.size(-1), b.size(-1));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+}
+
+// Both gradients of gmm with hidden sizes hin and hout, from such operands.
+std::pair<torch::Tensor, torch::Tensor> GradientsStrided(torch::Tensor grad, torch::Tensor a, torch::Tensor b,
+                                                         torch::Tensor batch_sizes, bool trans_b, int64_t hin, int64_t hout) {
+  const torch::Tensor &lhs = trans_b ? grad : a, &rhs = trans_b ? a : grad;
+  const int64_t lhs_cols = trans_b ? hout : hin, rhs_cols = trans_b ? hin : hout;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(grad.device());
+  torch::Tensor agrad = torch::empty({grad.size(0), hin}, grad.options());
+  torch::Tensor bgrad = torch::empty({batch_sizes.size(0), lhs_cols, rhs_cols}, grad.options());
+  CheckStrided(grad, b, agrad, batch_sizes, false, !trans_b, hout, hin);
+  CheckStrided(lhs, rhs, bgrad, batch_sizes, true, false, lhs_cols, rhs_cols);
+  torch::Tensor sizes = batch_sizes.is_cpu() ? batch_sizes.contiguous() : batch_sizes;
+  hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(grad.device().index()).stream();
+  TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
+  torch::Tensor workspace1, workspace2;
+  const gg_gmm_args g1 = StridedArguments(grad, b, agrad, sizes, false, !trans_b, hout, hin, stream, 0, &workspace1);
+  const gg_gmm_args g2 = StridedArguments(lhs, rhs, bgrad, sizes, true, false, lhs_cols, rhs_cols, stream,
+                                          workspace1.defined() ? 1 : 0, &workspace2);
+  const int rc = gg_gmm_pair_strided(&g1, grad.size(-1), b.size(-1), &g2, lhs.size(-1), rhs.size(-1));
+  TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
+  return {agrad, bgrad};
+}
+
 // gmm with GG_FLAG_* bits, for tests that compare the ways a call can be scheduled.
 void GroupedGemmWithFlags(torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes,
                           bool trans_a, bool trans_b, int64_t flags) {
@@ -572,6 +648,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gmm_autograd", &GroupedGemmAutograd, "The differentiable form of gmm_direct without trans_a.");
   m.def("gmm_gradients", &GroupedGemmGradients,
         "Both gradients of gmm, for operands the streaming kernels take as they are; None for others.");
+  m.def("gmm_strided", &GroupedGemmStrided, "gmm on operands whose rows are further apart than they are long.");
+  m.def("gmm_gradients_strided", &GradientsStrided, "Both gradients of gmm from such operands.");
   m.def("validate",
         [](torch::Tensor a, torch::Tensor b, torch::Tensor c, torch::Tensor batch_sizes, bool trans_a,
            bool trans_b) { Validate(a, b, c, batch_sizes, trans_a, trans_b, /*on_device=*/false); },

@@ -237,6 +237,19 @@ int gg_gmm(const gg_gmm_args* args);
 int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second);
 
 /*
+ * gg_gmm (and gg_gmm_pair) on operands whose rows are further apart than they are long: a_row and b_row elements
+ * from one row of a (of b, in any of its groups) to the next, multiples of 8, a and b on 16-byte boundaries,
+ * two-byte elements, no row indices, plain epilogue.  Hidden sizes and c are any: c is contiguous, its rows may
+ * start on 2-byte boundaries.  Where hidden_in is no multiple of 8 and rows run along the depth (a, and b with
+ * trans_b; not with trans_a), the elements behind each row up to the next multiple of 8 must be zero.
+ * For copies of operands whose own rows the streaming kernels cannot read (odd sizes): only those are copied, and the
+ * result needs no copy.
+ */
+int gg_gmm_strided(const gg_gmm_args* args, int64_t a_row, int64_t b_row);
+int gg_gmm_pair_strided(const gg_gmm_args* first, int64_t a_row1, int64_t b_row1, const gg_gmm_args* second, int64_t a_row2,
+                        int64_t b_row2);
+
+/*
  * gg_gmm with GG_EPILOGUE_SWIGLU that also stores the two products, rounded to the element type, for the
  * gradient (gg_swiglu_backward): gate_up (tokens, 2 * hidden_out), gate first, rows like those of c, 16-byte
  * aligned.  For calls for which gg_keeps_gate_up returns 1: two-byte elements, no row indices, sizes and

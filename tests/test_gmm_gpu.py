@@ -1537,6 +1537,44 @@ def test_even_depths_that_are_no_multiple_of_8_stream(ops, oracle, trans_b, dtyp
               f"case {idx}, gathered and scattered")
 
 
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
+@pytest.mark.parametrize("sizes,hin,hout", [
+    ([70, 0, 33, 260, 1, 148], 137, 201),     # small tiles
+    ([70, 0, 33, 260, 1, 148], 1, 7),         # less than a chunk
+    ([300, 520, 0, 90], 2051, 1023),          # short and full tiles, a last column of one
+    ([20, 13, 40, 9], 6401, 259),             # tiles cut along the depth: the sum stores odd rows too
+    ([2900, 40, 7], 137, 265),                # deep tiles of the weight gradient, cut
+    ([130, 126], 264, 333),                   # only the width is odd: a is read as it is
+])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_odd_rows_are_written_where_they_belong(ops, oracle, layout, sizes, hin, hout, shift):
+    # Outputs of odd width, on odd elements of a buffer: equal to the oracle, with nothing written in front, behind
+    # or into rows past the last group; what lies behind the operands' rows (NaNs here) reaches no sum.
+    _announce("odd rows in place", layout, sizes, hin, hout, shift)
+    trans_a, trans_b = layout == "tn", layout == "nt"
+    g = torch.Generator().manual_seed(hin)
+    bs = torch.tensor(sizes, dtype=torch.int64)
+    used, t = int(bs.sum()), int(bs.sum()) + 3
+    def guarded(*shape):   # a view with NaNs on both sides
+        n = int(np.prod(shape))
+        buffer = torch.full((n + 64,), float("nan"), dtype=torch.bfloat16, device="cuda")
+        view = buffer[32 + shift:32 + shift + n].view(*shape)
+        view.copy_(torch.randn(*shape, generator=g))
+        return view
+    a = guarded(t, hin)
+    b = guarded(*((t, hout) if trans_a else (len(sizes), hout, hin) if trans_b else (len(sizes), hin, hout)))
+    shape = (len(sizes), hin, hout) if trans_a else (t, hout)
+    n = int(np.prod(shape))
+    buffer = torch.full((n + 64,), 3.0, dtype=torch.bfloat16, device="cuda")
+    c = buffer[32 + shift:32 + shift + n].view(*shape)
+    for _ in range(2):
+        ops.backend.gmm(a, b, bs.cuda(), trans_a=trans_a, trans_b=trans_b, c=c)
+        want = oracle.gmm_loop(a, b, bs, trans_a=trans_a, trans_b=trans_b)
+        end = n if trans_a else used * hout
+        check(c if trans_a else c[:used], want if trans_a else want[:used], f"{layout} {hin} {hout}")
+        assert (buffer[:32 + shift] == 3).all() and (buffer[32 + shift + end:] == 3).all()
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "swiglu"])
 @pytest.mark.parametrize("hout", [8, 96, 200, 352])
 def test_rows_of_c_off_64_byte_boundaries(ops, oracle, layout, hout):
