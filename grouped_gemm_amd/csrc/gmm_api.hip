@@ -381,13 +381,19 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 18.1 and 39.0 / 24.9; 16 x 1024, 512 x 1024 (512): 28.3 / 25.2 and 70.7 / 40.6 (the deepest group's tiles set the
 // length of the launch: four times as many take a quarter of the time each); past that line even
 // depths lose: 64 x 256, 256 x 768 (768): 18.3 / 20.0; 16 x 256, 1024 x 1024 (1024): 19.7 / 22.6.  Groups of
-// kMiddlingGroups rows gain up to four rounds of small tiles, where the depth of a tile counts for more than its
+// kMiddlingGroups rows gain up to four rounds of small tiles (19 x 1896, 640 x 1024 accumulated in fp32 (760): 115 / 91), where the depth of a tile counts for more than its
 // traffic (both gradients in one launch): 9 x 613, 1792 x 960 (1008): 79 / 66; 11 x 980, 1088 x 1088 (891): 82 / 73; 6 x 1784, 1792 x 1088
 // (756): 120 / 111; 15 x 1627, 2368 x 256 (570): 91 / 96; of fewer rows 26 x 318, 192 x 1312 (572): 30 / 38.  Groups of
-// kDeepGroups rows and more keep the wide ones: where a few of them are much deeper than the rest,
-// those are cut along the depth (plan_deep_tiles).
+// kDeepGroups rows and more keep the wide ones where these fill the device: where a few of them are much deeper than
+// the rest, those are cut along the depth (plan_deep_tiles).  Where wide tiles leave half of it idle, small
+// ones, and pieces of them, which pay from 16 slices on, put the rest to work.  Wide / small and the number of
+// wide ones: 19 x 2569 rows, 384 x 128 (38): 53 / 25; 5 x 3106, 608 x 240 (15): 60 / 24; 3 x 4000, 1024 x 1024, Zipf 1.2 (48):
+// 82 / 53; 4 x 15000, 1024 x 512 (32): 101 / 72; 6 x 5000, 768 x 1024 (72): 89 / 64; 8 x 5000, 1024 x 1024 (128): 89 / 84; with fp32
+// accumulation 98 / 70 and 108 / 94; but 4 x 10000, 2048 x 1024 (128): 154 / 170.  Only where the caller says so
+// (GG_FLAG_FEW_TILES, as the PyTorch binding does): calls through the C ABI keep the order of their sums.
 constexpr int64_t kDeepGroups = 2560;
 constexpr int64_t kMiddlingGroups = 512;
+constexpr int64_t kVeryDeepGroups = 8192;
 constexpr int64_t kDeepProduct = 6144;       // weights are pulled through short tiles
 constexpr int64_t kDeepForSharing = 3072;    // small tiles one to a compute unit
 
@@ -395,9 +401,13 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   if (r.ragged_depth) return shape_of<WideRaggedDepth>();
   const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
   if (g.trans_a) {
-    const bool small = has_shape(g, r, SmallSquare::kId) && g.tokens < kDeepGroups * g.num_groups &&
-                       expected_tiles(g, SmallSquare::BM, SmallSquare::BN) <=
-                           (g.tokens >= kMiddlingGroups * g.num_groups && !g.accumulate_f32 ? 4 : 2) * kFullLaunch;
+    const int64_t small_tiles = expected_tiles(g, SmallSquare::BM, SmallSquare::BN);
+    const int64_t wide_tiles = expected_tiles(g, Wide::BM, Wide::BN);
+    const bool few = (g.flags & GG_FLAG_FEW_TILES) &&
+                     wide_tiles <= (g.tokens < kVeryDeepGroups * g.num_groups ? kFullLaunch / 2 : kFullLaunch / 4);
+    const bool small = has_shape(g, r, SmallSquare::kId) &&
+                       (few || (g.tokens < kDeepGroups * g.num_groups &&
+                                small_tiles <= (g.tokens >= kMiddlingGroups * g.num_groups ? 4 : 2) * kFullLaunch));
     return small ? shape_of<SmallSquare>() : shape_of<Wide>();
   }
   const int64_t short_tiles = expected_tiles(g, Short::BM, Short::BN / halves);
@@ -652,9 +662,10 @@ int launch_call(const gg_gmm_args& g, Plan* plan) {
       gp.a_rows = g.a_row_index;
       gp.b_rows = g.b_row_index;
       gp.c_rows = g.c_row_index;
-      gp.a_num_rows = plan->index_rows.a;
-      gp.b_num_rows = plan->index_rows.b;
-      gp.c_num_rows = plan->index_rows.c;
+      const IndexedRows& index_rows = plan->index_rows;
+      gp.a_num_rows = index_rows.a;
+      gp.b_num_rows = index_rows.b;
+      gp.c_num_rows = index_rows.c;
       // light workgroups (28 KiB of LDS): two per compute unit
       const int64_t grid = tiles < 2 * plan->cus ? tiles : 2 * plan->cus;
       GG_HIP(generic_ops(g.dtype)->launch(plan->layout, plan->route.vec, plan->epilogue, gp, hs, (int)grid, stream));

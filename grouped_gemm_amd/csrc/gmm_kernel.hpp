@@ -549,19 +549,24 @@ __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, in
   const int64_t slices = ((int64_t)s->row_start[E] - s->row_start[0] + (int64_t)E * (bk / 2)) / bk;
   const int64_t share = slices * per_group / grid;
   const int deepest = (s->most_rows + bk - 1) / bk;
-  int pieces = deepest / MIN_SLICES;
-  pieces = (pieces > kMaxDeepPieces ? kMaxDeepPieces : pieces) & ~1;
-  if (pieces == 0 || deepest <= share) return;
-  int most = grid / pieces;
-  most = most < p.ws_slots / pieces ? most : p.ws_slots / pieces;
-  most = most < kWsCounterBytes / 4 ? most : kWsCounterBytes / 4;
-  int front = 0;
-  for (int q = 0; q < E && front < most; ++q) {
-    const int depth = (s->rows[s->order[q]] + bk - 1) / bk;
-    if (2 * (int64_t)depth <= share || depth < pieces * MIN_SLICES) break;
-    front += per_group;
+  if (deepest <= share) return;
+  // As many pieces as end the launch soonest: its longest piece, or the deepest tile that there are no
+  // workgroups left to cut for (84 tiles of 100 slices: in 4 pieces each, 64 are cut and 20 set the length).
+  int pieces = 0, front = 0, best = deepest;
+  for (int n = kMaxDeepPieces; n >= 2; n >>= 1) {
+    int most = grid / n;
+    most = most < p.ws_slots / n ? most : p.ws_slots / n;
+    most = most < kWsCounterBytes / 4 ? most : kWsCounterBytes / 4;
+    int cut = 0, left = 0;   // tiles cut, depth of the first one left whole
+    for (int q = 0; q < E; ++q) {
+      left = (s->rows[s->order[q]] + bk - 1) / bk;
+      if (cut >= most || 2 * (int64_t)left <= share || left < n * MIN_SLICES) break;
+      cut += per_group;
+      if (cut <= most) left = 0;
+    }
+    const int each = (deepest + n - 1) / n, length = each > left ? each : left;
+    if (cut > 0 && length < best) best = length, pieces = n, front = cut < most ? cut : most;
   }
-  front = front < most ? front : most;
   if (front == 0) return;
   s->front_tiles = front;     // (every thread writes the same two values, and reads its own wave's)
   s->front_pieces = pieces;

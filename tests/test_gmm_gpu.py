@@ -2643,6 +2643,34 @@ def test_gpu_validation_errors(ops):
         ops.backend.gmm(a, b, bs, trans_a=True, trans_b=True)
 
 
+@pytest.mark.parametrize("sizes,hin,hout", [
+    ([2600, 2750, 2550, 2570, 3000, 2900], 392, 136),   # deep groups on few tiles: small ones, each in pieces
+    ([6400, 6300, 6380, 6500, 6410, 6300, 6350], 360, 432),   # more than there are workgroups for four pieces each
+    ([9000, 30, 0, 1400], 520, 648),                    # one much deeper group
+])
+def test_deep_weight_gradients_of_few_tiles(ops, oracle, sizes, hin, hout):
+    _announce("deep, few tiles", sizes, hin, hout)
+    lib = _c_abi()
+    c = torch.empty(len(sizes), hin, hout, dtype=torch.bfloat16, device="cuda")
+    rows = torch.empty(sum(sizes), 8, dtype=torch.bfloat16, device="cuda")
+    args = [_gmm_args(lib, rows, rows, c, torch.tensor(sizes), False, sum(sizes), hin, hout, True, False, flags=f) for f in (0, 128)]
+    assert [_tile(lib, x) for x in args] == [(256, 256), (128, 128)]
+    g = torch.Generator().manual_seed(hin)
+    bs, t = torch.tensor(sizes, dtype=torch.int64), sum(sizes)
+    a = torch.randn(t, hin, generator=g).to(torch.bfloat16).cuda()
+    b = torch.randn(t, hout, generator=g).to(torch.bfloat16).cuda()
+    want = oracle.gmm_loop(a, b, bs, trans_a=True)
+    first = ops.backend.gmm(a, b, bs.cuda(), trans_a=True)
+    check(first, want, f"weight gradient {sizes}")
+    assert torch.equal(ops.backend.gmm(a, b, bs, trans_a=True), first)
+    c = torch.full((len(sizes), hin, hout), 2.0, device="cuda")
+    ops.backend.accumulate_weight_gradient(a, b, bs.cuda(), c)
+    # fp32 sums in another order: on either side one rounding per addition, 2 ** -24 of a partial sum, and no more of
+    # them than products, which add up like a random walk; partial sums are as large as the largest sums
+    bound = 2 * max(sizes) ** 0.5 * 2.0 ** -24 * float(want.abs().max())
+    assert float(((c - 2.0) - want).abs().max()) <= bound
+
+
 @pytest.mark.parametrize("on_device", [False, True])
 @pytest.mark.parametrize("experts,rows,hin,hout,trans_b,skew", [
     (8, 1024, 128, 128, False, 0),       # small tiles of both
