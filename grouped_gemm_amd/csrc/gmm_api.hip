@@ -381,7 +381,8 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 18.1 and 39.0 / 24.9; 16 x 1024, 512 x 1024 (512): 28.3 / 25.2 and 70.7 / 40.6 (the deepest group's tiles set the
 // length of the launch: four times as many take a quarter of the time each); past that line even
 // depths lose: 64 x 256, 256 x 768 (768): 18.3 / 20.0; 16 x 256, 1024 x 1024 (1024): 19.7 / 22.6.  Groups of
-// kMiddlingGroups rows gain up to four rounds of small tiles (19 x 1896, 640 x 1024 accumulated in fp32 (760): 115 / 91), where the depth of a tile counts for more than its
+// kMiddlingGroups rows gain up to four rounds of small tiles (not accumulated in fp32, where full tiles add atomically:
+// 19 x 1896, 640 x 1024 (760): 115 / 91, but 10 x 2383, 184 x 5592 (880): 128 / 149), where the depth of a tile counts for more than its
 // traffic (both gradients in one launch): 9 x 613, 1792 x 960 (1008): 79 / 66; 11 x 980, 1088 x 1088 (891): 82 / 73; 6 x 1784, 1792 x 1088
 // (756): 120 / 111; 15 x 1627, 2368 x 256 (570): 91 / 96; of fewer rows 26 x 318, 192 x 1312 (572): 30 / 38.  Groups of
 // kDeepGroups rows and more keep the wide ones where these fill the device: where a few of them are much deeper than
@@ -407,7 +408,7 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
                      wide_tiles <= (g.tokens < kVeryDeepGroups * g.num_groups ? kFullLaunch / 2 : kFullLaunch / 4);
     const bool small = has_shape(g, r, SmallSquare::kId) &&
                        (few || (g.tokens < kDeepGroups * g.num_groups &&
-                                small_tiles <= (g.tokens >= kMiddlingGroups * g.num_groups ? 4 : 2) * kFullLaunch));
+                                small_tiles <= (g.tokens >= kMiddlingGroups * g.num_groups && !g.accumulate_f32 ? 4 : 2) * kFullLaunch));
     return small ? shape_of<SmallSquare>() : shape_of<Wide>();
   }
   const int64_t short_tiles = expected_tiles(g, Short::BM, Short::BN / halves);
