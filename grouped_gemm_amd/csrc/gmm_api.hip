@@ -689,6 +689,7 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
 // (MB of weights) 38 x 19, 1944 x 2496 (369): 205 / 200; 83 x 29, 168 x 4152 (116): 89 / 88; 27 x 51, 1024 x 1032 (57): 49 / 48;
 // 6 x 95, 208 x 2880 (7): 25 / 20.
 constexpr int64_t kPairWeightBytes = int64_t(128) << 20;
+constexpr int64_t kLongRounds = 8;   // (see pair_kernel)
 bool reads_then_writes(const gg_gmm_args& g) {
   return use_short_shape(g.num_groups, g.tokens, 0) && g.num_groups * g.hidden_in * g.hidden_out * 2 > kPairWeightBytes;
 }
@@ -704,6 +705,11 @@ const gg::PairOps* pair_kernel(const gg_gmm_args& g1, const Plan& p1, const gg_g
     return nullptr;
   if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace == p2.p.workspace) return nullptr;
   if (reads_then_writes(g1)) return nullptr;
+  // (launches of many rounds have nothing to gain: 8 x 4096 rows, 4096 -> 14336, forward and gradients 8383 in two, 8457 in
+  // one; 256 x 256, 7168 -> 2048: 6753 / 6777; 16 x 1024, 2048 -> 4096, 4 rounds of the first: 520 in two, 510 in one)
+  if (expected_tiles(g1, p1.shape.bm, p1.shape.bn) >= kLongRounds * kFullLaunch &&
+      expected_tiles(g2, p2.shape.bm, p2.shape.bn) >= kLongRounds * kFullLaunch)
+    return nullptr;
   // (small tiles have a compute unit each to themselves here, half as many as alone: too few to pull the weights of
   // deep products.  14 x 221 rows, 11392 -> 384: 118 / 130)
   if (p1.shape.id == Small::kId && g1.hidden_in > kDeepForSharing) return nullptr;
