@@ -205,8 +205,8 @@ struct Sched {
   int16_t order[kMaxGroups];
 };
 
-constexpr uint32_t kOutOfRange = 0x80000000u;  // beyond any descriptor size used here
-// ... and for the descriptors that span a whole tensor (rows reached through an index)
+constexpr uint32_t kOutOfRange = 0x80000000u;  // beyond the descriptor of one tile's rows
+// ... and for the descriptors that may be larger: of a whole tensor (rows reached through an index), of gate | up
 constexpr uint32_t kOutOfRangeIndexed = 0xfffffff0u;
 constexpr uint32_t kRsrcFlags = 0x00020000u;   // raw buffer, 32-bit data format
 // Cache policy of the output stores: non-temporal.  The output is written once and never read by
@@ -1650,7 +1650,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // index, the byte offset of row `row` of the tile in it and that of one of its columns (C_OOR: no
   // such row or column, nothing is stored).
   constexpr int CE = ACC_F32 ? 4 : 2;   // bytes per element of c
-  constexpr uint32_t C_OOR = INDEXED ? kOutOfRangeIndexed : kOutOfRange;
+  constexpr uint32_t C_OOR = INDEXED || KEEP ? kOutOfRangeIndexed : kOutOfRange;
+  // (the rows of a tile, of the largest width, end before it: 256 x 2^22 elements of c, twice as many of gate | up, whose
+  // widths are multiples of 8)
+  static_assert(INDEXED || (uint64_t)BM * (ACC_F32 ? 1 << 20 : (KEEP ? (1 << 22) - 8 : 1 << 22)) * (KEEP ? 4 : CE) <= C_OOR, "");
   auto c_rsrc = [&](const TileInfo& tile) {
     if constexpr (INDEXED) return make_rsrc(p.c, p.c_bytes);
     return make_rsrc(p.c + (tile.g.c_off + (int64_t)tile.m0 * tile.g.n) * CE,

@@ -2234,6 +2234,25 @@ def test_swiglu_keeps_gate_and_up(ops, experts, rows, hin, hout, dtype, trans_b)
         assert ((gate_up[:used].float() - want).abs() <= 2 * unit * want.abs() + 1e-5 * hin ** 0.5).all()
 
 
+@pytest.mark.parametrize("hout", [(1 << 21) + 8, (1 << 22) - 8])
+def test_swiglu_keeps_gate_and_up_of_the_widest_rows(ops, hout):
+    # Rows of gate | up so wide that those of one tile span more than 2 GiB: what the lanes past the last column
+    # hold must be dropped, not stored at the offset that says so where rows are shorter.  Whole numbers, so exact: sums below 256.
+    _announce("keep gate | up, widest rows", hout)
+    rows, hin = 256, 56
+    g = torch.Generator(device="cuda").manual_seed(3)
+    a = torch.randint(-1, 2, (rows, hin), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randint(-1, 2, (1, hin, 2 * hout), generator=g, device="cuda", dtype=torch.int8).to(torch.bfloat16)
+    args = _gmm_args(_c_abi(), a, w, torch.empty(rows, 8, dtype=torch.bfloat16, device="cuda"), torch.tensor([rows]), False, rows, hin,
+                     hout, False, False)
+    args.epilogue = 1
+    assert _tile(_c_abi(), args) == (256, 128)
+    _, gate_up = ops.backend.backend.gmm_swiglu_keep(a, w, torch.tensor([rows], device="cuda"), False)
+    for at in range(0, 2 * hout, 1 << 20):
+        want = a.float() @ w[0, :, at:at + (1 << 20)].float()
+        assert torch.equal(gate_up[:, at:at + (1 << 20)].float(), want), at
+
+
 def test_swiglu_gradients_from_kept_and_recomputed_products(ops):
     # The memory rule: kept where no larger than the operands; both ways give the same gradients.
     g = torch.Generator().manual_seed(5)
