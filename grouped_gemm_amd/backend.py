@@ -59,10 +59,13 @@ def _padded_size(n, itemsize):
     """The hidden size that n is padded to: what the streaming kernels need (16-byte rows), and where that adds
     little, rows of whole lines (128 bytes), or sectors (64), which neither loads nor stores share with the
     next row.  8 x 1024 rows, 2047 -> 5461, forward and gradients, padded to 5464 / 5504: 910 / 869 us
-    (with results padded too)."""
+    (with results padded too).  Where that would reach the limit of hidden sizes, 2 ** 22, whole chunks again."""
     align = 128 if n * itemsize >= 2048 else (64 if n * itemsize >= 512 else 16)
-    m = align // itemsize
-    return (n + m - 1) // m * m
+    for m in (align // itemsize, 16 // itemsize):
+        padded = (n + m - 1) // m * m
+        if padded < 1 << 22:
+            break
+    return padded
 
 
 def _needs_padding(a, b, c, batch_sizes, trans_a, trans_b):

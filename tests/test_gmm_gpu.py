@@ -1575,6 +1575,23 @@ def test_odd_rows_are_written_where_they_belong(ops, oracle, layout, sizes, hin,
         assert (buffer[:32 + shift] == 3).all() and (buffer[32 + shift + end:] == 3).all()
 
 
+@pytest.mark.parametrize("dtype,width", [(torch.bfloat16, (1 << 22) - 59), (torch.float16, (1 << 22) - 9),
+                                         (torch.float8_e4m3fn, (1 << 22) - 70)])
+def test_odd_sizes_next_to_the_limit(ops, dtype, width):
+    # Hidden sizes that rows of whole lines would take past 2 ** 22, as the width of a product, of its weight
+    # gradient and as the depth of its input gradient: whole numbers, sums below 2 ** 24, so exact before rounding.
+    _announce("next to the limit", dtype, width)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    draw = lambda *shape: torch.randint(-1, 2, shape, generator=g, device="cuda", dtype=torch.int8).to(torch.float32).to(dtype)
+    a, b, grad, sizes = draw(9, 24), draw(1, 24, width), draw(9, width), torch.tensor([9], device="cuda")
+    out = torch.bfloat16 if dtype == torch.float8_e4m3fn else dtype
+    wide = lambda t: t.double()
+    agrad, bgrad = ops.backend.gradients(grad, a, b, sizes, False, True, True)
+    assert torch.equal(ops.backend.gmm(a, b, sizes), (wide(a) @ wide(b[0])).to(out))
+    assert torch.equal(agrad, (wide(grad) @ wide(b[0]).t()).to(out))
+    assert torch.equal(bgrad[0], (wide(a).t() @ wide(grad)).to(out))
+
+
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "swiglu"])
 @pytest.mark.parametrize("hout", [8, 96, 200, 352])
 def test_rows_of_c_off_64_byte_boundaries(ops, oracle, layout, hout):

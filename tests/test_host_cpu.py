@@ -325,6 +325,19 @@ def test_row_index_bounds_reach_every_kernel():
     assert "strided < index_rows" in generic and "mem_row >= gp.c_num_rows" in generic
 
 
+def test_padded_sizes_stay_below_the_limit_of_hidden_sizes():
+    # A size that whole 16-byte chunks bring to a legal size (below 2 ** 22) is padded to a legal one.
+    from grouped_gemm_amd.backend import _padded_size
+    limit = 1 << 22
+    for itemsize in (1, 2):
+        chunk = 16 // itemsize
+        for n in (*range(1, 3000, 7), *range(limit - 300, limit)):
+            padded, least = _padded_size(n, itemsize), (n + chunk - 1) // chunk * chunk
+            assert padded >= least and padded % chunk == 0
+            assert padded < limit or least == limit, (n, itemsize)
+            assert padded - n <= max(chunk, n // 8), (n, itemsize)
+
+
 # ----------------------------------------------------------------- workloads
 
 def test_workload_generators():
