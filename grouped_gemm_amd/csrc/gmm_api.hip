@@ -9,7 +9,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
+#include <numeric>
+#include <vector>
 
 #include "gmm_generic.hpp"
 #include "gmm_variants.hpp"
@@ -751,6 +754,23 @@ int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn) {
   const TileShape shape = route.generic ? TileShape{-1, 0, 0} : pick_shape(*args, route);
   if (bm) *bm = shape.bm;
   if (bn) *bn = shape.bn / (args->epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1);
+  return GG_OK;
+}
+
+int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups,
+                      int partial_tiles, int tile_outputs, int* pieces, int* tiles) {
+  if (batch_sizes == nullptr || num_groups < 1 || num_groups > GG_MAX_GROUPS_PER_LAUNCH || tiles_per_group < 1 ||
+      tiles_per_group > (1 << 20) || workgroups < 1 || partial_tiles < 0 || pieces == nullptr || tiles == nullptr)
+    return fail(GG_EINVAL, "bad argument");
+  std::vector<int64_t> rows(batch_sizes, batch_sizes + num_groups);
+  std::sort(rows.begin(), rows.end(), std::greater<int64_t>());
+  if (rows.back() < 0 || rows.front() >= (int64_t(1) << 31) / num_groups) return fail(GG_EINVAL, "batch_sizes are negative or too large");
+  const int64_t all = std::accumulate(rows.begin(), rows.end(), int64_t(0));
+  const gg::DeepCut cut = gg::cut_deep_tiles([&](int q) { return (int)((rows[q] + gg::BK - 1) / gg::BK); }, (int)num_groups, all,
+                                             (int)tiles_per_group, workgroups, partial_tiles,
+                                             gg::min_slices_per_piece(tile_outputs), gg::BK);
+  *pieces = cut.pieces;
+  *tiles = cut.tiles;
   return GG_OK;
 }
 

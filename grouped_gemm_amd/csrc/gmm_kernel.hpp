@@ -131,6 +131,44 @@ __host__ __device__ inline int best_depth_pieces(int slices, int rows, int bn, i
 // fewest slices per piece, most pieces.
 constexpr int min_slices_per_piece(int tile_outputs) { return tile_outputs > 128 * 128 ? 48 : 16; }
 constexpr int kMaxDeepPieces = 4;
+// Tiles go out by descending depth, one workgroup each, so groups much deeper than the rest set the length of the launch.
+// depth(q): depth slices (of bk rows) of the q-th deepest of E groups, which have `rows` rows in all and per_group tiles each.  Where
+// the deepest tile is longer than a workgroup's even share of all slices, the tiles deeper than half of that share that leave every
+// piece min_slices are cut, as long as there are workgroups and partial tiles (`slots`) for their pieces.  Into as many
+// pieces as end the launch soonest: its longest piece, or the deepest tile that stays whole (84 tiles of 100 slices: in 4
+// pieces each, 64 are cut and 20 set the length, whatever the groups behind them are: 9000, 30, 0 and 1400 rows, 1536 x
+// 896: 95 us in four pieces, 51 in two).
+struct DeepCut {
+  int pieces, tiles;   // pieces per tile, tiles cut (0: none)
+};
+template <typename DEPTH>
+__host__ __device__ inline DeepCut cut_deep_tiles(const DEPTH& depth, int E, int64_t rows, int per_group, int grid, int slots,
+                                                  int min_slices, int bk) {
+  DeepCut chosen{0, 0};
+  const int deepest = depth(0);
+  // (half a slice per group for the rounding)
+  const int64_t share = (rows + (int64_t)E * (bk / 2)) / bk * per_group / grid;
+  if (deepest <= share) return chosen;
+  int best = deepest;
+  for (int n = kMaxDeepPieces; n >= 2; n >>= 1) {
+    int most = grid / n;
+    most = most < slots / n ? most : slots / n;
+    most = most < kWsCounterBytes / 4 ? most : kWsCounterBytes / 4;
+    int cut = 0, whole = 0;   // tiles cut, depth of the deepest one that is not
+    for (int q = 0; q < E; ++q) {
+      const int mine = depth(q);
+      const bool fits = cut < most && 2 * (int64_t)mine > share && mine >= n * min_slices;
+      if (fits) cut += per_group;
+      if (!fits || cut > most) {
+        whole = mine;
+        break;
+      }
+    }
+    const int each = (deepest + n - 1) / n, length = each > whole ? each : whole;
+    if (cut > 0 && length < best) best = length, chosen = DeepCut{n, cut < most ? cut : most};
+  }
+  return chosen;
+}
 
 // The last round of a persistent grid is filled only partly: `tiles % grid` workgroups have a
 // tile, the others idle.  When that rest is at most half of the grid, each of its tiles is cut
@@ -531,42 +569,18 @@ __device__ __forceinline__ void order_groups_by_depth(Sched* s, int num_groups, 
   __syncthreads();
 }
 
-// Weight-gradient layout with a workspace, after order_groups_by_depth: tiles go out by descending
-// depth, one workgroup each, so a group much deeper than the others sets the length of the launch
-// however its tiles are dealt (Zipf depths: the deepest tile 227 slices, 144 slices of work per
-// workgroup).  When the deepest tile is longer than a workgroup's even share of all depth slices,
-// the tiles deeper than half that share (and deep enough to pay for their fix-up) are cut into 2
-// or 4 depth pieces, which are handed out first, one per workgroup.  Run by every thread; the
-// same answer in each.
+// Weight-gradient layout with a workspace, after order_groups_by_depth: the deepest tiles in depth pieces (cut_deep_tiles), which
+// are handed out first, one per workgroup (Zipf depths: the deepest tile 227 slices, 144 slices of work per workgroup).  Run
+// by every thread; the same answer in each.
 template <int BM, int BN>
 __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, int grid, int bk, TailPlan* plan) {
-  constexpr int MIN_SLICES = min_slices_per_piece(BM * BN);
   const int E = p.num_groups;
   const int tiles = s->tile_start[E];
   if (E == 0 || tiles == 0 || p.ws_slots <= 0 || (p.flags & (kFlagWholeTiles | kFlagRowPieces))) return;
-  const int per_group = tiles / E;   // (every group has the same number of tiles in this layout)
-  // depth slices of all groups together: their rows, and half a slice per group for the rounding
-  const int64_t slices = ((int64_t)s->row_start[E] - s->row_start[0] + (int64_t)E * (bk / 2)) / bk;
-  const int64_t share = slices * per_group / grid;
-  const int deepest = (s->most_rows + bk - 1) / bk;
-  if (deepest <= share) return;
-  // As many pieces as end the launch soonest: its longest piece, or the deepest tile that there are no
-  // workgroups left to cut for (84 tiles of 100 slices: in 4 pieces each, 64 are cut and 20 set the length).
-  int pieces = 0, front = 0, best = deepest;
-  for (int n = kMaxDeepPieces; n >= 2; n >>= 1) {
-    int most = grid / n;
-    most = most < p.ws_slots / n ? most : p.ws_slots / n;
-    most = most < kWsCounterBytes / 4 ? most : kWsCounterBytes / 4;
-    int cut = 0, left = 0;   // tiles cut, depth of the first one left whole
-    for (int q = 0; q < E; ++q) {
-      left = (s->rows[s->order[q]] + bk - 1) / bk;
-      if (cut >= most || 2 * (int64_t)left <= share || left < n * MIN_SLICES) break;
-      cut += per_group;
-      if (cut <= most) left = 0;
-    }
-    const int each = (deepest + n - 1) / n, length = each > left ? each : left;
-    if (cut > 0 && length < best) best = length, pieces = n, front = cut < most ? cut : most;
-  }
+  const DeepCut cut = cut_deep_tiles([&](int q) { return (s->rows[s->order[q]] + bk - 1) / bk; }, E,
+                                     (int64_t)s->row_start[E] - s->row_start[0], tiles / E, grid, p.ws_slots,
+                                     min_slices_per_piece(BM * BN), bk);   // (every group has the same number of tiles here)
+  const int pieces = cut.pieces, front = cut.tiles;
   if (front == 0) return;
   s->front_tiles = front;     // (every thread writes the same two values, and reads its own wave's)
   s->front_pieces = pieces;

@@ -357,6 +357,13 @@ int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, 
  * kernels; looks at what gg_workspace_bytes_for looks at. */
 int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn);
 
+/* How a weight gradient (trans_a) with a workspace cuts its deepest tiles along the depth, for host-resident sizes and
+ * two-byte elements: `*tiles` of them, the deepest first, into `*pieces` pieces each (0: none), on `workgroups` workgroups, with room
+ * for `partial_tiles` partial tiles, where every group has tiles_per_group tiles of tile_outputs elements of c.  The
+ * function that the kernel itself runs; needs no device. */
+int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups,
+                      int partial_tiles, int tile_outputs, int* pieces, int* tiles);
+
 /* Message of the last failure on the calling thread ("" if none). */
 const char* gg_last_error(void);
 

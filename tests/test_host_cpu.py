@@ -338,6 +338,48 @@ def test_padded_sizes_stay_below_the_limit_of_hidden_sizes():
             assert padded - n <= max(chunk, n // 8), (n, itemsize)
 
 
+def _deep_cut(lib, rows, per_group, workgroups, partial_tiles, tile_outputs):
+    sizes, pieces, tiles = (ctypes.c_int64 * len(rows))(*rows), ctypes.c_int(-1), ctypes.c_int(-1)
+    assert lib.gg_debug_deep_cut(sizes, ctypes.c_int64(len(rows)), ctypes.c_int64(per_group), workgroups, partial_tiles,
+                                 tile_outputs, ctypes.byref(pieces), ctypes.byref(tiles)) == 0
+    return pieces.value, tiles.value
+
+
+def test_deep_tiles_are_cut_to_end_the_launch_soonest():
+    """Into how many pieces a weight gradient cuts its deepest tiles, against all tiles laid out one by one."""
+    lib = ctypes.CDLL(HIP_LIB)
+    small = 128 * 128
+    # one deep group of more tiles than there are workgroups for four pieces each, in front of shallow ones: two pieces of all
+    # 84 tiles (71 slices), not four of 64 (20 whole tiles of 141 slices)
+    assert _deep_cut(lib, [9000, 30, 0, 1400], 84, 256, 1024, small) == (2, 84)
+    assert _deep_cut(lib, [9000], 84, 256, 1024, small) == (2, 84)
+    assert _deep_cut(lib, [9000, 30, 0, 1400], 64, 256, 1024, small) == (4, 64)
+    assert _deep_cut(lib, [9000, 8900], 32, 256, 1024, small) == (4, 64)
+    assert _deep_cut(lib, [13000, 50, 12800], 32, 256, 256, 256 * 256) == (4, 64)
+    assert _deep_cut(lib, [3000] * 4, 64, 256, 1024, small) == (0, 0)      # a round of equal tiles
+    assert _deep_cut(lib, [9000, 30], 84, 256, 0, small) == (0, 0)         # nowhere to put partial tiles
+    assert _deep_cut(lib, [0, 0], 4, 256, 1024, small) == (0, 0)
+
+    rng = np.random.default_rng(11)
+    for _ in range(400):
+        groups = int(rng.integers(1, 40))
+        rows = (rng.pareto(1.0, groups) * 600).clip(0, 60000).astype(int).tolist()
+        per_group, workgroups, slots = int(rng.integers(1, 120)), int(rng.choice([256, 512])), int(rng.choice([0, 100, 256, 1024]))
+        tile_outputs = int(rng.choice([small, 256 * 256]))
+        least = 16 if tile_outputs == small else 48
+        depths = [-(-r // 64) for r in sorted(rows, reverse=True) for _ in range(per_group)]
+        share = (sum(rows) + groups * 32) // 64 * per_group // workgroups
+        chosen, best = (0, 0), depths[0]
+        for n in (4, 2):
+            deep_enough = sum(2 * d > share and d >= n * least for d in depths)
+            cut = min(deep_enough, workgroups // n, slots // n, 1024)
+            length = max(-(-depths[0] // n), depths[cut] if cut < len(depths) else 0)
+            if cut > 0 and length < best:
+                chosen, best = (n, cut), length
+        assert _deep_cut(lib, rows, per_group, workgroups, slots, tile_outputs) == (chosen if depths[0] > share else (0, 0))
+    assert lib.gg_debug_deep_cut(None, ctypes.c_int64(1), ctypes.c_int64(1), 256, 0, small, None, None) == -1
+
+
 # ----------------------------------------------------------------- workloads
 
 def test_workload_generators():
