@@ -461,7 +461,9 @@ struct Plan {
 // static_scratch: use the device's static scratch array as the workspace (gg_gmm_no_alloc).
 // gate_up: where gate | up are kept beside c (SwiGLU epilogue), or nullptr.
 // strides: where rows of a and b are further apart than they are long (gg_gmm_strided).
-int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_up = nullptr, const Strides* strides = nullptr) {
+// assumed: a device to plan for instead of the current one.
+int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_up = nullptr, const Strides* strides = nullptr,
+              const DeviceInfo* assumed = nullptr) {
   const int64_t num_groups = g.num_groups, tokens = g.tokens;
   const int64_t hidden_in = g.hidden_in, hidden_out = g.hidden_out;
   const int trans_a = g.trans_a != 0, trans_b = g.trans_b != 0;
@@ -513,8 +515,12 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
   }
 
   DeviceInfo info;
-  rc = device_info(&info);
-  if (rc != GG_OK) return rc;
+  if (assumed != nullptr) {
+    info = *assumed;
+  } else {
+    rc = device_info(&info);
+    if (rc != GG_OK) return rc;
+  }
   hipStream_t stream = static_cast<hipStream_t>(g.stream);
   const int layout = trans_a ? gg::kTN : (trans_b ? gg::kNT : gg::kNN);
   const int epilogue = out_f32 ? gg::kEpiAccF32 : (gate_up != nullptr ? gg::kEpiSwiGLUKeep : (swiglu ? gg::kEpiSwiGLU : gg::kEpiStore));
@@ -719,6 +725,50 @@ const gg::PairOps* pair_kernel(const gg_gmm_args& g1, const Plan& p1, const gg_g
   return find_pair(g1.dtype, p1.layout, p1.shape.id, p2.shape.id);
 }
 
+// Both calls of a pair, planned.
+struct PairPlan {
+  Plan first, second;
+  const gg::PairOps* pair = nullptr;   // the kernel that runs both in one launch; nullptr: one after the other
+  gg::HostSizes sizes;                 // (pair)
+};
+
+int plan_pair(const gg_gmm_args* first, const Strides* strides1, const gg_gmm_args* second, const Strides* strides2,
+              PairPlan* out, const DeviceInfo* assumed = nullptr) {
+  if (first == nullptr || second == nullptr) return fail(GG_EINVAL, "args is null");
+  if (first->struct_bytes != sizeof(gg_gmm_args) || second->struct_bytes != sizeof(gg_gmm_args))
+    return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is not the %zu this library expects", sizeof(gg_gmm_args));
+  Plan &p1 = out->first, &p2 = out->second;
+  int rc = plan_call(*first, false, &p1, nullptr, strides1, assumed);
+  if (rc == GG_OK) rc = plan_call(*second, false, &p2, nullptr, strides2, assumed);
+  if (rc != GG_OK) return rc;
+  // (also one after the other: the partial tiles of the first would be left where the second's counters have to be zero)
+  if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace != p2.p.workspace &&
+      p1.p.workspace < p2.p.workspace + second->workspace_bytes && p2.p.workspace < p1.p.workspace + first->workspace_bytes)
+    return fail(GG_EINVAL, "the workspaces of the two calls overlap in part");
+  out->pair = pair_kernel(*first, p1, *second, p2);
+  if (out->pair != nullptr) {
+    int64_t row1 = 0, row2 = 0, tiles1, tiles2;
+    rc = plan_launch(*first, &p1, 0, first->num_groups, &row1, &out->sizes, &tiles1);
+    if (rc == GG_OK) rc = plan_launch(*second, &p2, 0, second->num_groups, &row2, &out->sizes, &tiles2);
+    if (rc != GG_OK) return rc;
+    if (tiles1 == 0 || tiles2 == 0) out->pair = nullptr;
+  }
+  return GG_OK;
+}
+
+int run_pair(const gg_gmm_args* first, const Strides* strides1, const gg_gmm_args* second, const Strides* strides2) {
+  PairPlan plan;
+  int rc = plan_pair(first, strides1, second, strides2, &plan);
+  if (rc != GG_OK) return rc;
+  if (plan.pair != nullptr) {
+    GG_HIP(plan.pair->launch(plan.first.p, plan.second.p, plan.sizes, plan.first.cus * plan.pair->workgroups_per_cu,
+                             static_cast<hipStream_t>(first->stream)));
+    return GG_OK;
+  }
+  rc = launch_call(*first, &plan.first);
+  return rc == GG_OK ? launch_call(*second, &plan.second) : rc;
+}
+
 }  // namespace
 
 extern "C" {
@@ -754,6 +804,23 @@ int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn) {
   const TileShape shape = route.generic ? TileShape{-1, 0, 0} : pick_shape(*args, route);
   if (bm) *bm = shape.bm;
   if (bn) *bn = shape.bn / (args->epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1);
+  return GG_OK;
+}
+
+int gg_debug_pair(const gg_gmm_args* first, const gg_gmm_args* second, const int64_t* strides, int* shapes) {
+  if (shapes == nullptr) return fail(GG_EINVAL, "shapes is null");
+  const Strides strides1{strides ? strides[0] : 0, strides ? strides[1] : 0};
+  const Strides strides2{strides ? strides[2] : 0, strides ? strides[3] : 0};
+  DeviceInfo device;
+  device.cus = kFullLaunch;
+  PairPlan plan;
+  const int rc = plan_pair(first, strides ? &strides1 : nullptr, second, strides ? &strides2 : nullptr, &plan, &device);
+  if (rc != GG_OK) return rc;
+  const bool one = plan.pair != nullptr;
+  shapes[0] = one ? plan.first.shape.bm : 0;
+  shapes[1] = one ? plan.first.shape.bn : 0;
+  shapes[2] = one ? plan.second.shape.bm : 0;
+  shapes[3] = one ? plan.second.shape.bn : 0;
   return GG_OK;
 }
 
@@ -804,30 +871,6 @@ int gg_gmm_strided(const gg_gmm_args* args, int64_t a_row, int64_t b_row) {
   Plan plan;
   const int rc = plan_call(*args, false, &plan, nullptr, &strides);
   return rc != GG_OK ? rc : launch_call(*args, &plan);
-}
-
-static int run_pair(const gg_gmm_args* first, const Strides* strides1, const gg_gmm_args* second, const Strides* strides2) {
-  if (first == nullptr || second == nullptr) return fail(GG_EINVAL, "args is null");
-  if (first->struct_bytes != sizeof(gg_gmm_args) || second->struct_bytes != sizeof(gg_gmm_args))
-    return fail(GG_EINVAL, "gg_gmm_args.struct_bytes is not the %zu this library expects", sizeof(gg_gmm_args));
-  Plan p1, p2;
-  int rc = plan_call(*first, false, &p1, nullptr, strides1);
-  if (rc == GG_OK) rc = plan_call(*second, false, &p2, nullptr, strides2);
-  if (rc != GG_OK) return rc;
-  const gg::PairOps* pair = pair_kernel(*first, p1, *second, p2);
-  if (pair != nullptr) {
-    gg::HostSizes hs;
-    int64_t row1 = 0, row2 = 0, tiles1, tiles2;
-    rc = plan_launch(*first, &p1, 0, first->num_groups, &row1, &hs, &tiles1);
-    if (rc == GG_OK) rc = plan_launch(*second, &p2, 0, second->num_groups, &row2, &hs, &tiles2);
-    if (rc != GG_OK) return rc;
-    if (tiles1 > 0 && tiles2 > 0) {
-      GG_HIP(pair->launch(p1.p, p2.p, hs, p1.cus * pair->workgroups_per_cu, static_cast<hipStream_t>(first->stream)));
-      return GG_OK;
-    }
-  }
-  rc = launch_call(*first, &p1);
-  return rc == GG_OK ? launch_call(*second, &p2) : rc;
 }
 
 int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second) { return run_pair(first, nullptr, second, nullptr); }

@@ -232,7 +232,8 @@ int gg_gmm(const gg_gmm_args* args);
  * gg_gmm(first) followed by gg_gmm(second), in one launch where that is possible (a product with plain
  * rows and epilogue, then a weight gradient over the same batch_sizes, stream and tokens, two-byte elements:
  * the two gradients of a product).  Compute units that run out of tiles of the first then go on with the
- * second.  The two must not share a workspace; where they do, they are launched one after the other.
+ * second.  The two must not share a workspace; where they do, they are launched one after the other, and
+ * workspaces that overlap in part are refused (GG_EINVAL).
  * No counterpart in the reference, whose backward makes two calls (grouped_gemm/ops.py:19-29).
  */
 int gg_gmm_pair(const gg_gmm_args* first, const gg_gmm_args* second);
@@ -356,6 +357,12 @@ int gg_tile_shape(int64_t num_groups, int64_t tokens, int trans_a, int trans_b, 
 /* Output tile (rows, columns of c) that the call described by `args` runs on, 0 x 0 for the general
  * kernels; looks at what gg_workspace_bytes_for looks at. */
 int gg_debug_tile(const gg_gmm_args* args, int* bm, int* bn);
+
+/* Whether gg_gmm_pair runs the two calls in one launch (gg_gmm_pair_strided where strides is given: a_row1, b_row1,
+ * a_row2, b_row2): shapes[0 .. 3] are the tile heights and widths of the two, bm1, bn1, bm2, bn2, or zeros where they are
+ * launched one after the other.  Fails where the pair would, launches nothing and needs no device (256 compute
+ * units are assumed). */
+int gg_debug_pair(const gg_gmm_args* first, const gg_gmm_args* second, const int64_t* strides, int* shapes);
 
 /* How a weight gradient (trans_a) with a workspace cuts its deepest tiles along the depth, for host-resident sizes and
  * two-byte elements: `*tiles` of them, the deepest first, into `*pieces` pieces each (0: none), on `workgroups` workgroups, with room

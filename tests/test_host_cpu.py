@@ -338,6 +338,44 @@ def test_padded_sizes_stay_below_the_limit_of_hidden_sizes():
             assert padded - n <= max(chunk, n // 8), (n, itemsize)
 
 
+def _pair(lib, sizes, hin, hout, trans_b, dtype=0, workspaces=((0, 0), (0, 0)), strides=None, **kw):
+    """(status, tile shapes) of the two gradients of a product hin -> hout in one call, sizes on the host; addresses are
+    never dereferenced."""
+    rows = (ctypes.c_int64 * len(sizes))(*sizes)
+    both = []
+    for weight, (at, length) in zip((False, True), workspaces):
+        g = _Args()
+        g.struct_bytes, g.dtype = ctypes.sizeof(_Args), dtype
+        g.a, g.b, g.c = 4096, 8192, 12288
+        g.batch_sizes, g.num_groups, g.tokens = ctypes.addressof(rows), len(sizes), sum(sizes)
+        g.trans_a, g.trans_b = int(weight), int(not weight and not trans_b)
+        g.hidden_in, g.hidden_out = (hin, hout) if weight and not trans_b else (hout, hin)
+        g.workspace, g.workspace_bytes, g.flags = at, length, 128
+        for k, v in kw.items():
+            setattr(g, k, v)
+        both.append(g)
+    shapes = (ctypes.c_int * 4)(*[-1] * 4)
+    status = lib.gg_debug_pair(ctypes.byref(both[0]), ctypes.byref(both[1]), strides and (ctypes.c_int64 * 4)(*strides), shapes)
+    return status, tuple(shapes)
+
+
+def test_pairs_that_share_a_workspace():
+    """Two calls in one launch need workspaces that do not overlap: the same one twice means two launches; parts of one
+    are refused, as one call's partial tiles would land on the other's arrival counters."""
+    lib = ctypes.CDLL(HIP_LIB)
+    lib.gg_last_error.restype = ctypes.c_char_p
+    least, at = 4096 + 256 * 256 * 4, 1 << 32
+    deep = ([700, 0, 5300], 264, 8192, False)   # pieces in both: 128 slices, and up to 94
+    assert _pair(lib, *deep, workspaces=((at, least), (at + least, least))) == (0, (128, 256, 128, 128))
+    assert _pair(lib, *deep, workspaces=((at, least), (at, least))) == (0, (0, 0, 0, 0))
+    for shift in (256, 4096, least - 256):
+        for first, second in ((at, at + shift), (at + shift, at)):
+            assert _pair(lib, *deep, workspaces=((first, least), (second, least)))[0] == -1
+            assert b"overlap" in lib.gg_last_error()
+    # nothing is cut in either: neither touches a workspace
+    assert _pair(lib, [60, 50], 64, 72, True, workspaces=((at, least), (at + 256, least))) == (0, (64, 128, 128, 128))
+
+
 def _deep_cut(lib, rows, per_group, workgroups, partial_tiles, tile_outputs):
     sizes, pieces, tiles = (ctypes.c_int64 * len(rows))(*rows), ctypes.c_int(-1), ctypes.c_int(-1)
     assert lib.gg_debug_deep_cut(sizes, ctypes.c_int64(len(rows)), ctypes.c_int64(per_group), workgroups, partial_tiles,
