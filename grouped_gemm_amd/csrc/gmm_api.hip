@@ -889,6 +889,14 @@ uint64_t gg_workspace_bytes_for(const gg_gmm_args* args) {
   return !r.generic && may_cut_depth(g, r, pick_shape(g, r)) ? GG_WORKSPACE_BYTES : 0;
 }
 
+uint64_t gg_workspace_bytes_for_strided(const gg_gmm_args* args, int64_t a_row, int64_t b_row) {
+  if (args == nullptr || args->struct_bytes != sizeof(gg_gmm_args)) return 0;
+  const gg_gmm_args& g = *args;
+  if (g.hidden_in <= 0 || g.hidden_out <= 0 || !strides_fit(g, Strides{a_row, b_row})) return 0;
+  const Route r = strided_route(g);
+  return may_cut_depth(g, r, pick_shape(g, r)) ? GG_WORKSPACE_BYTES : 0;
+}
+
 int gg_gmm_no_alloc(const gg_gmm_args* args) {
   if (args == nullptr) return fail(GG_EINVAL, "args is null");
   if (args->struct_bytes != sizeof(gg_gmm_args))

@@ -245,11 +245,11 @@ gg_gmm_args Arguments(const torch::Tensor& a, const torch::Tensor& b, const torc
   return g;
 }
 
-// A workspace for calls that can cut tiles along the depth (deep products, weight gradients) and only for
-// them; the tensor has to live until the call is enqueued.
-torch::Tensor AttachWorkspace(gg_gmm_args* g, const torch::Device& device, hipStream_t stream, int which = 0) {
+// A workspace for calls that can make use of one (`bytes` of gg_workspace_bytes_for: deep products, weight gradients)
+// and only for them; the tensor has to live until the call is enqueued.
+torch::Tensor AttachWorkspace(gg_gmm_args* g, uint64_t bytes, const torch::Device& device, hipStream_t stream, int which = 0) {
   torch::Tensor workspace;
-  if (gg_workspace_bytes_for(g) > 0) {
+  if (bytes > 0) {
     workspace = Workspace(device, stream, which);
     if (workspace.defined()) {
       g->workspace = workspace.data_ptr();
@@ -267,7 +267,7 @@ void Run(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c,
   hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(a.device().index()).stream();
   TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
   gg_gmm_args g = Arguments(a, b, c, sizes, trans_a, trans_b, accumulate_f32, flags, rows, gate_up, stream);
-  const torch::Tensor workspace = AttachWorkspace(&g, a.device(), stream);
+  const torch::Tensor workspace = AttachWorkspace(&g, gg_workspace_bytes_for(&g), a.device(), stream);
   const int rc = gg_gmm(&g);
   TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
 }
@@ -282,8 +282,9 @@ void RunGradients(const torch::Tensor& grad, const torch::Tensor& b, const torch
   TORCH_CHECK(gg_init() == GG_OK, "grouped_gemm: ", gg_last_error());
   gg_gmm_args g1 = Arguments(grad, b, agrad, sizes, false, trans_b, false, 0, RowIndices(), false, stream);
   gg_gmm_args g2 = Arguments(lhs, rhs, bgrad, sizes, true, false, false, 0, RowIndices(), false, stream);
-  const torch::Tensor workspace1 = AttachWorkspace(&g1, grad.device(), stream);
-  const torch::Tensor workspace2 = AttachWorkspace(&g2, grad.device(), stream, workspace1.defined() ? 1 : 0);
+  const torch::Tensor workspace1 = AttachWorkspace(&g1, gg_workspace_bytes_for(&g1), grad.device(), stream);
+  const torch::Tensor workspace2 =
+      AttachWorkspace(&g2, gg_workspace_bytes_for(&g2), grad.device(), stream, workspace1.defined() ? 1 : 0);
   const int rc = gg_gmm_pair(&g1, &g2);
   TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
 }
@@ -421,20 +422,14 @@ void CheckStrided(const torch::Tensor& a, const torch::Tensor& b, const torch::T
               "grouped_gemm: c does not have the shape of the product");
 }
 
-// Arguments of such a call, with a workspace where the same call on multiples of 8 would have one.
+// Arguments of such a call, with a workspace where it can make use of one.
 gg_gmm_args StridedArguments(const torch::Tensor& a, const torch::Tensor& b, const torch::Tensor& c, const torch::Tensor& sizes,
                              bool trans_a, bool trans_b, int64_t hin, int64_t hout, hipStream_t stream, int which,
                              torch::Tensor* workspace) {
   gg_gmm_args g = Arguments(a, b, c, sizes, trans_a, trans_b, false, 0, RowIndices(), false, stream);
-  gg_gmm_args whole = g;
-  whole.hidden_in = (hin + 7) / 8 * 8;
-  whole.hidden_out = (hout + 7) / 8 * 8;
-  whole.c = nullptr;
-  *workspace = AttachWorkspace(&whole, a.device(), stream, which);
-  g.workspace = whole.workspace;
-  g.workspace_bytes = whole.workspace_bytes;
   g.hidden_in = hin;
   g.hidden_out = hout;
+  *workspace = AttachWorkspace(&g, gg_workspace_bytes_for_strided(&g, a.size(-1), b.size(-1)), a.device(), stream, which);
   return g;
 }
 
@@ -519,7 +514,7 @@ c10::optional<std::pair<torch::Tensor, torch::Tensor>> GroupedGemmSwiGLUKeep(con
   gg_gmm_args g = Arguments(a, b, c, sizes, false, trans_b, false, 0, RowIndices(), true, stream);
   if (!gg_keeps_gate_up(&g)) return c10::nullopt;
   torch::Tensor gate_up = torch::empty({a.size(0), cols}, a.options());
-  const torch::Tensor workspace = AttachWorkspace(&g, a.device(), stream);
+  const torch::Tensor workspace = AttachWorkspace(&g, gg_workspace_bytes_for(&g), a.device(), stream);
   const int rc = gg_gmm_keep_gate_up(&g, gate_up.data_ptr());
   TORCH_CHECK(rc == GG_OK, "grouped_gemm: ", gg_last_error());
   return std::make_pair(c, gate_up);

@@ -271,6 +271,8 @@ int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up);
  * reference, which asks CUTLASS for its workspace size per call (csrc/grouped_gemm.cu:347-349).
  */
 uint64_t gg_workspace_bytes_for(const gg_gmm_args* args);
+/* The same for gg_gmm_strided and the calls of gg_gmm_pair_strided, whatever their sizes; 0 where the strides do not fit. */
+uint64_t gg_workspace_bytes_for_strided(const gg_gmm_args* args, int64_t a_row, int64_t b_row);
 
 /*
  * gg_gmm for callers that cannot allocate and have no workspace to bring: code under HIP graph

@@ -274,6 +274,39 @@ def test_workspace_bytes_for_needs_no_device():
     assert want(dtype=2, hidden_in=12288) == full and want(dtype=2, hidden_in=12160) == 0
 
 
+def test_workspace_bytes_for_strided_operands():
+    """gg_workspace_bytes_for_strided: by the call's own sizes, whatever they are (gg_workspace_bytes_for has nothing for
+    hidden sizes that are no multiples of 8: its calls run those without pieces)."""
+    lib = ctypes.CDLL(HIP_LIB)
+    for f in (lib.gg_workspace_bytes_for_strided, lib.gg_workspace_bytes_for):
+        f.restype = ctypes.c_uint64
+    lib.gg_workspace_bytes_for_strided.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64]
+    lib.gg_workspace_bytes_for.argtypes = [ctypes.c_void_p]
+    full = 4096 + 256 * 256 * 256 * 4
+
+    def want(a_row, b_row, plain, **kw):
+        g = _Args()
+        g.struct_bytes = ctypes.sizeof(_Args)
+        g.a, g.b, g.c = 4096, 8192, 12288 + 2
+        g.num_groups, g.tokens, g.hidden_in, g.hidden_out = 8, 32768, 14335, 4095
+        for k, v in kw.items():
+            setattr(g, k, v)
+        assert lib.gg_workspace_bytes_for(ctypes.byref(g)) == plain
+        return lib.gg_workspace_bytes_for_strided(ctypes.byref(g), a_row, b_row)
+
+    assert lib.gg_workspace_bytes_for_strided(None, 8, 8) == 0
+    assert want(14336, 4096, 0) == full and want(14336, 14336, 0, trans_b=1) == full
+    assert want(14336, 4096, 0, trans_a=1) == full
+    assert want(6144, 4096, 0, hidden_in=6143) == full and want(6080, 4096, 0, hidden_in=6079) == 0
+    # groups of few rows: as for the same call on whole chunks
+    few = dict(num_groups=16, tokens=960, hidden_out=2047, dtype=1)
+    assert want(6144, 2048, 0, hidden_in=6144, **few) == want(6144, 2048, full, **{**few, "hidden_in": 6144, "hidden_out": 2048, "c": 12288})
+    assert want(14336, 4096, 0, struct_bytes=4) == 0 and want(14336, 4096, 0, flags=1) == 0
+    # (strides that gg_gmm_strided refuses, and what it does not take)
+    assert want(14328, 4096, 0) == 0 and want(14336, 4100, 0) == 0 and want(14336, 4096, 0, a=4096 + 8) == 0
+    assert want(14336, 4096, 0, dtype=2) == 0 and want(14336, 4096, 0, epilogue=1) == 0 and want(1 << 22, 4096, 0) == 0
+
+
 def test_tile_shapes_need_no_device():
     """The tile shape each call of the GPU tests of tile shapes runs on, so that a moved threshold cannot leave a
     shape without a test; and the general kernels, where a half of gate | up is no multiple of 8."""
