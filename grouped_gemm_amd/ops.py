@@ -5,6 +5,8 @@ backward is two more: the input gradient with the opposite layout of `b`, and th
 weight gradient with `trans_a` (per expert a_e^T @ grad_e, zeros for an expert
 without tokens).
 """
+from typing import Tuple
+
 import torch
 
 from grouped_gemm_amd import backend
@@ -162,7 +164,8 @@ def gmm_swiglu(a, w, batch_sizes, trans_b=False):
 # The same operator registered with torch.library, so that torch.compile sees one opaque node
 # with a known output shape instead of a call into an extension it cannot trace.  Not part of
 # the reference's surface (its ops.py stops at gmm above); results and gradients are those of
-# GroupedGemm, through the same backend calls.
+# GroupedGemm, through the same backend calls: where both gradients are wanted, one operator for the
+# two (one launch may plan its last round otherwise than two do: fp32 sums in another order).
 
 def _register_traceable():
     @torch.library.custom_op("grouped_gemm_amd::gmm", mutates_args=())
@@ -174,11 +177,25 @@ def _register_traceable():
     def _gmm_op_fake(a, b, batch_sizes, trans_a, trans_b):
         return backend._allocate_output(a, b, batch_sizes, trans_a, trans_b)
 
+    @torch.library.custom_op("grouped_gemm_amd::gmm_gradients", mutates_args=())
+    def _gradients_op(grad: torch.Tensor, a: torch.Tensor, b: torch.Tensor, batch_sizes: torch.Tensor,
+                      trans_b: bool) -> Tuple[torch.Tensor, torch.Tensor]:
+        return backend.gradients(grad, a, b, batch_sizes, trans_b, True, True)
+
+    @_gradients_op.register_fake
+    def _gradients_op_fake(grad, a, b, batch_sizes, trans_b):
+        lhs, rhs = (grad, a) if trans_b else (a, grad)
+        return (backend._allocate_output(grad, b, batch_sizes, False, not trans_b),
+                backend._allocate_output(lhs, rhs, batch_sizes, True, False))
+
+    def _refuse_gradients():   # only reached when a gradient is wanted
+        raise RuntimeError("grouped_gemm_amd::gmm is differentiable as a @ b or a @ b^T only "
+                           "(trans_a=False), as GroupedGemm is")
+
     def _gmm_op_setup_context(ctx, inputs, output):
         a, b, batch_sizes, trans_a, trans_b = inputs
-        if trans_a:   # only reached when a gradient is wanted
-            raise RuntimeError("grouped_gemm_amd::gmm is differentiable as a @ b or a @ b^T only "
-                               "(trans_a=False), as GroupedGemm is")
+        if trans_a:
+            _refuse_gradients()
         ctx.save_for_backward(a, b, batch_sizes)
         ctx.trans_b = trans_b
 
@@ -186,15 +203,20 @@ def _register_traceable():
         grad = grad.contiguous()
         a, b, batch_sizes = ctx.saved_tensors
         agrad = bgrad = None
-        if ctx.needs_input_grad[0]:
+        if ctx.needs_input_grad[0] and ctx.needs_input_grad[1]:
+            agrad, bgrad = _gradients_op(grad, a, b, batch_sizes, ctx.trans_b)
+        elif ctx.needs_input_grad[0]:
             agrad = _gmm_op(grad, b, batch_sizes, False, not ctx.trans_b)
-        if ctx.needs_input_grad[1]:
+        elif ctx.needs_input_grad[1]:
             lhs, rhs = (grad, a) if ctx.trans_b else (a, grad)
             bgrad = _gmm_op(lhs, rhs, batch_sizes, True, False)
         return agrad, bgrad, None, None, None
 
     torch.library.register_autograd("grouped_gemm_amd::gmm", _gmm_op_backward,
                                     setup_context=_gmm_op_setup_context)
+    # (gradients of both gradients: refused, as the weight gradient refuses its own)
+    torch.library.register_autograd("grouped_gemm_amd::gmm_gradients", lambda ctx, *grads: _refuse_gradients(),
+                                    setup_context=lambda ctx, inputs, output: _refuse_gradients())
     return _gmm_op
 
 

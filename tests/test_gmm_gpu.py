@@ -1294,6 +1294,35 @@ def test_traceable_operator_under_torch_compile(ops, trans_b):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("compiled", [False, True])
+def test_traceable_operator_gives_the_gradients_of_the_plain_one(ops, compiled):
+    # Bit for bit, also where both gradients in one launch add up in another order than in two: 3 groups,
+    # 512 -> 2048, whose input gradient is cut in pieces.  And one gradient alone, and gradients of gradients, which
+    # both forms of the weight gradient refuse.
+    g = torch.Generator().manual_seed(1)
+    sizes = torch.bincount(torch.randint(0, 3, (2000,), generator=g), minlength=3).cuda()
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    a0, b0, grad = draw(2000, 512), draw(3, 512, 2048), draw(2000, 2048)
+    traceable = lambda a, b: ops.gmm_traceable(a, b, sizes)
+    if compiled:
+        traceable = torch.compile(traceable, backend="aot_eager", fullgraph=True)
+    _announce("traceable gradients", compiled)
+    for wants in ((True, True), (True, False), (False, True)):
+        got = []
+        for fn in (lambda a, b: ops.gmm(a, b, sizes), traceable):
+            a, b = a0.clone().requires_grad_(wants[0]), b0.clone().requires_grad_(wants[1])
+            out = fn(a, b)
+            out.backward(grad)
+            got.append((out.detach(), a.grad, b.grad))
+        for x, y in zip(*got):
+            assert (x is None and y is None) or torch.equal(x, y), wants
+        assert (got[1][1] is not None, got[1][2] is not None) == wants
+    if not compiled:
+        a, b = a0.clone().requires_grad_(), b0.clone().requires_grad_()
+        with pytest.raises(RuntimeError, match="differentiable as a @ b"):
+            torch.autograd.grad(ops.gmm_traceable(a, b, sizes), (a, b), grad, create_graph=True)
+
+
 # ------------------------------------------------------------------- float16 operands
 
 @pytest.mark.parametrize("layout", [(False, False), (False, True), (True, False)])

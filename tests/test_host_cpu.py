@@ -492,6 +492,18 @@ def test_config1_fixture_matches_oracle(oracle):
 
 # ----------------------------------------------------------------- traceable operator
 
+def test_traceable_gradients_shapes_without_a_device():
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from grouped_gemm_amd import ops  # noqa: F401 (registers the operators)
+    for trans_b, shape in ((False, (4, 64, 96)), (True, (4, 96, 64))):
+        with FakeTensorMode():
+            a, b = torch.empty(100, 64, dtype=torch.bfloat16), torch.empty(shape, dtype=torch.bfloat16)
+            grad, sizes = torch.empty(100, 96, dtype=torch.bfloat16), torch.empty(4, dtype=torch.int64)
+            agrad, bgrad = torch.ops.grouped_gemm_amd.gmm_gradients(grad, a, b, sizes, trans_b)
+        assert agrad.shape == (100, 64) and bgrad.shape == shape
+
+
 def test_traceable_operator_shapes_without_a_device():
     # the torch.library form of the operator: output shapes for all three layouts from fake
     # tensors alone (what torch.compile needs), no kernel runs
