@@ -153,9 +153,13 @@ class GroupedGemmSwiGLU(torch.autograd.Function):
         return agrad, wgrad, None, None, None
 
 
-def gmm_swiglu(a, w, batch_sizes, trans_b=False):
-    """silu(a @ gate) * (a @ up) per expert, w = [gate | up]; see backend.gmm_swiglu."""
-    keep = torch.is_grad_enabled() and (a.requires_grad or w.requires_grad)
+def gmm_swiglu(a, w, batch_sizes, trans_b=False, keep_products=True):
+    """silu(a @ gate) * (a @ up) per expert, w = [gate | up]; see backend.gmm_swiglu.
+
+    keep_products: the two products may be held from forward to backward (4 bytes per element of the
+    result, at most as much as a and w take); False: the backward computes them again, and nothing but the operands is
+    held."""
+    keep = keep_products and torch.is_grad_enabled() and (a.requires_grad or w.requires_grad)
     return GroupedGemmSwiGLU.apply(a, w, batch_sizes, trans_b, keep)
 
 

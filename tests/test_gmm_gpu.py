@@ -2317,6 +2317,24 @@ def test_swiglu_gradients_from_kept_and_recomputed_products(ops):
         assert ops.gmm_swiglu(a, w, sizes).grad_fn is None
 
 
+def test_swiglu_holds_no_products_where_the_caller_says_so(ops):
+    # The operands alone are held between forward and backward, for the same results.
+    g = torch.Generator().manual_seed(6)
+    sizes = torch.tensor([300, 0, 212], dtype=torch.int64).cuda()
+    draw = lambda *shape: (torch.randn(*shape, generator=g) * 0.2).to(torch.bfloat16).cuda().requires_grad_(True)
+    a, w, upstream = draw(512, 256), draw(3, 256, 528), draw(512, 264).detach()
+    got = []
+    for keep in (True, False):
+        held = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: held.append(tuple(t.shape)) or t, lambda t: t):
+            out = ops.gmm_swiglu(a, w, sizes, keep_products=keep)
+        assert held == [(512, 256), (3, 256, 528), (3,)] + ([(512, 528)] if keep else [])
+        got.append((out.detach(), *torch.autograd.grad(out, (a, w), upstream)))
+    assert torch.equal(got[0][0], got[1][0])
+    for x, y in zip(got[0][1:], got[1][1:]):
+        check(x, y.float(), "gradients")
+
+
 @pytest.mark.parametrize("sizes", [[4096] * 8, [40] * 700, [60, 64, 33]])
 def test_swiglu_epilogue_divides_in_full_precision(ops, sizes):
     # silu(gate) * up of known pre-activations (rows times an identity), `up` chosen so that the product lies as
