@@ -693,11 +693,12 @@ int gmm_impl(const gg_gmm_args& g, bool static_scratch = false) {
 }
 
 // Groups of few rows and large weights: the first product does nothing but read weights, the second nothing but
-// write gradients, and reads queue behind writes.  Us, two launches and one: 134 x 58 rows, 600 x 8960: 765 / 800;
-// 108 x 23, 3792 x 9328: 3295 / 3356; 116 x 6, 2688 x 10304: 2025 / 2144; 70 x 12, 824 x 6416: 390 / 405; and with smaller ones
-// (MB of weights) 38 x 19, 1944 x 2496 (369): 205 / 200; 83 x 29, 168 x 4152 (116): 89 / 88; 27 x 51, 1024 x 1032 (57): 49 / 48;
-// 6 x 95, 208 x 2880 (7): 25 / 20.
-constexpr int64_t kPairWeightBytes = int64_t(128) << 20;
+// write gradients, and reads queue behind writes.  Two launches' time over one's, geometric mean, least and most of 110 products drawn
+// over 2 - 105 rows to a group, 6 - 200 groups, 128 - 7168 -> 128 - 10000, by MB of weights: below 64 1.09 (1.00 - 1.17), to
+// 128 1.07 (1.02 - 1.17), to 384 1.03 (0.97 - 1.07), to 700 1.00 (0.90 - 1.10), to 900 0.97 (0.86 - 1.03), to 1500 0.99 (0.90 - 1.02).
+// Us: 48 x 65 rows, 3600 -> 1184 (390): 211 in two, 202 in one; 13 x 9, 3856 -> 4744 (454): 233 / 252; 20 x 6, 2504 -> 9016 (861): 408 /
+// 466; 108 x 23, 3792 x 9328 (7290): 3295 / 3356.
+constexpr int64_t kPairWeightBytes = int64_t(384) << 20;
 constexpr int64_t kLongRounds = 8;   // (see pair_kernel)
 bool reads_then_writes(const gg_gmm_args& g) {
   return use_short_shape(g.num_groups, g.tokens, 0) && g.num_groups * g.hidden_in * g.hidden_out * 2 > kPairWeightBytes;
@@ -714,8 +715,10 @@ const gg::PairOps* pair_kernel(const gg_gmm_args& g1, const Plan& p1, const gg_g
     return nullptr;
   if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace == p2.p.workspace) return nullptr;
   if (reads_then_writes(g1)) return nullptr;
-  // (launches of many rounds have nothing to gain: 8 x 4096 rows, 4096 -> 14336, forward and gradients 8383 in two, 8457 in
-  // one; 256 x 256, 7168 -> 2048: 6753 / 6777; 16 x 1024, 2048 -> 4096, 4 rounds of the first: 520 in two, 510 in one)
+  // (launches of many rounds have little to gain.  Two launches' time over one's by the rounds of the shorter product, geometric mean,
+  // least and most of 50 products of 120 - 6000 rows to a group: 2 to 5 rounds 1.03 (0.98 - 1.09), 5 to 8 1.026 (1.013 - 1.042), 8 to 10
+  // 1.008 (1.000 - 1.016), 10 to 24 1.002 (0.994 - 1.010); 8 x 4096 rows, 4096 -> 14336 (8.25), forward and gradients: 8383 us
+  // in two, 8457 in one; 256 x 256, 7168 -> 2048 (42): 6753 / 6777)
   if (expected_tiles(g1, p1.shape.bm, p1.shape.bn) >= kLongRounds * kFullLaunch &&
       expected_tiles(g2, p2.shape.bm, p2.shape.bn) >= kLongRounds * kFullLaunch)
     return nullptr;

@@ -409,6 +409,19 @@ def test_pairs_that_share_a_workspace():
     assert _pair(lib, [60, 50], 64, 72, True, workspaces=((at, least), (at + 256, least))) == (0, (64, 128, 128, 128))
 
 
+def test_pairs_by_weights_and_rounds():
+    """Which gradients take one launch: few rows to a group up to 384 MB of weights, others below eight rounds of tiles of
+    either product."""
+    lib = ctypes.CDLL(HIP_LIB)
+    one = lambda *args, **kw: any(_pair(lib, *args, **kw)[1])
+    assert one([19] * 38, 1944, 2496, False) and one([65] * 45, 1064, 1184, True)
+    assert one([6] * 96, 1024, 2048, False) and not one([6] * 97, 1024, 2048, False)          # 384 MB and 388
+    assert not one([9] * 13, 3856, 4744, True) and not one([23] * 108, 3792, 9328, False)
+    assert one([1024] * 16, 2048, 4096, False) and not one([4096] * 8, 4096, 14336, False)   # 4 rounds of one, 8 of both
+    assert one([4096] * 8, 4096, 1408, False)                                                 # 8 and 3
+    assert not one([600] * 513, 64, 64, False)                                                # more groups than one launch takes
+
+
 def _deep_cut(lib, rows, per_group, workgroups, partial_tiles, tile_outputs):
     sizes, pieces, tiles = (ctypes.c_int64 * len(rows))(*rows), ctypes.c_int(-1), ctypes.c_int(-1)
     assert lib.gg_debug_deep_cut(sizes, ctypes.c_int64(len(rows)), ctypes.c_int64(per_group), workgroups, partial_tiles,
