@@ -2800,6 +2800,131 @@ def test_both_gradients_in_one_launch(ops, oracle, experts, rows, hin, hout, tra
         assert ((got - alone).abs() <= 2.0 ** -7 * alone.abs() + 1e-4 * alone.abs().max()).all()
 
 
+# Gradients that go out in one launch, one case per pair kernel of an element type, on multiples of 8 and on odd sizes: groups,
+# rows, hidden_in, hidden_out, trans_b, and the tile shapes of the input and of the weight gradient (gg_debug_pair has to
+# say so, here and without a device).
+_FULL, _SHORT, _SMALL, _SQUARE = (256, 256), (128, 256), (64, 128), (128, 128)
+_PAIR_SHAPES = [
+    (8, 8192, 2048, 1368, False, _FULL, _FULL),        # extra tiles for the workgroups that start early
+    (28, 6648, 776, 216, False, _FULL, _SQUARE),
+    (39, 370, 1192, 208, False, _SHORT, _FULL),
+    (3, 6000, 264, 6408, False, _SHORT, _SQUARE),      # deep on both sides: pieces of the input gradient, of the weight gradient too
+    (36, 69, 272, 520, False, _SMALL, _FULL),
+    (5, 300, 136, 264, False, _SMALL, _SQUARE),
+    (24, 2755, 1824, 216, True, _FULL, _FULL),
+    (9, 5519, 1792, 960, True, _FULL, _SQUARE),
+    (32, 4096, 768, 2048, True, _SHORT, _FULL),
+    (12, 8381, 264, 208, True, _SHORT, _SQUARE),
+    (39, 31, 520, 264, True, _SMALL, _FULL),
+    (5, 300, 136, 2056, True, _SMALL, _SQUARE),
+    (24, 120, 3200, 1024, True, _SHORT, _FULL),        # 157 MB of weights, few rows
+    (8, 8192, 2047, 1361, False, _FULL, _FULL),
+    (28, 6644, 805, 218, False, _FULL, _SQUARE),
+    (31, 400, 1601, 207, False, _SHORT, _FULL),
+    (2, 5900, 259, 6403, False, _SHORT, _SQUARE),
+    (26, 31, 411, 522, False, _SMALL, _FULL),
+    (5, 300, 137, 265, False, _SMALL, _SQUARE),
+    (26, 3133, 1615, 201, True, _FULL, _FULL),
+    (9, 5500, 1791, 961, True, _FULL, _SQUARE),
+    (26, 640, 1819, 207, True, _SHORT, _FULL),
+    (18, 8829, 261, 207, True, _SHORT, _SQUARE),
+    (35, 34, 523, 281, True, _SMALL, _FULL),
+    (5, 300, 137, 2051, True, _SMALL, _SQUARE),
+]
+
+
+def _row_stride(n):
+    return n if n % 8 == 0 else (n + 63) // 64 * 64
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("experts,rows,hin,hout,trans_b,first,second", _PAIR_SHAPES)
+def test_every_pair_kernel(oracle, experts, rows, hin, hout, trans_b, first, second, dtype):
+    # Through the C entry points, in the tiles that the case names, against the oracle: outputs between sentinels, on odd elements
+    # for odd sizes; NaNs behind the operands' rows, as near as they may be; counters of both workspaces zero afterwards.
+    _announce("pair kernel", experts, rows, hin, hout, trans_b, first, second, dtype)
+    lib = _c_abi()
+    odd = hin % 8 != 0 or hout % 8 != 0
+    g = torch.Generator().manual_seed(rows)
+    share = torch.rand(experts, generator=g) + 0.3
+    share[experts // 2] = 0
+    sizes = torch.bincount(torch.multinomial(share, rows - 3, replacement=True, generator=g), minlength=experts)
+    used = rows - 3
+
+    def operand(*shape):   # and the same with its rows further apart
+        t = torch.randn(*shape, generator=g).to(dtype).cuda()
+        n = shape[-1]
+        if not odd or n % 8 == 0:
+            return t, t
+        far = torch.full((*shape[:-1], _row_stride(n)), float("nan"), dtype=dtype, device="cuda")
+        far[..., :n], far[..., n:(n + 7) // 8 * 8] = t, 0
+        return t, far
+
+    def output(*shape):
+        n = int(np.prod(shape))
+        buffer = torch.full((n + 64,), 3.0, dtype=dtype, device="cuda")
+        at = 33 if odd else 32
+        return buffer, buffer[at:at + n].view(*shape)
+
+    (a, a_far), (grad, grad_far) = operand(rows, hin), operand(rows, hout)
+    b, b_far = operand(experts, *((hout, hin) if trans_b else (hin, hout)))
+    (buffer1, agrad), (buffer2, bgrad) = output(rows, hin), output(*b.shape)
+    lhs, rhs = (grad, a) if trans_b else (a, grad)
+    lhs_far, rhs_far = (grad_far, a_far) if trans_b else (a_far, grad_far)
+    on_device = trans_b
+    bs = sizes.cuda() if on_device else sizes
+    ws = [torch.zeros(4096 + 256 * 256 * 256 * 4, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    code, flags = int(dtype == torch.float16), 128
+    one = _gmm_args(lib, grad_far, b_far, agrad, bs, on_device, rows, hout, hin, False, not trans_b, flags, ws[0], code)
+    two = _gmm_args(lib, lhs_far, rhs_far, bgrad, bs, on_device, rows, lhs.shape[1], rhs.shape[1], True, False, flags, ws[1], code)
+    strides = [t.shape[-1] for t in (grad_far, b_far, lhs_far, rhs_far)]
+    shapes = (ctypes.c_int * 4)()
+    assert lib.gg_debug_pair(ctypes.byref(one), ctypes.byref(two), (ctypes.c_int64 * 4)(*strides) if odd else None, shapes) == 0
+    assert tuple(shapes) == first + second
+    want_a = oracle.gmm_loop(grad.float(), b.float(), sizes, trans_b=not trans_b)[:used]
+    want_b = oracle.gmm_loop(lhs.float(), rhs.float(), sizes, trans_a=True)
+    for _ in range(2):
+        if odd:
+            i64 = ctypes.c_int64
+            rc = lib.gg_gmm_pair_strided(ctypes.byref(one), i64(strides[0]), i64(strides[1]), ctypes.byref(two), i64(strides[2]), i64(strides[3]))
+        else:
+            rc = lib.gg_gmm_pair(ctypes.byref(one), ctypes.byref(two))
+        assert rc == 0, lib.gg_last_error()
+        torch.cuda.synchronize()
+        for got, want, what in ((agrad[:used], want_a, "input gradient"), (bgrad, want_b, "weight gradient")):
+            scale = max(1.0, float(want.pow(2).mean().sqrt()))
+            check(got.float() / scale, want / scale, what)
+        for buffer, inside in ((buffer1, used * hin), (buffer2, bgrad.numel())):
+            at = 33 if odd else 32
+            assert (buffer[:at] == 3).all() and (buffer[at + inside:] == 3).all()
+        assert not ws[0][:4096].any() and not ws[1][:4096].any()
+
+
+def test_two_calls_on_one_workspace(oracle):
+    # A pair that shares a workspace is launched one call after the other: the bits of the two calls alone.
+    _announce("pair, one workspace")
+    lib = _c_abi()
+    g = torch.Generator().manual_seed(23)
+    sizes, hin, hout = torch.tensor([700, 0, 5300]), 264, 8192
+    draw = lambda *shape: torch.randn(*shape, generator=g).to(torch.bfloat16).cuda()
+    a, grad, b = draw(6000, hin), draw(6000, hout), draw(3, hin, hout)
+    ws = torch.zeros(4096 + 256 * 256 * 256 * 4, dtype=torch.uint8, device="cuda")
+    outs = [(torch.zeros_like(a), torch.zeros_like(b)) for _ in range(2)]
+    for together, (agrad, bgrad) in zip((True, False), outs):
+        one = _gmm_args(lib, grad, b, agrad, sizes, False, 6000, hout, hin, False, True, 128, ws)
+        two = _gmm_args(lib, a, grad, bgrad, sizes, False, 6000, hin, hout, True, False, 128, ws)
+        calls = [lambda: lib.gg_gmm_pair(ctypes.byref(one), ctypes.byref(two))] if together else \
+            [lambda: lib.gg_gmm(ctypes.byref(one)), lambda: lib.gg_gmm(ctypes.byref(two))]
+        for call in calls:
+            assert call() == 0, lib.gg_last_error()
+        torch.cuda.synchronize()
+        assert not ws[:4096].any()
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    want = oracle.gmm_loop(a.float(), grad.float(), sizes, trans_a=True)
+    scale = float(want.pow(2).mean().sqrt())
+    check(outs[0][1].float() / scale, want / scale, "weight gradient")
+
+
 def test_both_gradients_in_one_launch_inside_a_graph(ops):
     sizes = torch.tensor([700, 0, 300, 500], dtype=torch.int64).cuda()
     g = torch.Generator().manual_seed(41)

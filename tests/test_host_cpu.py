@@ -422,6 +422,70 @@ def test_pairs_by_weights_and_rounds():
     assert not one([600] * 513, 64, 64, False)                                                # more groups than one launch takes
 
 
+def test_every_pair_kernel_has_a_case():
+    """The tiles that each case of the GPU test of pair kernels takes, so that a moved threshold cannot leave a kernel
+    without a test: every one of the library's pairs, of both element types, on multiples of 8 and on odd sizes."""
+    import re
+    from test_gmm_gpu import _PAIR_SHAPES, _row_stride
+    lib = ctypes.CDLL(HIP_LIB)
+    names = {(256, 256): "Wide", (128, 256): "Short", (64, 128): "Small", (128, 128): "SmallSquare"}
+    reached = {False: set(), True: set()}
+    for experts, rows, hin, hout, trans_b, first, second in _PAIR_SHAPES:
+        odd = hin % 8 != 0 or hout % 8 != 0
+        sizes = [rows // experts] * (experts - 1) + [rows - rows // experts * (experts - 1)]
+        in_row, out_row = _row_stride(hin), _row_stride(hout)
+        strides = (out_row, in_row if trans_b else out_row, *((out_row, in_row) if trans_b else (in_row, out_row))) if odd else None
+        for dtype in (0, 1):
+            assert _pair(lib, sizes, hin, hout, trans_b, dtype=dtype, strides=strides) == (0, first + second)
+            reached[odd].add(("kBF16 kF16".split()[dtype], "kNN" if trans_b else "kNT", names[first], names[second]))
+    built = open(os.path.join(ROOT, "grouped_gemm_amd", "csrc", "gmm_variants.def")).read()
+    pairs = set(re.findall(r"^GG_PAIR\(\d+, (\w+), (\w+), (\w+), (\w+)\)", built, flags=re.M))
+    assert len(pairs) == 24 and reached[False] == pairs and reached[True] == pairs
+
+
+def test_entry_points_beside_gg_gmm_refuse_bad_arguments():
+    """gg_gmm_pair, gg_gmm_strided, gg_gmm_pair_strided, gg_keeps_gate_up and gg_gmm_keep_gate_up: every case fails before the
+    device is looked for."""
+    lib = ctypes.CDLL(HIP_LIB)
+    lib.gg_last_error.restype = ctypes.c_char_p
+    rows = (ctypes.c_int64 * 2)(3, 5)
+    i64 = ctypes.c_int64
+
+    def args(**kw):
+        g = _Args()
+        g.struct_bytes = ctypes.sizeof(_Args)
+        g.a, g.b, g.c = 4096, 8192, 12288
+        g.batch_sizes, g.num_groups, g.tokens, g.hidden_in, g.hidden_out = ctypes.addressof(rows), 2, 8, 136, 264
+        for k, v in kw.items():
+            setattr(g, k, v)
+        return ctypes.byref(g)
+
+    for bad in (None, args(struct_bytes=8)):
+        assert lib.gg_gmm_pair(bad, args()) == -1 and lib.gg_gmm_pair(args(tokens=0), bad) == -1
+        assert lib.gg_gmm_pair_strided(bad, i64(136), i64(264), args(), i64(136), i64(264)) == -1
+        assert lib.gg_gmm_strided(bad, i64(136), i64(264)) == -1
+        assert lib.gg_debug_pair(bad, args(), None, (ctypes.c_int * 4)()) == -1
+        assert lib.gg_keeps_gate_up(bad) == 0 and lib.gg_gmm_keep_gate_up(bad, ctypes.c_void_p(4096)) == -1
+    assert lib.gg_debug_pair(args(), args(), None, None) == -1
+    assert lib.gg_gmm_pair(args(trans_a=1, trans_b=1), args(trans_a=1)) == -1      # the first call alone is wrong,
+    assert lib.gg_gmm_pair(args(tokens=0), args(trans_a=1, tokens=7)) == -1       # the second alone (sizes past its rows)
+    for a_row, b_row, kw in ((132, 264, {}), (128, 264, {}), (136, 256, {}), (136, 264 + 4, {}), (1 << 22, 264, {}),
+                             (136, 264, dict(a=4096 + 8)), (136, 264, dict(b=8192 + 2)), (136, 264, dict(dtype=2)),
+                             (136, 264, dict(epilogue=1)), (136, 264, dict(trans_a=1, accumulate_f32=1)),
+                             (136, 264, dict(a_row_index=64)), (136, 128, dict(trans_b=1)), (264, 136, dict(trans_a=1))):
+        assert lib.gg_gmm_strided(args(**kw), i64(a_row), i64(b_row)) == -1, (a_row, b_row, kw)
+        assert b"strides" in lib.gg_last_error()
+        assert lib.gg_gmm_pair_strided(args(**kw), i64(a_row), i64(b_row), args(), i64(136), i64(264)) == -1
+    swiglu = dict(epilogue=1)
+    assert lib.gg_keeps_gate_up(args(**swiglu)) == 1 and lib.gg_keeps_gate_up(args(dtype=1, **swiglu)) == 1
+    for kw in (dict(epilogue=0), dict(dtype=2, **swiglu), dict(hidden_in=132, **swiglu), dict(hidden_out=260, **swiglu),
+               dict(c=12288 + 8, **swiglu), dict(c_row_index=64, **swiglu)):
+        assert lib.gg_keeps_gate_up(args(**kw)) == 0 and lib.gg_gmm_keep_gate_up(args(**kw), ctypes.c_void_p(4096)) == -1
+    for at in (0, 4096 + 8, 4096 + 2):
+        assert lib.gg_gmm_keep_gate_up(args(**swiglu), ctypes.c_void_p(at)) == -1
+        assert b"16-byte" in lib.gg_last_error()
+
+
 def _deep_cut(lib, rows, per_group, workgroups, partial_tiles, tile_outputs):
     sizes, pieces, tiles = (ctypes.c_int64 * len(rows))(*rows), ctypes.c_int(-1), ctypes.c_int(-1)
     assert lib.gg_debug_deep_cut(sizes, ctypes.c_int64(len(rows)), ctypes.c_int64(per_group), workgroups, partial_tiles,
