@@ -12,7 +12,6 @@
 #include <functional>
 #include <mutex>
 #include <numeric>
-#include <vector>
 
 #include "gmm_generic.hpp"
 #include "gmm_variants.hpp"
@@ -394,7 +393,7 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // wide ones: 19 x 2569 rows, 384 x 128 (38): 53 / 25; 5 x 3106, 608 x 240 (15): 60 / 24; 3 x 4000, 1024 x 1024, Zipf 1.2 (48):
 // 82 / 53; 4 x 15000, 1024 x 512 (32): 101 / 72; 6 x 5000, 768 x 1024 (72): 89 / 64; 8 x 5000, 1024 x 1024 (128): 89 / 84; with fp32
 // accumulation 98 / 70 and 108 / 94; but 4 x 10000, 2048 x 1024 (128): 154 / 170.  Only where the caller says so
-// (GG_FLAG_FEW_TILES, as the PyTorch binding does): calls through the C ABI keep the order of their sums.
+// (GG_FLAG_FEW_TILES, as the PyTorch binding always does): of the rules here the only one that is an option of the C ABI.
 constexpr int64_t kDeepGroups = 2560;
 constexpr int64_t kMiddlingGroups = 512;
 constexpr int64_t kVeryDeepGroups = 8192;
@@ -832,10 +831,12 @@ int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t ti
   if (batch_sizes == nullptr || num_groups < 1 || num_groups > GG_MAX_GROUPS_PER_LAUNCH || tiles_per_group < 1 ||
       tiles_per_group > (1 << 20) || workgroups < 1 || partial_tiles < 0 || pieces == nullptr || tiles == nullptr)
     return fail(GG_EINVAL, "bad argument");
-  std::vector<int64_t> rows(batch_sizes, batch_sizes + num_groups);
-  std::sort(rows.begin(), rows.end(), std::greater<int64_t>());
-  if (rows.back() < 0 || rows.front() >= (int64_t(1) << 31) / num_groups) return fail(GG_EINVAL, "batch_sizes are negative or too large");
-  const int64_t all = std::accumulate(rows.begin(), rows.end(), int64_t(0));
+  int64_t rows[GG_MAX_GROUPS_PER_LAUNCH];
+  std::copy(batch_sizes, batch_sizes + num_groups, rows);
+  std::sort(rows, rows + num_groups, std::greater<int64_t>());
+  if (rows[num_groups - 1] < 0 || rows[0] >= (int64_t(1) << 31) / num_groups)
+    return fail(GG_EINVAL, "batch_sizes are negative or too large");
+  const int64_t all = std::accumulate(rows, rows + num_groups, int64_t(0));
   const gg::DeepCut cut = gg::cut_deep_tiles([&](int q) { return (int)((rows[q] + gg::BK - 1) / gg::BK); }, (int)num_groups, all,
                                              (int)tiles_per_group, workgroups, partial_tiles,
                                              gg::min_slices_per_piece(tile_outputs), gg::BK);

@@ -62,7 +62,9 @@ extern "C" {
 #define GG_FLAG_ONE_CLASS 2     /* hand out a tall group's short last tile row in place, not after all other tiles */
 #define GG_FLAG_ROW_PIECES 4    /* ignore the workspace: cut the last round's tiles along the rows only */
 #define GG_FLAG_GROUP_ORDER 8   /* hand out the groups' tiles in group order, also where the library would hand them out by their number of tile rows (many short groups, trans_a = 0) */
-#define GG_FLAG_FEW_TILES 128   /* trans_a = 1: smaller tiles also for deep groups whose full tiles would leave at least half of the device idle (up to three times as fast; sums in another order than without) */
+/* ... and one that is for speed: with trans_a, smaller tiles also for deep groups whose full tiles would leave at
+ * least half of the device idle, up to three times as fast (sums in another order than without). */
+#define GG_FLAG_FEW_TILES 128
 
 /*
  * One-time set-up for the current device: checks that it is a gfx950 and raises the LDS limit
@@ -228,10 +230,11 @@ typedef struct gg_gmm_args {
 int gg_gmm(const gg_gmm_args* args);
 
 /*
- * Two independent calls, neither of which reads what the other writes: the same results as
- * gg_gmm(first) followed by gg_gmm(second), in one launch where that is possible (a product with plain
+ * Two independent calls, neither of which reads what the other writes: gg_gmm(first) followed by
+ * gg_gmm(second), in one launch where that is possible (a product with plain
  * rows and epilogue, then a weight gradient over the same batch_sizes, stream and tokens, two-byte elements:
- * the two gradients of a product).  Compute units that run out of tiles of the first then go on with the
+ * the two gradients of a product).  One launch may cut the tiles of its last rounds into other depth pieces than two do:
+ * the same products, but where that is so fp32 sums in another order; the same bits on every call.  Compute units that run out of tiles of the first then go on with the
  * second.  The two must not share a workspace; where they do, they are launched one after the other, and
  * workspaces that overlap in part are refused (GG_EINVAL).
  * No counterpart in the reference, whose backward makes two calls (grouped_gemm/ops.py:19-29).
