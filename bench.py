@@ -34,10 +34,10 @@ PEAK_HBM_GBPS = 8000.0
 # the hash below (kernel_sources_sha16), and is reported only while the sources still have that
 # hash; the summary under profiles/ holds the figures, the commands and the commit.
 _TRAFFIC_KERNEL_SOURCES = ("gmm_kernel.hpp", "gmm_api.hip", "gmm_variants.hpp", "gmm_variants.def", "gmm_variant.hip")
-_TRAFFIC_KERNEL_SHA16 = "8f3effefeee82c43"
+_TRAFFIC_KERNEL_SHA16 = "87b0d1501df4f7c8"
 _TRAFFIC_SOURCE = ("profiles/gmm_kernel_mixtral_w1_hbm_traffic.md and profiles/gmm_kernel_configs_3_4_5_stats_and_traffic.md "
                    "(rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, kernel sources sha16 " + _TRAFFIC_KERNEL_SHA16 +
-                   ", commit 9f83f22; profiled once, not in this run)")
+                   ", commit d83e76f; profiled once, not in this run)")
 
 
 def kernel_sources_sha16():
@@ -55,10 +55,10 @@ def _traffic(fetch_kib, write_kib):
 
 
 MEASURED_TRAFFIC = {
-    2: {"fwd": _traffic(4042338, 917569), "agrad": _traffic(3318545, 276108), "bgrad": _traffic(2772976, 917552)},
-    3: {"fwd": _traffic(418102, 135175)},
-    4: {"bgrad": _traffic(2771937, 917540)},
-    5: {"fwd": _traffic(4241353, 262197), "agrad": _traffic(4816867, 917581), "bgrad": _traffic(1851677, 7345739)},
+    2: {"fwd": _traffic(4016084, 917548), "agrad": _traffic(3316306, 273422), "bgrad": _traffic(2762135, 917521)},
+    3: {"fwd": _traffic(410428, 135174)},
+    4: {"bgrad": _traffic(2756010, 917527)},
+    5: {"fwd": _traffic(4146437, 262172), "agrad": _traffic(4775926, 917592), "bgrad": _traffic(1851736, 7346337)},
 }
 
 
