@@ -13,7 +13,7 @@
 // arrive as zeros and no lane ever touches memory outside its group.  Fragments are read
 // from LDS with ds_read_b128 where the depth dimension is contiguous in memory and
 // with the transposing ds_read_b64_tr_b16 where it is not, feed
-// v_mfma_f32_32x32x16_bf16 with fp32 accumulators, and leave as bf16 through
+// v_mfma_f32_16x16x32_bf16 with fp32 accumulators, and leave as bf16 through
 // buffer stores that the descriptor clips at the group's last row (or are added to an fp32
 // output, in the accumulating form of the weight-gradient layout).
 #pragma once
@@ -261,6 +261,11 @@ constexpr int kDeviceScope = 16;
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+__device__ __forceinline__ const char* uniform_ptr(const char* p) {
+  const uint64_t b = reinterpret_cast<uint64_t>(p);
+  return reinterpret_cast<const char*>((uint64_t)(uint32_t)uniform((int)(uint32_t)b) | ((uint64_t)(uint32_t)uniform((int)(uint32_t)(b >> 32)) << 32));
+}
+
 // Buffer descriptor of `bytes` bytes at `base`, as the four dwords the hardware reads.
 // Both inputs are the same in every lane; reading them through the first lane tells the
 // compiler so and keeps the descriptor in scalar registers.
@@ -284,26 +289,35 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
                                            (uint32_t)uniform((int)bytes), kRsrcFlags);
 }
 
-// 16 bytes per lane from global memory straight into LDS at lds_addr + lane * 16.
+// 16 bytes per lane from global memory straight into LDS at lds_addr + OFFSET + lane * 16: the address, then
+// the load, which needs an instruction between the two.  Nothing else writes m0 (a reserved register: the compiler uses
+// it for nothing that occurs here).
 // Written as assembly on purpose: the compiler then keeps no record of pending writes
 // into LDS, and does not put a full wait for them in front of later LDS reads that touch
 // other buffers of the ring.  The waits that are needed are the explicit wait_vmcnt calls.
-__device__ __forceinline__ void load_to_lds_16(const rsrc_words& rsrc_in, uint32_t voffset,
-                                               uint32_t lds_addr) {
-  // (the descriptor is the same in every lane; saying so again here keeps it in scalar registers
-  // even where the compiler has parked it in vector registers for want of scalar ones)
-  rsrc_words rsrc;
-  rsrc[0] = uniform(rsrc_in[0]);
-  rsrc[1] = uniform(rsrc_in[1]);
-  rsrc[2] = uniform(rsrc_in[2]);
-  rsrc[3] = uniform(rsrc_in[3]);
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %0, %1, 0 offen lds"
-      :
-      : "v"(voffset), "s"(rsrc), "s"(lds_addr)
-      : "memory", "m0");
+template <int OFFSET>
+__device__ __forceinline__ void aim_lds(uint32_t lds_addr) {
+  asm volatile("s_add_u32 m0, %0, %1" : : "s"(lds_addr), "n"(OFFSET) : "memory", "m0", "scc");
+}
+// The hardware does not wait for a descriptor word that a vector instruction (v_readfirstlane, v_readlane) writes less
+// than five instructions before the load that reads it, and the compiler does not look into assembly: settle
+// puts the words where they stay, five instructions or more ahead of the first load that uses them (fetch_begin).  A test reads
+// the built library for loads that come too soon.
+template <int MORE = 0>   // instructions to wait here
+__device__ __forceinline__ void settle(rsrc_words& rsrc) {
+  if constexpr (MORE > 0) {
+    asm volatile("s_nop %1" : "+s"(rsrc) : "n"(MORE - 1));
+  } else {
+    asm volatile("" : "+s"(rsrc));
+  }
+}
+template <bool RIGHT_BEHIND>   // right behind aim_lds
+__device__ __forceinline__ void load_to_lds_16(const rsrc_words& rsrc, uint32_t voffset) {
+  if constexpr (RIGHT_BEHIND) {
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voffset), "s"(rsrc) : "memory");
+  } else {
+    asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(voffset), "s"(rsrc) : "memory");
+  }
 }
 
 __device__ __forceinline__ uint32_t lds_address(const void* p) {
@@ -331,6 +345,20 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(bf16x8 x, bf16x8 y, f32x16 acc) 
   } else {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x),
                                                   __builtin_bit_cast(f16x8, y), acc, 0, 0, 0);
+  }
+}
+
+// One 16x16x32 matrix instruction on fragments of 8 two-byte elements per lane: what the streaming kernel
+// multiplies two-byte elements with.  Per operation it moves half the accumulators of the 32x32x16 one in and out
+// of the register file, and power is what bounds these products: on operands like real activations, in
+// registers and nothing else running, 16x16x32 sustains 1970-2010 TFLOP/s (bf16), 32x32x16 1730-1800; on zeros,
+// at full clock, 2240 and 2275.
+template <int DT>
+__device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 x, bf16x8 y, f32x4 acc) {
+  if constexpr (DT == kBF16) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, acc, 0, 0, 0);
+  } else {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), acc, 0, 0, 0);
   }
 }
 
@@ -787,8 +815,9 @@ __global__ __launch_bounds__(64) void schedule_dump_kernel(GmmParams p, HostSize
 //
 // WidthMajor ("MC"): BK depth rows of W elements (M or N index contiguous).  LDS keeps
 // row-major rows of W*2 bytes; 64-byte segment s of depth row k sits at segment slot
-// s ^ g(k), g(k) = (k & 3) | ((k >> 1) & 4), so the 8 depth rows one transposing read
-// touches land in distinct bank groups.
+// s ^ (k & 3), and rows 8 .. 15 of every 16 start 32 bytes later (row_at), so the 8 depth rows (k .. k + 3 and
+// 8 below them) of which half a wave reads 16 columns at a time land in distinct groups of 8 banks, and the second
+// 16 columns of a block are 32 bytes behind the first ones in every lane.
 //
 // A lane's LDS slot is fixed by the hardware (wave base + lane * 16), so the swizzle is
 // applied by choosing which global chunk each lane fetches.
@@ -807,10 +836,10 @@ struct DepthMajor {
   static_assert(NT % CPR == 0 && (R * CPR) % NT == 0, "tile does not split over the block");
   static_assert(ROWS_PER_INSTR % (RP * CPR) == 0, "swizzle must not depend on the load index");
 
-  const char* base;   // first row of the tile, depth 0
+  const char* base;   // first row of the tile, next depth slice
   int ld;             // elements between rows ( = depth extent )
   int span;           // elements from the tile's first row to its last existing row
-  int depth;          // depth extent
+  int depth;          // depth values ahead of the cursor (below 0: past the end)
   int my_chunk;       // depth chunk (of 8) this lane fetches
   uint32_t voff0;     // byte offset of this lane's chunk for load 0
   uint32_t vrow[GATHER ? NI : 1];   // GATHER: byte offset of this lane's chunk per load
@@ -863,31 +892,41 @@ struct DepthMajor {
     up_step = (uint32_t)out_cols * (uint32_t)ld_ * 2u;
   }
 
-  // Fetch depth slice [kt*BK, kt*BK+BK) into the LDS tile at `dst` (wave-uniform).
-  // What all loads of depth slice kt share.
+  // Skip the first `slices` depth slices.
+  __device__ __forceinline__ void skip(int slices) {
+    base += (int64_t)slices * (BK * 2);
+    depth -= slices * BK;
+    if constexpr (GATHER) total_bytes = total_bytes > (uint32_t)slices * (BK * 2) ? total_bytes - (uint32_t)slices * (BK * 2) : 0u;
+  }
+  // What all loads of a depth slice share.
   struct Slice {
     rsrc_words rsrc;
     uint32_t v0;   // this lane's offset for load 0, or out of range in the depth tail
   };
-  __device__ __forceinline__ Slice slice(int kt) const {
-    const int left = uniform(depth - kt * BK);
+  // The next slice (past the depth: empty).
+  __device__ __forceinline__ Slice slice() {
+    const int left = depth = uniform(depth);
+    base = uniform_ptr(base);
     Slice sl;
     if constexpr (GATHER) {
       // the descriptor spans the tensor from this slice's first byte on; v0 is 0 for a chunk
       // inside the depth and out of range for one past it
-      const uint32_t skip = (uint32_t)kt * (BK * 2);
-      sl.rsrc = make_rsrc_words(base + skip, left > 0 && total_bytes > skip ? total_bytes - skip : 0u);
+      sl.rsrc = make_rsrc_words(base, left > 0 ? total_bytes : 0u);
       sl.v0 = (left >= BK || my_chunk * 8 < left) ? 0u : kOutOfRangeIndexed;
     } else {
       const int elems = left > 0 ? span + left : 0;
-      sl.rsrc = make_rsrc_words(base + (int64_t)kt * (BK * 2), elems > 0 ? (uint32_t)elems * 2u : 0u);
+      sl.rsrc = make_rsrc_words(base, elems > 0 ? (uint32_t)elems * 2u : 0u);
       sl.v0 = (left >= BK || my_chunk * 8 < left) ? voff0 : kOutOfRange;
     }
+    skip(1);
     return sl;
   }
-  // Load I of the NI that make up one slice, into the LDS tile at `dst` (wave-uniform).
+  // Load I of the NI that make up one slice goes kOffset<I> bytes behind wave_at of this wave in the LDS tile.
+  __device__ static constexpr __forceinline__ int wave_at(int wave) { return wave * 64 * 16; }
   template <int I>
-  __device__ __forceinline__ void load(const Slice& sl, const char* dst, int wave) const {
+  static constexpr int kOffset = I * NT * 16;
+  template <int I, bool RIGHT_BEHIND>
+  __device__ __forceinline__ void load(const Slice& sl) const {
     const uint32_t step = (uint32_t)(ROWS_PER_INSTR * ld) * 2u;
     uint32_t v;
     if constexpr (GATHER) {
@@ -898,7 +937,7 @@ struct DepthMajor {
     } else {
       v = sl.v0 + I * step;
     }
-    load_to_lds_16(sl.rsrc, v, uniform(lds_address(dst) + (I * NT + wave * 64) * 16));
+    load_to_lds_16<RIGHT_BEHIND>(sl.rsrc, v);
   }
 
   // A depth that is even but no multiple of 8: the 16-byte chunk that holds a row's last depth
@@ -920,19 +959,21 @@ struct DepthMajor {
 // F8 (one-byte elements, seen two to one as W two-byte elements per depth row): 32-byte segment
 // s of depth row k sits at segment slot s ^ (k & 7), so the 8 depth rows one byte-wise
 // transposing read touches land in 8 distinct groups of 8 banks.
+constexpr int width_major_bytes(int W, int BK, bool f8) { return W * BK * 2 + (f8 ? 0 : BK / 16 * 64); }
 template <int W, int BK, int NT, bool F8 = false>
 struct WidthMajor {
   static constexpr int CPRW = W / 8;                  // chunks per depth row
-  static constexpr int SEGS = W * 2 / 64;             // 64-byte segments per depth row
   static constexpr int ROWS_PER_INSTR = NT / CPRW;
+  static constexpr int ROWS_PER_WAVE = 64 / CPRW;     // ... of them by one wave
   static constexpr int NI = BK * CPRW / NT;
-  static constexpr int BYTES = W * BK * 2;
+  static constexpr int BYTES = width_major_bytes(W, BK, F8);
   static constexpr int PITCH = W * 2;
   static_assert(NT % CPRW == 0 && (BK * CPRW) % NT == 0, "tile does not split over the block");
-  static_assert(SEGS >= 4, "needs at least 128 columns");
+  static_assert(CPRW >= 16 && 8 % ROWS_PER_WAVE == 0, "at least 4 segments of 64 bytes; a wave's rows are all shifted or none");
 
-  __device__ static __forceinline__ int seg_swizzle(int krow) {
-    return (krow & 3) | (SEGS >= 8 ? ((krow >> 1) & 4) : 0);
+  // where depth row k starts in LDS
+  __device__ static constexpr __forceinline__ int row_at(int k) {
+    return F8 ? k * PITCH : k * PITCH + 32 * ((k >> 3) & 1) + 64 * (k >> 4);
   }
   // which 16-byte chunk of depth row krow the lane whose LDS slot is chunk p fetches
   __device__ static __forceinline__ int chunk_for_slot(int p, int krow) {
@@ -940,13 +981,13 @@ struct WidthMajor {
       static_assert(!F8 || CPRW == 16, "8 segments of 32 bytes per depth row");
       return (((p >> 1) ^ (krow & 7)) << 1) | (p & 1);
     } else {
-      return (((p >> 2) ^ seg_swizzle(krow)) << 2) | (p & 3);
+      return (((p >> 2) ^ (krow & 3)) << 2) | (p & 3);
     }
   }
 
-  const char* base;      // depth row 0 of the group, column 0
+  const char* base;      // depth row of the next slice, column 0
   int ld;                // elements between depth rows
-  int depth;             // depth rows of the group
+  int depth;             // depth rows of the group ahead of the cursor (below 0: past the end)
   uint32_t voff[NI];     // byte offset of this lane's chunk per load (kOutOfRange past the width)
 
   __device__ __forceinline__ void setup(const char* group_base, int ld_, int depth_, int col0,
@@ -987,25 +1028,40 @@ struct WidthMajor {
     }
   }
 
+  __device__ __forceinline__ void skip(int slices) {
+    base += (int64_t)slices * BK * ld * 2;
+    depth -= slices * BK;
+  }
   struct Slice {
     rsrc_words rsrc;
   };
-  __device__ __forceinline__ Slice slice(int kt) const {
-    int left = uniform(depth - kt * BK);
-    left = left < 0 ? 0 : (left > BK ? BK : left);
+  __device__ __forceinline__ Slice slice() {
+    const int left = uniform(depth), row = uniform(ld) * 2;
+    base = uniform_ptr(base);
     Slice sl;
-    sl.rsrc = make_rsrc_words(base + (int64_t)kt * BK * ld * 2, (uint32_t)(left * ld) * 2u);
+    int rows;   // 0 .. BK (in assembly: the compiler would work it out in vector registers)
+    asm("s_min_i32 %0, %1, %2\n\ts_max_i32 %0, %0, 0" : "=&s"(rows) : "s"(left), "n"(BK) : "scc");
+    sl.rsrc = make_rsrc_words(base, (uint32_t)(rows * row));
+    base += BK * row;
+    depth = left - BK;
     return sl;
   }
+  // (the rows of an instruction are a multiple of 8 apart from those of the next one)
+  static_assert(ROWS_PER_INSTR % 8 == 0 && (F8 || ROWS_PER_INSTR % 16 == 0 || ROWS_PER_INSTR * 2 == 16), "");
+  __device__ static constexpr __forceinline__ int wave_at(int wave) { return row_at(wave * ROWS_PER_WAVE); }
   template <int I>
-  __device__ __forceinline__ void load(const Slice& sl, const char* dst, int wave) const {
-    load_to_lds_16(sl.rsrc, voff[I], uniform(lds_address(dst) + (I * NT + wave * 64) * 16));
+  static constexpr int kOffset = row_at(I * ROWS_PER_INSTR);
+  template <int I, bool RIGHT_BEHIND>
+  __device__ __forceinline__ void load(const Slice& sl) const {
+    load_to_lds_16<RIGHT_BEHIND>(sl.rsrc, voff[I]);
   }
 };
 
 // ---------------------------------------------------------------- fragment readers
-// A fragment is the operand of one 32x32x16 MFMA: lane l holds 8 depth values
-// 8*(l/32) .. +7 of row (or column) l % 32.
+// A fragment is the operand of one 16x16x32 MFMA: lane l holds 8 depth values
+// 8*(l/16) .. +7 of row (or column) l % 16.  A wave's rows and columns come in blocks of 32, so the two
+// fragments of a block and of 32 depth values are numbered by "step": 2 s + h is half h (rows 16 h .. +15) of the
+// block at 32-deep step s.
 
 // STRIDE: distance between the blocks a wave owns, in 32-wide blocks (the waves along a
 // dimension take blocks alternately when STRIDE is their number, contiguously when it is 1).
@@ -1016,43 +1072,49 @@ template <int BK, int STRIDE, bool F8 = false>
 struct DepthMajorFrag {
   static constexpr int CPR = BK / 8;
   static constexpr int RP = (BK * 2 >= 256) ? 1 : 256 / (BK * 2);
-  static_assert((32 / RP) % CPR == 0, "blocks must share the swizzle of block 0");
-  uint32_t off[BK / 16];   // lane offset per 16-deep step, block 0
+  static_assert((16 / RP) % CPR == 0, "blocks and their halves must share the swizzle of block 0");
+  static constexpr int OFFSETS = F8 ? BK / 16 : BK / 32;
+  uint32_t off[OFFSETS];   // lane offset per step (two-byte elements: per pair of them), block 0
 
   __device__ __forceinline__ void setup(int first_row) {
     const int lane = threadIdx.x & 63;
-    const int row = first_row + (lane & 31);
+    const int row = first_row + (F8 ? lane & 31 : lane & 15);
     const int sw = (row / RP) % CPR;
 #pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int chunk = F8 ? 4 * (ks / 2) + 2 * (lane >> 5) + ks % 2 : ks * 2 + (lane >> 5);
-      off[ks] = (uint32_t)(row * (BK * 2) + ((chunk ^ sw) << 4));
+    for (int n = 0; n < OFFSETS; ++n) {
+      const int chunk = F8 ? 4 * (n / 2) + 2 * (lane >> 5) + n % 2 : 4 * n + (lane >> 4);
+      off[n] = (uint32_t)(row * (BK * 2) + ((chunk ^ sw) << 4));
     }
   }
   __device__ __forceinline__ bf16x8 read(const char* tile, int ks, int blk) const {
-    return *reinterpret_cast<const bf16x8*>(tile + off[ks] + blk * (STRIDE * 32) * (BK * 2));
+    const int first = blk * (STRIDE * 32) + (F8 ? 0 : 16 * (ks % 2));
+    return *reinterpret_cast<const bf16x8*>(tile + off[F8 ? ks : ks / 2] + first * (BK * 2));
   }
 };
 
 template <int W, int BK, int NBLK, int STRIDE>
 struct WidthMajorFrag {
   static constexpr int PITCH = W * 2;
-  static constexpr int SEGS = W * 2 / 64;
-  uint32_t off[NBLK];   // lane offset per 32-wide block, depth step 0
+  using Tile = WidthMajor<W, BK, 256>;
+  // blocks whose segments differ in what the swizzle changes; the others are whole groups of 4 segments behind them
+  static constexpr int OFFSETS = 4 / STRIDE < NBLK ? 4 / STRIDE : NBLK;
+  static_assert(4 % STRIDE == 0, "");
+  uint32_t off[OFFSETS];   // lane offset per 32-wide block, its first half, 32-deep step 0
 
+  // (16 lanes hand in the addresses of a block of 4 depth rows x 16 columns, lane i: depth row i / 4, columns
+  // 4 (i % 4) .. +3, and lane j of them receives column j)
   __device__ __forceinline__ void setup(int first_col) {
     const int lane = threadIdx.x & 63;
     const int l16 = lane & 15;
-    const int krow = 8 * (lane >> 5) + (l16 >> 2);
-    const int g = (krow & 3) | (SEGS >= 8 ? ((krow >> 1) & 4) : 0);
+    const int krow = 8 * (lane >> 4) + (l16 >> 2);   // (+ 4, + multiples of 32: neither changes swizzle or shift)
 #pragma unroll
-    for (int j = 0; j < NBLK; ++j) {
+    for (int j = 0; j < OFFSETS; ++j) {
       const int seg = (first_col >> 5) + j * STRIDE;
-      off[j] = (uint32_t)(krow * PITCH + ((seg ^ g) << 6) + 32 * ((lane >> 4) & 1) + 8 * (l16 & 3));
+      off[j] = (uint32_t)(Tile::row_at(krow) + ((seg ^ (krow & 3)) << 6) + 8 * (l16 & 3));
     }
   }
   __device__ __forceinline__ bf16x8 read(const char* tile, int ks, int blk) const {
-    const char* p = tile + off[blk] + ks * 16 * PITCH;
+    const char* p = tile + off[blk % OFFSETS] + (blk / OFFSETS) * 256 + 32 * (ks % 2) + (ks / 2) * Tile::row_at(32);
     const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
         (__attribute__((address_space(3))) bf16x4*)GG_LDS_PTR(p));
     const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
@@ -1104,6 +1166,16 @@ __device__ __forceinline__ void static_for(F&& f) {
   }(std::make_integer_sequence<int, N>{});
 }
 
+// Where the LOADS global loads that begin in a depth slice of S matrix instructions go: spread evenly from FROM to TO, beyond S
+// among the instructions of the slice after.
+template <int LOADS, int FROM, int WAIT, int TO, int S>
+struct LoadSlots {
+  // loads sent ahead of instruction m
+  static constexpr int before(int m) { return m <= FROM ? 0 : (m >= TO ? LOADS : LOADS * (m - FROM) / (TO - FROM)); }
+  // one load goes behind instruction m, and there is an instruction ahead of that one with no wait or branch in between
+  static constexpr bool alone(int m) { return m > FROM && m != WAIT && m != S && before(m + 1) == before(m) + 1; }
+};
+
 constexpr int kTileInfoDwords = 24;   // a tile's description on its way through LDS (pack_tile)
 
 template <int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, int WAVES_N>
@@ -1113,20 +1185,20 @@ struct GmmConfig {
   static constexpr int MB = WTM / 32, NB = WTN / 32;
   static constexpr bool A_DEPTH_MAJOR = LAYOUT != kTN;
   static constexpr bool B_DEPTH_MAJOR = LAYOUT == kNT;
-  static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2;
+  // (fp8 tiles of the same bytes without the shifts: a little less than this)
+  static constexpr int A_BYTES = A_DEPTH_MAJOR ? BM * BK * 2 : width_major_bytes(BM, BK, false);
+  static constexpr int B_BYTES = B_DEPTH_MAJOR ? BN * BK * 2 : width_major_bytes(BN, BK, false);
   static constexpr int STAGE_BYTES = A_BYTES + B_BYTES;
   // after the tile buffers: the schedule, then one strip per wave for the epilogue
   static constexpr int SCHED_OFFSET = STAGES * STAGE_BYTES;
   static constexpr int EPILOGUE_OFFSET = (SCHED_OFFSET + (int)sizeof(Sched) + 15) / 16 * 16;
   static constexpr int EPILOGUE_PITCH = 64 * 2 + 16;            // 64 bf16 columns + padding
   static constexpr int EPILOGUE_WAVE_BYTES = 32 * EPILOGUE_PITCH;
-  static constexpr bool STAGED_EPILOGUE =
-      NB % 2 == 0 && EPILOGUE_OFFSET + WAVES_M * WAVES_N * EPILOGUE_WAVE_BYTES <= 160 * 1024;
+  static_assert(NB % 2 == 0, "the epilogue's strips are 64 columns wide");
   // last: per wave, the descriptions of the tiles between the fetch and the compute cursor
   static constexpr int TILE_RING_SLOTS = 4;
   static constexpr int TILE_RING_OFFSET =
-      ((STAGED_EPILOGUE ? EPILOGUE_OFFSET + WAVES_M * WAVES_N * EPILOGUE_WAVE_BYTES
-                        : SCHED_OFFSET + (int)sizeof(Sched)) + 15) / 16 * 16;
+      (EPILOGUE_OFFSET + WAVES_M * WAVES_N * EPILOGUE_WAVE_BYTES + 15) / 16 * 16;
   static constexpr int LDS_BYTES = TILE_RING_OFFSET + WAVES_M * WAVES_N * TILE_RING_SLOTS * kTileInfoDwords * 4;
   static_assert(LDS_BYTES <= 160 * 1024, "a compute unit has 160 KiB of LDS");
   static constexpr int WORKGROUPS_PER_CU = 2 * LDS_BYTES <= 160 * 1024 ? 2 : 1;
@@ -1407,22 +1479,26 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   using BFrag = std::conditional_t<Cfg::B_DEPTH_MAJOR, DepthMajorFrag<BK, 1, F8>,
                                    std::conditional_t<F8, WidthMajorFrag8<BN, NB, 1>, WidthMajorFrag<BN, BK, NB, 1>>>;
   constexpr int LOADS_PER_STAGE = ALoad::NI + BLoad::NI;   // per lane, per depth slice
-  // A slice's loads go out in three parts, in steps 1, 2 and 3, or in four, in steps 1 to 3 and step 0
-  // of the slice after: loads T1, T2 and T3 begin parts 2, 3 and 4.  With three parts all loads of the
-  // next tile's first two slices precede the stores of a tile, and the first wait of the next tile lets
-  // those stores pass (counters go down in the order of issue); with a part of the loads behind the
-  // stores it waits for the memory to take the whole tile.  That pays where tiles are shallow and
-  // where the launch is bound by memory: weight gradients, 256 groups x 256 rows, 2048 x 7168: 2555 ->
-  // 2502 us, 64 x 768, 2048 x 1408: 290 -> 280; two rows each of 256 groups, 7168 -> 2048 (short
-  // tiles): 0 to 3 % by the box.  Full tiles of deep products run 0.3 % (bf16) to 1.3 % (fp8) faster with
-  // the steadier four parts (8 x 4096 rows, 4096 -> 14336).
-  constexpr bool THREE_PARTS = LAYOUT == kTN || BM < 256;
-  constexpr int T1 = THREE_PARTS ? LOADS_PER_STAGE / 3 : LOADS_PER_STAGE / 4;
-  constexpr int T2 = THREE_PARTS ? LOADS_PER_STAGE * 2 / 3 : LOADS_PER_STAGE / 2;
-  constexpr int T3 = THREE_PARTS ? LOADS_PER_STAGE : LOADS_PER_STAGE * 3 / 4;
-  static_assert(KS == 4 && STAGES == 2, "the step schedule below is written for BK = 64 and two buffers");
+  static_assert(KS == 4 && STAGES == 2, "the schedule of a slice (tile_body) is written for BK = 64 and two buffers");
   static_assert(LOADS_PER_STAGE >= 4 && LOADS_PER_STAGE < 32, "");
-  constexpr int UNITS = MB + NB;    // fragments of one 16-deep step
+  // The positions of a slice's schedule (see tile_body) in 32nds of its matrix instructions.  A buffer is handed over as
+  // early as LDS can deliver its fragments: what a fetch has time for counts for more than an even load on LDS
+  // (released at 8, 10, 13 and 14, ready at 24, 22, 19 and 18, us: 8 x 4096 rows, 4096 -> 14336, NN 2913 / 2943 / 2986 / 2978;
+  // 256 x 256, 7168 -> 2048, NT 2079 / 2030 / 2100 / 2160).  Tiles of few rows, whose launches are bound by latency: earlier still
+  // (6 and 26 against 8 and 24: 16 x 256 rows, 3072 -> 768: 32.8 / 34.1, NT 33.8 / 35.7; 32 x 128, 2048 -> 768: 28.5 / 28.4;
+  // against 10 and 22: 36.2, 37.7, 31.9).
+  constexpr bool EARLY = LAYOUT != kTN && BM < 256 && !F8;
+  constexpr int AT_READ_END = EARLY ? 6 : 8, AT_RELEASE = AT_READ_END, AT_READY = EARLY ? 26 : 24;
+  // Loads that reach into the next slice are steadier: ended at 32, 36 and 40, us: 8 x 4096 rows, 4096 -> 14336, NN 2743 / 2749 /
+  // 2779, input gradient 2685 / 2665 / 2675, 256 x 256 NT 1917 / 1897 / 1947, NN 1987 / 1921 / 1930.  Not where
+  // tiles are shallow or their launch is bound by memory (weight gradients, tiles of few rows): with loads behind the
+  // stores of a tile the first wait of the next one waits for the memory to take the whole tile, without it lets the
+  // stores pass (counters go down in the order of issue): 256 groups x 256 rows, 2048 x 7168: 2555 -> 2502 us.  Nor for fp8: 1431 /
+  // 1420 us with and without.
+  constexpr bool LATE_LOADS = LAYOUT != kTN && BM == 256 && !F8;
+  constexpr int AT_LOAD_END = LATE_LOADS ? 36 : 32;
+  constexpr int FIRST_LOADS = LoadSlots<LOADS_PER_STAGE, AT_RELEASE, AT_READY, AT_LOAD_END, 32>::before(32);   // ... by a slice's end
+  constexpr int UNITS = MB + NB;    // fragments of one set
 
   Sched* sched = reinterpret_cast<Sched*>(smem + Cfg::SCHED_OFFSET);
   build_schedule<LAYOUT, BM, BNS>(sched, p, hs, w);
@@ -1548,68 +1624,90 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       // (rows of b are as long as they are apart where row indices are used: a scalar register less)
       bload.setup(p.b + fti.g.b_off * ES, (INDEXED ? fti.g.n : p.ldb) * ES / 2, depth, fti.n0 * ES / 2, fti.g.n * ES / 2);
     }
+    if (fti.k0 != 0) {
+      aload.skip(fti.k0);
+      bload.skip(fti.k0);
+    }
   };
   // Slices past the depth (or past the last tile) are fetched with an empty descriptor:
   // zeros, no traffic, and the number of loads in flight is the same at every step.
   typename ALoad::Slice a_slice;
   typename BLoad::Slice b_slice;
-  auto fetch_begin = [&]() {   // descriptors of the cursor's slice
-    a_slice = aload.slice(fti.k0 + fetch_kt);
-    b_slice = bload.slice(fti.k0 + fetch_kt);
+  // Load J of the cursor's slice (A's loads first, then B's) into buffer `buf`: fetch_aim, then fetch_load.  A's descriptor
+  // comes with fetch_begin (then a wait, a barrier, a matrix instruction, fetch_aim and another instruction precede the first
+  // load), B's ahead of A's last load (then that load and two of each precede B's first).
+  auto fetch_begin = [&]() {
+    a_slice = aload.slice();
+    settle(a_slice.rsrc);
   };
-  // Load J of the cursor's slice (A's loads first, then B's) into buffer `buf`.
-  auto fetch_load = [&](auto j_tag, int buf) {
+  const uint32_t a_first = uniform(lds_address(smem) + ALoad::wave_at(wave)), b_first = uniform(lds_address(smem) + BLoad::wave_at(wave));
+  auto fetch_aim = [&](auto j_tag, int buf) {
     constexpr int J = decltype(j_tag)::value;
-    const char* st = smem + uniform(buf) * Cfg::STAGE_BYTES;
-    if constexpr (J < ALoad::NI) {
-      aload.template load<J>(a_slice, st, wave);
-    } else {
-      bload.template load<J - ALoad::NI>(b_slice, st + Cfg::A_BYTES, wave);
+    const uint32_t at = uniform(buf) * Cfg::STAGE_BYTES;
+    if constexpr (J == ALoad::NI - 1) {
+      b_slice = bload.slice();
+      settle(b_slice.rsrc);
     }
+    if constexpr (J < ALoad::NI) {
+      aim_lds<ALoad::template kOffset<J>>(uniform(a_first + at));
+    } else {
+      aim_lds<Cfg::A_BYTES + BLoad::template kOffset<J - ALoad::NI>>(uniform(b_first + at));
+    }
+  };
+  auto fetch_load = [&](auto j_tag, auto right_behind) {
+    constexpr int J = decltype(j_tag)::value;
+    if constexpr (J < ALoad::NI) {
+      aload.template load<J, decltype(right_behind)::value>(a_slice);
+    } else {
+      bload.template load<J - ALoad::NI, decltype(right_behind)::value>(b_slice);
+    }
+  };
+  auto fetch_whole = [&](auto j_tag, int buf) {
+    fetch_aim(j_tag, buf);
+    fetch_load(j_tag, std::true_type{});
   };
   auto fetch_advance = [&]() {
     // (said to be the same in every lane once more: where the compiler loses track of that, the
     // slice descriptors below are computed lane by lane and the branch becomes a masked one)
     fetch_kt = uniform(fetch_kt + 1);
-    if (fetch_kt == uniform(fti.nk) && uniform((int)fti.valid) != 0) {
+    // (once a tile: kept out of the loop's instructions, which a jump over it would fetch anew every slice)
+    if (__builtin_expect(fetch_kt == uniform(fti.nk) && uniform((int)fti.valid) != 0, 0)) {
       fetch_t = next_index(fetch_t);
       fetch_kt = 0;
       fetch_setup();
     }
   };
 
-  // Fragments: one register set per 16-deep step of a slice.  A "unit" is one fragment (one
-  // ds_read_b128, or two transposing 64-bit reads): the first ML of A's, then B's NB.
+  // Fragments: sets 0 and 1 are the halves of the first 32-deep (fp8: 64-deep) step of a slice, 2 and 3 those of the
+  // second.  A "unit" is one fragment (one ds_read_b128, or two transposing 64-bit reads).  Unit U of the pair of
+  // sets that begins with set SET, in the order in which the matrix instructions want them: B's first block, the
+  // first ML of A's, the rest of B's NB, both halves of each.
   bf16x8 fa[KS][MB], fb[KS][NB];
-  auto read_unit = [&](auto u_tag, auto set_tag, auto ml_tag, int buf) {   // set = 16-deep step it belongs to
-    constexpr int U = decltype(u_tag)::value, SET = decltype(set_tag)::value, ML = decltype(ml_tag)::value;
+  auto read_unit = [&](auto u_tag, auto set_tag, auto ml_tag, int buf) {
+    constexpr int U = decltype(u_tag)::value / 2, SET = decltype(set_tag)::value + decltype(u_tag)::value % 2;
+    constexpr int ML = decltype(ml_tag)::value;
     const char* sa = smem + buf * Cfg::STAGE_BYTES;
-    if constexpr (U < ML) {
-      fa[SET][U] = afrag.read(sa, SET, U);
+    if constexpr (U >= 1 && U <= ML) {
+      fa[SET][U - 1] = afrag.read(sa, SET, U - 1);
     } else {
-      fb[SET][U - ML] = bfrag.read(sa + Cfg::A_BYTES, SET, U - ML);
+      constexpr int J = U == 0 ? 0 : U - ML;
+      fb[SET][J] = bfrag.read(sa + Cfg::A_BYTES, SET, J);
     }
   };
 
   using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
   using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
   using IMB = std::integral_constant<int, MB>;
-  using IT1 = std::integral_constant<int, T1>;
-  using IT2 = std::integral_constant<int, T2>;
-  using ISecond = std::integral_constant<int, T2 - T1>;   // loads of the second part
-  using IThird = std::integral_constant<int, T3 - T2>;
-  using IT3 = std::integral_constant<int, T3>;
-  using ILast = std::integral_constant<int, LOADS_PER_STAGE - T3>;
 
-  // Both buffers are requested up front, except what step 0 issues.
+  // Both buffers are requested up front, except what the first slice's instructions send.
   fetch_setup();
   fetch_begin();
-  static_for<LOADS_PER_STAGE>([&](auto j) { fetch_load(j, 0); });
+  asm volatile("s_nop 4");
+  static_for<LOADS_PER_STAGE>([&](auto j) { fetch_whole(j, 0); });
   fetch_advance();
   fetch_begin();
-  static_for<T3>([&](auto j) { fetch_load(j, 1); });
+  asm volatile("s_nop 4");
+  static_for<FIRST_LOADS>([&](auto j) { fetch_whole(j, 1); });
 
   int tile_t = first_t;
   int tile_n = 0;   // tiles this workgroup has finished
@@ -1640,15 +1738,20 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       block_barrier();
     }
   };
-  wait_vmcnt<T3>();   // the first slice is in
+  wait_vmcnt<FIRST_LOADS>();   // the first slice is in
   block_barrier();
   if (RAGGED_DEPTH && tail_slice == 0) clear_tail(0);
   static_for<2 * UNITS>([&](auto u) {
-    constexpr int uu = decltype(u)::value;
-    read_unit(std::integral_constant<int, uu % UNITS>{}, std::integral_constant<int, uu / UNITS>{}, IMB{}, 0);
+    read_unit(u, I0{}, IMB{}, 0);
   });
 
   int x = 0;   // buffer of the slice being multiplied
+
+  // What a lane holds of a 32 x 32 block of the result: four groups q of 4 consecutive columns of a row.
+  auto group_row_of = [&](int at_lane, int q) { return F8 ? at_lane & 31 : 16 * (q / 2) + (at_lane & 15); };
+  auto group_col_of = [&](int at_lane, int q) { return F8 ? 8 * q + 4 * (at_lane >> 5) : 16 * (q % 2) + 4 * (at_lane >> 4); };
+  auto group_row = [&](int q) { return group_row_of(lane, q); };
+  auto group_col = [&](int q) { return group_col_of(lane, q); };
 
   // Partial tile of depth piece `piece` of the tile `ti` names: a lane's 16-byte group (i, j, q) sits
   // at ((i * NB + j) * 4 + q) * NT + thread, so one instruction of a wave moves 1 KiB of consecutive
@@ -1734,93 +1837,138 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // Row blocks this wave has stored of the tile before (0: none, or all of it has arrived), and the
   // store instructions of one (at least; more of them only make the wait that counts them stricter).
   int stored = 0;
-  constexpr int STORES = ACC_F32 ? 8 : (GATE_UP ? Cfg::WTN / 32 : (Cfg::STAGED_EPILOGUE ? NB / 2 * 4 : NB * 4));
-  static_assert(T2 + STORES * MB < 64, "vmcnt is a 6-bit field");
+  constexpr int STORES = ACC_F32 ? 8 : (GATE_UP ? Cfg::WTN / 32 : NB / 2 * 4);
+  static_assert(LOADS_PER_STAGE + STORES * MB < 64, "vmcnt is a 6-bit field");
 
   // One tile, for a wave that has ML row blocks with rows in them (the tile's row blocks go to
   // the wave rows alternately).  One copy of this body exists per value of ML; a tile picks
   // its copy once, so no accumulator ever lives across a choice.
   //
-  // Per slice (buffer X, the other buffer Y holds the next slice):
-  //   step 0  reads the fragments of steps 2 and 3 from X; after it nobody needs X any more
-  //   step 1  barrier: X goes to the fetch cursor, which starts the slice two ahead into it
-  //   step 3  barrier: Y is complete for every wave; reads the fragments of the next slice's
-  //           steps 0 and 1 from Y (all MB of A's: the next slice may be the next tile's)
-  // Steps 1 to 3 (and 0) each issue a part of a slice's loads, so the memory pipe sees a steady
-  // trickle, and X is released two steps before Y is needed, so loads stay in flight across the
-  // hand-over.
+  // A slice (buffer X, the other buffer Y holds the next slice) is S matrix instructions; the first half multiplies
+  // fragment sets 0 and 1, which are there when it begins, the second half sets 2 and 3:
+  //   to READ_END     the fragments of sets 2 and 3 are read from X
+  //   at RELEASE      all waves have them: X goes to the fetch cursor, which starts the slice two ahead into it, all
+  //                   of its loads by the end of this slice, i.e. ahead of the stores of a tile that ends with it
+  //   from READY      Y is complete for every wave: the fragments of the next slice's sets 0 and 1 are read from it
+  //                   (all MB of A's: the next slice may be the next tile's)
+  // Reads and loads are spread evenly over their spans.  LDS delivers the fragments of full tiles in half of a slice's
+  // matrix time and takes the loads in a quarter of it.
   auto tile_body = [&](auto ml_tag) {
     constexpr int ML = decltype(ml_tag)::value;
-    constexpr int SLOTS = ML * NB;    // MFMAs per 16-deep step
-    f32x16 acc[ML][NB];
+    // MFMAs: blocks of 32 x 32 outputs for fp8, of 16 x 16 for two-byte elements
+    constexpr int EDGE = F8 ? 1 : 2, MFMA_M = ML * EDGE, MFMA_N = NB * EDGE;
+    std::conditional_t<F8, f32x16, f32x4> acc[MFMA_M][MFMA_N];
 #pragma unroll
-    for (int i = 0; i < ML; ++i)
+    for (int i = 0; i < MFMA_M; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
+      for (int j = 0; j < MFMA_N; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int r = 0; r < (F8 ? 16 : 4); ++r) acc[i][j][r] = 0.0f;
+    // Group q (see group_row) of the 32 x 32 block (i, j), moved out of the accumulation registers here and no earlier:
+    // all of them at once would not fit beside the next tile's fragments.  (How that is said decides what the compiler
+    // makes of it: read in assembly, the plain epilogues of full tiles get by without moves and spills; tied
+    // to the accumulation registers, those that combine two products do.  Small tiles have room.)
+    auto take = [&](int i, int j, int q, float* v) {
+      auto& from = F8 ? acc[i][j] : acc[2 * i + q / 2][2 * j + q % 2];
+      constexpr bool TIED = !F8 && (GATE_UP || ((INDEXED || RAGGED_DEPTH) && BM > 128));
+      if constexpr (TIED) asm volatile("" : "+a"(from));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float x = from[F8 ? 4 * q + r : r];
+        if constexpr (F8 || (MB * NB > 4 && !TIED)) {
+          asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(x));
+        } else {
+          asm volatile("" : "+v"(x));
+          v[r] = x;
+        }
+      }
+    };
 
-    // One 16-deep step: SLOTS slots of one MFMA each, with this step's LDS reads and global
-    // loads placed behind the first MFMAs, in this order, so they run under the matrix pipe.
-    //   RML     A fragments per set that are read (ML, or MB for the next slice's)
-    //   SETS    sets read: 0 or 2, starting at READ_SET
-    //   LOADS   global loads FIRST_LOAD .. of the fetch cursor's slice, into buffer `fill`
-    auto step = [&](auto ks_tag, auto sets_tag, auto rml_tag, auto read_set_tag, auto first_load_tag,
-                    auto loads_tag, int src, int fill) {
-      constexpr int ks = decltype(ks_tag)::value, SETS = decltype(sets_tag)::value;
-      constexpr int RML = decltype(rml_tag)::value, RUNITS = RML + NB, READS = SETS * RUNITS;
-      constexpr int READ_SET = decltype(read_set_tag)::value;
-      constexpr int FIRST_LOAD = decltype(first_load_tag)::value, LOADS = decltype(loads_tag)::value;
-      // fp8: steps 2 s and 2 s + 1 share the 64-deep step s, half of the blocks each, and an
-      // instruction takes the halves 2 s and 2 s + 1 of both fragments
-      constexpr int STEP_SLOTS = F8 ? SLOTS / 2 : SLOTS;
-      static_for<STEP_SLOTS>([&](auto m_tag) {
-        constexpr int mm = decltype(m_tag)::value, m = F8 ? mm + (ks % 2) * STEP_SLOTS : mm;
-        // serpentine over the blocks: consecutive MFMAs share one operand, also across rows
-        constexpr int j = m / ML, i = (j % 2 == 0) ? m % ML : ML - 1 - m % ML;
+    constexpr int S = 2 * MFMA_M * MFMA_N;
+    constexpr int READ_END = S * AT_READ_END / 32, RELEASE = S * AT_RELEASE / 32, READY = S * AT_READY / 32, LOAD_END = S * AT_LOAD_END / 32;
+    static_assert(READ_END <= RELEASE && RELEASE <= READY && 2 * READY >= S && READ_END > 0 && READY < S && LOAD_END - S <= READ_END, "");
+    using Loads = LoadSlots<LOADS_PER_STAGE, RELEASE, READY, LOAD_END, S>;
+    static_assert(Loads::before(S) == FIRST_LOADS, "the copies of this body take over from one another");
+    // Matrix instructions FIRST .. LAST - 1, with the LDS reads and global loads placed behind them, in this
+    // order, so they run under the matrix pipe.
+    auto slots = [&](auto first_tag, auto last_tag, int y) {
+      constexpr int FIRST = decltype(first_tag)::value, LAST = decltype(last_tag)::value;
+      static_for<LAST - FIRST>([&](auto m_tag) {
+        constexpr int m = FIRST + decltype(m_tag)::value, n = m % (S / 2), set = m < S / 2 ? 0 : 2;
+        // serpentine over the 32 x 32 blocks and over the 16 x 16 ones in them: consecutive MFMAs share one operand, and the
+        // fragments are wanted no faster than they come (columns of 16 x 16 blocks want all of A's at once)
+        constexpr int quarter = F8 ? 0 : n % 4, block = F8 ? n : n / 4;
+        constexpr int j = block / ML, i = (j % 2 == 0) ? block % ML : ML - 1 - block % ML;
+        constexpr int hi = quarter / 2, hj = quarter == 1 || quarter == 2 ? 1 : 0;   // halves of A's and of B's block
         // operands swapped: the result block is held transposed, so a lane owns four
         // consecutive columns of one output row
-        if constexpr (F8) {
-          acc[i][j] = mfma_32x32x64_f8<DT>(fb[ks & ~1][j], fb[ks | 1][j], fa[ks & ~1][i], fa[ks | 1][i], acc[i][j]);
+        if constexpr (F8) {   // (takes both halves of both fragments)
+          acc[i][j] = mfma_32x32x64_f8<DT>(fb[set][j], fb[set + 1][j], fa[set][i], fa[set + 1][i], acc[i][j]);
         } else {
-          acc[i][j] = mfma_32x32x16<DT>(fb[ks][j], fa[ks][i], acc[i][j]);
+          f32x4& sum = acc[2 * i + hi][2 * j + hj];
+          sum = mfma_16x16x32<DT>(fb[set + hj][j], fa[set + hi][i], sum);
         }
-        constexpr int u0 = READS * mm / STEP_SLOTS, u1 = READS * (mm + 1) / STEP_SLOTS;
-        static_for<u1 - u0>([&](auto d) {
-          constexpr int u = u0 + decltype(d)::value;
-          read_unit(std::integral_constant<int, u % RUNITS>{},
-                    std::integral_constant<int, READ_SET + u / RUNITS>{}, rml_tag, src);
-        });
-        constexpr int l0 = LOADS * mm / STEP_SLOTS, l1 = LOADS * (mm + 1) / STEP_SLOTS;
-        static_for<l1 - l0>([&](auto d) {
-          fetch_load(std::integral_constant<int, FIRST_LOAD + l0 + decltype(d)::value>{}, fill);
-        });
+        if constexpr (m < READ_END) {
+          constexpr int U = 2 * (ML + NB), u0 = U * m / READ_END, u1 = U * (m + 1) / READ_END;
+          static_for<u1 - u0>([&](auto d) { read_unit(std::integral_constant<int, u0 + decltype(d)::value>{}, I2{}, ml_tag, x); });
+        } else if constexpr (m >= READY) {
+          constexpr int U = 2 * (MB + NB), u0 = U * (m - READY) / (S - READY), u1 = U * (m + 1 - READY) / (S - READY);
+          static_for<u1 - u0>([&](auto d) { read_unit(std::integral_constant<int, u0 + decltype(d)::value>{}, I0{}, IMB{}, y); });
+        }
+        // (a load on its own is aimed behind the instruction before: all of it behind one of 16 cycles would hold up the next)
+        constexpr int at = m < READ_END ? m + S : m;   // (loads of the slice before reach up to there)
+        const int to = m < READ_END ? y : x;
+        constexpr int l0 = Loads::before(at), l1 = Loads::before(at + 1);
+        if constexpr (Loads::alone(at)) {
+          __builtin_amdgcn_sched_barrier(0);   // (the instruction stays between the two)
+          fetch_load(std::integral_constant<int, l0>{}, std::false_type{});
+        } else {
+          static_for<l1 - l0>([&](auto d) { fetch_whole(std::integral_constant<int, l0 + decltype(d)::value>{}, to); });
+        }
+        if constexpr (m + 1 != READ_END && Loads::alone(at + 1)) fetch_aim(std::integral_constant<int, l1>{}, to);
         __builtin_amdgcn_sched_barrier(0);
       });
     };
+    using IReadEnd = std::integral_constant<int, READ_END>;
+    using IRelease = std::integral_constant<int, RELEASE>;
+    using IReady = std::integral_constant<int, READY>;
+    using IAll = std::integral_constant<int, S>;
 
     for (int kt = 0; kt < ti.nk; ++kt) {
       const int y = uniform(x ^ 1);   // (the same in every lane: keeps the LDS addresses scalar)
-      step(I0{}, I2{}, ml_tag, I2{}, IT3{}, ILast{}, x, y);
+      if constexpr (LATE_LOADS) {
+        // (the descriptor of the last loads comes from the iteration before, for all the compiler knows in vector
+        // registers; the first of them is behind a matrix instruction, fetch_aim and a wait)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) b_slice.rsrc[w] = uniform(b_slice.rsrc[w]);
+        settle<2>(b_slice.rsrc);
+      }
+      slots(I0{}, IReadEnd{}, y);
       fetch_advance();
+      fetch_begin();
+      slots(IReadEnd{}, IRelease{}, y);
       // every wave has all fragments of this slice in registers
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       block_barrier();
-      fetch_begin();
-      step(I1{}, I0{}, ml_tag, I0{}, I0{}, IT1{}, x, x);
-      step(I2{}, I0{}, ml_tag, I0{}, IT1{}, ISecond{}, x, x);
-      // the next slice has landed for every wave (only the two parts just issued may be pending and,
-      // THREE_PARTS, in a tile's first slice the stores of the tile before)
-      if (THREE_PARTS && kt == 0 && uniform(stored) == MB) {
-        wait_vmcnt<T2 + STORES * MB>();
-      } else if (THREE_PARTS && kt == 0 && uniform(stored) > 0) {
-        wait_vmcnt<T2 + STORES>();
+      slots(IRelease{}, IReady{}, y);
+      // the next slice has landed for every wave (only the loads just issued may be pending and, in the first
+      // slice after a tile that was stored, its stores)
+      constexpr int PENDING = Loads::before(READY);
+      // (in the weight-gradient layout the condition is one of the first slice's, which the compiler then takes out of the
+      // loop: with the other form it moves accumulators in and out of the loop, 332 moves a slice)
+      if (LATE_LOADS || (LAYOUT == kTN && kt > 0) || __builtin_expect(uniform(stored) == 0, 1)) {
+        wait_vmcnt<PENDING>();
       } else {
-        wait_vmcnt<T2>();
+        if (uniform(stored) == MB) {
+          wait_vmcnt<PENDING + STORES * MB>();
+        } else {
+          wait_vmcnt<PENDING + STORES>();
+        }
+        if (LAYOUT != kTN) stored = 0;   // (the next wait is for them too)
       }
       block_barrier();
       if (RAGGED_DEPTH && uniform(kt + 1 == ti.nk ? 0 : kt + 1) == tail_slice) clear_tail(y);
-      step(I3{}, I2{}, IMB{}, I0{}, IT2{}, IThird{}, y, x);
+      slots(IReady{}, IAll{}, y);
       x = uniform(y);
     }
 
@@ -1835,7 +1983,12 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         for (int j = 0; j < NB; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            f32x4 v;
+            if constexpr (F8) {
+              v = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            } else {
+              v = acc[2 * i + q / 2][2 * j + q % 2];
+            }
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), mine, partial_at(i, j, q), 0, kDeviceScope);
           }
       wait_vmcnt<0>();   // every wave's part has arrived before the arrival is counted
@@ -1861,7 +2014,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       return;
     }
 
-    // Epilogue.  A lane owns row (l % 32) of each 32x32 block and columns 8q + 4(l/32) .. +3.
+    // Epilogue.  A lane owns four groups of 4 columns of each 32x32 block (group_row, group_col).
     // The accumulators stay in the accumulation registers; each value is moved out right
     // where it is converted, so the epilogue needs only a few vector registers.
     {
@@ -1871,9 +2024,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       auto at = [&](uint32_t row_off, int col) { return c_at(ti, row_off, col); };
       auto take4 = [&](int i, int j, int q) {
         float v[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[i][j][4 * q + r]));
+        take(i, j, q, v);
         return round4<OUT_DT>(v[0], v[1], v[2], v[3]);
       };
       if constexpr (GATE_UP) {
@@ -1883,10 +2034,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         // whole lines: the 8-byte pieces the lanes hold, 16 bytes of a line per row and instruction,
         // were written at that size past L2 (16 x 1024 rows, 2048 -> 4096: 637 -> 574 us; decode,
         // 8 x 16 rows, 4096 -> 14336: 357 -> 348).
-        static_assert(Cfg::STAGED_EPILOGUE, "the gate | up epilogue uses the waves' LDS strips");
         constexpr int OUTW = Cfg::WTN / 2, CHUNKS = OUTW / 8, ROWS = 64 / CHUNKS, PITCH = Cfg::EPILOGUE_PITCH;
         char* strip = smem + Cfg::EPILOGUE_OFFSET + wave * Cfg::EPILOGUE_WAVE_BYTES;
-        const int in_row = lane & 31, in_half = lane >> 5;
         const int out_row = lane / CHUNKS, out_chunk = lane % CHUNKS;
         const int col = ti.n0 + wn * OUTW + out_chunk * 8;
         u32x4 held[32 / ROWS];   // (one strip behind, as below)
@@ -1916,7 +2065,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           __builtin_amdgcn_sched_barrier(0);
         };
         auto into_strip = [&](int jp, int q, u32x2 v) {
-          *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jp * 32 + 8 * q + 4 * in_half) * 2) = v;
+          *reinterpret_cast<u32x2*>(strip + group_row(q) * PITCH + (jp * 32 + group_col(q)) * 2) = v;
         };
 #pragma unroll
         for (int i = 0; i < ML; ++i) {
@@ -1949,11 +2098,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               float gate[4], up[4];
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(gate[r]) : "a"(acc[i][2 * jp][4 * q + r]));
-                asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(up[r]) : "a"(acc[i][2 * jp + 1][4 * q + r]));
-              }
+              take(i, 2 * jp, q, gate);
+              take(i, 2 * jp + 1, q, up);
               into_strip(jp, q, combine4(gate, up));
             }
           }
@@ -1973,21 +2119,17 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           // One 32 x 32 block at a time goes through the wave's LDS strip, in as the 16-byte pieces
           // the lanes hold, out as one float per lane, 32 lanes to a row: an instruction then adds
           // to two complete 128-byte lines.
-          static_assert(Cfg::STAGED_EPILOGUE, "the accumulating epilogue uses the waves' LDS strips");
           char* strip = smem + Cfg::EPILOGUE_OFFSET + wave * Cfg::EPILOGUE_WAVE_BYTES;
           constexpr int PITCH = Cfg::EPILOGUE_PITCH;   // 32 floats and 16 bytes of padding
-          const int in_row = lane & 31, in_half = lane >> 5;
 #pragma unroll
           for (int i = 0; i < ML; ++i) {
 #pragma unroll
             for (int j = 0; j < NB; ++j) {
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
-                f32x4 v;
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v[r]) : "a"(acc[i][j][4 * q + r]));
-                *reinterpret_cast<f32x4*>(strip + in_row * PITCH + (8 * q + 4 * in_half) * 4) = v;
+                float v[4];
+                take(i, j, q, v);
+                *reinterpret_cast<f32x4*>(strip + group_row(q) * PITCH + group_col(q) * 4) = f32x4{v[0], v[1], v[2], v[3]};
               }
               // (offsets from one per block on: worked out per instruction they do not change from tile to
               // tile, and the compiler keeps them in more registers than there are: reloading those it
@@ -2007,47 +2149,44 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           }
         } else {
           // c += product in fp32.  The 4 consecutive columns a lane holds are 16 bytes of c:
-          // read them, add, write them back; lanes l and l + 32 cover 32 contiguous bytes of a
-          // row, four such instructions one 128-byte line.  All reads of a 32-row block row are
+          // read them, add, write them back; the lanes of an instruction cover 64 (fp8: 32) contiguous bytes of a
+          // row, the instructions of a block 128-byte lines.  All reads of a 32-row block row are
           // issued before the first addition: 16 in flight per lane measured faster than a
           // rolling 8 + 8.
 #pragma unroll
           for (int i = 0; i < ML; ++i) {
-            const int row = (wm + i * WAVES_M) * 32 + (lane & 31);
-            uint32_t off[NB][4];
+            // (offsets are worked out again for the stores: kept, they take more registers than there are)
+            auto offset = [&](int at_lane, int j, int q) {
+              const int row = (wm + i * WAVES_M) * 32 + group_row_of(at_lane, q);
+              const int col = ti.n0 + wn * Cfg::WTN + j * 32 + group_col_of(at_lane, q);
+              return col < ti.g.n ? (uint32_t)(row * ti.g.n + col) * 4u : kOutOfRange;
+            };
             u32x4 old[NB][4];
 #pragma unroll
             for (int j = 0; j < NB; ++j)
 #pragma unroll
-              for (int q = 0; q < 4; ++q) {
-                const int col = ti.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
-                off[j][q] = col < ti.g.n ? (uint32_t)(row * ti.g.n + col) * 4u : kOutOfRange;
-                old[j][q] = __builtin_amdgcn_raw_buffer_load_b128(rc, off[j][q], 0, 0);
-              }
+              for (int q = 0; q < 4; ++q) old[j][q] = __builtin_amdgcn_raw_buffer_load_b128(rc, offset(lane, j, q), 0, 0);
             __builtin_amdgcn_sched_barrier(0);
+            int at_lane = lane;
+            asm volatile("" : "+v"(at_lane));
 #pragma unroll
             for (int j = 0; j < NB; ++j)
 #pragma unroll
               for (int q = 0; q < 4; ++q) {
-                f32x4 sum = __builtin_bit_cast(f32x4, old[j][q]);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                  float v;
-                  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(acc[i][j][4 * q + r]));
-                  sum[r] += v;
-                }
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum), rc, off[j][q], 0, 0);
+                float v[4];
+                take(i, j, q, v);
+                const f32x4 sum = __builtin_bit_cast(f32x4, old[j][q]) + f32x4{v[0], v[1], v[2], v[3]};
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum), rc, offset(at_lane, j, q), 0, 0);
               }
             __builtin_amdgcn_sched_barrier(0);
           }
         }
-      } else if constexpr (Cfg::STAGED_EPILOGUE) {
+      } else {
         // Through a strip of LDS private to the wave: 32 rows x 64 columns go in as the
         // 8-byte pieces the lanes hold and come out as 16 bytes per lane, 8 lanes per row, so
         // that one store instruction writes 8 complete 128-byte lines.
         char* strip = smem + Cfg::EPILOGUE_OFFSET + wave * Cfg::EPILOGUE_WAVE_BYTES;
         constexpr int PITCH = Cfg::EPILOGUE_PITCH;
-        const int in_row = lane & 31, in_half = lane >> 5;
         const int out_row = lane >> 3, out_chunk = lane & 7;
         // an even width that is not a multiple of 8: rows of c then start on 4-byte boundaries
         // only, and the last 16-byte chunk of a row holds 2, 4 or 6 columns
@@ -2101,7 +2240,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
             for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
               for (int q = 0; q < 4; ++q)
-                *reinterpret_cast<u32x2*>(strip + in_row * PITCH + (jj * 32 + 8 * q + 4 * in_half) * 2) =
+                *reinterpret_cast<u32x2*>(strip + group_row(q) * PITCH + (jj * 32 + group_col(q)) * 2) =
                     take4(i, 2 * jp + jj, q);
             if (i + jp > 0) store_held();
             held_col = ti.n0 + wn * Cfg::WTN + jp * 64 + out_chunk * 8;
@@ -2116,20 +2255,6 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
           }
         }
         store_held();
-      } else {
-#pragma unroll
-        for (int i = 0; i < ML; ++i) {
-          const uint32_t row_off = row_offset((wm + i * WAVES_M) * 32 + (lane & 31));
-#pragma unroll
-          for (int j = 0; j < NB; ++j) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const int col = ti.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
-              __builtin_amdgcn_raw_buffer_store_b64(take4(i, j, q), rc, at(row_off, col), 0, kStoreStreaming);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-          }
-        }
       }
       stored = ANY_ROWS && (p.flags & kFlagAnyRows) != 0 ? 0 : ML;   // (not every store is sent there: nothing to count on)
     }
@@ -2194,8 +2319,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
 #pragma unroll
           for (int q = 0; q < 4; ++q) sum[j][q] = (sum[j][q] + v0[j][q]) + v1[j][q];
       }
-      // a lane owns row (l % 32) of each 32x32 block and columns 8q + 4(l/32) .. +3
-      const uint32_t row_off = c_row(ft, (wm + i * WAVES_M) * 32 + (lane & 31));
+      // (groups 0 and 1 of a lane share their row, and 2 and 3; for fp8 all four)
+      const uint32_t rows_off[2] = {c_row(ft, (wm + i * WAVES_M) * 32 + group_row(0)), c_row(ft, (wm + i * WAVES_M) * 32 + group_row(2))};
       if constexpr (GATE_UP) {
 #pragma unroll
         for (int jp = 0; jp < NB / 2; ++jp)
@@ -2204,7 +2329,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
             float gate[4], up[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) gate[r] = sum[2 * jp][q][r], up[r] = sum[2 * jp + 1][q][r];
-            const int col = ft.n0 + wn * (Cfg::WTN / 2) + jp * 32 + 8 * q + 4 * (lane >> 5);
+            const uint32_t row_off = rows_off[q / 2];
+            const int col = ft.n0 + wn * (Cfg::WTN / 2) + jp * 32 + group_col(q);
             __builtin_amdgcn_raw_buffer_store_b64(combine4(gate, up), rc, c_at(ft, row_off, col), 0, kStoreMerging);
             if constexpr (KEEP) {
               const __amdgpu_buffer_rsrc_t rg = gate_up_rsrc(ft);
@@ -2219,7 +2345,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         for (int j = 0; j < NB; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const int col = ft.n0 + wn * Cfg::WTN + j * 32 + 8 * q + 4 * (lane >> 5);
+            const uint32_t row_off = rows_off[q / 2];
+            const int col = ft.n0 + wn * Cfg::WTN + j * 32 + group_col(q);
             const uint32_t off = c_at(ft, row_off, col);
             if (ANY_ROWS && (p.flags & kFlagAnyRows) != 0) {
               const u32x2 v = round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]);

@@ -7,6 +7,7 @@ import importlib.util
 import inspect
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -594,3 +595,59 @@ def test_traceable_operator_shapes_without_a_device():
         wgrad = torch.ops.grouped_gemm_amd.gmm(a, torch.empty(100, 96, dtype=torch.bfloat16), bs, True, False)
         assert wgrad.shape == (4, 64, 96) and wgrad.dtype == torch.bfloat16
 
+
+
+def _early_loads(lines):
+    """Loads straight to LDS in a disassembly that come too soon: less than five wait states behind a vector instruction
+    that writes a word of their descriptor (the hardware does not wait for it, and the compiler does not look into the
+    assembly that these loads are written in), or right behind the write of m0 that aims them."""
+    code = []
+    for line in lines:
+        m = re.match(r"\s+([a-z]\w+)\s*(.*?)\s*(//.*)?$", line)
+        if m:
+            code.append((m.group(1), m.group(2)))
+    early, loads = [], 0
+    for i, (op, args) in enumerate(code):
+        if op != "buffer_load_dwordx4" or not args.endswith(" lds"):
+            continue
+        loads += 1
+        first, last = map(int, re.search(r", s\[(\d+):(\d+)\]", args).groups())
+        waited, aimed, k = 0, None, i - 1
+        while k >= 0 and (waited < 5 or aimed is None):
+            before, to = code[k]
+            m = re.match(r"s(\d+)\b", to)
+            if waited < 5 and before.startswith("v_read") and m and first <= int(m.group(1)) <= last:
+                early.append(code[k:i + 1])
+            if aimed is None and re.match(r"m0\b", to):
+                aimed = waited
+            waited += 1 + int(to, 0) if before == "s_nop" else 1
+            k -= 1
+        if aimed == 0:
+            early.append(code[i - 1:i + 1])
+    return early, loads
+
+
+def test_loads_to_lds_are_late_enough(tmp_path):
+    # the check itself ...
+    load = "\tbuffer_load_dwordx4 v1, s[8:11], 0 offen lds"
+    aim = "\ts_add_u32 m0, s3, 16"
+    for between, bad in [([aim, "\ts_nop 0"], 1), ([aim, "\ts_nop 2"], 1), ([aim, "\ts_nop 3"], 0), (["\ts_nop 4", aim], 1)]:
+        early, loads = _early_loads(["\tv_readfirstlane_b32 s9, v0"] + between + [load])
+        assert (len(early), loads) == (bad, 1), between
+    # ... and every kernel that was built
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    library = os.path.join(ROOT, "grouped_gemm_amd", "libgrouped_gemm_hip.so")
+    copy = tmp_path / "library.so"
+    copy.write_bytes(open(library, "rb").read())
+    subprocess.run([objdump, "--offloading", str(copy)], check=True, capture_output=True)
+    objects = [f for f in sorted(tmp_path.iterdir()) if "gfx950" in f.name]
+    assert objects
+    total = 0
+    for f in objects:
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(f)], check=True, capture_output=True, text=True).stdout
+        early, loads = _early_loads(text.splitlines())
+        assert not early, (f.name, early[:3])
+        total += loads
+    assert total > 1000
