@@ -388,12 +388,13 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // traffic (both gradients in one launch): 9 x 613, 1792 x 960 (1008): 79 / 66; 11 x 980, 1088 x 1088 (891): 82 / 73; 6 x 1784, 1792 x 1088
 // (756): 120 / 111; 15 x 1627, 2368 x 256 (570): 91 / 96; of fewer rows 26 x 318, 192 x 1312 (572): 30 / 38.  Groups of
 // kDeepGroups rows and more keep the wide ones where these fill the device: where a few of them are much deeper than
-// the rest, those are cut along the depth (plan_deep_tiles).  Where wide tiles leave half of it idle, small
+// the rest, those are cut along the depth (plan_pieces_by_length).  Where wide tiles leave half of it idle, small
 // ones, and pieces of them, which pay from 16 slices on, put the rest to work.  Wide / small and the number of
 // wide ones: 19 x 2569 rows, 384 x 128 (38): 53 / 25; 5 x 3106, 608 x 240 (15): 60 / 24; 3 x 4000, 1024 x 1024, Zipf 1.2 (48):
 // 82 / 53; 4 x 15000, 1024 x 512 (32): 101 / 72; 6 x 5000, 768 x 1024 (72): 89 / 64; 8 x 5000, 1024 x 1024 (128): 89 / 84; with fp32
 // accumulation 98 / 70 and 108 / 94; but 4 x 10000, 2048 x 1024 (128): 154 / 170.  Only where the caller says so
 // (GG_FLAG_FEW_TILES, as the PyTorch binding always does): of the rules here the only one that is an option of the C ABI.
+// Without it the groups' depths are cut by plan_deep_tiles, into as many pieces of every tile that is cut.
 constexpr int64_t kDeepGroups = 2560;
 constexpr int64_t kMiddlingGroups = 512;
 constexpr int64_t kVeryDeepGroups = 8192;
@@ -565,6 +566,7 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
                 "the header's flags are the kernel's");
   p.flags = g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ONE_CLASS | GG_FLAG_ROW_PIECES | GG_FLAG_GROUP_ORDER);
   if (merge_stores(g)) p.flags |= gg::kFlagMergeStores;
+  if (trans_a && (g.flags & GG_FLAG_FEW_TILES)) p.flags |= gg::kFlagPiecesByLength;
   if (strides != nullptr && (hidden_out % 8 != 0 || (reinterpret_cast<uintptr_t>(g.c) & 15))) p.flags |= gg::kFlagAnyRows;
   const bool depth_pieces = !generic && may_cut_depth(g, route, shape);
   p.sched_out = nullptr;

@@ -101,6 +101,7 @@ enum : int {   // debugging switches, for comparing the ways a call can be sched
   kFlagGroupOrder = 8,    // NN and NT layouts: never hand out the groups' tiles by tile rows
   kFlagByTileRows = 16,   // set by the host side (never by callers): hand them out by tile rows
   kFlagAnyRows = 64,      // set by the host side: rows of c on 2-byte boundaries, of any length
+  kFlagPiecesByLength = 128,   // set by the host side: plan_pieces_by_length instead of plan_deep_tiles
   kFlagMergeStores = 32,  // set by the host side: kStoreMerging instead of kStoreStreaming (merge_stores in gmm_api.hip)
 };
 
@@ -231,7 +232,11 @@ struct Sched {
   // cut along the depth into front_pieces pieces each; tile indices 0 .. front_tiles *
   // front_pieces - 1 name those pieces, the tiles behind follow whole, and the last round is not
   // cut.  (Kept here, not in registers: the tile loop has no scalar registers to spare.)
-  int32_t front_tiles, front_pieces;
+  // With plan_pieces_by_length front_pieces is 0, indices 0 .. front_tiles - 1 name the pieces of the first cut_groups
+  // positions of `order`: position q's begin at tile_start[q], runt_start[q] of every tile (first all tiles' first
+  // pieces, then all their second ones: neighbours share rows of both operands).
+  int32_t front_tiles, front_pieces, cut_groups;
+  int32_t group_tiles;                 // tiles per group
   int32_t most_rows;                   // rows of the largest group
   // order[q] is the group whose tiles are handed out q-th.  Weight-gradient layout: by descending
   // depth.  Every group has the same number of tiles there and a tile's cost is its group's depth,
@@ -525,9 +530,11 @@ __device__ __forceinline__ void build_schedule(Sched* s, const GmmParams& p, con
       rrun += runt_tiles[i];
     }
   }
+  if (lane == 0) s->group_tiles = (int)main_tiles[0];   // (weight-gradient layout: the same for every group)
   if (lane == 63) {
     s->front_tiles = 0;
     s->front_pieces = 1;
+    s->cut_groups = 0;
     s->most_rows = (int)most;
     s->row_start[E] = (int)(all < tokens ? all : tokens);
     s->tile_start[E] = (int)tincl;
@@ -615,6 +622,103 @@ __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, in
   plan->pieces = 1;   // the last round stays whole: a workgroup has at most one tile to fix
   plan->by_depth = true;
   plan->main_tiles = plan->total = front * pieces + (tiles - front);
+}
+
+// ... and with kFlagPiecesByLength: pieces of about one length, as many of a tile as it has such lengths, so that groups of
+// all depths end together, also where there are few tiles and the deepest are many times as long as the rest (small
+// hidden sizes and many rows).  The length is one of the deepest tile's halves to sixteenths, the one with which the launch
+// is expected to end soonest: the longest of the first round (a piece and its fix-up, or the deepest whole tile) and an even share
+// of what is left, in depth slices.  us per launch, plan_deep_tiles / this one:
+// 21 Zipf (1.2) groups, 51204 rows, 128 x 560: 45.4 / 34.3; 56, 19094 rows, 704 x 1376: 124 / 92; 64, 49152 rows, 2048 x 1408: 320 /
+// 314; 7 even groups, 44642 rows, 360 x 424: 37.3 / 33.2; 15, 40804, 416 x 136 (cut as the last round by both): 24.1 / 24.5.
+template <int OUTPUTS>
+struct PieceCosts {   // in slices: a tile's turnover, a fix-up (constant, per piece), a partial tile's way through memory
+  static constexpr bool FULL = OUTPUTS > 128 * 128;
+  static constexpr float TILE = FULL ? 4 : 3, FIX = FULL ? 14 : 4, FIX_PIECE = FULL ? 3 : 1.5f, PARTIAL = FULL ? 6 : 3;
+  static constexpr int SHORTEST = FULL ? 16 : 6;   // piece
+};
+__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(x, [](uint32_t a, uint32_t b) { return a + b; }), 63);
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; }), 63);
+}
+template <int BM, int BN>
+__device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams& p, int grid, int bk, TailPlan* plan) {
+  using Costs = PieceCosts<BM * BN>;
+  const int E = p.num_groups, tiles = s->tile_start[E], per_group = s->group_tiles, lane = threadIdx.x & 63;
+  if (E == 0 || tiles == 0 || p.ws_slots <= 0 || (p.flags & (kFlagWholeTiles | kFlagRowPieces))) return;
+  // (every wave works out the same plan; each lane has up to 8 positions of the order, 64 apart)
+  const int per = (E + 63) >> 6;
+  uint32_t depth[8], sum = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    depth[i] = 0;
+    if (i < per && lane + 64 * i < E) depth[i] = (uint32_t)(s->rows[s->order[lane + 64 * i]] + bk - 1) / bk;
+    sum += depth[i];
+  }
+  const int deepest = __builtin_amdgcn_readfirstlane((int)depth[0]);
+  if (deepest < 4 * Costs::SHORTEST) return;
+  const float share = ((float)wave_sum(sum) * per_group + Costs::TILE * tiles) / grid;
+  // What follows the first round when the first `from` positions are cut: the share of all, less that of the first round (those and as many
+  // whole tiles as there are workgroups left).
+  auto rest = [&](uint32_t from, uint32_t pieces) {
+    const uint32_t to = from + (uint32_t)max(0, grid - (int)pieces * per_group) / per_group;
+    uint32_t first = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < per) first += (uint32_t)(lane + 64 * i) < to ? depth[i] : 0;
+    return fmaxf(0.0f, share - Costs::TILE + (Costs::PARTIAL * pieces - (float)wave_sum(first)) * per_group / grid);
+  };
+  // as it is: the tiles of a launch of one round may be cut already
+  const bool one_round = tiles <= grid;
+  float best = plan->by_depth && plan->main_tiles == 0 ? deepest / plan->pieces + Costs::FIX + Costs::FIX_PIECE * plan->pieces
+                                                       : deepest + Costs::TILE + (one_round ? 0.0f : rest(0, 0));
+  best *= 15.0f / 16.0f;
+  int length = 0, cut = 0, pieces = 0;
+#pragma unroll 1
+  for (int n = 2; n <= kMaxDepthPieces; n += n < 4 ? 1 : (n < 8 ? 2 : 4)) {
+    const int l = (deepest + n - 1) / n;
+    if (l < Costs::SHORTEST) break;
+    const uint32_t above = (uint32_t)(l + l / 2);
+    uint32_t t = 0, c = 0, longest = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < per) {
+        const bool is_cut = depth[i] > above;
+        t += is_cut ? (depth[i] + l - 1) / l : 0;
+        c += is_cut ? 1 : 0;
+        longest = is_cut || depth[i] < longest ? longest : depth[i];
+      }
+    t = wave_sum(t), c = wave_sum(c), longest = wave_max(longest);
+    if ((uint64_t)t * per_group > (uint64_t)min(grid, p.ws_slots) || (uint64_t)c * per_group > kWsCounterBytes / 4) continue;
+    float end = fmaxf(l + Costs::FIX + Costs::FIX_PIECE * n, longest + Costs::TILE);
+    if (tiles - (int)c * per_group + (int)t * per_group > grid) end += rest(c, t);
+    if (c > 0 && end < best) best = end, length = l, cut = (int)c, pieces = (int)t;
+  }
+  if (length == 0) return;
+  __syncthreads();   // (tile_start has been read by every wave)
+  uint32_t start = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if (i < per) {
+      const int q = lane + 64 * i;
+      const uint32_t mine = q < cut ? (depth[i] + length - 1) / length : 0;
+      const uint32_t upto = wave_scan(mine, [](uint32_t a, uint32_t b) { return a + b; });
+      if (q < cut) {
+        s->tile_start[q] = (int)(start + upto - mine) * per_group;
+        s->runt_start[q] = (int)mine;
+      }
+      start += (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+    }
+  // (every wave writes the same values, and reads its own)
+  s->tile_start[cut] = pieces * per_group;
+  s->front_tiles = pieces * per_group;
+  s->front_pieces = 0;
+  s->cut_groups = cut;
+  plan->pieces = 1;   // the last round stays whole: a workgroup has at most one tile to fix
+  plan->by_depth = true;
+  plan->main_tiles = plan->total = pieces * per_group + (tiles - cut * per_group);
 }
 
 // NN and NT layouts with many short groups: the groups by ascending number of tile rows, groups
@@ -1217,7 +1321,8 @@ struct TileInfo {
   int nk;           // depth slices, at least 1 so that an empty group still stores zeros
   int pieces;       // depth pieces this tile is cut into (1: whole depth, store directly)
   int piece;        // which of them this is
-  int rank;         // index of the tile among the tiles of the last round
+  int rank;         // index of the tile among the tiles that are cut
+  int slot, slots_apart;   // where its pieces' partial tiles are in the workspace
   bool valid;
 };
 
@@ -1237,7 +1342,7 @@ __device__ __forceinline__ void pack_tile(const TileInfo& t, int32_t* w) {
   w[6] = t.g.m, w[7] = t.g.n, w[8] = t.g.k, w[9] = t.g.row0;
   w[10] = t.m0, w[11] = t.n0, w[12] = t.rows_valid, w[13] = t.blocks, w[14] = t.depth, w[15] = t.k0;
   w[16] = t.nk, w[17] = t.pieces, w[18] = t.piece, w[19] = t.rank, w[20] = t.valid ? 1 : 0;
-  w[21] = w[22] = w[23] = 0;
+  w[21] = t.slot, w[22] = t.slots_apart, w[23] = 0;
 }
 __device__ __forceinline__ TileInfo unpack_tile(const int32_t* w) {
   auto u = [&](int i) { return uniform(w[i]); };
@@ -1246,7 +1351,7 @@ __device__ __forceinline__ TileInfo unpack_tile(const int32_t* w) {
   t.g.a_off = u64(0), t.g.b_off = u64(2), t.g.c_off = u64(4);
   t.g.m = u(6), t.g.n = u(7), t.g.k = u(8), t.g.row0 = u(9);
   t.m0 = u(10), t.n0 = u(11), t.rows_valid = u(12), t.blocks = u(13), t.depth = u(14), t.k0 = u(15);
-  t.nk = u(16), t.pieces = u(17), t.piece = u(18), t.rank = u(19), t.valid = u(20) != 0;
+  t.nk = u(16), t.pieces = u(17), t.piece = u(18), t.rank = u(19), t.valid = u(20) != 0, t.slot = u(21), t.slots_apart = u(22);
   return t;
 }
 
@@ -1285,6 +1390,8 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
   ti.pieces = 1;
   ti.piece = 0;
   ti.rank = 0;
+  ti.slot = 0;
+  ti.slots_apart = 1;
   if (t >= plan.total) {
     ti.g = GroupGeom{0, 0, 0, 0, 0, 0, 0};
     ti.m0 = ti.n0 = ti.rows_valid = ti.depth = 0;
@@ -1299,10 +1406,33 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
   if (front_tiles > 0) {
     const int front_pieces = uniform(sched->front_pieces);
     const int cut = front_tiles * front_pieces;
-    if (t < cut) {
+    if (front_pieces == 0) {   // (plan_pieces_by_length)
+      const int per_group = uniform(sched->group_tiles), groups = uniform(sched->cut_groups);
+      if (t < front_tiles) {
+        // (positions whose pieces end at t or before; no loop here, see tile_body)
+        int q = 0;
+#pragma unroll
+        for (int i = 0; i < kMaxGroups; i += 64)
+          if (i < groups) {
+            const int lane = threadIdx.x & 63, at = i + lane;
+            q += __popcll(__ballot(at < groups && sched->tile_start[at + 1] <= t));
+          }
+        q = uniform(q);
+        const int first = uniform(sched->tile_start[q]);
+        pieces = uniform(sched->runt_start[q]);
+        piece = (t - first) / per_group;
+        ti.slot = t - piece * per_group;
+        ti.slots_apart = per_group;
+        t = q * per_group + (ti.slot - first);
+        ti.rank = t;
+      } else {
+        t = t - front_tiles + groups * per_group;
+      }
+    } else if (t < cut) {
       pieces = front_pieces;
       piece = t % pieces;
       ti.rank = t / pieces;
+      ti.slot = t - piece;
       t = ti.rank;
     } else {
       t = t - cut + front_tiles;
@@ -1311,13 +1441,14 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
     const int r = t - plan.main_tiles;
     piece = r % plan.pieces;
     ti.rank = r / plan.pieces;
+    ti.slot = r - piece;
     t = plan.main_tiles + ti.rank;
   }
   const int first_class = uniform(sched->tile_start[p.num_groups]);
   int u;
   if (LAYOUT == kTN) {
-    // (every group has the same number of tiles, tile_start[1], and there are no runt rows)
-    const int per_group = uniform(sched->tile_start[1]);
+    // (every group has the same number of tiles, and there are no runt rows)
+    const int per_group = uniform(sched->group_tiles);
     cur.e = t / per_group;
     u = t - cur.e * per_group;
   } else if (t < first_class) {
@@ -1530,7 +1661,11 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   if constexpr (PART::SECOND) plan.main_tiles += head_tiles, plan.total += head_tiles;
   if constexpr (!DEPTH_PIECES) plan.by_depth = false;   // (known at compile time: no depth-piece code is kept)
   if constexpr (LAYOUT == kTN && DEPTH_PIECES) {
-    plan_deep_tiles<BM, BN>(sched, p, G, BK_ELEMS, &plan);
+    if (p.flags & kFlagPiecesByLength) {
+      plan_pieces_by_length<BM, BN>(sched, p, G, BK_ELEMS, &plan);
+    } else {
+      plan_deep_tiles<BM, BN>(sched, p, G, BK_ELEMS, &plan);
+    }
     plan.pieces = uniform(plan.pieces), plan.main_tiles = uniform(plan.main_tiles), plan.total = uniform(plan.total);
     // (cut deep tiles go out first, at most one piece to a workgroup)
     if (PART::SECOND && uniform(sched->front_tiles) > 0) head_tiles = 0;
@@ -1757,8 +1892,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // at ((i * NB + j) * 4 + q) * NT + thread, so one instruction of a wave moves 1 KiB of consecutive
   // bytes.
   auto partial_rsrc = [&](const TileInfo& tile, int piece) {
-    return make_rsrc(p.workspace + kWsCounterBytes + (int64_t)(tile.rank * tile.pieces + piece) * (BM * BN * 4),
-                     BM * BN * 4);
+    return make_rsrc(p.workspace + kWsCounterBytes + (int64_t)(tile.slot + piece * tile.slots_apart) * (BM * BN * 4),
+                     piece < tile.pieces ? BM * BN * 4 : 0);   // (no such piece: zeros)
   };
   auto partial_at = [&](int i, int j, int q) -> uint32_t { return (((i * NB + j) * 4 + q) * NT + threadIdx.x) * 16; };
   bool fix_pending = false;   // this workgroup's depth piece was the last of its tile to arrive
@@ -1955,7 +2090,8 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       // slice after a tile that was stored, its stores)
       constexpr int PENDING = Loads::before(READY);
       // (in the weight-gradient layout the condition is one of the first slice's, which the compiler then takes out of the
-      // loop: with the other form it moves accumulators in and out of the loop, 332 moves a slice)
+      // loop, as long as there is no loop in this one: with that wait in the loop it moves accumulators in and out of it, 332
+      // moves a slice)
       if (LATE_LOADS || (LAYOUT == kTN && kt > 0) || __builtin_expect(uniform(stored) == 0, 1)) {
         wait_vmcnt<PENDING>();
       } else {
@@ -2286,7 +2422,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
 
   // Fix-up of a tile that was cut along the depth: the tile this workgroup left in
   // Sched::fix_tile when its piece arrived last (a workgroup has at most one).  The partial tiles
-  // are added up in piece order, two per step (their count is even), whichever piece does the
+  // are added up in piece order, two per step, whichever piece does the
   // adding, so the result does not depend on timing.  One block row of 32 rows at a time: NB * 4
   // groups of 16 bytes per lane and piece.
   if (DEPTH_PIECES && fix_pending) {

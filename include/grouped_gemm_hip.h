@@ -63,7 +63,8 @@ extern "C" {
 #define GG_FLAG_ROW_PIECES 4    /* ignore the workspace: cut the last round's tiles along the rows only */
 #define GG_FLAG_GROUP_ORDER 8   /* hand out the groups' tiles in group order, also where the library would hand them out by their number of tile rows (many short groups, trans_a = 0) */
 /* ... and one that is for speed: with trans_a, smaller tiles also for deep groups whose full tiles would leave at
- * least half of the device idle, up to three times as fast (sums in another order than without). */
+ * least half of the device idle, up to three times as fast, and groups of unequal depths in pieces of one length (see
+ * workspace; sums in another order than without). */
 #define GG_FLAG_FEW_TILES 128
 
 /*
@@ -188,7 +189,8 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *                 depend on timing.  With trans_a = 1, when a group is so much deeper than the
  *                 rest that its tiles alone would set the length of the launch, the tiles of
  *                 such groups are cut the same way and handed out first (instead of the last
- *                 round's).  The first 4096 bytes (arrival counters) must be zero
+ *                 round's); with GG_FLAG_FEW_TILES into pieces of one length, so that a deeper group is cut
+ *                 into more of them.  The first 4096 bytes (arrival counters) must be zero
  *                 before the first call and are zero again after every call; the rest needs no
  *                 initialisation.  GG_WORKSPACE_BYTES serves every call; a smaller workspace
  *                 (at least 4096 + one 256 KiB tile; plain calls on two-byte operands whose
@@ -372,7 +374,7 @@ int gg_debug_pair(const gg_gmm_args* first, const gg_gmm_args* second, const int
 /* How a weight gradient (trans_a) with a workspace cuts its deepest tiles along the depth, for host-resident sizes and
  * two-byte elements: `*tiles` of them, the deepest first, into `*pieces` pieces each (0: none), on `workgroups` workgroups, with room
  * for `partial_tiles` partial tiles, where every group has tiles_per_group tiles of tile_outputs elements of c.  The
- * function that the kernel itself runs; needs no device. */
+ * function that the kernel itself runs without GG_FLAG_FEW_TILES; needs no device. */
 int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups,
                       int partial_tiles, int tile_outputs, int* pieces, int* tiles);
 

@@ -2754,6 +2754,57 @@ def test_deep_weight_gradients_of_few_tiles(ops, oracle, sizes, hin, hout):
     assert float(((c - 2.0) - want).abs().max()) <= bound
 
 
+@pytest.mark.parametrize("sizes,hin,hout,side,partial", [
+    ([14000, 300, 200, 0, 150, 6500, 100, 120], 264, 520, 128, 15 * (8 + 4)),    # pieces of 28 slices, 219 and 102 of them
+    ([64] * 50 + [20000] + [64] * 50, 256, 256, 128, 4 * 16),
+    ([9000, 4200, 2000, 1000, 500, 250] * 2 + [64] * 30, 704, 1376, 256, 18 * (4 + 4 + 2 + 2)),   # 141 and 66 slices, 36 a piece
+    ([9000, 7000, 5200, 2600, 1300] + [200] * 60, 136, 264, 128, 6 * (8 + 7 + 5 + 3)),            # odd numbers of pieces
+    ([5000] * 3 + [0] * 5, 128, 264, 128, 3 * 24),              # every tile with rows
+    ([90 + 7 * i for i in range(509)] + [20000, 0, 17000], 64, 72, 128, 8 + 7),   # most groups there can be, 8 to a lane
+    ([1500] + [100] * 7, 264, 520, 128, 15 * 4),                # 24 slices: the least depth that is cut,
+    ([1460] + [100] * 7, 264, 520, 128, 0),                     # and less
+    ([30000], 128, 128, 128, 16),                               # the last round's cut is as good
+    ([5000, 5000, 5000, 5000], 2048, 2048, 256, 0),             # deep, but no deeper than a workgroup's share
+])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_weight_gradients_in_pieces_by_length(oracle, sizes, hin, hout, side, partial, accumulate):
+    # Pieces of one length, of every group that is longer: through the C ABI with a workspace of the test's own. As many
+    # partial tiles in it as there are pieces, the counters zero again, the same bits on every call, zero-row groups
+    # zero (or as they were), and against whole tiles no further than fp32 sums in another order.
+    _announce("pieces by length", sizes if len(sizes) < 10 else len(sizes), hin, hout, accumulate)
+    lib = _c_abi()
+    g = torch.Generator().manual_seed(hin + hout)
+    bs, t = torch.tensor(sizes, dtype=torch.int64), sum(sizes)
+    a = torch.randn(t, hin, generator=g).to(torch.bfloat16).cuda()
+    b = torch.randn(t, hout, generator=g).to(torch.bfloat16).cuda()
+    ws = torch.zeros(1024 + 256 * 256 * 256, dtype=torch.float32, device="cuda")
+    outs = []
+    for flags in (128, 128, 128 | 1):   # the last: whole tiles
+        c = torch.full((len(sizes), hin, hout), 7.0, dtype=torch.float32 if accumulate else torch.bfloat16, device="cuda")
+        args = _gmm_args(lib, a, b, c, bs.cuda() if accumulate else bs, accumulate, t, hin, hout, True, False, flags=flags, workspace=ws)
+        args.accumulate_f32 = int(accumulate)
+        assert lib.gg_gmm(ctypes.byref(args)) == 0, lib.gg_last_error()
+        torch.cuda.synchronize()
+        outs.append(c)
+        assert not bool(ws[:1024].any()), "arrival counters left nonzero"
+        if len(outs) == 1:
+            assert _tile(lib, args) == (side, side)
+            assert int((ws[1024:].view(-1, side * side) != 0).any(dim=1).sum()) == partial
+    cut, again, whole = outs
+    assert torch.equal(cut, again)
+    ends = bs.cumsum(0).tolist()
+    want = torch.stack([a[e - n:e].float().t() @ b[e - n:e].float() for e, n in zip(ends, sizes)])
+    # one rounding of 2 ** -24 of a partial sum for each product and fewer of them than those, as a random walk (7: what c held)
+    bound = 2 * max(sizes) ** 0.5 * 2.0 ** -24 * (7.0 + float(want.abs().max()))
+    if accumulate:
+        assert float(((cut - 7.0) - want).abs().max()) <= bound
+        assert float((cut - whole).abs().max()) <= bound
+    else:
+        check(cut, want, f"in pieces {hin} x {hout}")
+        assert float((cut.float() - whole.float()).abs().max()) <= 2 ** -7 * float(want.abs().max())
+    assert bool((cut[bs == 0] == (7.0 if accumulate else 0.0)).all())
+
+
 @pytest.mark.parametrize("on_device", [False, True])
 @pytest.mark.parametrize("experts,rows,hin,hout,trans_b,skew", [
     (8, 1024, 128, 128, False, 0),       # small tiles of both
