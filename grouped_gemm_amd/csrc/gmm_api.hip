@@ -429,10 +429,9 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
 // allowed.  Judged as for a crowded device (the sizes, and so the tiles of the last round, may be known on the
 // device only): a call that could be cut only where its last round holds few tiles does without.
 bool may_cut_depth(const gg_gmm_args& g, const Route& r, const TileShape& shape) {
-  // (the fix-up of depth pieces stores 4 columns at a time: whole tiles and row pieces for ragged widths.
-  // Ragged depths: the kernel looks for the ragged chunks in the slice hidden_in / 64 of tiles that start
-  // at depth 0.)
-  if (r.generic || r.ragged_width || r.ragged_depth || g.num_groups <= 0) return false;
+  // (the fix-up of depth pieces stores 4 columns at a time where rows go through indices: whole tiles and row pieces
+  // for ragged widths then)
+  if (r.generic || (r.ragged_width && r.indexed) || g.num_groups <= 0) return false;
   if (g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ROW_PIECES)) return false;
   const bool scattered = r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU;
   if (scattered && shape.id == Wide::kId) return false;
@@ -586,18 +585,19 @@ int plan_call(const gg_gmm_args& g, bool static_scratch, Plan* out, void* gate_u
     hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(gg::kWsCounterBytes / 4), 0, stream,
                        reinterpret_cast<int*>(info.scratch));
     GG_HIP(hipGetLastError());
-  } else if (g.workspace != nullptr && !generic && !route.ragged_width && !route.ragged_depth) {
-    if (reinterpret_cast<uintptr_t>(g.workspace) & 255)
-      return fail(GG_ELIMIT, "the workspace must be 256-byte aligned");
+  } else if (g.workspace != nullptr && !generic) {
+    const bool ragged = route.ragged_width || route.ragged_depth;   // (takes any workspace; one that does not fit is not used)
+    const bool misaligned = (reinterpret_cast<uintptr_t>(g.workspace) & 255) != 0;
+    if (misaligned && !ragged) return fail(GG_ELIMIT, "the workspace must be 256-byte aligned");
     const uint64_t slot_bytes = (uint64_t)bm * bn * (swiglu ? 2 : 1) * 4;
     // (one tile of the wide shape, or of the short one where groups average few rows: what a caller can tell
     // without the rules of pick_shape, whose tiles are no larger)
     const bool few_rows = !swiglu && !indexed && elem_bytes == 2 && use_short_shape(num_groups, tokens, trans_a);
     const uint64_t least = gg::kWsCounterBytes + (few_rows ? (uint64_t)Short::BM * Short::BN : (uint64_t)Wide::BM * Wide::BN) * 4;
-    if (g.workspace_bytes < least)
+    if (g.workspace_bytes < least && !ragged)
       return fail(GG_ELIMIT, "the workspace holds %llu bytes, the smallest useful one %llu",
                   (unsigned long long)g.workspace_bytes, (unsigned long long)least);
-    const uint64_t slots = (g.workspace_bytes - gg::kWsCounterBytes) / slot_bytes;
+    const uint64_t slots = misaligned || g.workspace_bytes < least ? 0 : (g.workspace_bytes - gg::kWsCounterBytes) / slot_bytes;
     p.workspace = static_cast<char*>(g.workspace);
     // one arrival counter per tile of the last round: at most grid / 2 of them, 1024 fit
     p.ws_slots = !depth_pieces ? 0 : (slots > 1024 ? 1024 : (int32_t)slots);
@@ -747,8 +747,12 @@ int plan_pair(const gg_gmm_args* first, const Strides* strides1, const gg_gmm_ar
   if (rc != GG_OK) return rc;
   // (also one after the other: the partial tiles of the first would be left where the second's counters have to be zero)
   if (p1.p.ws_slots > 0 && p2.p.ws_slots > 0 && p1.p.workspace != p2.p.workspace &&
-      p1.p.workspace < p2.p.workspace + second->workspace_bytes && p2.p.workspace < p1.p.workspace + first->workspace_bytes)
-    return fail(GG_EINVAL, "the workspaces of the two calls overlap in part");
+      p1.p.workspace < p2.p.workspace + second->workspace_bytes && p2.p.workspace < p1.p.workspace + first->workspace_bytes) {
+    // (ragged sizes take any workspace, see plan_call)
+    const bool ragged1 = p1.route.ragged_width || p1.route.ragged_depth, ragged2 = p2.route.ragged_width || p2.route.ragged_depth;
+    if (!ragged1 && !ragged2) return fail(GG_EINVAL, "the workspaces of the two calls overlap in part");
+    (ragged1 ? p1 : p2).p.ws_slots = 0;
+  }
   out->pair = pair_kernel(*first, p1, *second, p2);
   if (out->pair != nullptr) {
     int64_t row1 = 0, row2 = 0, tiles1, tiles2;

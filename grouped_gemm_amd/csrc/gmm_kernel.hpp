@@ -1651,7 +1651,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
 
   // (tiles that are combined or scattered on their way out are cut along the depth in the shapes for
   // few rows and few tiles only: full ones would pay for it with the fix-up's scalar registers)
-  constexpr bool DEPTH_PIECES = !RAGGED_DEPTH && !((GATE_UP || INDEXED) && BM > 128);
+  constexpr bool DEPTH_PIECES = !((GATE_UP || INDEXED) && BM > 128);
   const int all_tiles = uniform(sched->tile_start[p.num_groups]) + uniform(sched->runt_start[p.num_groups]);
   // SECOND: indices below head_tiles go to the workgroups that start early, the others to all of them
   Head head{0, 0};
@@ -1771,7 +1771,9 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // Load J of the cursor's slice (A's loads first, then B's) into buffer `buf`: fetch_aim, then fetch_load.  A's descriptor
   // comes with fetch_begin (then a wait, a barrier, a matrix instruction, fetch_aim and another instruction precede the first
   // load), B's ahead of A's last load (then that load and two of each precede B's first).
+  bool tail_fetched = false;   // RAGGED_DEPTH: the cursor's slice holds the end of the depth
   auto fetch_begin = [&]() {
+    if constexpr (RAGGED_DEPTH) tail_fetched = uniform(aload.depth) > 0 && uniform(aload.depth) < BK;
     a_slice = aload.slice();
     settle(a_slice.rsrc);
   };
@@ -1839,8 +1841,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   fetch_begin();
   asm volatile("s_nop 4");
   static_for<LOADS_PER_STAGE>([&](auto j) { fetch_whole(j, 0); });
+  const bool tail_first = tail_fetched;
   fetch_advance();
   fetch_begin();
+  bool tail_next = tail_fetched;   // ... the slice after the one that is multiplied does
   asm volatile("s_nop 4");
   static_for<FIRST_LOADS>([&](auto j) { fetch_whole(j, 1); });
 
@@ -1857,12 +1861,13 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
     return unpack_tile(words);
   };
   TileInfo ti = next_tile();
-  // RAGGED_DEPTH: hidden_in is even but no multiple of 8.  No depth pieces then (every tile starts at
-  // depth 0), so the ragged chunks are in slice hidden_in / BK of every tile.  Once a buffer holds
-  // that slice, complete for every wave, what its ragged chunks picked up from the rows behind is
-  // cleared before any wave reads a fragment from it.
+  // RAGGED_DEPTH: hidden_in is even but no multiple of 8.  The ragged chunks are in the slice that ends the depth, which
+  // the fetch cursor knows by what is left of it (a depth piece may begin anywhere and has that slice only if it is
+  // its tile's last).  Once a buffer holds that slice, complete for every wave, what its ragged chunks picked up from
+  // the rows behind is cleared before any wave reads a fragment from it.
+  // Whole tiles / pieces, us: 28 Zipf (1.2) groups, 5434 rows, 13374 -> 272, fp16, b transposed: 314 / 201, not: 223 / 182;
+  // 16 groups, 8192 rows, 9998 -> 2048: 542 / 466.
   static_assert(!RAGGED_DEPTH || (LAYOUT != kTN && !F8 && !GATE_UP && !INDEXED), "");
-  const int tail_slice = RAGGED_DEPTH ? p.hidden_in / BK : -1;
   auto clear_tail = [&](int buf) {
     if constexpr (RAGGED_DEPTH) {
       char* st = smem + uniform(buf) * Cfg::STAGE_BYTES;
@@ -1875,7 +1880,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   };
   wait_vmcnt<FIRST_LOADS>();   // the first slice is in
   block_barrier();
-  if (RAGGED_DEPTH && tail_slice == 0) clear_tail(0);
+  if (RAGGED_DEPTH && tail_first) clear_tail(0);
   static_for<2 * UNITS>([&](auto u) {
     read_unit(u, I0{}, IMB{}, 0);
   });
@@ -1934,6 +1939,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // any boundary, the last ones of a row by elements.  8 x 1024 rows, 2047 -> 5461, forward and gradients: 834 us with
   // padded results copied back (120 of them the copies), 760 so.
   constexpr bool ANY_ROWS = EPI == kEpiStore && !INDEXED && !RAGGED_DEPTH && !F8;
+  // ... or that are no whole groups of 4 columns, which the fix-up of depth pieces stores (whole tiles / pieces, us: weight
+  // gradients of 21 Zipf (1.2) groups, 51204 rows, 128 x 558: 125 / 38, 64, 49152 rows, 2046 x 1406: 492 / 364; 16 groups, 600 rows,
+  // 6144 -> 518: 46.8 / 33.8).
+  constexpr bool FIX_ANY_ROWS = EPI == kEpiStore && !INDEXED && !F8;
   auto store_any = [&](const TileInfo& tile, uint32_t row_off, int col, int most, u32x4 v) {
     struct Chunk {
       u32x4 v;
@@ -2103,7 +2112,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         if (LAYOUT != kTN) stored = 0;   // (the next wait is for them too)
       }
       block_barrier();
-      if (RAGGED_DEPTH && uniform(kt + 1 == ti.nk ? 0 : kt + 1) == tail_slice) clear_tail(y);
+      if constexpr (RAGGED_DEPTH) {
+        if (tail_next) clear_tail(y);
+        tail_next = tail_fetched;
+      }
       slots(IReady{}, IAll{}, y);
       x = uniform(y);
     }
@@ -2484,7 +2496,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
             const uint32_t row_off = rows_off[q / 2];
             const int col = ft.n0 + wn * Cfg::WTN + j * 32 + group_col(q);
             const uint32_t off = c_at(ft, row_off, col);
-            if (ANY_ROWS && (p.flags & kFlagAnyRows) != 0) {
+            if (FIX_ANY_ROWS && ((p.flags & kFlagAnyRows) != 0 || uniform(ft.g.n & 3) != 0)) {
               const u32x2 v = round4<OUT_DT>(sum[j][q][0], sum[j][q][1], sum[j][q][2], sum[j][q][3]);
               store_any(ft, row_off, col, 4, u32x4{v[0], v[1], 0u, 0u});
             } else if constexpr (ACC_F32) {

@@ -195,7 +195,7 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *                 initialisation.  GG_WORKSPACE_BYTES serves every call; a smaller workspace
  *                 (at least 4096 + one 256 KiB tile; plain calls on two-byte operands whose
  *                 groups average few rows, see gg_tile_shape: 128 KiB) serves fewer pieces;
- *                 256-byte aligned.
+ *                 256-byte aligned.  (Calls of even hidden sizes that are no multiples of 8 ignore one that is smaller or off.)
  *                 Calls that share a workspace must not overlap in time (same stream is enough).
  *   flags         GG_FLAG_* bits.
  */
@@ -267,7 +267,7 @@ int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up);
 
 /*
  * Bytes of workspace the call described by `args` can make use of: 0 when no launch of it ever
- * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8, or a
+ * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8 with row indices, or a
  * product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte
  * elements for full tiles, fewer for groups of few rows; the depth of the trans_a layout being what
  * one group could hold, i.e. all rows), GG_WORKSPACE_BYTES otherwise.  Looks at the sizes, flags

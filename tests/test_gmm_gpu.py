@@ -2805,6 +2805,66 @@ def test_weight_gradients_in_pieces_by_length(oracle, sizes, hin, hout, side, pa
     assert bool((cut[bs == 0] == (7.0 if accumulate else 0.0)).all())
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("layout,sizes,hin,hout", [
+    ("nn", [40, 0, 300, 75], 6402, 264), ("nt", [40, 0, 300, 75], 6402, 264),       # only the depth is no multiple of 8: 101 slices
+    ("nn", [33, 90], 6414, 1030), ("nt", [33, 90], 6414, 1030),                     # neither is
+    ("nn", [700, 1], 13374, 270), ("nt", [257], 6146, 14),                          # 209 slices; two depth values in the last one
+    ("nn", [130, 5], 6400, 518), ("nt", [20, 13, 40, 9], 6400, 262),                # only the width
+    ("tn", [2900, 40, 0, 7], 138, 266), ("tn", [9000, 300], 520, 270),
+])
+def test_even_sizes_in_depth_pieces(oracle, layout, sizes, hin, hout, dtype):
+    # Even sizes that are no multiples of 8, on 4-byte boundaries, in depth pieces: partial tiles in the workspace and its
+    # counters zero again, the oracle's result (a NaN at the start of a row reaches that row's outputs only, also
+    # where the row before ends in the same chunk), nothing behind c's rows, the same bits on every call.  A workspace off
+    # 256-byte boundaries, or too small, is not used.
+    _announce("even sizes in pieces", layout, sizes, hin, hout, dtype)
+    lib = _c_abi()
+    lib.gg_workspace_bytes_for.argtypes, lib.gg_workspace_bytes_for.restype = [ctypes.c_void_p], ctypes.c_uint64
+    g = torch.Generator().manual_seed(hin + hout)
+    bs, t, tn = torch.tensor(sizes, dtype=torch.int64), sum(sizes), layout == "tn"
+    a = torch.randn(t, hin, generator=g).to(dtype)
+    b_shape = (t, hout) if tn else ((len(sizes), hout, hin) if layout == "nt" else (len(sizes), hin, hout))
+    b = (torch.randn(b_shape, generator=g) * (t if tn else hin) ** -0.5).to(dtype)
+    if not tn:
+        a[t // 2, :2] = float("nan")
+    want = oracle.gmm_loop(a, b, bs, trans_a=tn, trans_b=layout == "nt")
+    finite = torch.isfinite(want)
+    assert int((~finite).sum()) == (0 if tn else hout)
+
+    def off_by_4(x):   # on a 4-byte boundary and no wider one
+        buf = torch.empty(x.numel() + 2, dtype=dtype, device="cuda")
+        buf[2:] = x.flatten()
+        return buf[2:].view(x.shape)
+
+    da, db, sizes_on_device = off_by_4(a), off_by_4(b), bs.cuda()
+    ws = torch.zeros(1024 + 256 * 256 * 256, dtype=torch.float32, device="cuda")
+    outs = []
+    for use in ("pieces", "pieces", "off", "small", "none"):
+        buf = torch.full((want.numel() + 4,), 7.0, dtype=dtype, device="cuda")
+        c = buf[2:-2].view(want.shape)
+        ws.zero_()
+        args = _gmm_args(lib, da, db, c, sizes_on_device, True, t, hin, hout, tn, layout == "nt", workspace=None if use == "none" else ws,
+                         dtype=0 if dtype == torch.bfloat16 else 1)
+        assert lib.gg_workspace_bytes_for(ctypes.byref(args)) > 0
+        if use == "off":
+            args.workspace += 64
+            args.workspace_bytes -= 64
+        if use == "small":
+            args.workspace_bytes = 4096 + 1024
+        assert lib.gg_gmm(ctypes.byref(args)) == 0, lib.gg_last_error()
+        torch.cuda.synchronize()
+        assert not bool(ws[:1024].any()), "arrival counters left nonzero"
+        assert bool(ws.any()) == (use == "pieces"), use
+        assert bool((buf[:2] == 7.0).all()) and bool((buf[-2:] == 7.0).all())
+        got = c.cpu()
+        assert bool((torch.isfinite(got) == finite).all()), use
+        zero = torch.zeros((), dtype=torch.float32)
+        outs.append(torch.where(finite, got.float(), zero))
+        check(outs[-1], torch.where(finite, want.float(), zero), use)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[4]) and torch.equal(outs[3], outs[4])
+
+
 @pytest.mark.parametrize("on_device", [False, True])
 @pytest.mark.parametrize("experts,rows,hin,hout,trans_b,skew", [
     (8, 1024, 128, 128, False, 0),       # small tiles of both

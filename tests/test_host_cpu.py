@@ -277,7 +277,7 @@ def test_workspace_bytes_for_needs_no_device():
 
 def test_workspace_bytes_for_strided_operands():
     """gg_workspace_bytes_for_strided: by the call's own sizes, whatever they are (gg_workspace_bytes_for has nothing for
-    hidden sizes that are no multiples of 8: its calls run those without pieces)."""
+    odd hidden sizes: its calls run those on the general kernels)."""
     lib = ctypes.CDLL(HIP_LIB)
     for f in (lib.gg_workspace_bytes_for_strided, lib.gg_workspace_bytes_for):
         f.restype = ctypes.c_uint64
