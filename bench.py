@@ -427,7 +427,7 @@ def main():
     pipe_random = mfma_rate(False, 10)
     pipe_zeros = mfma_rate(True, 10)
     out["matrix_pipe_alone"] = {
-        "what": "v_mfma_f32_32x32x16_bf16 on register operands, 256 workgroups of 4 waves, 10 launches of about 2.5 ms",
+        "what": "v_mfma_f32_16x16x32_bf16 on register operands, 256 workgroups of 4 waves, 10 launches of about 2.5 ms",
         "random_operands_TFLOP/s": round(pipe_random, 1),
         "zero_operands_TFLOP/s": round(pipe_zeros, 1),
         "random_operands_frac_of_peak": round(pipe_random / PEAK_BF16_TFLOPS, 4),

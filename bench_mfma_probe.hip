@@ -1,5 +1,5 @@
 // A probe, not a GEMM: the rate at which this chip sustains the matrix instruction the kernels are
-// built on (v_mfma_f32_32x32x16_bf16), with all operands and accumulators held in registers and
+// built on (v_mfma_f32_16x16x32_bf16), with all operands and accumulators held in registers and
 // no memory traffic at all.  On operands whose bits vary like real activations the chip lowers
 // its clock to stay inside its power limit; on all-zero operands it does not.  The first figure
 // is therefore the ceiling of any bf16 GEMM on this device and data, whatever its memory system
@@ -14,9 +14,9 @@
 namespace {
 
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
-using f32x16 = __attribute__((ext_vector_type(16))) float;
+using f32x4 = __attribute__((ext_vector_type(4))) float;
 
-constexpr int kProbeWaves = 4, kProbeBlocks = 4;   // 4 x 4 blocks of 32 x 32 per wave: 256 accumulator registers
+constexpr int kProbeWaves = 4, kProbeBlocks = 8;   // 8 x 8 blocks of 16 x 16 per wave: 256 accumulator registers
 
 // Eight bf16 values distributed like randn * 0.02 (the sum of four uniform numbers stands in for
 // the normal distribution), from a per-lane integer hash: signs, exponents and mantissas then
@@ -40,25 +40,27 @@ __global__ __launch_bounds__(kProbeWaves * 64) void mfma_probe_kernel(int iterat
   bf16x8 a[kProbeBlocks], b[kProbeBlocks];
 #pragma unroll
   for (int i = 0; i < kProbeBlocks; ++i) {
-    a[i] = probe_operand(id * 8u + i, zeros != 0);
-    b[i] = probe_operand(id * 8u + 4u + i, zeros != 0);
+    a[i] = probe_operand(id * 16u + i, zeros != 0);
+    b[i] = probe_operand(id * 16u + 8u + i, zeros != 0);
   }
-  f32x16 acc[kProbeBlocks][kProbeBlocks];
+  f32x4 acc[kProbeBlocks][kProbeBlocks];
 #pragma unroll
   for (int i = 0; i < kProbeBlocks; ++i)
 #pragma unroll
     for (int j = 0; j < kProbeBlocks; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
   for (int it = 0; it < iterations; ++it) {
 #pragma unroll
     for (int j = 0; j < kProbeBlocks; ++j)
 #pragma unroll
-      for (int i = 0; i < kProbeBlocks; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
-    // new operand values every step, as a depth loop would bring them (the elements of two
+      for (int i = 0; i < kProbeBlocks; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    // new operand values every step, as a depth loop would bring them (the elements of four
     // fragments rotate: register moves only)
     a[0] = __builtin_shufflevector(a[0], a[0], 1, 2, 3, 4, 5, 6, 7, 0);
+    a[4] = __builtin_shufflevector(a[4], a[4], 1, 2, 3, 4, 5, 6, 7, 0);
     b[1] = __builtin_shufflevector(b[1], b[1], 1, 2, 3, 4, 5, 6, 7, 0);
+    b[5] = __builtin_shufflevector(b[5], b[5], 1, 2, 3, 4, 5, 6, 7, 0);
   }
   float s = 0.0f;
 #pragma unroll
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(kProbeWaves * 64) void mfma_probe_kernel(int iterat
 // Launches the probe `launches` + 1 times on `stream` (the first untimed) with one workgroup per
 // compute unit and returns the rate of the timed ones in TFLOP/s through `tflops`.
 hipError_t run_mfma_probe(int cus, int zeros, int launches, float* sink, hipStream_t stream, float* tflops) {
-  constexpr int kIterations = 8192;
+  constexpr int kIterations = 4096;
   hipEvent_t e0, e1;
   hipError_t err = hipEventCreate(&e0);
   if (err != hipSuccess) return err;
@@ -94,7 +96,7 @@ hipError_t run_mfma_probe(int cus, int zeros, int launches, float* sink, hipStre
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (err != hipSuccess) return err;
-  const double flop = (double)launches * cus * kProbeWaves * (double)kIterations * kProbeBlocks * kProbeBlocks * (2.0 * 32 * 32 * 16);
+  const double flop = (double)launches * cus * kProbeWaves * (double)kIterations * kProbeBlocks * kProbeBlocks * (2.0 * 16 * 16 * 32);
   *tflops = (float)(flop / ((double)ms * 1e-3) / 1e12);
   return hipSuccess;
 }
