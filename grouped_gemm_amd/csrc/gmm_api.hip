@@ -35,6 +35,8 @@ using gg::Short;
 using gg::Small;
 using gg::SmallSquare;
 using gg::Wide;
+using gg::ShortRaggedDepth;
+using gg::SmallRaggedDepth;
 using gg::WideRaggedDepth;
 
 thread_local char g_err[512] = "";
@@ -275,7 +277,7 @@ Route classify(const gg_gmm_args& g) {
   // stores.  Along the depth (rows of a, and of b stored transposed; not in the weight-gradient
   // layout, where both operands run along their widths) such a chunk would add the next row's
   // first values to the sums: a kernel variant clears them in LDS before the slice is multiplied
-  // (WideRaggedDepth; plain rows only, no row indices).
+  // (WideRaggedDepth and its like; plain rows only, no row indices).
   const bool aligned = hidden_in % 8 == 0 && hidden_out % 8 == 0 && (r.address_bits & 15) == 0;
   r.relaxed = !aligned && r.elem_bytes == 2 && !swiglu && !g.accumulate_f32 && (r.address_bits & 3) == 0 &&
               hidden_out % 2 == 0 && hidden_in % 2 == 0;
@@ -377,6 +379,9 @@ bool has_shape(const gg_gmm_args& g, const Route& r, int id) {
 // 13.4 / 12.5 / 11.9; 16 x 200, 3072 -> 768 (348, 99): 38.3 / 32.8 / 35.3; 32 x 128, 2048 -> 768 (480, 144): 30.4 /
 // 29.8 / 32.7; 16 x 256, 2048 -> 1024 (576, 160): 31.2 / 30.8 / 38.8; 64 x 64, 1024 -> 1024 (768, 256): 28.1 / 26.8 /
 // 42.2; 32 x 250, 1024 -> 1024 (1256, 312): 30.2 / 32.6 / 42.3; 32 x 128, 768 -> 2048 (1280, 384): 24.3 / 29.9 / 36.9.
+// Depths that are even but no multiples of 8 go by the same lines.  Full tiles / these, us: 28 Zipf (1.2) groups, 5434 rows, 13374 -> 272
+// (short): 182 / 130, b stored transposed 201 / 174; 64 x 16, 6402 -> 518: 128 / 105; 128 x 2, 2046 -> 5462: 472 / 403; 32 x 94, 770 -> 2050:
+// 34.1 / 32.1; small ones: 8 x 187, 1022 -> 1030: 16.2 / 12.7, in short ones 18.1; 4 x 75, 130 -> 262: 8.8 / 6.7 and 9.2.
 // (The line of one round of short tiles is not sharp: 5 x 409, 272 -> 3520 (952, 252), b stored transposed: 16.7 / 17.8.)
 // Weight gradients: small tiles up to two rounds of them.  Wide / small, groups of even and of Zipf (0.8)
 // depths: 8 x 512 rows, 512 x 1024 (256 small tiles): 19.4 / 12.4 and 30.8 / 17.3; 16 x 512, 768 x 640 (480): 19.4 /
@@ -402,7 +407,6 @@ constexpr int64_t kDeepProduct = 6144;       // weights are pulled through short
 constexpr int64_t kDeepForSharing = 3072;    // small tiles one to a compute unit
 
 TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
-  if (r.ragged_depth) return shape_of<WideRaggedDepth>();
   const int halves = g.epilogue == GG_EPILOGUE_SWIGLU ? 2 : 1;   // of a tile's width: gate and up
   if (g.trans_a) {
     const int64_t small_tiles = expected_tiles(g, SmallSquare::BM, SmallSquare::BN);
@@ -418,11 +422,11 @@ TileShape pick_shape(const gg_gmm_args& g, const Route& r) {
   const bool streams_weights = g.tokens <= Small::BM * g.num_groups && g.hidden_in >= kDeepProduct && 2 * short_tiles >= kFullLaunch;
   const int64_t most_small = g.hidden_in >= kDeepForSharing ? kFullLaunch : kFullLaunch * 3 / 2;
   if (has_shape(g, r, Small::kId) && !streams_weights && expected_tiles(g, Small::BM, Small::BN / halves) <= most_small)
-    return shape_of<Small>();
+    return r.ragged_depth ? shape_of<SmallRaggedDepth>() : shape_of<Small>();
   if (has_shape(g, r, Short::kId) && (use_short_shape(g.num_groups, g.tokens, 0) ||
                                       short_tiles <= kFullLaunch))
-    return shape_of<Short>();
-  return shape_of<Wide>();
+    return r.ragged_depth ? shape_of<ShortRaggedDepth>() : shape_of<Short>();
+  return r.ragged_depth ? shape_of<WideRaggedDepth>() : shape_of<Wide>();
 }
 
 // Whether tiles of a call may be cut along the depth: what gg_workspace_bytes_for promises and what a launch is

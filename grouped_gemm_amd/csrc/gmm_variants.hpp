@@ -23,11 +23,15 @@ struct Short {
   static constexpr int kId = 1, BM = 128, BN = 256, WAVES_M = 1, WAVES_N = 4;
   static constexpr bool RAGGED_DEPTH = false;
 };
-// The wide shape for a hidden_in that is even but no multiple of 8, in the layouts whose rows run
+// The wide, the short and the small shape for a hidden_in that is even but no multiple of 8, in the layouts whose rows run
 // along the depth: the kernel then clears, in LDS, what the last 16-byte chunk of a row picks up
-// from the next row (DepthMajor::clear_depth_tail), and cuts no tile along the depth.
+// from the next row (DepthMajor::clear_depth_tail).
 struct WideRaggedDepth : Wide {
   static constexpr int kId = 2;
+  static constexpr bool RAGGED_DEPTH = true;
+};
+struct ShortRaggedDepth : Short {
+  static constexpr int kId = 5;
   static constexpr bool RAGGED_DEPTH = true;
 };
 
@@ -37,6 +41,10 @@ struct WideRaggedDepth : Wide {
 struct Small {
   static constexpr int kId = 3, BM = 64, BN = 128, WAVES_M = 2, WAVES_N = 2;
   static constexpr bool RAGGED_DEPTH = false;
+};
+struct SmallRaggedDepth : Small {
+  static constexpr int kId = 6;
+  static constexpr bool RAGGED_DEPTH = true;
 };
 struct SmallSquare {
   static constexpr int kId = 4, BM = 128, BN = 128, WAVES_M = 2, WAVES_N = 2;

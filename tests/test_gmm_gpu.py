@@ -2810,6 +2810,8 @@ def test_weight_gradients_in_pieces_by_length(oracle, sizes, hin, hout, side, pa
     ("nn", [40, 0, 300, 75], 6402, 264), ("nt", [40, 0, 300, 75], 6402, 264),       # only the depth is no multiple of 8: 101 slices
     ("nn", [33, 90], 6414, 1030), ("nt", [33, 90], 6414, 1030),                     # neither is
     ("nn", [700, 1], 13374, 270), ("nt", [257], 6146, 14),                          # 209 slices; two depth values in the last one
+    ("nn", [40] * 12, 6402, 5462), ("nt", [40] * 12, 6402, 5462),                   # short tiles
+    ("nn", [4096, 200], 6150, 4090), ("nt", [4096, 200], 6150, 4096),               # full tiles, a second round of them cut
     ("nn", [130, 5], 6400, 518), ("nt", [20, 13, 40, 9], 6400, 262),                # only the width
     ("tn", [2900, 40, 0, 7], 138, 266), ("tn", [9000, 300], 520, 270),
 ])
@@ -2828,7 +2830,8 @@ def test_even_sizes_in_depth_pieces(oracle, layout, sizes, hin, hout, dtype):
     b = (torch.randn(b_shape, generator=g) * (t if tn else hin) ** -0.5).to(dtype)
     if not tn:
         a[t // 2, :2] = float("nan")
-    want = oracle.gmm_loop(a, b, bs, trans_a=tn, trans_b=layout == "nt")
+    where = "cuda" if t * hin * hout > 1 << 32 else "cpu"
+    want = oracle.gmm_loop(a.to(where), b.to(where), bs, trans_a=tn, trans_b=layout == "nt").cpu()
     finite = torch.isfinite(want)
     assert int((~finite).sum()) == (0 if tn else hout)
 
@@ -2847,6 +2850,8 @@ def test_even_sizes_in_depth_pieces(oracle, layout, sizes, hin, hout, dtype):
         args = _gmm_args(lib, da, db, c, sizes_on_device, True, t, hin, hout, tn, layout == "nt", workspace=None if use == "none" else ws,
                          dtype=0 if dtype == torch.bfloat16 else 1)
         assert lib.gg_workspace_bytes_for(ctypes.byref(args)) > 0
+        if not tn and hin % 8:
+            assert _tile(lib, args) == ((256, 256) if t > 4000 else (128, 256) if hout == 5462 else (64, 128))
         if use == "off":
             args.workspace += 64
             args.workspace_bytes -= 64
