@@ -34,10 +34,10 @@ PEAK_HBM_GBPS = 8000.0
 # the hash below (kernel_sources_sha16), and is reported only while the sources still have that
 # hash; the summary under profiles/ holds the figures, the commands and the commit.
 _TRAFFIC_KERNEL_SOURCES = ("gmm_kernel.hpp", "gmm_api.hip", "gmm_variants.hpp", "gmm_variants.def", "gmm_variant.hip")
-_TRAFFIC_KERNEL_SHA16 = "87b0d1501df4f7c8"
+_TRAFFIC_KERNEL_SHA16 = "c86646acb4fc393d"
 _TRAFFIC_SOURCE = ("profiles/gmm_kernel_mixtral_w1_hbm_traffic.md and profiles/gmm_kernel_configs_3_4_5_stats_and_traffic.md "
                    "(rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, kernel sources sha16 " + _TRAFFIC_KERNEL_SHA16 +
-                   ", commit d83e76f; profiled once, not in this run)")
+                   ", commit 3664088; profiled once, not in this run)")
 
 
 def kernel_sources_sha16():
@@ -55,10 +55,10 @@ def _traffic(fetch_kib, write_kib):
 
 
 MEASURED_TRAFFIC = {
-    2: {"fwd": _traffic(4016084, 917548), "agrad": _traffic(3316306, 273422), "bgrad": _traffic(2762135, 917521)},
-    3: {"fwd": _traffic(410428, 135174)},
-    4: {"bgrad": _traffic(2756010, 917527)},
-    5: {"fwd": _traffic(4146437, 262172), "agrad": _traffic(4775926, 917592), "bgrad": _traffic(1851736, 7346337)},
+    2: {"fwd": _traffic(4463456, 917582), "agrad": _traffic(3321526, 273642), "bgrad": _traffic(2856366, 917560)},
+    3: {"fwd": _traffic(445579, 135178)},
+    4: {"bgrad": _traffic(2848553, 917566)},
+    5: {"fwd": _traffic(4310785, 262210), "agrad": _traffic(5053021, 917902), "bgrad": _traffic(1851763, 7345855)},
 }
 
 
