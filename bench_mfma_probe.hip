@@ -57,13 +57,15 @@ __global__ __launch_bounds__(kProbeWaves * 64) void mfma_probe_kernel(int iterat
       for (int i = 0; i < kProbeBlocks; ++i)
         // (in assembly: with all 256 accumulation registers in use the compiler would move some of them about in the loop)
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(b[j]), "v"(a[i]));
-    // new operand values every step, as a depth loop would bring them (the elements of four
-    // fragments rotate: register moves only)
-    a[0] = __builtin_shufflevector(a[0], a[0], 1, 2, 3, 4, 5, 6, 7, 0);
-    a[4] = __builtin_shufflevector(a[4], a[4], 1, 2, 3, 4, 5, 6, 7, 0);
-    b[1] = __builtin_shufflevector(b[1], b[1], 1, 2, 3, 4, 5, 6, 7, 0);
-    b[5] = __builtin_shufflevector(b[5], b[5], 1, 2, 3, 4, 5, 6, 7, 0);
-    asm volatile("s_nop 7" : "+v"(a[0]), "+v"(a[4]), "+v"(b[1]), "+v"(b[5]));   // (nothing else keeps them ahead of their readers)
+    // new operand values now and then, as a depth loop would bring them (the elements of four
+    // fragments rotate: register moves only, few enough not to cost time)
+    if (it % 8 == 0) {
+      a[0] = __builtin_shufflevector(a[0], a[0], 1, 2, 3, 4, 5, 6, 7, 0);
+      a[4] = __builtin_shufflevector(a[4], a[4], 1, 2, 3, 4, 5, 6, 7, 0);
+      b[1] = __builtin_shufflevector(b[1], b[1], 1, 2, 3, 4, 5, 6, 7, 0);
+      b[5] = __builtin_shufflevector(b[5], b[5], 1, 2, 3, 4, 5, 6, 7, 0);
+      asm volatile("s_nop 7" : "+v"(a[0]), "+v"(a[4]), "+v"(b[1]), "+v"(b[5]));   // (nothing else keeps them ahead of their readers)
+    }
   }
   asm volatile("s_nop 15\n\ts_nop 15");   // the last instructions' results
   float s = 0.0f;
