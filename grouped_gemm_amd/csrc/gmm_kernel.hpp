@@ -711,11 +711,12 @@ __device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams&
       }
       start += (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
     }
-  // (every wave writes the same values, and reads its own)
+  // (every wave writes the same values)
   s->tile_start[cut] = pieces * per_group;
   s->front_tiles = pieces * per_group;
   s->front_pieces = 0;
   s->cut_groups = cut;
+  __syncthreads();   // (find_tile's lanes read what other lanes have written)
   plan->pieces = 1;   // the last round stays whole: a workgroup has at most one tile to fix
   plan->by_depth = true;
   plan->main_tiles = plan->total = pieces * per_group + (tiles - cut * per_group);

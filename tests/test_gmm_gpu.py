@@ -2761,6 +2761,7 @@ def test_deep_weight_gradients_of_few_tiles(ops, oracle, sizes, hin, hout):
     ([9000, 7000, 5200, 2600, 1300] + [200] * 60, 136, 264, 128, 6 * (8 + 7 + 5 + 3)),            # odd numbers of pieces
     ([5000] * 3 + [0] * 5, 128, 264, 128, 3 * 24),              # every tile with rows
     ([90 + 7 * i for i in range(509)] + [20000, 0, 17000], 64, 72, 128, 8 + 7),   # most groups there can be, 8 to a lane
+    ([20000, 9000, 9000], 264, 520, 128, 15 * (8 + 4 + 4)),     # every group in pieces: nothing follows them
     ([1500] + [100] * 7, 264, 520, 128, 15 * 4),                # 24 slices: the least depth that is cut,
     ([1460] + [100] * 7, 264, 520, 128, 0),                     # and less
     ([30000], 128, 128, 128, 16),                               # the last round's cut is as good
