@@ -437,6 +437,8 @@ bool may_cut_depth(const gg_gmm_args& g, const Route& r, const TileShape& shape)
   // for ragged widths then)
   if (r.generic || (r.ragged_width && r.indexed) || g.num_groups <= 0) return false;
   if (g.flags & (GG_FLAG_WHOLE_TILES | GG_FLAG_ROW_PIECES)) return false;
+  // (callers that bring a workspace to every call may share one where these sizes had no use for it)
+  if ((r.ragged_width || r.ragged_depth) && !(g.flags & GG_FLAG_EVEN_PIECES)) return false;
   const bool scattered = r.indexed || g.epilogue == GG_EPILOGUE_SWIGLU;
   if (scattered && shape.id == Wide::kId) return false;
   const int64_t slice = r.elem_bytes == 1 ? 2 * gg::BK : gg::BK;   // depth elements per slice

@@ -239,7 +239,7 @@ gg_gmm_args Arguments(const torch::Tensor& a, const torch::Tensor& b, const torc
   g.a_num_rows = a.size(0);
   g.c_num_rows = trans_a ? 0 : c.size(0);
   g.b_num_rows = trans_a ? (int32_t)b.size(0) : 0;
-  g.flags = (int32_t)flags | GG_FLAG_FEW_TILES;
+  g.flags = (int32_t)flags | GG_FLAG_FEW_TILES | GG_FLAG_EVEN_PIECES;
   g.stream = static_cast<void*>(stream);
   if (sizes.is_cuda()) g.size_status = SizeStatusWord();
   return g;

@@ -66,6 +66,10 @@ extern "C" {
  * least half of the device idle, up to three times as fast, and groups of unequal depths in pieces of one length (see
  * workspace; sums in another order than without). */
 #define GG_FLAG_FEW_TILES 128
+/* ... another: calls of even hidden sizes that are no multiples of 8 use their workspace too (or the static scratch of
+ * gg_gmm_no_alloc), with all that it asks for: zeroed counters, no calls on it that overlap in time.  Without it
+ * such calls neither read nor write one, whatever it holds. */
+#define GG_FLAG_EVEN_PIECES 256
 
 /*
  * One-time set-up for the current device: checks that it is a gfx950 and raises the LDS limit
@@ -195,7 +199,8 @@ int gg_gmm_bf16_acc_f32(const void* a, const void* b, float* c, const int64_t* b
  *                 initialisation.  GG_WORKSPACE_BYTES serves every call; a smaller workspace
  *                 (at least 4096 + one 256 KiB tile; plain calls on two-byte operands whose
  *                 groups average few rows, see gg_tile_shape: 128 KiB) serves fewer pieces;
- *                 256-byte aligned.  (Calls of even hidden sizes that are no multiples of 8 ignore one that is smaller or off.)
+ *                 256-byte aligned.  Calls of even hidden sizes that are no multiples of 8 use one only with
+ *                 GG_FLAG_EVEN_PIECES, and ignore one that is smaller or off.
  *                 Calls that share a workspace must not overlap in time (same stream is enough).
  *   flags         GG_FLAG_* bits.
  */
@@ -267,8 +272,8 @@ int gg_gmm_keep_gate_up(const gg_gmm_args* args, void* gate_up);
 
 /*
  * Bytes of workspace the call described by `args` can make use of: 0 when no launch of it ever
- * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8 with row indices, or a
- * product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte
+ * cuts tiles along the depth (general kernels, hidden sizes that are no multiples of 8 with row indices or without
+ * GG_FLAG_EVEN_PIECES, or a product too shallow for depth pieces to pay: about 90 depth slices of 64 two-byte or 128 one-byte
  * elements for full tiles, fewer for groups of few rows; the depth of the trans_a layout being what
  * one group could hold, i.e. all rows), GG_WORKSPACE_BYTES otherwise.  Looks at the sizes, flags
  * and pointers' alignment only; args->workspace is ignored.  A caller that keeps workspaces

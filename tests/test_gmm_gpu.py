@@ -2849,7 +2849,7 @@ def test_even_sizes_in_depth_pieces(oracle, layout, sizes, hin, hout, dtype):
         c = buf[2:-2].view(want.shape)
         ws.zero_()
         args = _gmm_args(lib, da, db, c, sizes_on_device, True, t, hin, hout, tn, layout == "nt", workspace=None if use == "none" else ws,
-                         dtype=0 if dtype == torch.bfloat16 else 1)
+                         dtype=0 if dtype == torch.bfloat16 else 1, flags=256)
         assert lib.gg_workspace_bytes_for(ctypes.byref(args)) > 0
         if not tn and hin % 8:
             assert _tile(lib, args) == ((256, 256) if t > 4000 else (128, 256) if hout == 5462 else (64, 128))
@@ -2869,6 +2869,34 @@ def test_even_sizes_in_depth_pieces(oracle, layout, sizes, hin, hout, dtype):
         outs.append(torch.where(finite, got.float(), zero))
         check(outs[-1], torch.where(finite, want.float(), zero), use)
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[4]) and torch.equal(outs[3], outs[4])
+
+
+@pytest.mark.parametrize("layout,sizes,hin,hout", [
+    ("nn", [40, 0, 300, 75], 6402, 264), ("nt", [130, 5], 6402, 262), ("nn", [130, 5], 6400, 518), ("tn", [2900, 40, 0, 7], 138, 266)])
+def test_even_sizes_leave_a_workspace_alone(layout, sizes, hin, hout):
+    # Without GG_FLAG_EVEN_PIECES: neither what a workspace holds (counters that are not zero) nor calls beside it on the
+    # same one can matter, since it is not touched; gg_gmm_no_alloc goes without pieces as well.
+    _announce("even sizes, no pieces", layout, sizes, hin, hout)
+    lib = _c_abi()
+    lib.gg_workspace_bytes_for.argtypes, lib.gg_workspace_bytes_for.restype = [ctypes.c_void_p], ctypes.c_uint64
+    bs, t, tn = torch.tensor(sizes, dtype=torch.int64), sum(sizes), layout == "tn"
+    g = torch.Generator(device="cuda").manual_seed(hin)
+    a = torch.randn(t, hin, device="cuda", generator=g).bfloat16()
+    b_shape = (t, hout) if tn else ((len(sizes), hout, hin) if layout == "nt" else (len(sizes), hin, hout))
+    b = torch.randn(b_shape, device="cuda", generator=g).bfloat16()
+    ws = torch.full((1024 + 256 * 256 * 256,), 0x01010101, dtype=torch.int32, device="cuda")
+    outs = []
+    for entry, workspace in ((lib.gg_gmm, None), (lib.gg_gmm, ws), (lib.gg_gmm_no_alloc, None)):
+        for flags in (0, 128):
+            c = torch.full((len(sizes), hin, hout) if tn else (t, hout), 7.0, dtype=torch.bfloat16, device="cuda")
+            args = _gmm_args(lib, a, b, c, bs, False, t, hin, hout, tn, layout == "nt", workspace=workspace, flags=flags)
+            assert lib.gg_workspace_bytes_for(ctypes.byref(args)) == 0
+            assert entry(ctypes.byref(args)) == 0, lib.gg_last_error()
+            torch.cuda.synchronize()
+            outs.append((flags, c))
+    assert bool((ws == 0x01010101).all())
+    for flags, c in outs:
+        assert torch.equal(c, outs[0][1] if flags == 0 else outs[1][1])
 
 
 @pytest.mark.parametrize("on_device", [False, True])

@@ -273,6 +273,11 @@ def test_workspace_bytes_for_needs_no_device():
     assert want(hidden_in=14336, hidden_out=2048, epilogue=1) == 0
     assert want(hidden_in=14336, flags=1) == 0 and want(hidden_in=14336, flags=4) == 0
     assert want(dtype=2, hidden_in=12288) == full and want(dtype=2, hidden_in=12160) == 0
+    # even sizes that are no multiples of 8: only where the caller says so
+    for sizes in (dict(hidden_in=14334), dict(hidden_in=14336, hidden_out=4094), dict(trans_a=1, hidden_out=4098)):
+        assert want(**sizes) == 0 and want(flags=128, **sizes) == 0 and want(flags=256, **sizes) == full
+        assert want(flags=256 | 1, **sizes) == 0 and want(flags=256, c_row_index=64 * (sizes.get("trans_a") is None), **sizes) == (
+            full if "trans_a" in sizes else 0)
 
 
 def test_workspace_bytes_for_strided_operands():
