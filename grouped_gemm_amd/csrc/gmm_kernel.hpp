@@ -1065,7 +1065,11 @@ struct DepthMajor {
 // s of depth row k sits at segment slot s ^ (k & 7), so the 8 depth rows one byte-wise
 // transposing read touches land in 8 distinct groups of 8 banks.
 constexpr int width_major_bytes(int W, int BK, bool f8) { return W * BK * 2 + (f8 ? 0 : BK / 16 * 64); }
-template <int W, int BK, int NT, bool F8 = false>
+//
+// The offset of a lane's chunk differs from load to load by whole rows only, so ONE_OFFSET holds that of load 0 and adds the rest.  An
+// addition ahead of every load costs full tiles of many slices 3 % (8 x 4096 rows, 4096 x 14336: 2621 us against 2720), and is
+// for the kernel that would spill the offsets: reading, adding and writing fp32 leaves no registers for them.
+template <int W, int BK, int NT, bool F8 = false, bool ONE_OFFSET = false>
 struct WidthMajor {
   static constexpr int CPRW = W / 8;                  // chunks per depth row
   static constexpr int ROWS_PER_INSTR = NT / CPRW;
@@ -1093,7 +1097,7 @@ struct WidthMajor {
   const char* base;      // depth row of the next slice, column 0
   int ld;                // elements between depth rows
   int depth;             // depth rows of the group ahead of the cursor (below 0: past the end)
-  uint32_t voff[NI];     // byte offset of this lane's chunk per load (kOutOfRange past the width)
+  uint32_t voff[ONE_OFFSET ? 1 : NI];   // byte offset of this lane's chunk per load (kOutOfRange past the width)
 
   __device__ __forceinline__ void setup(const char* group_base, int ld_, int depth_, int col0,
                                         int width) {
@@ -1103,7 +1107,7 @@ struct WidthMajor {
     const int tid = threadIdx.x;
     const int krow0 = tid / CPRW, p = tid % CPRW;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
+    for (int i = 0; i < (ONE_OFFSET ? 1 : NI); ++i) {
       const int krow = krow0 + i * ROWS_PER_INSTR;
       const int c = chunk_for_slot(p, krow);
       const int col = col0 + c * 8;
@@ -1124,7 +1128,7 @@ struct WidthMajor {
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int krow = krow0 + i * ROWS_PER_INSTR;
-      static_assert(!F8, "gate | up columns are for two-byte elements");
+      static_assert(!F8 && !ONE_OFFSET, "gate | up columns are for two-byte elements");
       const int c = chunk_for_slot(p, krow);   // 16-byte chunk of the tile row
       const int block = c >> 2;                                        // 32-column block of the tile
       const int out = col0 + (block >> 1) * 32 + (c & 3) * 8;          // output column it belongs to
@@ -1158,7 +1162,13 @@ struct WidthMajor {
   static constexpr int kOffset = row_at(I * ROWS_PER_INSTR);
   template <int I, bool RIGHT_BEHIND>
   __device__ __forceinline__ void load(const Slice& sl) const {
-    load_to_lds_16<RIGHT_BEHIND>(sl.rsrc, voff[I]);
+    if constexpr (ONE_OFFSET) {
+      // (rows of up to 2^22 values: past the width it stays between 2^31 and 2^32, beyond every descriptor)
+      static_assert((uint64_t)(BK - 1) * (F8 ? 1 : 2) * (1 << 22) < kOutOfRange, "");
+      load_to_lds_16<RIGHT_BEHIND>(sl.rsrc, voff[0] + I * ((uint32_t)(ROWS_PER_INSTR * ld) * 2u));
+    } else {
+      load_to_lds_16<RIGHT_BEHIND>(sl.rsrc, voff[I]);
+    }
   }
 };
 
@@ -1600,12 +1610,17 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   static_assert(!KEEP || (!F8 && !INDEXED), "gate | up are kept for two-byte elements and rows in place");
   static_assert(!GATE_UP || NB % 2 == 0, "a wave needs the gate and the up block of its columns");
   constexpr int BNS = GATE_UP ? BN / 2 : BN;   // output columns per tile, what the schedule counts in
+  // fp32 accumulation by reading, adding and writing in full tiles, whose epilogue holds a block row of c (16 values of 16 bytes).  With
+  // every load's offset held beside it 19 registers spill, and each block row begins with a reload that waits for the stores of
+  // the one before.  us with / without: 234 groups, 12160 rows, 1152 x 296: 201 / 186; 49, 7883 rows, 1920 x 8920: 1639 / 1614; 22,
+  // 18760 rows, 960 x 1496: 105 / 101.
+  constexpr bool ONE_OFFSET = EPI == kEpiAccF32 && BM == 256;
   // (width-major tiles of one-byte elements: half as many two-byte elements per depth row, twice
   // the depth rows)
   using ALoad = std::conditional_t<Cfg::A_DEPTH_MAJOR, DepthMajor<BM, BK, NT, INDEXED>,
-                                   WidthMajor<BM * ES / 2, BK_ELEMS, NT, F8>>;
+                                   WidthMajor<BM * ES / 2, BK_ELEMS, NT, F8, ONE_OFFSET>>;
   using BLoad = std::conditional_t<Cfg::B_DEPTH_MAJOR, DepthMajor<BN, BK, NT, false, GATE_UP>,
-                                   WidthMajor<BN * ES / 2, BK_ELEMS, NT, F8>>;
+                                   WidthMajor<BN * ES / 2, BK_ELEMS, NT, F8, ONE_OFFSET>>;
   using AFrag = std::conditional_t<Cfg::A_DEPTH_MAJOR, DepthMajorFrag<BK, WAVES_M, F8>,
                                    std::conditional_t<F8, WidthMajorFrag8<BM, MB, WAVES_M>, WidthMajorFrag<BM, BK, MB, WAVES_M>>>;
   using BFrag = std::conditional_t<Cfg::B_DEPTH_MAJOR, DepthMajorFrag<BK, 1, F8>,

@@ -632,6 +632,19 @@ def _early_loads(lines):
     return early, loads
 
 
+def _code_objects(folder):
+    """llvm-objdump and the device code of the built library, one file per translation unit."""
+    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    copy = folder / "library.so"
+    copy.write_bytes(open(os.path.join(ROOT, "grouped_gemm_amd", "libgrouped_gemm_hip.so"), "rb").read())
+    subprocess.run([objdump, "--offloading", str(copy)], check=True, capture_output=True)
+    objects = [f for f in sorted(folder.iterdir()) if "gfx950" in f.name]
+    assert objects
+    return objdump, objects
+
+
 def test_loads_to_lds_are_late_enough(tmp_path):
     # the check itself ...
     load = "\tbuffer_load_dwordx4 v1, s[8:11], 0 offen lds"
@@ -640,15 +653,7 @@ def test_loads_to_lds_are_late_enough(tmp_path):
         early, loads = _early_loads(["\tv_readfirstlane_b32 s9, v0"] + between + [load])
         assert (len(early), loads) == (bad, 1), between
     # ... and every kernel that was built
-    objdump = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
-    if not os.path.exists(objdump):
-        pytest.skip("no llvm-objdump")
-    library = os.path.join(ROOT, "grouped_gemm_amd", "libgrouped_gemm_hip.so")
-    copy = tmp_path / "library.so"
-    copy.write_bytes(open(library, "rb").read())
-    subprocess.run([objdump, "--offloading", str(copy)], check=True, capture_output=True)
-    objects = [f for f in sorted(tmp_path.iterdir()) if "gfx950" in f.name]
-    assert objects
+    objdump, objects = _code_objects(tmp_path)
     total = 0
     for f in objects:
         text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(f)], check=True, capture_output=True, text=True).stdout
@@ -656,3 +661,16 @@ def test_loads_to_lds_are_late_enough(tmp_path):
         assert not early, (f.name, early[:3])
         total += loads
     assert total > 1000
+
+
+def test_reading_accumulation_keeps_its_registers(tmp_path):
+    """Full tiles that add to fp32 by reading, adding and writing (epilogue 1 of the template's arguments) have no scratch memory: with
+    some, each block row of c began with a reload that waited for all stores of the one before."""
+    objdump, objects = _code_objects(tmp_path)
+    found = {}
+    for f in objects:
+        notes = subprocess.run([objdump.replace("objdump", "readelf"), "--notes", str(f)], check=True, capture_output=True, text=True).stdout
+        for name, scratch in re.findall(r"\.name:\s+(_Z\w+)\n.*?\.private_segment_fixed_size:\s+(\d+)", notes, flags=re.S):
+            found[name] = int(scratch)
+    reading = {name: n for name, n in found.items() if re.search(r"10gmm_kernelILi\dELi2ELi256E(Li\d+E){5}Li1E", name)}
+    assert len(reading) == 4 and not any(reading.values()), reading
