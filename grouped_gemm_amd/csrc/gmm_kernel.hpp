@@ -1640,9 +1640,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // 2779, input gradient 2685 / 2665 / 2675, 256 x 256 NT 1917 / 1897 / 1947, NN 1987 / 1921 / 1930.  Not where
   // tiles are shallow or their launch is bound by memory (weight gradients, tiles of few rows): with loads behind the
   // stores of a tile the first wait of the next one waits for the memory to take the whole tile, without it lets the
-  // stores pass (counters go down in the order of issue): 256 groups x 256 rows, 2048 x 7168: 2555 -> 2502 us.  Nor for fp8: 1431 /
-  // 1420 us with and without.
-  constexpr bool LATE_LOADS = LAYOUT != kTN && BM == 256 && !F8;
+  // stores pass (counters go down in the order of issue): 256 groups x 256 rows, 2048 x 7168: 2555 -> 2502 us.  fp8, ended at 32 and
+  // 36: 8 Zipf (1.2) groups, 22637 rows, 4720 -> 352, one tile to a workgroup: 54.1 / 51.4; 8 x 4096 rows, 4096 -> 14336, NT 1394 / 1399,
+  // 8 x 2048, 4096 -> 3072 NN 174 / 174, 16 x 1024, 2048 -> 2048 NT 68.7 / 68.6.
+  constexpr bool LATE_LOADS = LAYOUT != kTN && BM == 256;
   constexpr int AT_LOAD_END = LATE_LOADS ? 36 : 32;
   constexpr int FIRST_LOADS = LoadSlots<LOADS_PER_STAGE, AT_RELEASE, AT_READY, AT_LOAD_END, 32>::before(32);   // ... by a slice's end
   constexpr int UNITS = MB + NB;    // fragments of one set
