@@ -857,6 +857,63 @@ int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t ti
   return GG_OK;
 }
 
+int gg_debug_pieces(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups, int units,
+                    int partial_tiles, int tile_outputs, int tail_pieces, int32_t* pieces, int32_t* places, int64_t capacity) {
+  if (batch_sizes == nullptr || num_groups < 1 || num_groups > GG_MAX_GROUPS_PER_LAUNCH || tiles_per_group < 1 ||
+      tiles_per_group > (1 << 20) || workgroups < 1 || units < 1 || partial_tiles < 0 || tail_pieces < 1 || pieces == nullptr)
+    return fail(GG_EINVAL, "bad argument");
+  int64_t rows[GG_MAX_GROUPS_PER_LAUNCH];
+  std::copy(batch_sizes, batch_sizes + num_groups, rows);
+  std::sort(rows, rows + num_groups, std::greater<int64_t>());
+  if (rows[num_groups - 1] < 0 || rows[0] >= (int64_t(1) << 31) / num_groups)
+    return fail(GG_EINVAL, "batch_sizes are negative or too large");
+  struct {
+    uint32_t groups, depth[GG_MAX_GROUPS_PER_LAUNCH], upto[GG_MAX_GROUPS_PER_LAUNCH + 1];
+    uint32_t at(uint32_t q) const { return q < groups ? depth[q] : 0; }
+    uint32_t first(uint32_t n) const { return upto[std::min(n, groups)]; }
+  } depths;
+  depths.groups = (uint32_t)num_groups;
+  depths.upto[0] = 0;
+  for (int64_t q = 0; q < num_groups; ++q) {
+    depths.depth[q] = (uint32_t)((rows[q] + gg::BK - 1) / gg::BK);
+    depths.upto[q + 1] = depths.upto[q] + depths.depth[q];
+  }
+  const gg::PieceLaunch launch{(int)(num_groups * tiles_per_group), (int)tiles_per_group, workgroups, units, partial_tiles};
+  auto choose = [&](auto outputs) {   // length in slices, 0: nothing is cut
+    using Costs = gg::PieceCosts<decltype(outputs)::value>;
+    const int deepest = (int)depths.at(0);
+    if (partial_tiles == 0 || deepest < 4 * Costs::SHORTEST) return 0;
+    const float share = ((float)depths.first((uint32_t)num_groups) * launch.per_group + Costs::TILE * launch.tiles) / workgroups;
+    float best = gg::kPiecesPay * gg::uncut_end<Costs::OUT>(depths, launch, tail_pieces, share);
+    int chosen = 0;
+    for (int k = 0; k < gg::kPieceLengths; ++k) {
+      const int n = gg::piece_count<Costs::OUT>(k), length = (deepest + n - 1) / n;
+      int cut = 0, all = 0;
+      for (; gg::is_cut(depths.at((uint32_t)cut), length); ++cut) all += ((int)depths.at((uint32_t)cut) + length - 1) / length;
+      const float end = gg::pieces_end<Costs::OUT>(depths, launch, n, length, cut, all, share);
+      if (end < best) best = end, chosen = length;
+    }
+    return chosen;
+  };
+  const int length = tile_outputs > Small::BM * Small::BN * 2 ? choose(std::integral_constant<int, Wide::BM * Wide::BN>{})
+                                                              : choose(std::integral_constant<int, SmallSquare::BM * SmallSquare::BN>{});
+  int64_t index = 0;
+  for (int64_t q = 0; q < num_groups; ++q) {
+    const uint32_t d = depths.at((uint32_t)q);
+    pieces[q] = length > 0 && gg::is_cut(d, length) ? (int32_t)((d + length - 1) / length) : 0;
+    const int64_t first = index;
+    for (; index < first + pieces[q] * tiles_per_group; ++index) {
+      if (places == nullptr) continue;
+      if (index >= capacity) return fail(GG_EINVAL, "more than %lld pieces", (long long)capacity);
+      const gg::PieceAt at = gg::piece_at((int)index, (int)first, (int)tiles_per_group);
+      const int32_t place[4] = {(int32_t)(q * tiles_per_group) + at.tile, at.piece, pieces[q],
+                                at.slot + at.piece * (int)tiles_per_group};
+      std::copy(place, place + 4, places + 4 * index);
+    }
+  }
+  return GG_OK;
+}
+
 int gg_gmm(const gg_gmm_args* args) {
   if (args == nullptr) return fail(GG_EINVAL, "args is null");
   if (args->struct_bytes != sizeof(gg_gmm_args))

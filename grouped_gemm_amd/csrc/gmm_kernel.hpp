@@ -171,6 +171,70 @@ __host__ __device__ inline DeepCut cut_deep_tiles(const DEPTH& depth, int E, int
   return chosen;
 }
 
+// Pieces of one length instead (GG_FLAG_FEW_TILES): as many of a tile as it has such lengths, so that groups of all depths end
+// together, also where there are few tiles and the deepest are many times as long as the rest (small hidden sizes and many
+// rows).  The deepest groups are cut; those that are no more than half as long again as a piece stay whole.
+// In depth slices of such a tile: a tile's turnover; a fix-up, constant and per piece; a partial tile's way through memory; the shortest
+// piece.
+template <int OUTPUTS>
+struct PieceCosts {
+  static constexpr int OUT = OUTPUTS;
+  static constexpr bool FULL = OUTPUTS > 128 * 128;
+  static constexpr float TILE = FULL ? 4 : 3, FIX = FULL ? 14 : 4, FIX_PIECE = FULL ? 3 : 1.5f, PARTIAL = FULL ? 6 : 3;
+  static constexpr int SHORTEST = FULL ? 16 : 6;
+};
+// The lengths tried: the deepest tile's halves to sixteenths.  (No fifths of full tiles: 56 Zipf (1.2) groups, 19094 rows, 704 x 1376, 5
+// and 3 pieces of the deepest two against 4 and 2: 93.5 us and 91.5.)
+constexpr int kPieceLengths = 8;
+template <int OUTPUTS>
+__host__ __device__ constexpr int piece_count(int k) {
+  return k < 5 ? k + 2 - (PieceCosts<OUTPUTS>::FULL && k == 3 ? 1 : 0) : 4 * (k - 3);
+}
+__host__ __device__ constexpr bool is_cut(uint32_t depth, uint32_t length) { return depth > length + length / 2; }
+// The one with which the launch is expected to end soonest: the longest of the first round (a piece and its fix-up, or the deepest whole
+// tile), and an even share of what is left.  More pieces than compute units: two of them share a unit and take twice as long (7
+// groups of 6377 rows, 12 small tiles each: 3 pieces 31.0 us, 4 of them 36.0; 2 of 20000, 22 each: 5 pieces 44.5, 6 of them 48.3).
+// `depths` is the groups' depths, deepest first: at(q) that of position q (0 behind the last), first(n) the sum of n.
+struct PieceLaunch {
+  int tiles, per_group, grid, units, slots;
+};
+template <int OUTPUTS, typename DEPTHS>
+__host__ __device__ inline float pieces_end(const DEPTHS& depths, const PieceLaunch& of, int n, int length, int cut, int pieces, float share) {
+  using Costs = PieceCosts<OUTPUTS>;
+  const uint32_t front = (uint32_t)pieces * (uint32_t)of.per_group;
+  const int most = of.grid < of.slots ? of.grid : of.slots;
+  const bool fits = (uint64_t)(uint32_t)pieces * of.per_group <= (uint64_t)most && (uint64_t)(uint32_t)cut * of.per_group <= kWsCounterBytes / 4;
+  if (n > 1 && (length < Costs::SHORTEST || cut == 0 || !fits)) return 1e30f;
+  const float whole = (float)depths.at(cut) + Costs::TILE;
+  const float piece = cut > 0 ? ((int)front > of.units ? 2.0f : 1.0f) * length + Costs::FIX + Costs::FIX_PIECE * n : 0.0f;
+  float end = piece > whole ? piece : whole;
+  if (of.tiles - cut * of.per_group + (int)front > of.grid) {
+    // what follows: the share of all, less that of the first round (the pieces and whole tiles for the workgroups left)
+    const uint32_t to = (uint32_t)cut + (uint32_t)(of.grid - (int)front) / of.per_group;
+    const float after = share - Costs::TILE + (Costs::PARTIAL * pieces - (float)depths.first(to)) * of.per_group / of.grid;
+    end += after > 0 ? after : 0.0f;
+  }
+  return end;
+}
+// ... and of a launch as it is: whole tiles, or all of them in `tail` pieces.
+template <int OUTPUTS, typename DEPTHS>
+__host__ __device__ inline float uncut_end(const DEPTHS& depths, const PieceLaunch& of, int tail, float share) {
+  using Costs = PieceCosts<OUTPUTS>;
+  if (tail <= 1) return pieces_end<OUTPUTS>(depths, of, 1, 0, 0, 0, share);
+  return (of.tiles * tail > of.units ? 2.0f : 1.0f) * (float)depths.at(0) / tail + Costs::FIX + Costs::FIX_PIECE * tail;
+}
+// (a change has to pay by a tenth: 6 groups of 6000 rows, 8 small tiles each, stay in 4 pieces: 25.7 us, in 5 26.7)
+constexpr float kPiecesPay = 0.9f;
+// Index t of the pieces of one group's tiles, the first of which is `first`: first all tiles' first pieces, then all their second ones
+// (neighbours share rows of both operands).
+struct PieceAt {
+  int piece, tile, slot;   // which piece of which tile of the group; place of that tile's first partial tile, the others are per_group apart
+};
+__host__ __device__ inline PieceAt piece_at(int t, int first, int per_group) {
+  const int piece = (t - first) / per_group, slot = t - piece * per_group;
+  return PieceAt{piece, slot - first, slot};
+}
+
 // The last round of a persistent grid is filled only partly: `tiles % grid` workgroups have a
 // tile, the others idle.  When that rest is at most half of the grid, each of its tiles is cut
 // into pieces that go to different workgroups.  With a workspace (and a deep product) the cut
@@ -624,102 +688,106 @@ __device__ __forceinline__ void plan_deep_tiles(Sched* s, const GmmParams& p, in
   plan->main_tiles = plan->total = front * pieces + (tiles - front);
 }
 
-// ... and with kFlagPiecesByLength: pieces of about one length, as many of a tile as it has such lengths, so that groups of
-// all depths end together, also where there are few tiles and the deepest are many times as long as the rest (small
-// hidden sizes and many rows).  The length is one of the deepest tile's halves to sixteenths, the one with which the launch
-// is expected to end soonest: the longest of the first round (a piece and its fix-up, or the deepest whole tile) and an even share
-// of what is left, in depth slices.  us per launch, plan_deep_tiles / this one:
-// 21 Zipf (1.2) groups, 51204 rows, 128 x 560: 45.4 / 34.3; 56, 19094 rows, 704 x 1376: 124 / 92; 64, 49152 rows, 2048 x 1408: 320 /
-// 314; 7 even groups, 44642 rows, 360 x 424: 37.3 / 33.2; 15, 40804, 416 x 136 (cut as the last round by both): 24.1 / 24.5.
-template <int OUTPUTS>
-struct PieceCosts {   // in slices: a tile's turnover, a fix-up (constant, per piece), a partial tile's way through memory
-  static constexpr bool FULL = OUTPUTS > 128 * 128;
-  static constexpr float TILE = FULL ? 4 : 3, FIX = FULL ? 14 : 4, FIX_PIECE = FULL ? 3 : 1.5f, PARTIAL = FULL ? 6 : 3;
-  static constexpr int SHORTEST = FULL ? 16 : 6;   // piece
+// x / y, rounded up, for small quotients
+__device__ __forceinline__ uint32_t ceil_quotient(uint32_t x, uint32_t y) {
+  uint32_t q = (uint32_t)((float)x * __builtin_amdgcn_rcpf((float)y));   // (one off at most)
+  q += q * y < x ? 1 : 0;
+  q += q * y < x ? 1 : 0;
+  return q - (q > 0 && (q - 1) * y >= x ? 1 : 0);
+}
+__device__ __forceinline__ uint32_t wave_sums(uint32_t x) {
+  return wave_scan(x, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t lane_of(uint32_t x, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)x, lane); }
+
+// What a launch's groups hold, in LDS: depth[q] of position q of the order, upto[q] the sum of those before it.
+struct GroupDepths {
+  const uint32_t *depth, *upto;
+  uint32_t groups, sum;
+  __device__ __forceinline__ uint32_t at(uint32_t q) const { return q < groups ? depth[q] : 0; }
+  __device__ __forceinline__ uint32_t first(uint32_t n) const { return n < groups ? upto[n] : sum; }
 };
-__device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(x, [](uint32_t a, uint32_t b) { return a + b; }), 63);
-}
-__device__ __forceinline__ uint32_t wave_max(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(x, [](uint32_t a, uint32_t b) { return a > b ? a : b; }), 63);
-}
-template <int BM, int BN>
-__device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams& p, int grid, int bk, TailPlan* plan) {
-  using Costs = PieceCosts<BM * BN>;
+
+// ... and with kFlagPiecesByLength: pieces of one length (pieces_end).  All lengths are looked at together, one lane each: one after
+// the other, each with sums over the lanes that wait for those before, they were 3 us of every such launch, now 1.  us per launch,
+// plan_deep_tiles / this one: 21 Zipf (1.2) groups, 51204 rows, 128 x 560: 46 / 32; 56, 19094 rows, 704 x 1376: 121 / 90; 64, 49152 rows,
+// 2048 x 1408: 332 / 302; 7 even groups, 44642 rows, 360 x 424: 38.0 / 31.6; 4 of 8483, 128 x 1384: 31.2 / 30.7 (one after the other:
+// 33.0); 2 of 20000, 256 x 1408: 49.7 / 45.5 (51.5); 15, 40804, 416 x 136 (cut as the last round by both): 24.5 / 23.8.
+// `scratch` is for 2 kMaxGroups words (the tile buffers are not in use yet); ends with a barrier.
+template <int BM, int BN, int WGS_PER_CU>
+__device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams& p, int grid, int bk, uint32_t* scratch, TailPlan* plan) {
   const int E = p.num_groups, tiles = s->tile_start[E], per_group = s->group_tiles, lane = threadIdx.x & 63;
   if (E == 0 || tiles == 0 || p.ws_slots <= 0 || (p.flags & (kFlagWholeTiles | kFlagRowPieces))) return;
-  // (every wave works out the same plan; each lane has up to 8 positions of the order, 64 apart)
+  // (every wave works out the same plan and writes the same words)
+  uint32_t *depth = scratch, *upto = scratch + kMaxGroups;
   const int per = (E + 63) >> 6;
-  uint32_t depth[8], sum = 0;
+  auto depth_of = [&](int q) { return q < E ? (uint32_t)(s->rows[s->order[q]] + bk - 1) / bk : 0u; };
+  const uint32_t deepest = (uint32_t)uniform((int)depth_of(0));
+  if (deepest < 4 * PieceCosts<BM * BN>::SHORTEST) return;
+  // lanes 0 .. kPieceLengths - 1: a length each
+  const int mine = lane < kPieceLengths ? lane : kPieceLengths - 1, n = piece_count<BM * BN>(mine);
+  const uint32_t length = (deepest + n - 1) / n;
+  uint32_t cut = 0, parts[kPieceLengths], sum = 0;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    depth[i] = 0;
-    if (i < per && lane + 64 * i < E) depth[i] = (uint32_t)(s->rows[s->order[lane + 64 * i]] + bk - 1) / bk;
-    sum += depth[i];
-  }
-  const int deepest = __builtin_amdgcn_readfirstlane((int)depth[0]);
-  if (deepest < 4 * Costs::SHORTEST) return;
-  const float share = ((float)wave_sum(sum) * per_group + Costs::TILE * tiles) / grid;
-  // What follows the first round when the first `from` positions are cut: the share of all, less that of the first round (those and as many
-  // whole tiles as there are workgroups left).
-  auto rest = [&](uint32_t from, uint32_t pieces) {
-    const uint32_t to = from + (uint32_t)max(0, grid - (int)pieces * per_group) / per_group;
-    uint32_t first = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < per) first += (uint32_t)(lane + 64 * i) < to ? depth[i] : 0;
-    return fmaxf(0.0f, share - Costs::TILE + (Costs::PARTIAL * pieces - (float)wave_sum(first)) * per_group / grid);
-  };
-  // as it is: the tiles of a launch of one round may be cut already
-  const bool one_round = tiles <= grid;
-  float best = plan->by_depth && plan->main_tiles == 0 ? deepest / plan->pieces + Costs::FIX + Costs::FIX_PIECE * plan->pieces
-                                                       : deepest + Costs::TILE + (one_round ? 0.0f : rest(0, 0));
-  best *= 15.0f / 16.0f;
-  int length = 0, cut = 0, pieces = 0;
+  for (int k = 0; k < kPieceLengths; ++k) parts[k] = 0;
 #pragma unroll 1
-  for (int n = 2; n <= kMaxDepthPieces; n += n < 4 ? 1 : (n < 8 ? 2 : 4)) {
-    const int l = (deepest + n - 1) / n;
-    if (l < Costs::SHORTEST) break;
-    const uint32_t above = (uint32_t)(l + l / 2);
-    uint32_t t = 0, c = 0, longest = 0;
+  for (int i = 0; i < per; ++i) {
+    const int q = lane + 64 * i;
+    const uint32_t d = depth_of(q), up = wave_sums(d);
+    depth[q] = d;
+    upto[q] = sum + up - d;
+    sum += lane_of(up, 63);
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < per) {
-        const bool is_cut = depth[i] > above;
-        t += is_cut ? (depth[i] + l - 1) / l : 0;
-        c += is_cut ? 1 : 0;
-        longest = is_cut || depth[i] < longest ? longest : depth[i];
-      }
-    t = wave_sum(t), c = wave_sum(c), longest = wave_max(longest);
-    if ((uint64_t)t * per_group > (uint64_t)min(grid, p.ws_slots) || (uint64_t)c * per_group > kWsCounterBytes / 4) continue;
-    float end = fmaxf(l + Costs::FIX + Costs::FIX_PIECE * n, longest + Costs::TILE);
-    if (tiles - (int)c * per_group + (int)t * per_group > grid) end += rest(c, t);
-    if (c > 0 && end < best) best = end, length = l, cut = (int)c, pieces = (int)t;
-  }
-  if (length == 0) return;
-  __syncthreads();   // (tile_start has been read by every wave)
-  uint32_t start = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-    if (i < per) {
-      const int q = lane + 64 * i;
-      const uint32_t mine = q < cut ? (depth[i] + length - 1) / length : 0;
-      const uint32_t upto = wave_scan(mine, [](uint32_t a, uint32_t b) { return a + b; });
-      if (q < cut) {
-        s->tile_start[q] = (int)(start + upto - mine) * per_group;
-        s->runt_start[q] = (int)mine;
-      }
-      start += (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+    for (int k = 0; k < kPieceLengths; ++k) {
+      const uint32_t l = lane_of(length, k);
+      const bool yes = is_cut(d, l);
+      const uint32_t all = (uint32_t)__popcll(__ballot(yes));
+      cut += mine == k ? all : 0;
+      parts[k] += yes ? ceil_quotient(d, l) : 0;
     }
-  // (every wave writes the same values)
-  s->tile_start[cut] = pieces * per_group;
-  s->front_tiles = pieces * per_group;
-  s->front_pieces = 0;
-  s->cut_groups = cut;
-  __syncthreads();   // (find_tile's lanes read what other lanes have written)
-  plan->pieces = 1;   // the last round stays whole: a workgroup has at most one tile to fix
-  plan->by_depth = true;
-  plan->main_tiles = plan->total = pieces * per_group + (tiles - cut * per_group);
+  }
+  uint32_t pieces = 0;
+#pragma unroll
+  for (int k = 0; k < kPieceLengths; ++k) {
+    const uint32_t all = lane_of(wave_sums(parts[k]), 63);
+    pieces = mine == k ? all : pieces;
+  }
+  __syncthreads();   // (all lanes' words are there, and tile_start has been read by every wave)
+  const GroupDepths depths{depth, upto, (uint32_t)E, sum};
+  const PieceLaunch launch{tiles, per_group, grid, grid / WGS_PER_CU, p.ws_slots};
+  const float share = ((float)sum * per_group + PieceCosts<BM * BN>::TILE * tiles) / grid;
+  const float end = pieces_end<BM * BN>(depths, launch, n, (int)length, (int)cut, (int)pieces, share);
+  float best = kPiecesPay * uncut_end<BM * BN>(depths, launch, plan->by_depth && plan->main_tiles == 0 ? plan->pieces : 1, share);
+  int chosen = -1;
+#pragma unroll
+  for (int k = 0; k < kPieceLengths; ++k) {
+    const float at_k = __builtin_bit_cast(float, lane_of(__builtin_bit_cast(uint32_t, end), k));
+    chosen = at_k < best ? k : chosen;
+    best = fminf(best, at_k);
+  }
+  chosen = uniform(chosen);
+  if (chosen >= 0) {
+    const int l = (int)lane_of(length, chosen), groups = (int)lane_of(cut, chosen), all = (int)lane_of(pieces, chosen);
+    uint32_t start = 0;
+#pragma unroll 1
+    for (int i = 0; 64 * i < groups; ++i) {
+      const int q = lane + 64 * i;
+      const uint32_t of_tile = q < groups ? ceil_quotient(depth[q], l) : 0, up = wave_sums(of_tile);
+      if (q < groups) {
+        s->tile_start[q] = (int)(start + up - of_tile) * per_group;
+        s->runt_start[q] = (int)of_tile;
+      }
+      start += lane_of(up, 63);
+    }
+    s->tile_start[groups] = all * per_group;
+    s->front_tiles = all * per_group;
+    s->front_pieces = 0;
+    s->cut_groups = groups;
+    plan->pieces = 1;   // the last round stays whole: a workgroup has at most one tile to fix
+    plan->by_depth = true;
+    plan->main_tiles = plan->total = all * per_group + (tiles - groups * per_group);
+  }
+  __syncthreads();   // (find_tile's lanes read what other lanes have written; the scratch is free again)
 }
 
 // NN and NT layouts with many short groups: the groups by ascending number of tile rows, groups
@@ -1429,12 +1497,12 @@ __device__ __forceinline__ TileInfo find_tile(const Sched* sched, const GmmParam
             q += __popcll(__ballot(at < groups && sched->tile_start[at + 1] <= t));
           }
         q = uniform(q);
-        const int first = uniform(sched->tile_start[q]);
+        const PieceAt at = piece_at(t, uniform(sched->tile_start[q]), per_group);
         pieces = uniform(sched->runt_start[q]);
-        piece = (t - first) / per_group;
-        ti.slot = t - piece * per_group;
+        piece = at.piece;
+        ti.slot = at.slot;
         ti.slots_apart = per_group;
-        t = q * per_group + (ti.slot - first);
+        t = q * per_group + at.tile;
         ti.rank = t;
       } else {
         t = t - front_tiles + groups * per_group;
@@ -1679,7 +1747,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   if constexpr (!DEPTH_PIECES) plan.by_depth = false;   // (known at compile time: no depth-piece code is kept)
   if constexpr (LAYOUT == kTN && DEPTH_PIECES) {
     if (p.flags & kFlagPiecesByLength) {
-      plan_pieces_by_length<BM, BN>(sched, p, G, BK_ELEMS, &plan);
+      plan_pieces_by_length<BM, BN, PART::WGS_PER_CU>(sched, p, G, BK_ELEMS, reinterpret_cast<uint32_t*>(smem), &plan);
     } else {
       plan_deep_tiles<BM, BN>(sched, p, G, BK_ELEMS, &plan);
     }

@@ -383,6 +383,14 @@ int gg_debug_pair(const gg_gmm_args* first, const gg_gmm_args* second, const int
 int gg_debug_deep_cut(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups,
                       int partial_tiles, int tile_outputs, int* pieces, int* tiles);
 
+/* ... and with GG_FLAG_FEW_TILES, on `workgroups` workgroups of `units` compute units: pieces[q] is the number of pieces of each tile of the
+ * q-th deepest group (0: it stays whole).  tail_pieces: what every tile is cut into in a launch of one round where this changes nothing
+ * (1: whole).  places, where not null, receives four numbers for each of the pieces in the order in which they are handed out, `capacity`
+ * of them at most: the tile (q tiles_per_group + index in its group), the piece, the tile's number of pieces, the place of its
+ * partial tile. */
+int gg_debug_pieces(const int64_t* batch_sizes, int64_t num_groups, int64_t tiles_per_group, int workgroups, int units,
+                    int partial_tiles, int tile_outputs, int tail_pieces, int32_t* pieces, int32_t* places, int64_t capacity);
+
 /* Message of the last failure on the calling thread ("" if none). */
 const char* gg_last_error(void);
 

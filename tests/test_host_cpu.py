@@ -534,6 +534,66 @@ def test_deep_tiles_are_cut_to_end_the_launch_soonest():
     assert lib.gg_debug_deep_cut(None, ctypes.c_int64(1), ctypes.c_int64(1), 256, 0, small, None, None) == -1
 
 
+def _pieces(lib, rows, per_group, workgroups, units, partial_tiles, tile_outputs, tail=1):
+    sizes, pieces = (ctypes.c_int64 * len(rows))(*rows), (ctypes.c_int32 * len(rows))()
+    places = (ctypes.c_int32 * (4 * workgroups))()
+    assert lib.gg_debug_pieces(sizes, ctypes.c_int64(len(rows)), ctypes.c_int64(per_group), workgroups, units, partial_tiles,
+                               tile_outputs, tail, pieces, places, ctypes.c_int64(workgroups)) == 0
+    return list(pieces), np.array(places[:4 * per_group * sum(pieces)]).reshape(-1, 4)
+
+
+def test_pieces_of_one_length():
+    """How a weight gradient is cut into pieces of one length: every piece once, in its own place, within what there is."""
+    lib = ctypes.CDLL(HIP_LIB)
+    small, full = 128 * 128, 256 * 256
+    # pieces per tile, deepest group first (in brackets us of the launch, and of others)
+    assert _pieces(lib, [8483] * 4, 11, 512, 256, 1024, small, 8)[0] == [5] * 4              # (29.8; 4: 30.3, 3: 34.5)
+    assert _pieces(lib, [20000] * 2, 22, 512, 256, 1024, small, 8)[0] == [5] * 2             # (44.5; 4: 49, 6: 48.3)
+    assert _pieces(lib, [6377] * 7, 12, 512, 256, 1024, small, 4)[0] == [3] * 7              # (31.0; 2: 36.5, 4: 36.0)
+    assert _pieces(lib, [17150, 7470, 4590, 3250, 2490, 2000, 1660, 1390], 8, 512, 256, 1024, small)[0] == [12, 6, 4, 3, 2, 0, 0, 0]
+    assert _pieces(lib, [6000] * 6, 8, 512, 256, 1024, small, 4)[0] == [0] * 6              # the last round's cut is as good (25.7; 5: 26.7)
+    assert _pieces(lib, [4000] * 4, 16, 512, 256, 1024, small, 4)[0] == [0] * 4
+    zipf = [5696, 2432, 1600, 1088, 832, 704, 640, 512] + [300] * 48
+    assert _pieces(lib, zipf, 18, 256, 256, 256, full)[0][:3] == [4, 2, 0]                   # (91.5; 5 and 3: 93.5)
+    assert _pieces(lib, [3000] * 4, 64, 512, 256, 0, small)[0] == [0] * 4                    # nowhere to put partial tiles
+    assert _pieces(lib, [1500, 20], 4, 512, 256, 1024, small)[0][0] > 1 and _pieces(lib, [1500], 4, 256, 256, 1024, full)[0] == [0]
+    assert _pieces(lib, [0, 0], 4, 512, 256, 1024, small)[0] == [0, 0]
+    rng = np.random.default_rng(5)
+    seen = dict(all_cut=0, some_cut=0, none=0, few_slots=0)
+    for trial in range(600):
+        groups = int(rng.integers(1, 513 if trial % 4 == 0 else 40))
+        rows = (rng.pareto(0.7, groups) * rng.choice([60, 600, 4000])).clip(0, 2**31 // groups - 1).astype(int).tolist()
+        if trial % 3 == 0:
+            rows = rng.integers(4000, 12000, groups := int(rng.integers(1, 12))).tolist()
+        tile_outputs = int(rng.choice([small, full]))
+        units = 256
+        workgroups = units * (2 if tile_outputs == small else 1)
+        per_group, slots = int(rng.choice([1, 4, 11, 30, 120])), int(rng.choice([1, 20, 100, 256, 1024]))
+        pieces, places = _pieces(lib, rows, per_group, workgroups, units, slots, tile_outputs, int(rng.choice([1, 1, 2, 4])))
+        depths = [-(-r // 64) for r in sorted(rows, reverse=True)]
+        cut = sum(n > 0 for n in pieces)
+        assert all(n > 0 for n in pieces[:cut])                    # the deepest groups
+        assert cut * per_group <= 1024                            # one arrival counter per tile
+        assert len(places) <= min(workgroups, slots)              # at most one piece to a workgroup, a place for each
+        assert all(2 <= n <= 17 for n in pieces[:cut])
+        if cut:
+            length = max(-(-d // n) for d, n in zip(depths, pieces[:cut]))
+            assert length >= (6 if tile_outputs == small else 16)
+            assert all(d > 1.5 * (length - 1) for d in depths[:cut]) and all(d < 2 * length + 2 for d in depths[cut:])
+            tile, piece, of, slot = places.T
+            assert len({(t, p) for t, p in zip(tile, piece)}) == len(places) and sorted(slot) == list(range(len(places)))
+            assert (of == np.array(pieces)[tile // per_group]).all() and (piece < of).all() and tile.max() < cut * per_group
+        seen["all_cut"] += cut == groups
+        seen["none"] += cut == 0
+        seen["some_cut"] += 0 < cut < groups
+        seen["few_slots"] += cut > 0 and len(places) > slots // 2
+    assert all(n >= 40 for n in seen.values()), seen
+    bad = (ctypes.c_int32 * 4)()
+    assert lib.gg_debug_pieces(None, ctypes.c_int64(1), ctypes.c_int64(1), 512, 256, 1, small, 1, bad, None, ctypes.c_int64(0)) == -1
+    one = (ctypes.c_int64 * 1)(9000)
+    assert lib.gg_debug_pieces(one, ctypes.c_int64(1), ctypes.c_int64(4), 512, 256, 1024, small, 1, bad, (ctypes.c_int32 * 4)(), ctypes.c_int64(1)) == -1
+
+
 # ----------------------------------------------------------------- workloads
 
 def test_workload_generators():
