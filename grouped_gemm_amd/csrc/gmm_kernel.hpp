@@ -1701,8 +1701,10 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
   // (released at 8, 10, 13 and 14, ready at 24, 22, 19 and 18, us: 8 x 4096 rows, 4096 -> 14336, NN 2913 / 2943 / 2986 / 2978;
   // 256 x 256, 7168 -> 2048, NT 2079 / 2030 / 2100 / 2160).  Tiles of few rows, whose launches are bound by latency: earlier still
   // (6 and 26 against 8 and 24: 16 x 256 rows, 3072 -> 768: 32.8 / 34.1, NT 33.8 / 35.7; 32 x 128, 2048 -> 768: 28.5 / 28.4;
-  // against 10 and 22: 36.2, 37.7, 31.9).
-  constexpr bool EARLY = LAYOUT != kTN && BM < 256 && !F8;
+  // against 10 and 22: 36.2, 37.7, 31.9).  Not short tiles of the NN layout, which mostly stream weights: 128 groups x 30 rows, 4096 ->
+  // 2048: 358 / 351, 16 rows: 353 / 345; 64 x 50, 7168 -> 2048: 314 / 308; 8 x 40, 4096 -> 14336: 170 / 168; but as the first of a pair,
+  // which is bound by latency again (16 x 200, 1024 -> 3072 transposed, forward and both gradients: 104 / 106).
+  constexpr bool EARLY = LAYOUT != kTN && BM < 256 && !F8 && !(LAYOUT == kNN && BM == 128 && !PART::FIRST);
   constexpr int AT_READ_END = EARLY ? 6 : 8, AT_RELEASE = AT_READ_END, AT_READY = EARLY ? 26 : 24;
   // Loads that reach into the next slice are steadier: ended at 32, 36 and 40, us: 8 x 4096 rows, 4096 -> 14336, NN 2743 / 2749 /
   // 2779, input gradient 2685 / 2665 / 2675, 256 x 256 NT 1917 / 1897 / 1947, NN 1987 / 1921 / 1930.  Not where
