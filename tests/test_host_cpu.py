@@ -663,33 +663,69 @@ def test_traceable_operator_shapes_without_a_device():
 
 
 def _early_loads(lines):
-    """Loads straight to LDS in a disassembly that come too soon: less than five wait states behind a vector instruction
-    that writes a word of their descriptor (the hardware does not wait for it, and the compiler does not look into the
-    assembly that these loads are written in), or right behind the write of m0 that aims them."""
-    code = []
+    """Loads straight to LDS in a disassembly (branch targets as labels) that are not what they were written as, on any way that leads to
+    them: less than five wait states behind a vector instruction that writes a word of their descriptor (the hardware does not wait for it,
+    and the compiler does not look into the assembly that these loads are written in), right behind the write of m0 that aims
+    them, aimed by another instruction than theirs, or by one that has aimed a load already."""
+    functions, code, labels = [], [], {}
     for line in lines:
         m = re.match(r"\s+([a-z]\w+)\s*(.*?)\s*(//.*)?$", line)
         if m:
             code.append((m.group(1), m.group(2)))
-    early, loads = [], 0
-    for i, (op, args) in enumerate(code):
-        if op != "buffer_load_dwordx4" or not args.endswith(" lds"):
-            continue
-        loads += 1
-        first, last = map(int, re.search(r", s\[(\d+):(\d+)\]", args).groups())
-        waited, aimed, k = 0, None, i - 1
-        while k >= 0 and (waited < 5 or aimed is None):
-            before, to = code[k]
-            m = re.match(r"s(\d+)\b", to)
-            if waited < 5 and before.startswith("v_read") and m and first <= int(m.group(1)) <= last:
-                early.append(code[k:i + 1])
-            if aimed is None and re.match(r"m0\b", to):
-                aimed = waited
-            waited += 1 + int(to, 0) if before == "s_nop" else 1
-            k -= 1
-        if aimed == 0:
-            early.append(code[i - 1:i + 1])
-    return early, loads
+        elif m := re.match(r"(?:[0-9a-f]+ )?<(L\d+)>:", line):
+            labels[m.group(1)] = len(code)
+        elif re.match(r"[0-9a-f]+ <", line):
+            functions.append((code, labels))
+            code, labels = [], {}
+    functions.append((code, labels))
+    bad, loads = [], 0
+    for code, labels in functions:
+        jumps = {}
+        for i, (op, args) in enumerate(code):
+            if op == "s_branch" or op.startswith("s_cbranch"):
+                jumps.setdefault(labels[args.split()[0]], []).append(i)
+
+        def ways_to(i):
+            falls = i > 0 and code[i - 1][0] not in ("s_branch", "s_endpgm", "s_setpc_b64")
+            return jumps.get(i, []) + ([i - 1] if falls else [])
+
+        def to_lds(op, args):
+            return op == "buffer_load_dwordx4" and args.endswith(" lds")
+
+        def wrong(i):
+            first, last = map(int, re.search(r", s\[(\d+):(\d+)\]", code[i][1]).groups())
+            todo, least = [(k, 0, False) for k in ways_to(i)], {}
+            if not todo:
+                return True
+            while todo:
+                k, waited, aimed = todo.pop()
+                if least.get((k, aimed), 9) <= waited:
+                    continue
+                least[k, aimed] = waited
+                op, args = code[k]
+                m = re.match(r"s(?:(\d+)|\[(\d+):(\d+)\])", args) if op.startswith("v_") else None
+                if m and waited < 5 and int(m.group(1) or m.group(2)) <= last and int(m.group(1) or m.group(3)) >= first:
+                    return True
+                if not aimed and re.match(r"m0\b", args):
+                    if op != "s_add_u32" or waited == 0:
+                        return True
+                    aimed = True
+                elif not aimed and to_lds(op, args):
+                    return True
+                waited = min(waited + (1 + int(args, 0) if op == "s_nop" else 1), 5)
+                if waited < 5 or not aimed:
+                    ways = ways_to(k)
+                    if not ways and not aimed:
+                        return True
+                    todo += [(way, waited, aimed) for way in ways]
+            return False
+
+        for i, (op, args) in enumerate(code):
+            if to_lds(op, args):
+                loads += 1
+                if wrong(i):
+                    bad.append(code[max(i - 8, 0):i + 1])
+    return bad, loads
 
 
 def _code_objects(folder):
@@ -709,14 +745,26 @@ def test_loads_to_lds_are_late_enough(tmp_path):
     # the check itself ...
     load = "\tbuffer_load_dwordx4 v1, s[8:11], 0 offen lds"
     aim = "\ts_add_u32 m0, s3, 16"
-    for between, bad in [([aim, "\ts_nop 0"], 1), ([aim, "\ts_nop 2"], 1), ([aim, "\ts_nop 3"], 0), (["\ts_nop 4", aim], 1)]:
-        early, loads = _early_loads(["\tv_readfirstlane_b32 s9, v0"] + between + [load])
-        assert (len(early), loads) == (bad, 1), between
+    word = "\tv_readfirstlane_b32 s9, v0"
+    for code, bad in [
+            ([word, aim, "\ts_nop 0", load], 1), ([word, aim, "\ts_nop 2", load], 1), ([word, aim, "\ts_nop 3", load], 0),
+            (["\tv_readfirstlane_b32 s12, v0", aim, "\ts_nop 0", load], 0), (["\tv_cmp_eq_u32_e64 s[10:11], v0, v1", aim, "\ts_nop 0", load], 1),
+            (["\ts_nop 4", aim, load], 1),                                             # right behind its aim
+            ([aim, "\ts_mov_b32 m0, s4", "\ts_nop 4", load], 1),                        # aimed elsewhere
+            (["\ts_nop 4", load], 1), ([aim, "\ts_nop 0", load, "\ts_nop 0", load], 1),   # not aimed, aimed once for two
+            # the word is written at the end of a loop, far from its beginning in the text, and jumped over in between
+            ([aim, "<L0>:", "\ts_nop 0", load, "\ts_nop 7", aim, word, "\ts_cbranch_scc1 L0"], 1),
+            ([aim, "<L0>:", "\ts_nop 3", load, "\ts_nop 7", aim, word, "\ts_cbranch_scc1 L0"], 0),
+            ([aim, "<L0>:", "\ts_nop 3", load, "\ts_nop 7", "\ts_cbranch_scc1 L0"], 1),   # (aimed for the first time round only)
+            ([word, "\ts_branch L1", "\ts_nop 7", "<L1>:", aim, "\ts_nop 0", load], 1),
+            (["\ts_cbranch_scc0 L1", word, "\ts_nop 4", "\ts_branch L2", "<L1>:", "\ts_nop 0", "<L2>:", aim, "\ts_nop 0", load], 0)]:
+        early, loads = _early_loads(code)
+        assert (len(early), loads) == (bad, sum(line == load for line in code)), code
     # ... and every kernel that was built
     objdump, objects = _code_objects(tmp_path)
     total = 0
     for f in objects:
-        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(f)], check=True, capture_output=True, text=True).stdout
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", "--symbolize-operands", str(f)], check=True, capture_output=True, text=True).stdout
         early, loads = _early_loads(text.splitlines())
         assert not early, (f.name, early[:3])
         total += loads
