@@ -708,11 +708,12 @@ struct GroupDepths {
   __device__ __forceinline__ uint32_t first(uint32_t n) const { return n < groups ? upto[n] : sum; }
 };
 
-// ... and with kFlagPiecesByLength: pieces of one length (pieces_end).  All lengths are looked at together, one lane each: one after
-// the other, each with sums over the lanes that wait for those before, they were 3 us of every such launch, now 1.  us per launch,
-// plan_deep_tiles / this one: 21 Zipf (1.2) groups, 51204 rows, 128 x 560: 46 / 32; 56, 19094 rows, 704 x 1376: 121 / 90; 64, 49152 rows,
-// 2048 x 1408: 332 / 302; 7 even groups, 44642 rows, 360 x 424: 38.0 / 31.6; 4 of 8483, 128 x 1384: 31.2 / 30.7 (one after the other:
-// 33.0); 2 of 20000, 256 x 1408: 49.7 / 45.5 (51.5); 15, 40804, 416 x 136 (cut as the last round by both): 24.5 / 23.8.
+// ... and with kFlagPiecesByLength: pieces of one length (pieces_end).  All lengths are looked at together, eight lanes each: one
+// after the other, each with sums over the lanes that wait for those before, they were 3 us of every such launch.  A lane for each
+// length and every group in a lane took 1 us, and so many scalar registers that others were spilled all over the pair kernels (1.2 us of
+// launches that cut nothing).  us per launch, plan_deep_tiles / this one: 21 Zipf (1.2) groups, 51204 rows, 128 x 560: 46 / 32; 56, 19094
+// rows, 704 x 1376: 124 / 90; 64, 49152 rows, 2048 x 1408: 331 / 310; 7 even groups, 44642 rows, 360 x 424: 38.0 / 30.7; 4 of 8483, 128 x
+// 1384: 31.2 / 30.0; 2 of 20000, 256 x 1408: 49.6 / 44.3; 15, 40804, 416 x 136 (cut as the last round by both): 24.5 / 23.3.
 // `scratch` is for 2 kMaxGroups words (the tile buffers are not in use yet); ends with a barrier.
 template <int BM, int BN, int WGS_PER_CU>
 __device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams& p, int grid, int bk, uint32_t* scratch, TailPlan* plan) {
@@ -724,12 +725,7 @@ __device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams&
   auto depth_of = [&](int q) { return q < E ? (uint32_t)(s->rows[s->order[q]] + bk - 1) / bk : 0u; };
   const uint32_t deepest = (uint32_t)uniform((int)depth_of(0));
   if (deepest < 4 * PieceCosts<BM * BN>::SHORTEST) return;
-  // lanes 0 .. kPieceLengths - 1: a length each
-  const int mine = lane < kPieceLengths ? lane : kPieceLengths - 1, n = piece_count<BM * BN>(mine);
-  const uint32_t length = (deepest + n - 1) / n;
-  uint32_t cut = 0, parts[kPieceLengths], sum = 0;
-#pragma unroll
-  for (int k = 0; k < kPieceLengths; ++k) parts[k] = 0;
+  uint32_t sum = 0;
 #pragma unroll 1
   for (int i = 0; i < per; ++i) {
     const int q = lane + 64 * i;
@@ -737,35 +733,32 @@ __device__ __forceinline__ void plan_pieces_by_length(Sched* s, const GmmParams&
     depth[q] = d;
     upto[q] = sum + up - d;
     sum += lane_of(up, 63);
-#pragma unroll
-    for (int k = 0; k < kPieceLengths; ++k) {
-      const uint32_t l = lane_of(length, k);
-      const bool yes = is_cut(d, l);
-      const uint32_t all = (uint32_t)__popcll(__ballot(yes));
-      cut += mine == k ? all : 0;
-      parts[k] += yes ? ceil_quotient(d, l) : 0;
-    }
-  }
-  uint32_t pieces = 0;
-#pragma unroll
-  for (int k = 0; k < kPieceLengths; ++k) {
-    const uint32_t all = lane_of(wave_sums(parts[k]), 63);
-    pieces = mine == k ? all : pieces;
   }
   __syncthreads();   // (all lanes' words are there, and tile_start has been read by every wave)
+  // Eight lanes to each length, every eighth group for each of them.
+  static_assert(kPieceLengths == 8, "");
+  const int k = lane / 8, n = piece_count<BM * BN>(k);
+  const uint32_t length = (deepest + n - 1) / n;
+  uint32_t cut = 0, pieces = 0;
+#pragma unroll 1
+  for (int q = lane % 8;; q += 8) {
+    const uint32_t d = q < E ? depth[q] : 0;
+    const bool yes = is_cut(d, length);
+    if (__ballot(yes) == 0) break;   // (nor any of the groups behind these)
+    cut += yes ? 1 : 0;
+    pieces += yes ? ceil_quotient(d, length) : 0;
+  }
+#pragma unroll
+  for (int d = 1; d < 8; d *= 2) cut += (uint32_t)__shfl_xor((int)cut, d), pieces += (uint32_t)__shfl_xor((int)pieces, d);
   const GroupDepths depths{depth, upto, (uint32_t)E, sum};
   const PieceLaunch launch{tiles, per_group, grid, grid / WGS_PER_CU, p.ws_slots};
   const float share = ((float)sum * per_group + PieceCosts<BM * BN>::TILE * tiles) / grid;
   const float end = pieces_end<BM * BN>(depths, launch, n, (int)length, (int)cut, (int)pieces, share);
-  float best = kPiecesPay * uncut_end<BM * BN>(depths, launch, plan->by_depth && plan->main_tiles == 0 ? plan->pieces : 1, share);
-  int chosen = -1;
-#pragma unroll
-  for (int k = 0; k < kPieceLengths; ++k) {
-    const float at_k = __builtin_bit_cast(float, lane_of(__builtin_bit_cast(uint32_t, end), k));
-    chosen = at_k < best ? k : chosen;
-    best = fminf(best, at_k);
-  }
-  chosen = uniform(chosen);
+  const float uncut = uncut_end<BM * BN>(depths, launch, plan->by_depth && plan->main_tiles == 0 ? plan->pieces : 1, share);
+  // the least, the first of equals: by its bits, the lowest three of which are its number
+  const uint32_t mine = (__builtin_bit_cast(uint32_t, end) & ~7u) | (uint32_t)k;
+  const uint32_t least = ~lane_of(wave_scan(~mine, [](uint32_t a, uint32_t b) { return a > b ? a : b; }), 63);
+  const int chosen = uniform(__builtin_bit_cast(float, least & ~7u) < kPiecesPay * uncut ? (int)(least & 7u) * 8 : -1);
   if (chosen >= 0) {
     const int l = (int)lane_of(length, chosen), groups = (int)lane_of(cut, chosen), all = (int)lane_of(pieces, chosen);
     uint32_t start = 0;
@@ -2187,7 +2180,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       constexpr int PENDING = Loads::before(READY);
       // (in the weight-gradient layout the condition is one of the first slice's, which the compiler then takes out of the
       // loop, as long as there is no loop in this one: with that wait in the loop it moves accumulators in and out of it, 332
-      // moves a slice)
+      // moves a slice.)
       if (LATE_LOADS || (LAYOUT == kTN && kt > 0) || __builtin_expect(uniform(stored) == 0, 1)) {
         wait_vmcnt<PENDING>();
       } else {
