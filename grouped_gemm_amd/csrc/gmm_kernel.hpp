@@ -2131,6 +2131,11 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
         } else {
           f32x4& sum = acc[2 * i + hi][2 * j + hj];
           sum = mfma_16x16x32<DT>(fb[set + hj][j], fa[set + hi][i], sum);
+          // (the first slice of a weight gradient's tile is a copy of the loop's, see the wait below: said to be in accumulation registers
+          // from there on, half as many of its sums are moved to others and back, each behind a matrix result.  One slice, 128
+          // groups x 30 rows, 2048 x 1408: 132.3 / 129.5 us; two, 64 x 64, 4096 x 4096: 389.7 / 385.2; four or more: the same.  As
+          // the second of a pair, where there are 12 moves either way, and with the epilogues that accumulate it gains nothing.)
+          if constexpr (LAYOUT == kTN && BM == 256 && EPI == kEpiStore && !PART::SECOND && m < S / 2) asm volatile("" : "+a"(sum));
         }
         if constexpr (m < READ_END) {
           constexpr int U = 2 * (ML + NB), u0 = U * m / READ_END, u1 = U * (m + 1) / READ_END;
@@ -2180,7 +2185,9 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& p, const HostSizes& h
       constexpr int PENDING = Loads::before(READY);
       // (in the weight-gradient layout the condition is one of the first slice's, which the compiler then takes out of the
       // loop, as long as there is no loop in this one: with that wait in the loop it moves accumulators in and out of it, 332
-      // moves a slice.)
+      // moves a slice.  Without a copy and without a move, the waits chosen among in assembly and every accumulator's zeros its
+      // own, the loop is slower for the branches in each slice: 8 x 4096 rows, 4096 x 14336: 2632 / 2702 us; 256 x 256, 2048 x 7168:
+      // 2561 / 2600)
       if (LATE_LOADS || (LAYOUT == kTN && kt > 0) || __builtin_expect(uniform(stored) == 0, 1)) {
         wait_vmcnt<PENDING>();
       } else {

@@ -771,6 +771,19 @@ def test_loads_to_lds_are_late_enough(tmp_path):
     assert total > 1000
 
 
+def test_first_slice_of_weight_gradients_moves_few_sums(tmp_path):
+    """Weight gradients on full tiles: sums that the slices move from their accumulation registers to others, and back."""
+    objdump, objects = _code_objects(tmp_path)
+    moves = {}
+    for f in objects:
+        text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(f)], check=True, capture_output=True, text=True).stdout
+        for name, body in re.findall(r"^[0-9a-f]+ <(_ZN2gg10gmm_kernelILi[01]ELi2ELi256ELi256E(?:Li\d+E){4}Li0E\w+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)",
+                                     text, flags=re.S | re.M):
+            blocks = [re.findall(r"^\s+(\w+)", b, flags=re.M) for b in re.split(r"\bs_c?branch\w*", body)]
+            moves[name] = sum(b.count("v_accvgpr_read_b32") for b in blocks if sum("mfma" in op for op in b) >= 32)
+    assert len(moves) == 2 and max(moves.values()) <= 12, moves
+
+
 def test_reading_accumulation_keeps_its_registers(tmp_path):
     """Full tiles that add to fp32 by reading, adding and writing (epilogue 1 of the template's arguments) have no scratch memory: with
     some, each block row of c began with a reload that waited for all stores of the one before."""
