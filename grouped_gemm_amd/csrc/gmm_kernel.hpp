@@ -420,8 +420,8 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(bf16x8 x, bf16x8 y, f32x16 acc) 
 // One 16x16x32 matrix instruction on fragments of 8 two-byte elements per lane: what the streaming kernel
 // multiplies two-byte elements with.  Per operation it moves half the accumulators of the 32x32x16 one in and out
 // of the register file, and power is what bounds these products: on operands like real activations, in
-// registers and nothing else running, 16x16x32 sustains 1970-2010 TFLOP/s (bf16), 32x32x16 1730-1800; on zeros,
-// at full clock, 2240 and 2275.
+// registers and nothing else running, 16x16x32 sustains 1930-1950 TFLOP/s (bf16; on zeros, at full clock, 2331-2335), 32x32x16
+// 1635-1740 (the rate probe of the benchmark, each at its time).
 template <int DT>
 __device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 x, bf16x8 y, f32x4 acc) {
   if constexpr (DT == kBF16) {
