@@ -34,10 +34,10 @@ PEAK_HBM_GBPS = 8000.0
 # the hash below (kernel_sources_sha16), and is reported only while the sources still have that
 # hash; the summary under profiles/ holds the figures, the commands and the commit.
 _TRAFFIC_KERNEL_SOURCES = ("gmm_kernel.hpp", "gmm_api.hip", "gmm_variants.hpp", "gmm_variants.def", "gmm_variant.hip")
-_TRAFFIC_KERNEL_SHA16 = "c86646acb4fc393d"
+_TRAFFIC_KERNEL_SHA16 = "2c67e678e1632f30"
 _TRAFFIC_SOURCE = ("profiles/gmm_kernel_mixtral_w1_hbm_traffic.md and profiles/gmm_kernel_configs_3_4_5_stats_and_traffic.md "
                    "(rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, kernel sources sha16 " + _TRAFFIC_KERNEL_SHA16 +
-                   ", commit 3664088; profiled once, not in this run)")
+                   ", commit 8e6560a; profiled once, not in this run)")
 
 
 def kernel_sources_sha16():
@@ -55,10 +55,10 @@ def _traffic(fetch_kib, write_kib):
 
 
 MEASURED_TRAFFIC = {
-    2: {"fwd": _traffic(4463456, 917582), "agrad": _traffic(3321526, 273642), "bgrad": _traffic(2856366, 917560)},
-    3: {"fwd": _traffic(445579, 135178)},
-    4: {"bgrad": _traffic(2848553, 917566)},
-    5: {"fwd": _traffic(4310785, 262210), "agrad": _traffic(5053021, 917902), "bgrad": _traffic(1851763, 7345855)},
+    2: {"fwd": _traffic(4355407, 917525), "agrad": _traffic(3329409, 273445), "bgrad": _traffic(2869692, 917519)},
+    3: {"fwd": _traffic(444303, 135186)},
+    4: {"bgrad": _traffic(2849146, 917520)},
+    5: {"fwd": _traffic(4261433, 262199), "agrad": _traffic(4924570, 917932), "bgrad": _traffic(1851758, 7346140)},
 }
 
 

@@ -420,7 +420,7 @@ __device__ __forceinline__ f32x16 mfma_32x32x16(bf16x8 x, bf16x8 y, f32x16 acc) 
 // One 16x16x32 matrix instruction on fragments of 8 two-byte elements per lane: what the streaming kernel
 // multiplies two-byte elements with.  Per operation it moves half the accumulators of the 32x32x16 one in and out
 // of the register file, and power is what bounds these products: on operands like real activations, in
-// registers and nothing else running, 16x16x32 sustains 1930-1950 TFLOP/s (bf16; on zeros, at full clock, 2331-2335), 32x32x16
+// registers and nothing else running, 16x16x32 sustains 1930-1970 TFLOP/s (bf16; on zeros, at full clock, 2331-2352), 32x32x16
 // 1635-1740 (the rate probe of the benchmark, each at its time).
 template <int DT>
 __device__ __forceinline__ f32x4 mfma_16x16x32(bf16x8 x, bf16x8 y, f32x4 acc) {
@@ -2027,7 +2027,7 @@ __device__ __forceinline__ void gmm_tiles(const GmmParams& given, const HostSize
   // padded results copied back (120 of them the copies), 760 so.
   constexpr bool ANY_ROWS = EPI == kEpiStore && !INDEXED && !RAGGED_DEPTH && !F8;
   // ... or that are no whole groups of 4 columns, which the fix-up of depth pieces stores (whole tiles / pieces, us: weight
-  // gradients of 21 Zipf (1.2) groups, 51204 rows, 128 x 558: 125 / 38, 64, 49152 rows, 2046 x 1406: 492 / 364; 16 groups, 600 rows,
+  // gradients of 21 Zipf (1.2) groups, 51204 rows, 128 x 558: 125 / 38; 64, 49152 rows, 2046 x 1406: 492 / 364; 16 groups, 600 rows,
   // 6144 -> 518: 46.8 / 33.8).
   constexpr bool FIX_ANY_ROWS = EPI == kEpiStore && !INDEXED && !F8;
   auto store_any = [&](const TileInfo& tile, uint32_t row_off, int col, int most, u32x4 v) {
