@@ -1659,12 +1659,16 @@ template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, i
           int EPI, bool INDEXED, bool RAGGED_DEPTH, typename PART>
 __device__ __forceinline__ void gmm_tiles(const GmmParams& given, const HostSizes& hs, char* smem, const int w, const int G, const PART& part) {
   GmmParams p = given;
-  // Eight words that the kernel arguments are read in together, told apart: the first of these pairs otherwise spills them as
-  // one and reads all eight back wherever it wants one (1950 reads of spilled words, with this 1060; 16 x 1024 rows, forward and gradients of
-  // a permuted layer, 1024 -> 2048: 629 / 625 us).  In the other pairs they are spilled one by one as it is.
-  if constexpr (PART::FIRST && LAYOUT == kNT && BM == 256)
-    asm volatile("" : "+s"(p.first_group), "+s"(p.num_groups), "+s"(p.hidden_in), "+s"(p.hidden_out), "+s"(p.group_m), "+s"(p.flags),
-                 "+s"(p.ws_slots), "+s"(p.b_cols));
+  // Words that the kernel arguments are read in together, told apart: the first of these pairs otherwise spills eight of them as one and
+  // reads all eight back wherever it wants one (1950 reads of spilled words, with this 710).  Which of them is what the
+  // allocator takes well; in the other pairs they are spilled one by one as it is.
+  if constexpr (PART::FIRST && LAYOUT == kNT && BM == 256) {
+    if constexpr (DT == kBF16) {
+      asm volatile("" : "+s"(p.hidden_in), "+s"(p.hidden_out), "+s"(p.ws_slots), "+s"(p.flags), "+s"(p.lda), "+s"(p.ldb));
+    } else {
+      asm volatile("" : "+s"(p.hidden_in), "+s"(p.hidden_out), "+s"(p.ws_slots), "+s"(p.flags));
+    }
+  }
   using Cfg = GmmConfig<LAYOUT, BM, BN, BK, STAGES, WAVES_M, WAVES_N>;
   constexpr int NT = Cfg::NT, MB = Cfg::MB, NB = Cfg::NB, KS = BK / 16;
   constexpr bool ACC_F32 = EPI == kEpiAccF32 || EPI == kEpiAccF32Atomic, KEEP = EPI == kEpiSwiGLUKeep, GATE_UP = EPI == kEpiSwiGLU || KEEP;
