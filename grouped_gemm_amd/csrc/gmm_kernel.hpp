@@ -193,7 +193,8 @@ __host__ __device__ constexpr int piece_count(int k) {
 __host__ __device__ constexpr bool is_cut(uint32_t depth, uint32_t length) { return depth > length + length / 2; }
 // The one with which the launch is expected to end soonest: the longest of the first round (a piece and its fix-up, or the deepest whole
 // tile), and an even share of what is left.  More pieces than compute units: two of them share a unit and take twice as long (7
-// groups of 6377 rows, 12 small tiles each: 3 pieces 31.0 us, 4 of them 36.0; 2 of 20000, 22 each: 5 pieces 44.5, 6 of them 48.3).
+// groups of 6377 rows, 12 small tiles each: 3 pieces 31.0 us, 4 of them 36.0; 2 of 20000, 22 each: 5 pieces 44.5, 6 of them 48.3).  Where
+// there are more tiles than that, whole ones share units too, and nothing sets the pieces apart.
 // `depths` is the groups' depths, deepest first: at(q) that of position q (0 behind the last), first(n) the sum of n.
 struct PieceLaunch {
   int tiles, per_group, grid, units, slots;
@@ -206,7 +207,8 @@ __host__ __device__ inline float pieces_end(const DEPTHS& depths, const PieceLau
   const bool fits = (uint64_t)(uint32_t)pieces * of.per_group <= (uint64_t)most && (uint64_t)(uint32_t)cut * of.per_group <= kWsCounterBytes / 4;
   if (n > 1 && (length < Costs::SHORTEST || cut == 0 || !fits)) return 1e30f;
   const float whole = (float)depths.at(cut) + Costs::TILE;
-  const float piece = cut > 0 ? ((int)front > of.units ? 2.0f : 1.0f) * length + Costs::FIX + Costs::FIX_PIECE * n : 0.0f;
+  const bool shared = (int)front > of.units && of.tiles <= of.units;
+  const float piece = cut > 0 ? (shared ? 2.0f : 1.0f) * length + Costs::FIX + Costs::FIX_PIECE * n : 0.0f;
   float end = piece > whole ? piece : whole;
   if (of.tiles - cut * of.per_group + (int)front > of.grid) {
     // what follows: the share of all, less that of the first round (the pieces and whole tiles for the workgroups left)

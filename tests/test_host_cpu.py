@@ -553,6 +553,7 @@ def test_pieces_of_one_length():
     assert _pieces(lib, [17150, 7470, 4590, 3250, 2490, 2000, 1660, 1390], 8, 512, 256, 1024, small)[0] == [12, 6, 4, 3, 2, 0, 0, 0]
     assert _pieces(lib, [6000] * 6, 8, 512, 256, 1024, small, 4)[0] == [0] * 6              # the last round's cut is as good (25.7; 5: 26.7)
     assert _pieces(lib, [4000] * 4, 16, 512, 256, 1024, small, 4)[0] == [0] * 4
+    assert _pieces(lib, [4215, 1834, 1129, 799, 611, 491, 408, 347, 302, 266], 132, 512, 256, 1024, small)[0][:2] == [2, 0]   # whole ones share too
     zipf = [5696, 2432, 1600, 1088, 832, 704, 640, 512] + [300] * 48
     assert _pieces(lib, zipf, 18, 256, 256, 256, full)[0][:3] == [4, 2, 0]                   # (91.5; 5 and 3: 93.5)
     assert _pieces(lib, [3000] * 4, 64, 512, 256, 0, small)[0] == [0] * 4                    # nowhere to put partial tiles
