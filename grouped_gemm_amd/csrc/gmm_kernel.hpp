@@ -1662,8 +1662,8 @@ template <int DT, int LAYOUT, int BM, int BN, int BK, int STAGES, int WAVES_M, i
 __device__ __forceinline__ void gmm_tiles(const GmmParams& given, const HostSizes& hs, char* smem, const int w, const int G, const PART& part) {
   GmmParams p = given;
   // Words that the kernel arguments are read in together, told apart: the first of these pairs otherwise spills eight of them as one and
-  // reads all eight back wherever it wants one (1950 reads of spilled words, with this 710).  Which of them is what the
-  // allocator takes well; in the other pairs they are spilled one by one as it is.
+  // reads all eight back wherever it wants one (1950 reads of spilled words, with this 710 to 1560, by what else the
+  // kernel holds); in the other pairs they are spilled one by one as it is.
   if constexpr (PART::FIRST && LAYOUT == kNT && BM == 256) {
     if constexpr (DT == kBF16) {
       asm volatile("" : "+s"(p.hidden_in), "+s"(p.hidden_out), "+s"(p.ws_slots), "+s"(p.flags), "+s"(p.lda), "+s"(p.ldb));
